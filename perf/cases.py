@@ -1,0 +1,552 @@
+"""Timed workloads of the verify path, each through a public entry point.
+
+A case is one call a user's program makes: a 2-bit product, an MoE block, an attention block, the
+head, sampled acceptance, or a whole engine pass (prefill, greedy verify).  Sizes are those of the
+synthetic benchmark model (hidden 2048, 64 experts top-8 of 1024, group 64, window 1024, fp16 head
+of 151936 ids) and of the Maple checkpoint defaults (256 experts of 512, group 128, window 512
+with every fourth layer full attention, 4-bit head), at the row counts the path sees: one row
+(plain decode), 9 (a K = 8 chain), 17 (a 16-node tree), 64 (a prefill chunk), and between.
+"""
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import torch
+
+from momij_amd import _lib, synth
+from momij_amd.engine import MapleLikeConfig, VerifyEngine, random_model
+from momij_amd.ops import Context
+
+VOCAB = 151936
+H, NQ, NKV, D = 2048, 16, 4, 128
+EPS, ROPE_BASE = 1e-6, 1e6
+
+_context = None
+
+
+def context() -> Context:
+    """One context per program; the program's own torch work runs on the context's stream, so
+    inputs and outputs need no events."""
+    global _context
+    if _context is None:
+        _context = Context(0)
+        torch.cuda.set_stream(_context.stream)
+    return _context
+
+
+# ------------------------------------------------------------------------------------ cases
+def listed():
+    return [
+        # the smallest call: one activation row through one 2-bit matrix
+        dict(name="gemv", kind="gather", M=1, ktop=1, E=1, K=2048, N=5632, gs=64, add=False,
+             per=False),
+        # the expert product as the engine's op-level callers issue it: 9 rows routed top-8
+        dict(name="gather_routed", kind="gather", M=9, ktop=8, E=64, K=2048, N=2048, gs=64,
+             add=False, per=False),
+        # the MoE block of one decode step, and of a 64-row prefill chunk
+        dict(name="moe_decode", kind="moe", M=1, E=64, I=1024, gs=64, alpha=False),
+        dict(name="moe_prefill", kind="moe", M=64, E=64, I=1024, gs=64, alpha=False),
+        # Maple's experts (256 of 512, group 128, one alpha a row) under a 16-node tree
+        dict(name="moe_maple_tree", kind="moe", M=17, E=256, I=512, gs=128, alpha=True),
+        # attention of a K = 8 chain in the sliding window's ring; of a prefill chunk deep in a
+        # full-attention (NoPE) layer
+        dict(name="attn_chain", kind="attn", M=9, L=2048, window=1024, rope=64, gs=64, tree=False),
+        dict(name="attn_prefill_full", kind="attn", M=64, L=6000, window=0, rope=0, gs=128,
+             tree=False),
+        # the head of a sampled verify (logits kept, log-sum-exp); the checkpoint's 4-bit head
+        # over a large draft tree
+        dict(name="head_fp16", kind="head", bits=16, M=9, K=2048, V=VOCAB, lse=True, logits=True,
+             banned=0),
+        dict(name="head_q4_tree", kind="head", bits=4, M=33, K=2048, V=VOCAB, lse=False,
+             logits=True, banned=16),
+        # sampled acceptance of a chain: penalties over the prompt's tokens, then the bonus
+        # token from the nucleus
+        dict(name="accept_top_p", kind="accept", rows=9, V=VOCAB, top_p=0.9, rep=1.1, pres=0.1,
+             freq=0.1, n_hist=1500, uniform_q=True),
+        # whole calls: a greedy verify pass of the K = 8 chain in a four-layer stack of the
+        # benchmark model; a Maple prompt through one period of its layer mix, prompt logits kept
+        dict(name="engine_verify", kind="verify", layers=4, M=9, L=1100, tree=False),
+        dict(name="engine_prefill", kind="prefill", layers=4, n=200),
+    ]
+
+
+def _log(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(["gather", "gather", "moe", "moe", "moe", "attn", "attn", "attn", "head",
+                       "head", "accept", "verify", "prefill"])
+    if kind == "gather":
+        K, gs = rng.choice([512, 1024, 2048, 2048, 4096]), rng.choice([64, 128])
+        N = 16 * _log(rng, 4, 352)
+        if rng.random() < 0.4:  # a dense projection
+            return dict(kind=kind, M=_log(rng, 1, 64), ktop=1, E=1, K=K, N=N, gs=gs,
+                        add=rng.random() < 0.5, per=False)
+        E = rng.choice([8, 16, 64, 128])
+        N = min(N, 16 * ((1 << 29) // (E * K * 16)))
+        return dict(kind=kind, M=_log(rng, 1, 64), ktop=rng.choice([1, 2, 4, 8]), E=E, K=K, N=N,
+                    gs=gs, add=False, per=rng.random() < 0.3)
+    if kind == "moe":
+        E, I, gs = rng.choice([(64, 1024, 64), (64, 1024, 64), (256, 512, 128), (128, 1024, 64),
+                               (40, 1024, 64), (16, 1024, 128), (64, 512, 64)])
+        return dict(kind=kind, M=_log(rng, 1, 64), E=E, I=I, gs=gs, alpha=rng.random() < 0.3)
+    if kind == "attn":
+        window, rope = rng.choice([(1024, 64), (512, 64), (0, 0), (1024, 128), (0, 32)])
+        return dict(kind=kind, M=_log(rng, 1, 64), L=_log(rng, 8, 6000), window=window, rope=rope,
+                    gs=rng.choice([64, 128]), tree=rng.random() < 0.4)
+    if kind == "head":
+        bits, M = rng.choice([16, 4]), _log(rng, 1, 64)
+        return dict(kind=kind, bits=bits, M=M, K=rng.choice([1024, 2048, 2048]),
+                    V=_log(rng, 8000, VOCAB), lse=rng.random() < 0.5, logits=rng.random() < 0.5,
+                    banned=rng.choice([0, 0, 16]))
+    if kind == "accept":
+        pen = rng.random() < 0.5
+        return dict(kind=kind, rows=_log(rng, 1, 33), V=_log(rng, 8000, VOCAB),
+                    top_p=rng.choice([1.0, 0.9, 0.6]), rep=1.1 if pen else 1.0,
+                    pres=0.1 if pen else 0.0, freq=0.1 if pen else 0.0,
+                    n_hist=_log(rng, 16, 4000) if pen else 0, uniform_q=rng.random() < 0.7)
+    if kind == "verify":
+        return dict(kind=kind, layers=rng.randint(1, 4), M=_log(rng, 1, 33), L=_log(rng, 40, 1100),
+                    tree=rng.random() < 0.4)
+    return dict(kind="prefill", layers=rng.randint(1, 4), n=_log(rng, 16, 200))
+
+
+# ----------------------------------------------------------------------------------- inputs
+class _Rand:
+    """Seeded generators of one state: the device's and the host's."""
+
+    def __init__(self, seed):
+        self.gen = torch.Generator(device="cuda")
+        self.gen.manual_seed(seed)
+        self.np = np.random.default_rng(seed)
+
+    def normal(self, shape, std=1.0):
+        return synth.torch_normal(self.gen, shape, std)
+
+    def qweight(self, lead, N, K, gs):
+        return synth.torch_qweight(self.gen, lead, N, K, gs)
+
+    def norm_w(self, n):
+        return (1.0 + 0.1 * torch.randn(n, generator=self.gen, device="cuda")).half()
+
+    def ints(self, hi, n):
+        return torch.randint(0, hi, (n,), generator=self.gen, device="cuda", dtype=torch.int32)
+
+
+def _alpha_experts(r, E, N, K, gs):
+    """One alpha a row: scale alpha and bias -alpha in every group (the checkpoint's row_alpha)."""
+    w, _, _ = r.qweight((E,), N, K, gs)
+    al = (torch.rand((E, N), generator=r.gen, device="cuda") * 0.015 + 0.005).half()
+    s = al[..., None].expand(E, N, K // gs).contiguous()
+    return w, s, -s, al
+
+
+def _moe_weights(r, E, I, gs, alpha, eps=EPS):
+    mw = dict(norm_w=r.norm_w(H), router_w=r.normal((E, H), 0.02), E=E, top_k=8, H=H, I=I, gs=gs,
+              eps=eps)
+    for name, N, K in (("up_gate", 2 * I, H), ("down", H, I)):
+        if alpha:
+            w, s, b, mw[name + "_alpha"] = _alpha_experts(r, E, N, K, gs)
+        else:
+            w, s, b = r.qweight((E,), N, K, gs)
+        mw[name + "_w"], mw[name + "_s"], mw[name + "_b"] = w, s, b
+    return mw
+
+
+def _attn_weights(r, gs):
+    qw, qs, qb = r.qweight((), (NQ + 2 * NKV) * D, H, gs)
+    ow, os_, ob = r.qweight((), H, NQ * D, gs)
+    return dict(norm_w=r.norm_w(H), qkv_w=qw, qkv_s=qs, qkv_b=qb, q_norm_w=r.norm_w(D),
+                k_norm_w=r.norm_w(D), o_w=ow, o_s=os_, o_b=ob)
+
+
+def _head4(r, V, K):
+    w = torch.randint(-(2**31), 2**31 - 1, (V, K // 8), generator=r.gen, device="cuda",
+                      dtype=torch.int64).to(torch.int32)
+    s = (torch.rand((V, K // 64), generator=r.gen, device="cuda") * 0.003 + 0.001).half()
+    return w, s, (-7.5 * s.float()).half()
+
+
+def _parents(r, M, tree):
+    """A chain, or a tree of which every node hangs off one of the six rows before it."""
+    if not tree:
+        return None
+    return [-1] + [int(r.np.integers(max(0, i - 6), i)) for i in range(1, M)]
+
+
+def _inputs(case, seed):
+    """Everything the call reads, from the seed alone (also what exact() starts from)."""
+    r = _Rand(seed)
+    kind = case["kind"]
+    if kind == "gather":
+        M, k, E, K, N = (case[x] for x in ("M", "ktop", "E", "K", "N"))
+        w, s, b = r.qweight((E,), N, K, case["gs"])
+        inds = torch.rand((M, E), generator=r.gen, device="cuda").topk(k, dim=1).indices
+        return dict(w=w, s=s, b=b, x=r.normal((M * k if case["per"] else M, K)),
+                    inds=inds.to(torch.int32).contiguous(), y0=r.normal((M * k, N)))
+    if kind == "moe":
+        return dict(mw=_moe_weights(r, case["E"], case["I"], case["gs"], case["alpha"]),
+                    x=r.normal((case["M"], H)))
+    if kind == "attn":
+        M, L, win = case["M"], case["L"], case["window"]
+        C = win + 64 if win else (L + M + 63) // 64 * 64
+        return dict(cfg=dict(H=H, nQ=NQ, nKV=NKV, D=D, rope_dim=case["rope"], rope_base=ROPE_BASE,
+                             eps=EPS, window=win, C=C, gs=case["gs"]),
+                    aw=_attn_weights(r, case["gs"]), h0=r.normal((M, H)),
+                    kc=r.normal((NKV, C, D)), vc=r.normal((NKV, C, D)),
+                    parents=_parents(r, M, case["tree"]))
+    if kind == "head":
+        M, K, V = case["M"], case["K"], case["V"]
+        d = dict(x=r.normal((M, K)), banned=r.ints(V, case["banned"]) if case["banned"] else None)
+        if case["bits"] == 16:
+            d["w"] = r.normal((V, K), 0.02)
+        else:
+            d["w"], d["s"], d["b"] = _head4(r, V, K)
+        return d
+    if kind == "accept":
+        rows, V = case["rows"], case["V"]
+        logits = torch.randn((rows, V), generator=r.gen, device="cuda") * 2.5
+        draft = r.ints(V, rows)
+        # the target likes the drafted tokens: the usual case of a useful drafter
+        logits[torch.arange(rows, device="cuda"), draft.long()] += 16.0
+        hist = None
+        if case["n_hist"]:
+            tok = np.sort(r.np.choice(V, case["n_hist"], replace=False)).astype(np.int32)
+            hist = (tok, r.np.integers(1, 4, case["n_hist"]).astype(np.int32))
+        return dict(logits=logits.contiguous(), draft=draft[: rows - 1].contiguous(), hist=hist,
+                    counter=int(r.np.integers(1 << 30)))
+    if kind == "verify":
+        cfg = MapleLikeConfig(n_layers=case["layers"])
+        return dict(cfg=cfg, weights=random_model(cfg, seed=seed), scales=(None, None),
+                    prompt=r.np.integers(0, VOCAB, case["L"]).tolist(),
+                    draft=r.np.integers(0, VOCAB, case["M"] - 1).tolist(),
+                    parents=_parents(r, case["M"], case["tree"]))
+    n = case["n"]
+    wins, ropes = MapleLikeConfig.maple_layer_mix(case["layers"], 512, 64)
+    cfg = MapleLikeConfig(n_layers=case["layers"], E=256, I=512, gs=128, window=512,
+                          kv_capacity=512 + 64, layer_window=wins, layer_rope_dim=ropes,
+                          head_bits=4)
+    layers = [dict(attn=_attn_weights(r, 128), moe=_moe_weights(r, 256, 512, 128, True))
+              for _ in range(case["layers"])]
+    w4, s4, b4 = _head4(r, VOCAB, H)
+    return dict(cfg=cfg, weights=(layers, r.normal((VOCAB, H)), r.norm_w(H), w4), scales=(s4, b4),
+                prompt=r.np.integers(0, VOCAB, n).tolist())
+
+
+class _DeviceArray:
+    """A device buffer of the engine as torch sees it."""
+
+    def __init__(self, p, shape):
+        self.__cuda_array_interface__ = dict(data=(p, False), shape=shape, typestr="<f2", version=2)
+
+
+def _kv_views(eng, cfg):
+    shape = (cfg.n_kv_heads, cfg.kv_capacity, cfg.head_dim)
+    return [tuple(torch.as_tensor(_DeviceArray(p, shape), device="cuda") for p in eng.kv(l))
+            for l in range(cfg.n_layers)]
+
+
+def prepare(case, seed):
+    ctx = context()
+    st = dict(case=case, ctx=ctx, **_inputs(case, seed))
+    kind = case["kind"]
+
+    def out(shape, dtype=torch.float32):
+        return torch.zeros(shape, dtype=dtype, device="cuda")
+
+    if kind == "gather":
+        st["y"] = torch.empty_like(st["y0"])
+    elif kind == "moe":
+        st.update(y=torch.empty_like(st["x"]), inds=out((case["M"], 8), torch.int32),
+                  scores=out((case["M"], 8)))
+    elif kind == "attn":
+        st["h"] = torch.empty_like(st["h0"])
+    elif kind == "head":
+        M = case["M"]
+        st.update(argmax=out(M, torch.int32), max=out(M), lse=out(M) if case["lse"] else None,
+                  logits=out((M, case["V"])) if case["logits"] else None)
+    elif kind == "accept":
+        st["out"] = out(2, torch.int32)
+    else:
+        cfg = st["cfg"]
+        eng = VerifyEngine(ctx, cfg, *st["weights"], *st["scales"])
+        st["eng"], st["kv"] = eng, _kv_views(eng, cfg)
+        if kind == "prefill":
+            st["logits"] = out((_lib.MJ_MAX_ROWS, cfg.vocab))
+            eng.set_capture(logits=st["logits"])
+        else:
+            # a useful drafter: the first half of the draft follows the target
+            y = eng.prefill(st["prompt"])
+            st["y"], st["L"], t = y, eng.offset, y
+            par = st["parents"] or list(range(-1, case["M"] - 1))
+            row = 0
+            for _ in range((case["M"] - 1) // 2):
+                t = eng.step_chain_feeds([t])[0]
+                kids = [c for c in range(row + 1, case["M"]) if par[c] == row]
+                if not kids:
+                    break
+                row = kids[0]
+                st["draft"][row - 1] = t
+            eng.rewind(st["L"])
+    return st
+
+
+# -------------------------------------------------------------------------------- one pass
+def run(st):
+    case, ctx = st["case"], st["ctx"]
+    kind = case["kind"]
+    if kind == "gather":
+        if case["add"]:  # the residual the product is added to is new on every call
+            st["y"].copy_(st["y0"])
+        ctx.gather_qmm2(st["x"], st["w"], st["s"], st["b"], st["inds"], st["y"], case["M"],
+                        case["ktop"], case["K"], case["N"], case["gs"],
+                        lhs_per_expert=case["per"],
+                        epilogue=_lib.MJ_EPI_ADD if case["add"] else _lib.MJ_EPI_STORE)
+        return st["y"]
+    if kind == "moe":
+        ctx.moe_block(st["mw"], st["x"], st["y"], case["M"],
+                      _lib.MJ_MOE_PRENORM | _lib.MJ_MOE_RESIDUAL, st["inds"], st["scores"])
+        return dict(y=st["y"], inds=st["inds"], scores=st["scores"])
+    if kind == "attn":
+        st["h"].copy_(st["h0"])  # the block works in place on the residual stream
+        ctx.attn_block(st["cfg"], st["aw"], st["h"], st["kc"], st["vc"], case["L"], st["parents"],
+                       case["M"])
+        return dict(h=st["h"], k=st["kc"], v=st["vc"])
+    if kind == "head":
+        tail = dict(out_max=st["max"], out_logits=st["logits"], banned=st["banned"],
+                    n_banned=case["banned"], temperature=0.7, out_lse=st["lse"])
+        if case["bits"] == 16:
+            ctx.lm_head_verify(st["x"], st["w"], case["M"], case["K"], case["V"], st["argmax"],
+                               **tail)
+        else:
+            ctx.lm_head_verify_q4(st["x"], st["w"], st["s"], st["b"], case["M"], case["K"],
+                                  case["V"], st["argmax"], **tail)
+        return dict(argmax=st["argmax"], max=st["max"], lse=st["lse"], logits=st["logits"])
+    if kind == "accept":
+        ctx.accept_sampled_ex(st["logits"], case["rows"], case["V"], st["draft"],
+                              _lib.MJ_Q_UNIFORM if case["uniform_q"] else _lib.MJ_Q_POINT, 7,
+                              st["counter"], st["out"], 0.7, top_p=case["top_p"], rep=case["rep"],
+                              pres=case["pres"], freq=case["freq"], hist=st["hist"])
+        return st["out"]
+    eng = st["eng"]
+    if kind == "prefill":
+        eng.rewind(0)
+        nxt = eng.prefill(st["prompt"])
+        n = case["n"]
+        return dict(next=nxt, logits=st["logits"][: (n - 1) % _lib.MJ_MAX_ROWS + 1],
+                    kv=[(k[:, :n], v[:, :n]) for k, v in st["kv"]])
+    # a production pass replays a graph, which the logits capture would switch off: what it leaves
+    # are the tokens and every layer's cache
+    eng.rewind(st["L"])
+    acc, toks = eng.verify_greedy(st["y"], st["draft"], st["parents"])
+    return dict(accepted=acc, tokens=toks, kv=st["kv"])
+
+
+# ------------------------------------------------------------------------- work, tolerance
+def _experts(E, k, M):
+    return E * (1.0 - (1.0 - k / E) ** M)
+
+
+def _qbytes(N, K, gs, alpha=False):
+    return N * (K / 4 + (2 if alpha else 4 * K / gs))
+
+
+def _moe_work(M, E, I, gs, alpha):
+    u = _experts(E, 8, M)
+    b = u * (_qbytes(2 * I, H, gs, alpha) + _qbytes(H, I, gs, alpha)) + E * H * 2 + M * H * 4
+    return b, 2.0 * M * (8 * 3 * H * I + E * H)
+
+
+def _attn_work(M, L, window, gs):
+    keys = min(L, window) if window else L
+    b = (_qbytes((NQ + 2 * NKV) * D, H, gs) + _qbytes(H, NQ * D, gs) + M * H * 4 +
+         2 * NKV * D * 2 * (keys + M))
+    f = 2.0 * M * H * D * (2 * NQ + 2 * NKV) + 4.0 * M * NQ * D * (keys + M / 2)
+    return b, f
+
+
+def _head_work(M, K, V, bits, logits):
+    w = V * K * 2 if bits == 16 else V * (K / 2 + K / 16)
+    return w + M * K * 2 + (M * V * 4 if logits else 0), 2.0 * M * K * V
+
+
+def work(case):
+    kind = case["kind"]
+    if kind == "gather":
+        M, k, K, N = case["M"], case["ktop"], case["K"], case["N"]
+        b = (_experts(case["E"], k, M) * _qbytes(N, K, case["gs"]) +
+             (M * k if case["per"] else M) * K * 2 + M * k * N * (4 if case["add"] else 2))
+        f = 2.0 * M * k * N * K
+    elif kind == "moe":
+        b, f = _moe_work(case["M"], case["E"], case["I"], case["gs"], case["alpha"])
+    elif kind == "attn":
+        b, f = _attn_work(case["M"], case["L"], case["window"], case["gs"])
+    elif kind == "head":
+        b, f = _head_work(case["M"], case["K"], case["V"], case["bits"], case["logits"])
+    elif kind == "accept":
+        b, f = case["rows"] * case["V"] * 4.0, case["rows"] * case["V"] * 10.0
+    else:
+        b = f = 0.0
+        verify = kind == "verify"
+        left, at = (case["M"], case["L"]) if verify else (case["n"], 0)
+        last = 0
+        while left > 0:
+            last = min(left, _lib.MJ_MAX_ROWS)
+            for l in range(case["layers"]):
+                win = 1024 if verify else (512 if (l + 1) % 4 else 0)
+                ab, af = _attn_work(last, at, win, 64 if verify else 128)
+                mb, mf = (_moe_work(last, 64, 1024, 64, False) if verify else
+                          _moe_work(last, 256, 512, 128, True))
+                b, f = b + ab + mb, f + af + mf
+            left, at = left - last, at + last
+        hb, hf = _head_work(last, H, VOCAB, 16 if verify else 4, not verify)
+        b, f = b + hb, f + hf
+    return {"bytes": b, "flops": f}
+
+
+def tolerance(case):
+    kind = case["kind"]
+    if kind == "accept":
+        return "exact"  # fixed-order sums by definition
+    # about four times the distance from exact() that the path shows
+    if kind == "head":
+        return {"rel": 2e-6, "max": 1e-4}  # fp32 sums of fp16 products
+    if kind == "gather":
+        return {"rel": 1e-3, "max": 2e-2}  # one fp16 rounding of the result
+    if kind in ("moe", "attn"):
+        return {"rel": 1e-3, "max": 3e-2, "differ": 0.01}  # fp16 between the block's stages
+    return {"rel": 1.6e-2, "max": 0.5, "differ": 0.01}  # rounding carried through four layers
+
+
+# -------------------------------------------------------------------- the same in 64 bits
+def _dequant(w, s, b, gs):
+    shifts = torch.arange(0, 32, 2, device=w.device, dtype=torch.int32)
+    q = ((w[..., None] >> shifts) & 3).reshape(*w.shape[:-1], -1).double()
+    rep = (lambda t: t.double().repeat_interleave(gs, dim=-1))
+    return rep(s) * q + rep(b)
+
+
+def _rms(x, w, eps=EPS):
+    return x / torch.sqrt(x.square().mean(-1, keepdim=True) + eps) * w.double()
+
+
+def _moe64(mw, x):
+    gs = mw["gs"]
+    xn = _rms(x, mw["norm_w"])
+    logits = xn @ mw["router_w"].double().T
+    top = logits.sort(dim=1, descending=True, stable=True)
+    inds = top.indices[:, :8]
+    g = torch.softmax(logits, 1).gather(1, inds)
+    scores = g / g.sum(1, keepdim=True)
+    y = x.clone()
+    for e in inds.unique().tolist():
+        row, slot = (inds == e).nonzero(as_tuple=True)
+        ug = xn[row] @ _dequant(mw["up_gate_w"][e], mw["up_gate_s"][e], mw["up_gate_b"][e], gs).T
+        up, gate = ug[:, : mw["I"]].clamp(-7, 7), ug[:, mw["I"]:].clamp(max=7)
+        act = gate * torch.sigmoid(gate) * up
+        dn = act @ _dequant(mw["down_w"][e], mw["down_s"][e], mw["down_b"][e], gs).T
+        y.index_add_(0, row, dn * scores[row, slot][:, None])
+    return y, inds.to(torch.int32), scores
+
+
+def _rope64(v, pos, rope):
+    if rope == 0:
+        return v
+    half = rope // 2
+    inv = ROPE_BASE ** (-torch.arange(half, device=v.device, dtype=torch.float64) / half)
+    th = pos.double()[:, None, None] * inv
+    a, b = v[..., :half], v[..., half:rope]
+    return torch.cat([a * th.cos() - b * th.sin(), b * th.cos() + a * th.sin(), v[..., rope:]], -1)
+
+
+def _attn64(cfg, aw, h, K, V, L, parents, M):
+    """h, K, V after the block; K, V [nKV][C][128] in 64 bits, updated in place."""
+    gs, win, C = cfg["gs"], cfg["window"], cfg["C"]
+    par = parents or list(range(-1, M - 1))
+    depth, anc = [0] * M, [[0]]
+    for r in range(1, M):
+        depth[r] = depth[par[r]] + 1
+        anc.append(anc[par[r]] + [r])
+    dev = h.device
+    pos = L + torch.tensor(depth, device=dev)
+    qkv = _rms(h, aw["norm_w"]) @ _dequant(aw["qkv_w"], aw["qkv_s"], aw["qkv_b"], gs).T
+    q, k, v = (t.reshape(M, -1, D) for t in qkv.split([NQ * D, NKV * D, NKV * D], 1))
+    q = _rope64(_rms(q, aw["q_norm_w"]), pos, cfg["rope_dim"])
+    k = _rope64(_rms(k, aw["k_norm_w"]), pos, cfg["rope_dim"])
+    lo = max(0, L - win + 1) if win else 0
+    old = torch.arange(lo, L, device=dev)
+    ok = torch.zeros((M, len(old) + M), dtype=torch.bool, device=dev)
+    ok[:, : len(old)] = old[None] > (pos[:, None] - win if win else -1)
+    for r in range(M):
+        ok[r, len(old) + torch.tensor(anc[r], device=dev)] = True
+    kk = torch.cat([K[:, old % C], k.transpose(0, 1)], 1).repeat_interleave(NQ // NKV, 0)
+    vv = torch.cat([V[:, old % C], v.transpose(0, 1)], 1).repeat_interleave(NQ // NKV, 0)
+    sc = torch.matmul(q.transpose(0, 1).contiguous(), kk.transpose(1, 2).contiguous()) * D ** -0.5
+    p = torch.softmax(sc.masked_fill(~ok[None], -math.inf), -1)
+    o = torch.matmul(p, vv.contiguous()).transpose(0, 1).reshape(M, NQ * D)
+    slots = (L + torch.arange(M, device=dev)) % C
+    K[:, slots], V[:, slots] = k.transpose(0, 1), v.transpose(0, 1)
+    return h + o @ _dequant(aw["o_w"], aw["o_s"], aw["o_b"], gs).T
+
+
+def _head64(x, w, s=None, b=None, step=8192):
+    """x W^T of an fp16 head, or of a 4-bit one of group 64, a slice of the vocabulary at a time."""
+    shifts = torch.arange(0, 32, 4, device=x.device, dtype=torch.int32)
+    out = []
+    for v in range(0, w.shape[0], step):
+        if s is None:
+            wv = w[v:v + step].double()
+        else:
+            q = ((w[v:v + step, :, None] >> shifts) & 15).flatten(1).double()
+            rep = (lambda t: t[v:v + step].double().repeat_interleave(64, dim=-1))
+            wv = q * rep(s) + rep(b)
+        out.append(x @ wv.T)
+    return torch.cat(out, 1)
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    if kind in ("accept", "verify"):
+        return None  # whole values; a pass whose caches are mostly its input
+    context()
+    d = _inputs(case, seed)
+    if kind == "gather":
+        rows = d["inds"].reshape(-1)
+        x = d["x"].double()
+        x = x if case["per"] else x.repeat_interleave(case["ktop"], 0)
+        y = torch.empty((rows.numel(), case["N"]), dtype=torch.float64, device="cuda")
+        for e in rows.unique().tolist():
+            at = rows == e
+            y[at] = x[at] @ _dequant(d["w"][e], d["s"][e], d["b"][e], case["gs"]).T
+        return y + d["y0"].double() if case["add"] else y
+    if kind == "moe":
+        y, inds, scores = _moe64(d["mw"], d["x"].double())
+        return dict(y=y, inds=inds, scores=scores)
+    if kind == "attn":
+        K, V = d["kc"].double(), d["vc"].double()
+        h = _attn64(d["cfg"], d["aw"], d["h0"].double(), K, V, case["L"], d["parents"], case["M"])
+        return dict(h=h, k=K, v=V)
+    if kind == "head":
+        lg = _head64(d["x"].double(), d["w"], d.get("s"), d.get("b"))
+        ban = lg.clone()
+        if d["banned"] is not None:
+            ban[:, d["banned"].long()] = -math.inf
+        return dict(argmax=ban.argmax(1).to(torch.int32), max=ban.amax(1),
+                    lse=torch.logsumexp(ban / 0.7, 1) if case["lse"] else None,
+                    logits=lg if case["logits"] else None)
+    cfg = d["cfg"]
+    layers, embed, fnorm, w4 = d["weights"]
+    n = case["n"]
+    h = embed[torch.tensor(d["prompt"], device="cuda")].double()
+    kv = []
+    for l, lw in enumerate(layers):
+        K = torch.zeros((NKV, cfg.kv_capacity, D), dtype=torch.float64, device="cuda")
+        V = torch.zeros_like(K)
+        h = _attn64(cfg.attn_cfg(l), lw["attn"], h, K, V, 0, None, n)
+        h = _moe64(lw["moe"], h)[0]
+        kv.append((K[:, :n], V[:, :n]))
+    last = (n - 1) % _lib.MJ_MAX_ROWS + 1
+    logits = _head64(_rms(h[n - last:], fnorm), w4, *d["scales"])
+    return dict(next=None, logits=logits, kv=kv)
