@@ -236,16 +236,18 @@ def _inputs(case, seed):
 
 
 class _DeviceArray:
-    """A device buffer of the engine as torch sees it."""
+    """A device buffer of the engine as torch sees it: the tensor holds this object, and so the
+    engine that owns the memory, for as long as any view of it lives."""
 
-    def __init__(self, p, shape):
+    def __init__(self, eng, p, shape):
+        self.owner = eng
         self.__cuda_array_interface__ = dict(data=(p, False), shape=shape, typestr="<f2", version=2)
 
 
 def _kv_views(eng, cfg):
     shape = (cfg.n_kv_heads, cfg.kv_capacity, cfg.head_dim)
-    return [tuple(torch.as_tensor(_DeviceArray(p, shape), device="cuda") for p in eng.kv(l))
-            for l in range(cfg.n_layers)]
+    return [tuple(torch.as_tensor(_DeviceArray(eng, p, shape), device="cuda")
+                  for p in eng.kv(l)) for l in range(cfg.n_layers)]
 
 
 def prepare(case, seed):
