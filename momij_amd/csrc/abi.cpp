@@ -308,15 +308,25 @@ mj_status mj_gather_qmm2(mj_ctx* ctx, const void* x, const uint32_t* w, const vo
     s = mj_hip(ctx, launch_qx_prep((const uint16_t*)x, xperm, xsum, rows_x, K, ctx->abort_dev,
                                    ctx->stream), "qx prep");
     if (s != MJ_OK) return s;
-    s = mj_hip(ctx, launch_bucket_inds(inds, P, bk, ctx->abort_dev, ctx->stream), "bucket");
-    if (s != MJ_OK) return s;
+    const int epi = epilogue == MJ_EPI_ADD ? EPI_ADD : EPI_STORE;
+    // the tile kernel forms its row sets from the ids itself
+    const bool tile = gather3_supported(epi, K, N, gs);
+    if (!tile) {
+        s = mj_hip(ctx, launch_bucket_inds(inds, P, bk, ctx->abort_dev, ctx->stream), "bucket");
+        if (s != MJ_OK) return s;
+    }
     GatherArgs g{};
     g.xperm = xperm;
     g.xsum = xsum;
     g.w = w;
     g.s = (const uint16_t*)scales;
     g.b = (const uint16_t*)biases;
-    g.bk = bk;
+    if (tile) {
+        g.inds = inds;
+        g.npairs = P;
+    } else {
+        g.bk = bk;
+    }
     g.y = (uint16_t*)y;
     g.K = K;
     g.N = N;
@@ -324,8 +334,7 @@ mj_status mj_gather_qmm2(mj_ctx* ctx, const void* x, const uint32_t* w, const vo
     g.x_div = lhs_per_expert ? 1 : ktop;
     g.abort = ctx->abort_dev;
     const int nb = P < MJ_MAX_EXPERTS ? P : MJ_MAX_EXPERTS;
-    return mj_hip(ctx, launch_gather(g, epilogue == MJ_EPI_ADD ? EPI_ADD : EPI_STORE, P, nb,
-                                     ctx->stream), "gather launch");
+    return mj_hip(ctx, launch_gather(g, epi, P, nb, ctx->stream), "gather launch");
 }
 
 // Arguments and shape of an MoE block call (shared by mj_moe_block and its no-alloc variant).
@@ -424,9 +433,6 @@ void moe_scratch_layout(Arena& a, int H, int I, int E, int k, int M, MoeScratch&
     ms.act = (uint16_t*)a.take((size_t)M * k * I * 2);
     ms.act_sum = (float2*)a.take((size_t)M * k * (I / 64) * sizeof(float2));
     ms.down = (uint16_t*)a.take((size_t)M * k * H * 2);
-    ms.ecnt = (int*)a.take((size_t)E * 4);
-    ms.eplist = (int*)a.take((size_t)E * MJ_MAX_ROWS * 4);
-    ms.srec = (int*)a.take((size_t)64 * 64 * 4);
 }
 
 mj_status moe_scratch(mj_ctx* ctx, int H, int I, int E, int k, int M, MoeScratch& ms) {
@@ -462,12 +468,11 @@ mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint1
     const bool fused = route_supported(H, E, k);
     const bool up_tile = gather3_supported(EPI_SWIGLU, H, 2 * I, w->gs);
     const bool dn_tile = gather3_supported(EPI_STORE, I, H, w->gs);
-    // tile path: the top-k launch also lists each expert's (row, slot) pairs for the gathers.
-    // One row takes it too, so a row's result does not depend on how many rows share its pass
-    // (a verify row equals the one-row decode step at its position, bit for bit).
+    // tile path: one row takes it too, so a row's result does not depend on how many rows share
+    // its pass (a verify row equals the one-row decode step at its position, bit for bit)
     const bool tile = fused && M >= MJ_TILE_MIN_ROWS && M <= MJ_MAX_ROWS && up_tile && dn_tile;
     // the common expert shape, up to 32 rows over at most 64 experts: one launch ranks the
-    // logits (its blocks build the slot records in LDS) and runs both products
+    // logits (its blocks form the slot records themselves) and runs both products
     const bool moe_fused =
         MJ_MOE_FUSED && tile && E <= 64 &&
         (w->up_gate_alpha == nullptr) == (w->down_alpha == nullptr) &&
@@ -486,10 +491,6 @@ mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint1
         ra.inds = inds;
         ra.scores = scores;
         ra.logits = ms.logits;
-        // E <= 64: slot records for the persistent gathers; more experts: per-expert lists
-        ra.srec = tile && E <= 64 ? ms.srec : nullptr;
-        ra.ecnt = tile && E > 64 ? ms.ecnt : nullptr;
-        ra.eplist = tile && E > 64 ? ms.eplist : nullptr;
         ra.M = M;
         ra.E = E;
         ra.k = k;
@@ -574,12 +575,11 @@ mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint1
         up.w = w->up_gate_w;
         up.s = (const uint16_t*)w->up_gate_s;
         up.b = (const uint16_t*)w->up_gate_b;
-        if (tile) {
-            up.srec = E <= 64 ? ms.srec : nullptr;
-            up.ecnt = E > 64 ? ms.ecnt : nullptr;
-            up.eplist = E > 64 ? ms.eplist : nullptr;
-        } else {
+        if (!tile) {
             up.bk = ms.bk;
+        } else if (!topk_in_up) {
+            up.inds = inds;
+            up.npairs = M * k;
         }
         up.alpha = tile ? (const uint16_t*)w->up_gate_alpha : nullptr;
         up.y = ms.act;
@@ -596,11 +596,10 @@ mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint1
             up.rk = k;
             up.rinds = inds;
             up.rscores = scores;
-            up.rsrec = ms.srec;
         }
         if (!moe_fused) {
             if (prof) prof->begin(PROF_UP, st);
-            s = mj_hip(ctx, launch_gather(up, EPI_SWIGLU, M, tile ? E : nb, st), "up gather");
+            s = mj_hip(ctx, launch_gather(up, EPI_SWIGLU, M, nb, st), "up gather");
             if (prof) prof->end(st);
             if (s != MJ_OK) return s;
         }
@@ -611,7 +610,11 @@ mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint1
             if (s != MJ_OK) return s;
         }
         GatherArgs dn = up;
-        dn.rlogits = nullptr;  // the down product reads the records the up product wrote
+        dn.rlogits = nullptr;  // the down product takes the ids the routing wrote
+        if (tile) {
+            dn.inds = inds;
+            dn.npairs = M * k;
+        }
         dn.xperm = ms.act;
         dn.xsum = dn_tile ? nullptr : ms.act_sum;
         dn.w = w->down_w;
@@ -633,7 +636,7 @@ mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint1
             if (s != MJ_OK) return s;
         } else {
             if (prof) prof->begin(PROF_DOWN, st);
-            s = mj_hip(ctx, launch_gather(dn, EPI_STORE, M, tile ? E : nb, st), "down gather");
+            s = mj_hip(ctx, launch_gather(dn, EPI_STORE, M, nb, st), "down gather");
             if (prof) prof->end(st);
             if (s != MJ_OK) return s;
         }

@@ -126,6 +126,19 @@ __device__ __forceinline__ void lds_only_barrier() {
 // static LDS of the routing words of a launch that ranks up to FR rows itself
 constexpr size_t g5_fused_rec_bytes(int FR) { return 64 * (4 + 8 + (FR > 16 ? 8 : 0)); }
 
+// Pair table of a persistent launch whose slots follow from the pairs' expert ids (REC_IDS),
+// built by every block from a.inds: byte i of id[l] = expert of pair l + 64 i, bit i of on[l] = the
+// pair has one; slot[s] = expert | part << 8, experts in increasing id, an expert with more than
+// `ps` pairs taking several slots (parts) of ps pairs.  Kept small: with 2.6 KB of it the up
+// product staged 7 rows a pass instead of 8 (64 rows over 64 experts: 41 -> 47 us).
+#define MJ_IDS_PS_MIN 8
+struct IdsLds {
+    uint64_t id[64];
+    uint8_t on[64];
+    uint16_t slot[MJ_MAX_EXPERTS + MJ_MAX_PAIRS / MJ_IDS_PS_MIN];
+    int nslot, ps;
+};
+
 // How one call of the tile-gather body fits into a launch.  MODE 0: the whole launch (the
 // standalone kernels).  The fused MoE kernel calls the up || gate body (MODE 1) and then the down
 // body (MODE 2) in every block; io carries the routing words from the first to the second.
@@ -133,13 +146,21 @@ struct FuseIO {
     uint32_t em = 0;   // lane t: rows that picked expert t (bit r)
     uint64_t er = 0;   // ... and expert t's rank in rows 0 .. 15 (3 bits at 3r)
     uint64_t er1 = 0;  // ... and in rows 16 .. 31 (3 bits at 3 (r - 16))
+    IdsLds* ids = nullptr;  // the launch's pair table (REC_IDS)
 };
+
+// Where a persistent launch's slot records come from.  REC_RANK: the launch ranks the router
+// logits itself (passes of at most FR rows over at most 64 experts).  REC_IDS: from the expert id
+// of every (row, slot) pair in global memory (any rows and experts a pass may have).
+enum { REC_NONE = 0, REC_RANK = 1, REC_IDS = 2 };
 
 // FR: rows the fused routing ranks at most (16: two a wave, ranks in er; 32: four a wave, rows
 // 16 .. 31's ranks in er1)
-template <int KPL, int GS, int EPI, int WPB, int KS, bool PER, bool ROWA, bool FUS, int MODE,
+template <int KPL, int GS, int EPI, int WPB, int KS, int REC, bool ROWA, int MODE,
           int FR = MJ_G5_FUSED_ROWS>
 __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO& io) {
+    constexpr bool PER = REC != REC_NONE;
+    constexpr bool FUS = REC == REC_RANK && MODE != 2;  // ranks the logits in its prologue
     static_assert(FR == 16 || FR == 32, "fused routing rows");
     using S = G5Shape<KPL, GS, EPI, WPB, KS>;
     constexpr int R = S::R, K = S::K, KB = S::KB, KBW = S::KBW, TPB = S::TPB, XS = S::XS;
@@ -151,25 +172,20 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int q = lane >> 4, n = lane & 15;
     const int tt = wv % TPB, kh = wv / TPB;   // weight tile and K-slice of this wave
-    const int ncb = a.N / (16 * TPB);
+    const int ncb = (a.N + 16 * TPB - 1) / (16 * TPB);
     const int u = blockIdx.x / ncb;
     int cb = blockIdx.x % ncb;
     const bool own_sums = a.xsum == nullptr;  // block sums formed here from the staged rows
 
-    // Persistent expert mode (PER): the work items are (routed-expert slot i / ncb, column
-    // block i % ncb); block b takes items b, b + gridDim.x, ... until a slot with no pairs.
-    // One load per lane brings a slot's record: pair j in lane j, the expert id and the pair
-    // count in the high halves of lanes 0 and 1; the next item's record is fetched while the
-    // current item computes.  Expert mode: block u serves expert u, whose ecnt[u] (row, slot)
-    // pairs are listed at eplist[u * MJ_ROWS ..]; count and list are loaded together, and an
-    // expert nobody picked ends here.  Bucket mode: block u serves the u-th expert of a Buckets
-    // table.  Dense: rows 0 .. dense_rows-1 in groups of R, block u taking group u (the blocks
-    // of a group stream the same weights, concurrently with the other groups' blocks).
-    const int* plist = nullptr;
-    int lpair = 0;  // expert modes: pair j of the list in lane j
-    const bool dense_mode = !PER && a.ecnt == nullptr && a.bk == nullptr;
-    const int rbase = dense_mode ? R * u : 0;  // dense: first row of the block's group
-    int e = 0, np = dense_mode ? min(R, a.dense_rows - rbase) : a.dense_rows;
+    // Persistent expert mode (PER): the work items are (slot i / ncb, column block i % ncb);
+    // block b takes items b, b + gridDim.x, ... until the slots end.  A slot is a routed expert
+    // with the pairs that picked it; its record (pair j in lane j, the expert id and the pair
+    // count in the high halves of lanes 0 and 1) is formed from registers or LDS.  Dense: rows
+    // 0 .. dense_rows-1 in groups of R, block u taking group u (the blocks of a group stream the
+    // same weights, concurrently with the other groups' blocks).
+    int lpair = 0;  // pair j of the item's record in lane j
+    const int rbase = PER ? 0 : R * u;  // dense: first row of the block's group
+    int e = 0, np = PER ? 0 : min(R, a.dense_rows - rbase);
     int item = blockIdx.x;
     int rec_n = 0;  // the next item's record (persistent mode)
     extern __shared__ __align__(16) char g5lds[];
@@ -179,8 +195,7 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
     // t in lane t, the rows that picked it (em: bit r) and t's rank in each of them (er: 3 bits
     // a row).  A slot's record follows from these in registers: slots number the routed experts
     // in increasing id (as the route kernel's), a record lists its pairs (row * k + rank) by
-    // row.  The last block also writes inds / scores and the global records for the down
-    // product.
+    // row.  The last block also writes inds / scores.
     struct FusedRoute {
         // per expert t, set by LDS atomics as the rows are ranked: the rows that picked t (bit
         // r) and t's rank in each (3 bits at 3r for rows 0 .. 15, at 3 (r - 16) in er1 beyond)
@@ -190,20 +205,46 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
     };
     // (an instantiation of its own, FUS: the routing code stays out of the other kernels)
     constexpr bool FUSABLE = FUS;
-    static_assert(!FUS || (PER && EPI == EPI_SWIGLU), "fused routing: persistent up || gate");
+    static_assert(!FUS || EPI == EPI_SWIGLU, "fused routing: persistent up || gate");
     __shared__ __align__(16) std::conditional_t<FUSABLE, FusedRoute, char> s_fr;
     constexpr bool fused = FUS;
-    static_assert(MODE == 0 || (MODE == 1 && FUS) || (MODE == 2 && PER && EPI == EPI_STORE),
+    static_assert(MODE == 0 || (MODE == 1 && FUS) || (MODE == 2 && REC == REC_RANK && EPI == EPI_STORE),
                   "fused MoE phases: up || gate with routing, then down");
-    // slot records from the routing words in registers: the ranking kernel itself, or the down
-    // phase of the fused MoE launch (words handed over by its up phase)
-    constexpr bool RREC = FUS || MODE == 2;
     uint32_t em = MODE == 2 ? io.em : 0u;
     uint64_t er = MODE == 2 ? io.er : 0ull;
     uint64_t er1 = MODE == 2 ? io.er1 : 0ull;
-    // record of slot sl in the global records' form: pair j in lane j, expert id and pair count
-    // in the high halves of lanes 0 and 1 (count 0 past the last routed expert)
-    auto fused_rec = [&](int sl) -> int {
+    // record of slot sl: pair j in lane j, expert id and pair count in the high halves of lanes 0
+    // and 1 (count 0 past the last slot)
+    auto slot_rec = [&](int sl) -> int {
+      if constexpr (REC == REC_IDS) {
+        // lane l holds the ids of pairs l + 64 i; the pairs of the slot's expert are numbered
+        // in increasing index by ballots and sent to the lane of their number in the part.
+        // Lanes with nothing to send, in round i, send to the lane below the round's first
+        // (63 in the first round: it is only taken when every lane sends)
+        if (sl >= io.ids->nslot) return 0;
+        const int se = __builtin_amdgcn_readfirstlane((int)io.ids->slot[sl]);
+        const int ex = se & 255, ps = io.ids->ps, base = (se >> 8) * ps;
+        const uint64_t iv = io.ids->id[lane];
+        const uint32_t onv = io.ids->on[lane];
+        int tot = -base, got = 0;  // pairs before round i, from the part's first
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint64_t bal =
+                __ballot((int)((uint32_t)(iv >> (8 * i)) & 255u) == ex && ((onv >> i) & 1u) != 0u);
+            if (bal == 0ull) continue;  // wave-uniform
+            const int pos = tot + (int)__builtin_amdgcn_mbcnt_hi(
+                                      (uint32_t)(bal >> 32),
+                                      __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0));
+            const int next = tot + __popcll(bal);
+            const bool send = ((bal >> lane) & 1ull) != 0ull && (unsigned)pos < (unsigned)ps;
+            const int dst = send ? pos : tot > 0 ? tot - 1 : 63;
+            const int v = __builtin_amdgcn_ds_permute(4 * dst, lane + 64 * i);
+            if (lane >= tot && lane < next) got = v;
+            tot = next;
+        }
+        const int cnt = min(ps, tot);
+        return (lane < cnt ? got : 0) | (lane == 0 ? ex << 16 : lane == 1 ? cnt << 16 : 0);
+      } else {
         const uint64_t on = __ballot(em != 0u);
         const int mys = __popcll(on & ((1ull << lane) - 1ull));
         const uint64_t hit = __ballot(em != 0u && mys == sl);
@@ -223,7 +264,76 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
         const int pr = rr * a.rk + (int)(((rr < 16 ? rx0 : rx1) >> (3 * (rr & 15))) & 7u);
         const int got = __builtin_amdgcn_ds_permute((mine ? pos : 63) * 4, pr);
         return got | (lane == 0 ? ex << 16 : lane == 1 ? __popc(rm) << 16 : 0);
+      }
     };
+    // the pair table, once a launch
+    if constexpr (REC == REC_IDS) {
+        IdsLds& t = *io.ids;
+        static_assert(NT >= MJ_MAX_PAIRS && MJ_MAX_EXPERTS == 256, "a pair and an expert a thread");
+        const int idv = tid < a.npairs ? a.inds[tid] : -1;
+        uint32_t* s_cnt = (uint32_t*)g5lds;  // pairs per expert, where the weight tiles go later
+        if (tid < MJ_MAX_EXPERTS) s_cnt[tid] = 0u;
+        // one reading of the abort word decides for the block (its waves meet at barriers)
+        if (tid == 0) t.nslot = aborted(a.abort) ? -1 : 0;
+        __syncthreads();
+        if (t.nslot < 0) return;
+        const bool ok = (unsigned)idv < (unsigned)MJ_MAX_EXPERTS;
+        if (tid < MJ_MAX_PAIRS) ((uint8_t*)t.id)[8 * (tid & 63) + (tid >> 6)] = (uint8_t)idv;
+        if (ok) atomicAdd(&s_cnt[idv], 1u);
+        // (pairs without an expert: their bits of the lanes' bytes go through the scratch)
+        uint8_t* s_ok = (uint8_t*)(s_cnt + MJ_MAX_EXPERTS);
+        if (tid < MJ_MAX_PAIRS) s_ok[tid] = ok ? 1 : 0;
+        __syncthreads();
+        if (wv == 1) {
+            uint32_t b = 0u;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) b |= (uint32_t)s_ok[64 * i + lane] << i;
+            t.on[lane] = (uint8_t)b;
+        }
+        if (wv == 0) {
+            // lane l numbers the slots of experts l, l + 64, l + 128, l + 192.  Parts of 64 pairs;
+            // of the RA rows one pass takes where the slots' items would leave half of the blocks
+            // idle (few experts, many rows): the parts' weights then come from L2
+            int c[4], routed = 0, first = 0;
+            uint64_t on[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                c[i] = (int)s_cnt[lane + 64 * i];
+                on[i] = __ballot(c[i] > 0);
+                routed += __popcll(on[i]);
+            }
+            const int ps = 2 * routed * ncb <= (int)gridDim.x ? max(RA, MJ_IDS_PS_MIN) : 64;
+            if (__ballot(max(max(c[0], c[1]), max(c[2], c[3])) > ps) == 0ull) {
+                // no expert in parts (every pass of an MoE block): no sums across lanes
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (c[i] > 0)
+                        t.slot[first + __popcll(on[i] & ((1ull << lane) - 1ull))] =
+                            (uint16_t)(lane + 64 * i);
+                    first += __popcll(on[i]);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int parts = (c[i] + ps - 1) / ps;
+                    int incl = parts;
+#pragma unroll
+                    for (int o = 1; o < 64; o <<= 1) {
+                        const int y = __shfl_up(incl, o, MJ_WAVE);
+                        if (lane >= o) incl += y;
+                    }
+                    for (int p = 0; p < parts; ++p)
+                        t.slot[first + incl - parts + p] = (uint16_t)((lane + 64 * i) | (p << 8));
+                    first += __shfl(incl, 63, MJ_WAVE);
+                }
+            }
+            if (lane == 0) {
+                t.nslot = first;
+                t.ps = ps;
+            }
+        }
+        __syncthreads();
+    }
     if constexpr (FUSABLE) {
         static_assert(sizeof(FusedRoute) == g5_fused_rec_bytes(FR), "record bytes");
         static_assert(FR <= 4 * WPB, "at most four rows a wave");
@@ -286,33 +396,11 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
             io.em = em;
             io.er = er;
             io.er1 = er1;
-            if (wr && wv == 0) {
-                const uint64_t on = __ballot(em != 0u);
-                const int total = __popcll(on);
-                if (em != 0u) {
-                    int* gr = a.rsrec + __popcll(on & ((1ull << lane) - 1ull)) * MJ_ROWS;
-                    const int cnt = __popc(em);
-                    int c = 0;
-#pragma unroll
-                    for (int r = 0; r < FR; ++r) {
-                        if ((em >> r) & 1u) {
-                            gr[c] = (r * k + (int)(((r < 16 ? er : er1) >> (3 * (r & 15))) & 7u)) |
-                                    (c == 0 ? lane << 16 : c == 1 ? cnt << 16 : 0);
-                            ++c;
-                        }
-                    }
-                    if (cnt == 1) gr[1] = 1 << 16;
-                }
-                if (lane >= total) {  // slots past the last routed expert: count 0
-                    a.rsrec[lane * MJ_ROWS] = 0;
-                    a.rsrec[lane * MJ_ROWS + 1] = 0;
-                }
-            }
             // the row scratch is free for the weight tiles: every wave is past the barrier above
         }
     }
     {
-        const int ab = !fused && a.abort ? *a.abort : 0;  // fused: checked with the logits
+        const int ab = !PER && a.abort ? *a.abort : 0;  // persistent: checked with the routing
         if constexpr (PER) {
             if constexpr (MODE == 2) {
                 // blocks with one up item fewer come free first: they take the first down items
@@ -321,23 +409,11 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
                 const int G = (int)gridDim.x, rem = (nS * a.fup_ncb) % G;
                 item = (int)blockIdx.x >= rem ? (int)blockIdx.x - rem : (int)blockIdx.x + (G - rem);
             }
-            const int rec = RREC ? fused_rec(min(item / ncb, 63))
-                                 : a.srec[min(item / ncb, 63) * MJ_ROWS + lane];
+            const int rec = slot_rec(REC == REC_IDS ? item / ncb : min(item / ncb, 63));
             e = __builtin_amdgcn_readlane(rec, 0) >> 16;
-            np = item / ncb < 64 ? __builtin_amdgcn_readlane(rec, 1) >> 16 : 0;
+            np = REC == REC_IDS || item / ncb < 64 ? __builtin_amdgcn_readlane(rec, 1) >> 16 : 0;
             lpair = rec & 0xFFFF;
             cb = item % ncb;
-        } else if (a.ecnt != nullptr) {
-            e = u;
-            np = a.ecnt[u];
-            lpair = a.eplist[u * MJ_ROWS + lane];
-        } else if (a.bk != nullptr) {
-            const Buckets* bk = a.bk;
-            const int cnt = bk->count, ee = bk->expert[u], s0 = bk->start[u], s1 = bk->start[u + 1];
-            if (u >= cnt) return;  // whole block
-            e = ee;
-            np = s1 - s0;
-            plist = bk->pair + s0;
         }
         if (ab || np <= 0) return;  // whole block
     }
@@ -365,19 +441,18 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
     // epilogue does not wait on a dependent load (older than the weights, they change no wait
     // count)
     constexpr bool RES_PF = EPI == EPI_ADD && !PER;
-    const bool res_pf = RES_PF && a.ecnt == nullptr && a.bk == nullptr && kh == 0;
+    const bool res_pf = RES_PF && kh == 0;
     uint32_t resv[4] = {0u, 0u, 0u, 0u};
     auto stage_load = [&](int pb, int npass, int b, int lp, int npp, bool first = false) {
         uint16_t* xs = xs_of(b);
         float2* xsl = xsl_of(b);
         const int myr = min(pb + (lane < R ? lane : 0), npp - 1);
-        const int prl =
-            (PER || a.ecnt) ? __shfl(lp, myr, MJ_WAVE) : (plist ? plist[myr] : rbase + myr);
+        const int prl = PER ? __shfl(lp, myr, MJ_WAVE) : rbase + myr;
         if constexpr (RES_PF) {
             // (after the pair list: the wait for a list load would cover these too)
             if (first && res_pf) {
                 // rows of the lane's outputs: q (a pass of at most 4 rows), else 4q .. 4q+3
-                const int col = (cb * TPB + tt) * 16 + n;
+                const int col = min((cb * TPB + tt) * 16, a.N - 16) + n;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int i = npass <= 4 ? q : 4 * q + r;
@@ -435,7 +510,8 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
                 const int j0 = (cbb * TPB + tt) * 8;
                 return (size_t)ee * a.N + (r < 8 ? j0 + r : I + j0 + r - 8);
             } else {
-                return (size_t)ee * a.N + (cbb * TPB + tt) * 16 + r;
+                // (a last column block may have fewer tiles: its other waves repeat the last)
+                return (size_t)ee * a.N + min((cbb * TPB + tt) * 16, a.N - 16) + r;
             }
         };
         __builtin_amdgcn_sched_barrier(0);  // loads issued before stay ahead in the vmcnt queue
@@ -556,18 +632,11 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
             own_block_sums(npass);
             lds_barrier<G + NSB>();
         }
-        // persistent mode: the next item's record, fetched behind this item's weights (one
-        // vector load younger than them: PF).  With fused routing the record is formed from
-        // registers once the weights have landed; the load is then a stand-in that keeps the
-        // queue's count, and its value is consumed (times zero) so that it stays
-        // (the down phase of the fused launch forms every record from registers: no load)
-        constexpr int PF = PER && MODE != 2 ? 1 : 0;
-        if constexpr (PER && MODE != 2) {
-            if (pb == 0) {
-                const int* rp = fused ? (const int*)a.rlogits
-                                      : a.srec + min((item + (int)gridDim.x) / ncb, 63) * MJ_ROWS + lane;
-                rec_n = *rp;
-            }
+        // ranked routing's up product: a stand-in load behind this item's weights (PF: one vector
+        // load younger than them), whose value is consumed (times zero) so that it stays
+        constexpr int PF = FUS ? 1 : 0;
+        if constexpr (FUS) {
+            if (pb == 0) rec_n = *(const int*)a.rlogits;
         }
         wait_vmcnt<G + PF>();      // scales and biases have landed
         u4v sv[SCW], bv[SCW];
@@ -637,19 +706,22 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
         // scales and first half of the code groups are requested once this item's first half
         // is done (its scales are in registers, its first half's codes read), the rest after
         // its MFMAs; the item waits for its own groups first, so later waits count nothing new
-        constexpr bool SPLIT = PER && (MODE == 1 || MODE == 2) && G >= 2;
+        constexpr bool SPLIT = PER && (MODE != 0 || REC == REC_IDS) && G >= 2;
         constexpr int GP = G / 2;  // code groups a part (four parts measured slower)
         bool stage_next = false;
         int np_next = 0;
         auto next_item = [&]() {
             if constexpr (PER) {
                 const int nx = item + (int)gridDim.x;
-                if constexpr (MODE == 2) {
-                    rec_n = fused_rec(min(nx / ncb, 63));
-                } else if (fused)
-                    rec_n = fused_rec(min(nx / ncb, 63)) | (rec_n & (int)opaque(0u));
+                if constexpr (REC == REC_IDS) {
+                    rec_n = slot_rec(nx / ncb);
+                } else if constexpr (MODE == 2) {
+                    rec_n = slot_rec(min(nx / ncb, 63));
+                } else {
+                    rec_n = slot_rec(min(nx / ncb, 63)) | (rec_n & (int)opaque(0u));
+                }
                 np_next = __builtin_amdgcn_readlane(rec_n, 1) >> 16;
-                stage_next = pb + RA >= np && nx / ncb < 64 && np_next > 0;
+                stage_next = pb + RA >= np && (REC == REC_IDS || nx / ncb < 64) && np_next > 0;
             }
         };
         // sum_B s_B * (sum q x)_B: per 64-block f16 MFMA sums, scaled in fp32, one column group
@@ -813,7 +885,7 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
                 const int i = NR == 1 ? q : 4 * q + r;
-                if (kh == 0 && i < npass) {
+                if (kh == 0 && i < npass && col < a.N) {
                     uint16_t* yp = a.y + (size_t)s_pair[buf][i] * a.N + col;
                     if constexpr (EPI == EPI_ADD) {
                         const uint16_t res = res_pf && pb == 0 ? (uint16_t)resv[r] : *yp;
@@ -839,7 +911,7 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
     }
     if constexpr (!PER) break;
     item += gridDim.x;
-    if (item / ncb >= 64) break;
+    if (REC != REC_IDS && item / ncb >= 64) break;
     np = __builtin_amdgcn_readlane(rec_n, 1) >> 16;
     if (np <= 0) break;
     e = __builtin_amdgcn_readlane(rec_n, 0) >> 16;
@@ -850,13 +922,14 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
   }
 }
 
-template <int KPL, int GS, int EPI, int WPB, int KS, bool PER = false, bool ROWA = false,
-          bool FUS = false>
-// four waves per SIMD: two 8-wave blocks (or one 16-wave block) per CU
+template <int KPL, int GS, int EPI, int WPB, int KS, int REC = REC_NONE, bool ROWA = false>
+// four waves per SIMD: two 8-wave blocks per CU
 __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_gather5(
     GatherArgs a, int RA, int multi) {
     FuseIO io;
-    g5_body<KPL, GS, EPI, WPB, KS, PER, ROWA, FUS, 0>(a, RA, multi, io);
+    __shared__ __align__(16) std::conditional_t<REC == REC_IDS, IdsLds, char> s_ids;
+    if constexpr (REC == REC_IDS) io.ids = &s_ids;
+    g5_body<KPL, GS, EPI, WPB, KS, REC, ROWA, 0>(a, RA, multi, io);
 }
 
 // Fused MoE launch (H = 2048, I = 1024): the up || gate product with its routing, then the down
@@ -870,9 +943,14 @@ template <int GS, bool ROWA, int FR>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_moe_fused(
     GatherArgs up, GatherArgs dn, int ra_up, int ra_dn, int multi_up, int multi_dn) {
     FuseIO io;
-    g5_body<8, GS, EPI_SWIGLU, 8, 2, true, ROWA, true, 1, FR>(up, ra_up, multi_up, io);
+    g5_body<8, GS, EPI_SWIGLU, 8, 2, REC_RANK, ROWA, 1, FR>(up, ra_up, multi_up, io);
     __syncthreads();  // every wave is done with the up phase's LDS
-    g5_body<4, GS, EPI_STORE, 8, 1, true, ROWA, false, 2, FR>(dn, ra_dn, multi_dn, io);
+    g5_body<4, GS, EPI_STORE, 8, 1, REC_RANK, ROWA, 2, FR>(dn, ra_dn, multi_dn, io);
+}
+
+// static LDS of a persistent kernel: its pair lists and what its records are formed from
+constexpr size_t g5_stat(int rec, int FR) {
+    return 256 + (rec == REC_IDS ? sizeof(IdsLds) : g5_fused_rec_bytes(FR));
 }
 
 // dynamic LDS a tile-gather launch may take (the device has 160 KB per workgroup)
@@ -891,107 +969,96 @@ static int persistent_blocks() {
     return 2 * cus;
 }
 
-template <int KPL, int GS, int EPI, int WPB, int KS, bool PER = false, bool ROWA = false>
-static hipError_t launch_g5(const GatherArgs& a, int rows, int n_buckets, hipStream_t st) {
+template <int KPL, int GS, int EPI, int WPB, int KS, int REC = REC_NONE, bool ROWA = false>
+static hipError_t launch_g5(const GatherArgs& a, int rows, int slots, hipStream_t st) {
     using S = G5Shape<KPL, GS, EPI, WPB, KS>;
-    const int ncb = a.N / (16 * S::TPB);
-    // staged rows per pass: for the expert products as many as keep two blocks per CU (more
-    // rows on one expert are rare and take extra passes); dense projections take up to 16
+    constexpr bool PER = REC != REC_NONE;
+    const int ncb = (a.N + 16 * S::TPB - 1) / (16 * S::TPB);
+    // staged rows per pass: for the persistent products as many as keep two blocks per CU (more
+    // rows on one expert take extra passes); dense projections take up to 16
     const int want = rows < 1 ? 1 : rows;
     int RA = want < S::R ? want : S::R;
-    const bool expert = a.ecnt != nullptr || a.srec != nullptr;
-    // two blocks a CU for the expert products; static LDS: the pair lists (128 bytes) and, in
-    // the persistent up || gate kernels, the fused routing's records
-    const size_t stat = 256 + (PER && EPI == EPI_SWIGLU ? g5_fused_rec_bytes(MJ_G5_FUSED_ROWS) : 0);
-    const size_t limit =
-        (EPI == EPI_SWIGLU || EPI == EPI_STORE) && expert ? 80 * 1024 - stat : G5_LDS_MAX;
+    const size_t limit = PER ? 80 * 1024 - g5_stat(REC, MJ_G5_FUSED_ROWS) : G5_LDS_MAX;
     while (RA > 1 && S::lds(RA, want > RA || PER) > limit) --RA;
     const bool multi = want > RA;
-    int grid = n_buckets * ncb;
+    int grid = slots * ncb;
     if (PER && grid > persistent_blocks()) grid = persistent_blocks();
-    if constexpr (PER && EPI == EPI_SWIGLU) {
-        if (a.rlogits != nullptr) {
-            launch_timed(k_gather5<KPL, GS, EPI, WPB, KS, PER, ROWA, true>, dim3(grid),
-                         dim3(WPB * 64), S::lds(RA, multi || PER), st, a, RA, (int)multi);
-            return hipGetLastError();
-        }
-    }
-    launch_timed(k_gather5<KPL, GS, EPI, WPB, KS, PER, ROWA>, dim3(grid), dim3(WPB * 64),
+    launch_timed(k_gather5<KPL, GS, EPI, WPB, KS, REC, ROWA>, dim3(grid), dim3(WPB * 64),
                  S::lds(RA, multi || PER), st, a, RA, (int)multi);
     return hipGetLastError();
 }
 
-// Shapes the tile kernel covers: SWIGLU / ADD at K = 2048, STORE at K = 512, 1024 or 2048; N
-// a multiple of the block's rows; group size 64 or 128.
+// Shapes the tile kernel covers: SWIGLU at K = 2048, STORE / ADD at K = 512, 1024 or 2048; N a
+// multiple of a tile's 16 rows (of a block's 64 for SWIGLU); group size 64 or 128.
 bool gather3_supported(int epi, int K, int N, int gs) {
     if (gs != 64 && gs != 128) return false;
     switch (epi) {
         case EPI_SWIGLU: return K == 2048 && N % 64 == 0;
-        case EPI_ADD: return K == 2048 && N % 64 == 0;
-        case EPI_STORE: return (K == 512 || K == 1024 || K == 2048) && N % 64 == 0;
+        case EPI_ADD:
+        case EPI_STORE: return (K == 512 || K == 1024 || K == 2048) && N % 16 == 0;
     }
     return false;
 }
 
-hipError_t launch_gather3(const GatherArgs& a, int epi, int max_rows_per_bucket, int n_buckets,
-                          hipStream_t st) {
+hipError_t launch_gather3(const GatherArgs& a, int epi, int rows, hipStream_t st) {
     if (!gather3_supported(epi, a.K, a.N, a.gs)) return hipErrorInvalidValue;
-    int rows = max_rows_per_bucket;
-    // expert products over routed-expert slot records (at most 64 experts): persistent
-    const bool per = a.srec != nullptr;
-    if (per && (n_buckets > 64 || (epi != EPI_SWIGLU && epi != EPI_STORE)))
+    const bool rank = a.rlogits != nullptr, per = rank || a.inds != nullptr;
+    // ranked routing: the up || gate product ranks the router logits itself
+    if (rank && (epi != EPI_SWIGLU || a.rM < 1 || a.rM > MJ_G5_FUSED_ROWS || a.rE < 1 ||
+                 a.rE > 64 || a.rk < 1 || a.rk > 8 || a.rk > a.rE || a.x_div != a.rk ||
+                 a.rinds == nullptr || a.rscores == nullptr))
         return hipErrorInvalidValue;
-    // fused routing: the up || gate product ranks the router logits itself
-    if (a.rlogits != nullptr &&
-        (!per || epi != EPI_SWIGLU || a.rM < 1 || a.rM > MJ_G5_FUSED_ROWS || a.rE < 1 ||
-         a.rE > 64 || a.rk < 1 || a.rk > 8 || a.rk > a.rE || a.x_div != a.rk ||
-         a.rinds == nullptr || a.rscores == nullptr || a.rsrec == nullptr))
-        return hipErrorInvalidValue;
+    if (per && !rank && (a.npairs < 1 || a.npairs > MJ_MAX_PAIRS)) return hipErrorInvalidValue;
+    if (!per && epi == EPI_SWIGLU) return hipErrorInvalidValue;
+    // slots the launch may have: each a routed expert, or a part of one's pairs
+    const int slots = rank ? 64 : a.npairs;
+#define MJ_G5(KPL, E, W, KS64, KS128, REC, A)                                               \
+    return a.gs == 64 ? launch_g5<KPL, 64, E, W, KS64, REC, A>(a, rows, slots, st)          \
+                      : launch_g5<KPL, 128, E, W, KS128, REC, A>(a, rows, slots, st);
     // row-alpha expert weights (scale alpha, bias -alpha in every group of a row): the
     // fold kernels read one alpha per row instead of the group scales and biases
-    if (a.alpha != nullptr && (a.srec != nullptr || a.ecnt != nullptr) &&
-        (epi == EPI_SWIGLU || epi == EPI_STORE)) {
-#define MJ_G5A(KPL, E, KS64, KS128)                                                        \
-    {                                                                                      \
-        if (per)                                                                           \
-            return a.gs == 64 ? launch_g5<KPL, 64, E, 8, KS64, true, true>(a, rows, n_buckets, st) \
-                              : launch_g5<KPL, 128, E, 8, KS128, true, true>(a, rows, n_buckets, st); \
-        return a.gs == 64 ? launch_g5<KPL, 64, E, 8, KS64, false, true>(a, rows, n_buckets, st)    \
-                          : launch_g5<KPL, 128, E, 8, KS128, false, true>(a, rows, n_buckets, st); \
+    const bool al = a.alpha != nullptr && per && epi != EPI_ADD;
+    if (epi == EPI_SWIGLU) {
+        if (rank && al) { MJ_G5(8, EPI_SWIGLU, 8, 2, 2, REC_RANK, true) }
+        if (rank) { MJ_G5(8, EPI_SWIGLU, 8, 2, 2, REC_RANK, false) }
+        if (al) { MJ_G5(8, EPI_SWIGLU, 8, 2, 2, REC_IDS, true) }
+        MJ_G5(8, EPI_SWIGLU, 8, 2, 2, REC_IDS, false)
     }
-        if (epi == EPI_SWIGLU) MJ_G5A(8, EPI_SWIGLU, 2, 2)
-        if (a.K == 512) MJ_G5A(2, EPI_STORE, 1, 1)
-        if (a.K == 1024) MJ_G5A(4, EPI_STORE, 1, 1)
-        MJ_G5A(8, EPI_STORE, 2, 2)
-#undef MJ_G5A
+    if (per && epi == EPI_STORE && al) {
+        if (a.K == 512) { MJ_G5(2, EPI_STORE, 8, 1, 1, REC_IDS, true) }
+        if (a.K == 1024) { MJ_G5(4, EPI_STORE, 8, 1, 1, REC_IDS, true) }
+        MJ_G5(8, EPI_STORE, 8, 2, 2, REC_IDS, true)
     }
-#define MJ_G5(KPL, E, W, KS64, KS128)                                                      \
-    if (per && (E == EPI_SWIGLU || E == EPI_STORE))                                         \
-        return a.gs == 64 ? launch_g5<KPL, 64, E, W, KS64, true>(a, rows, n_buckets, st)    \
-                          : launch_g5<KPL, 128, E, W, KS128, true>(a, rows, n_buckets, st); \
-    return a.gs == 64 ? launch_g5<KPL, 64, E, W, KS64>(a, rows, n_buckets, st)              \
-                      : launch_g5<KPL, 128, E, W, KS128>(a, rows, n_buckets, st);
+    if (per && epi == EPI_STORE) {
+        if (a.K == 512) { MJ_G5(2, EPI_STORE, 8, 1, 1, REC_IDS, false) }
+        if (a.K == 1024) { MJ_G5(4, EPI_STORE, 8, 1, 1, REC_IDS, false) }
+        MJ_G5(8, EPI_STORE, 8, 2, 2, REC_IDS, false)
+    }
+    if (per) {
+        if (a.K == 512) { MJ_G5(2, EPI_ADD, 8, 1, 1, REC_IDS, false) }
+        if (a.K == 1024) { MJ_G5(4, EPI_ADD, 8, 1, 1, REC_IDS, false) }
+        MJ_G5(8, EPI_ADD, 8, 2, 2, REC_IDS, false)
+    }
+#undef MJ_G5
     // dense projections (qkv, o-proj: a few MB at most) spread over many small blocks, four
     // waves of one 16-row tile (group 64) or two (group 128): the unpack work of a block is
     // then short, and the launch fills the chip.  More than 16 rows: one set of blocks per
     // 16-row group, running side by side (each re-reads the small weight matrix) instead of
     // one block unpacking its tile again for every further 16 rows.
-    const bool dense = a.srec == nullptr && a.ecnt == nullptr && a.bk == nullptr;
-    if (dense) {
-        n_buckets = (a.dense_rows + 15) / 16;
-        rows = rows < 16 ? rows : 16;
+    const int groups = (a.dense_rows + 15) / 16;
+    rows = rows < 16 ? rows : 16;
+#define MJ_G5D(KPL, E, W, KS64, KS128)                                                    \
+    return a.gs == 64 ? launch_g5<KPL, 64, E, W, KS64>(a, rows, groups, st)               \
+                      : launch_g5<KPL, 128, E, W, KS128>(a, rows, groups, st);
+    if (epi == EPI_ADD) {
+        if (a.K == 512) { MJ_G5D(2, EPI_ADD, 8, 1, 1) }
+        if (a.K == 1024) { MJ_G5D(4, EPI_ADD, 8, 1, 1) }
+        MJ_G5D(8, EPI_ADD, 4, 4, 2)
     }
-    switch (epi) {
-        case EPI_SWIGLU: MJ_G5(8, EPI_SWIGLU, 8, 2, 2)
-        case EPI_ADD: MJ_G5(8, EPI_ADD, 4, 4, 2)
-        case EPI_STORE:
-            if (a.K == 512) { MJ_G5(2, EPI_STORE, 8, 1, 1) }
-            if (a.K == 1024) { MJ_G5(4, EPI_STORE, 8, 1, 1) }
-            if (dense) { MJ_G5(8, EPI_STORE, 4, 4, 2) }
-            MJ_G5(8, EPI_STORE, 8, 2, 2)
-    }
-#undef MJ_G5
-    return hipErrorInvalidValue;
+    if (a.K == 512) { MJ_G5D(2, EPI_STORE, 8, 1, 1) }
+    if (a.K == 1024) { MJ_G5D(4, EPI_STORE, 8, 1, 1) }
+    MJ_G5D(8, EPI_STORE, 4, 4, 2)
+#undef MJ_G5D
 }
 
 // static LDS of the fused MoE kernel: both phases' pair lists and the routing words
@@ -1057,8 +1124,7 @@ bool moe_fused_supported(int H, int I, int E, int gs, int M, bool rowa) {
 hipError_t launch_moe_fused(const GatherArgs& up, const GatherArgs& dn, int rows, hipStream_t st) {
     const bool rowa = up.alpha != nullptr;
     if (!moe_fused_supported(up.K, dn.K, up.rE, up.gs, up.rM, rowa) || up.N != 2 * dn.K ||
-        dn.N != up.K || up.rlogits == nullptr || up.srec == nullptr ||
-        dn.srec == nullptr)
+        dn.N != up.K || up.rlogits == nullptr)
         return hipErrorInvalidValue;
     if (up.gs == 64)
         return rowa ? launch_moe_fused_t<64, true>(up, dn, rows, st)
@@ -1067,10 +1133,9 @@ hipError_t launch_moe_fused(const GatherArgs& up, const GatherArgs& dn, int rows
                 : launch_moe_fused_t<128, false>(up, dn, rows, st);
 }
 
-template <int KPL, int GS, int EPI, int WPB, int KS, bool PER = false, bool ROWA = false,
-          bool FUS = false>
+template <int KPL, int GS, int EPI, int WPB, int KS, int REC = REC_NONE, bool ROWA = false>
 static hipError_t g5_attr() {
-    return hipFuncSetAttribute((const void*)k_gather5<KPL, GS, EPI, WPB, KS, PER, ROWA, FUS>,
+    return hipFuncSetAttribute((const void*)k_gather5<KPL, GS, EPI, WPB, KS, REC, ROWA>,
                                hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)std::min(G5Shape<KPL, GS, EPI, WPB, KS>::lds(16, true),
                                              G5_LDS_MAX));
@@ -1078,20 +1143,29 @@ static hipError_t g5_attr() {
 
 hipError_t set_gather3_attributes() {
     hipError_t e = hipSuccess;
-#define MJ_A(KPL, E, W, KS64, KS128)                                 \
-    if (e == hipSuccess) e = g5_attr<KPL, 64, E, W, KS64>();          \
-    if (e == hipSuccess) e = g5_attr<KPL, 128, E, W, KS128>();        \
-    if (e == hipSuccess) e = g5_attr<KPL, 64, E, W, KS64, true>();    \
-    if (e == hipSuccess) e = g5_attr<KPL, 128, E, W, KS128, true>();
-    MJ_A(8, EPI_SWIGLU, 8, 2, 2) MJ_A(8, EPI_ADD, 4, 4, 2) MJ_A(2, EPI_STORE, 8, 1, 1)
-    MJ_A(4, EPI_STORE, 8, 1, 1) MJ_A(8, EPI_STORE, 8, 2, 2) MJ_A(8, EPI_STORE, 4, 4, 2)
+#define MJ_A(KPL, E, W, KS64, KS128, REC, A)                                  \
+    if (e == hipSuccess) e = g5_attr<KPL, 64, E, W, KS64, REC, A>();          \
+    if (e == hipSuccess) e = g5_attr<KPL, 128, E, W, KS128, REC, A>();
+    MJ_A(8, EPI_ADD, 4, 4, 2, REC_NONE, false)
+    MJ_A(2, EPI_ADD, 8, 1, 1, REC_NONE, false)
+    MJ_A(4, EPI_ADD, 8, 1, 1, REC_NONE, false)
+    MJ_A(2, EPI_STORE, 8, 1, 1, REC_NONE, false)
+    MJ_A(4, EPI_STORE, 8, 1, 1, REC_NONE, false)
+    MJ_A(8, EPI_STORE, 4, 4, 2, REC_NONE, false)
+    MJ_A(8, EPI_SWIGLU, 8, 2, 2, REC_RANK, false)
+    MJ_A(8, EPI_SWIGLU, 8, 2, 2, REC_RANK, true)
+    MJ_A(8, EPI_SWIGLU, 8, 2, 2, REC_IDS, false)
+    MJ_A(8, EPI_SWIGLU, 8, 2, 2, REC_IDS, true)
+    MJ_A(2, EPI_STORE, 8, 1, 1, REC_IDS, false)
+    MJ_A(4, EPI_STORE, 8, 1, 1, REC_IDS, false)
+    MJ_A(8, EPI_STORE, 8, 2, 2, REC_IDS, false)
+    MJ_A(2, EPI_STORE, 8, 1, 1, REC_IDS, true)
+    MJ_A(4, EPI_STORE, 8, 1, 1, REC_IDS, true)
+    MJ_A(8, EPI_STORE, 8, 2, 2, REC_IDS, true)
+    MJ_A(2, EPI_ADD, 8, 1, 1, REC_IDS, false)
+    MJ_A(4, EPI_ADD, 8, 1, 1, REC_IDS, false)
+    MJ_A(8, EPI_ADD, 8, 2, 2, REC_IDS, false)
 #undef MJ_A
-#define MJ_AA(KPL, E, KS64, KS128)                                              \
-    if (e == hipSuccess) e = g5_attr<KPL, 64, E, 8, KS64, true, true>();        \
-    if (e == hipSuccess) e = g5_attr<KPL, 128, E, 8, KS128, true, true>();      \
-    if (e == hipSuccess) e = g5_attr<KPL, 64, E, 8, KS64, false, true>();       \
-    if (e == hipSuccess) e = g5_attr<KPL, 128, E, 8, KS128, false, true>();
-    MJ_AA(8, EPI_SWIGLU, 2, 2) MJ_AA(2, EPI_STORE, 1, 1) MJ_AA(4, EPI_STORE, 1, 1)
     // the fused MoE kernels
     {
         int ra_up = 0, ra_dn = 0;
@@ -1107,12 +1181,5 @@ hipError_t set_gather3_attributes() {
         for (const void* k : ks)
             if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     }
-    // the fused-routing up || gate kernels
-    if (e == hipSuccess) e = g5_attr<8, 64, EPI_SWIGLU, 8, 2, true, false, true>();
-    if (e == hipSuccess) e = g5_attr<8, 128, EPI_SWIGLU, 8, 2, true, false, true>();
-    if (e == hipSuccess) e = g5_attr<8, 64, EPI_SWIGLU, 8, 2, true, true, true>();
-    if (e == hipSuccess) e = g5_attr<8, 128, EPI_SWIGLU, 8, 2, true, true, true>();
-    MJ_AA(8, EPI_STORE, 2, 2)
-#undef MJ_AA
     return e;
 }

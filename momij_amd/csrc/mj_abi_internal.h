@@ -56,9 +56,6 @@ struct MoeScratch {
     uint16_t* act;       // [M*k][I] (qx for M > 1, plain for M == 1)
     float2* act_sum;     // [M*k][I/64]
     uint16_t* down;      // [M*k][H]
-    int* ecnt;           // pairs per expert [E]
-    int* eplist;         // pair lists per expert [E][MJ_ROWS]
-    int* srec;           // routed-expert slot records [64][64] (E <= 64)
     bool want_plain = false;  // also write the normed rows plain into xn (debug capture)
 };
 

@@ -85,23 +85,19 @@ struct StepResult {
 };
 
 
-// Row sets of a gather launch (grid = groups x column blocks):
-//   ecnt != nullptr (tile kernel): group u = expert u with ecnt[u] pairs listed, in no
-//   particular order, at eplist[u * MJ_ROWS ..] (pair = row * top_k + slot);
-//   bk != nullptr: group u = bucket u of the table;  neither: dense, one group of dense_rows.
+// Row sets of a gather launch:
+//   tile kernel, persistent: the pairs (pair = row * top_k + slot) of each routed expert, from
+//   `inds` or ranked from the router logits;  tile kernel, dense: rows 0 .. dense_rows-1 of
+//   expert 0;  general kernel: bk != nullptr: group u = bucket u of the table, else dense.
 struct GatherArgs {
     const uint16_t* xperm;  // qx activations [rows_x][K]
     const float2* xsum;     // [rows_x][K/64] {sum x, sum base*x}
     const uint32_t* w;      // [E][N][K/16]
     const uint16_t* s;      // [E][N][K/gs]
     const uint16_t* b;
-    const Buckets* bk;      // fallback kernel: rows grouped by expert (nullptr: dense)
-    const int* ecnt;        // tile kernel: pairs per expert [E]
-    const int* eplist;      // tile kernel: pair lists [E][MJ_ROWS]
-    const int* srec;        // tile kernel, persistent: one record per routed-expert slot
-                            // [64][64]: lane j = pair j (low 16 bits); lane 0 also holds the
-                            // expert id, lane 1 the pair count (high 16 bits); count 0 past the
-                            // last routed expert
+    const Buckets* bk;      // general kernel: rows grouped by expert (nullptr: dense)
+    const int32_t* inds;    // tile kernel, persistent: expert of every pair [npairs] (pairs whose
+    int npairs;             // id is outside [0, MJ_MAX_EXPERTS) are left out)
     int dense_rows;         // dense: rows 0 .. dense_rows-1 of expert 0
     const uint16_t* alpha;  // row-alpha weights [E][N] fp16 (scale alpha, bias -alpha in
                             // every group): the tile expert kernels read it instead of s / b
@@ -110,14 +106,13 @@ struct GatherArgs {
     int K, N, gs;
     int x_div;              // x row of pair p = p / x_div
     const int* abort;
-    // persistent expert mode with fused routing (rlogits set, at most MJ_G5_FUSED_ROWS rows,
-    // E <= 64): every block ranks the router logits [rM][rE] itself and builds the slot records
-    // in LDS; block 0 writes inds / scores [rM][rk] and the records (rsrec) for the next product
+    // persistent, ranked routing (rlogits set, at most MJ_G5_FUSED_ROWS rows, in the fused MoE
+    // launch MJ_MOE_FUSED_ROWS; E <= 64): every block ranks the router logits [rM][rE] itself;
+    // the last block writes inds / scores [rM][rk]
     const float* rlogits;
     int rM, rE, rk;
     int32_t* rinds;
     float* rscores;
-    int* rsrec;
     // fused MoE launch (up || gate then down in one kernel): the up product's column blocks,
     // and the bound of a down item's wait for act rows still holding the router launch's
     // marker, in re-stagings of its rows
@@ -155,8 +150,7 @@ bool gather3_supported(int epi, int K, int N, int gs);
 // (the shapes, and two blocks of the launch resident a CU: its waits assume every block runs)
 bool moe_fused_supported(int H, int I, int E, int gs, int M, bool rowa);
 hipError_t launch_moe_fused(const GatherArgs& up, const GatherArgs& dn, int rows, hipStream_t st);
-hipError_t launch_gather3(const GatherArgs& a, int epi, int max_rows_per_bucket, int n_buckets,
-                          hipStream_t st);
+hipError_t launch_gather3(const GatherArgs& a, int epi, int rows, hipStream_t st);
 
 // RoPE angles of a pass: rope_cs[r * MJ_ROPE_F + f] = {cos, sin} of (L + depth[r]) *
 // inv_freq[f] for row r and frequency f < rope_dim / 2, written by the pass's embedding kernel
@@ -299,10 +293,6 @@ struct RouteArgs {
     int32_t* inds;           // [M][k]
     float* scores;           // [M][k]
     float* logits;           // [M][E] router logits
-    int* ecnt;               // pairs per expert [E] (route lists)
-    int* eplist;             // pair lists [E][MJ_ROWS] (route lists)
-    int* srec;               // slot records of the persistent gathers [64][64] (E <= 64;
-                             // nullable: then ecnt / eplist, when set, are written instead)
     int M, E, k;
     float eps;
     const int* abort;
@@ -311,8 +301,7 @@ struct RouteArgs {
 };
 bool route_supported(int H, int E, int k);
 hipError_t launch_route_logits(const RouteArgs& a, int H, hipStream_t st);
-// inds and scores of every row from the logits, and (when a.ecnt is set, M <= MJ_ROWS) the
-// per-expert pair lists ecnt / eplist
+// inds and scores of every row from the logits
 hipError_t launch_route_topk(const RouteArgs& a, hipStream_t st);
 // y = [x_resid +] combine of the k expert rows (as launch_score_combine), then the norm of y
 // into `no`; H must be 2048.

@@ -102,37 +102,56 @@ hipError_t launch_router(const uint16_t* W, const uint16_t* x, float* logits, in
     return hipGetLastError();
 }
 
-// Group pair indices 0..P-1 by expert id (ids in s_ids, LDS): experts in increasing id, pairs
-// in increasing index inside each expert.  Ids outside [0, E) are left out.  Whole block.
+// Group pair indices 0..P-1 by expert id (ids in s_ids, LDS): experts in increasing id, an
+// expert's pairs in no particular order (each pair's output is computed the same way wherever it
+// is listed).  Ids outside [0, E) are left out.  Whole 256-thread block, thread t = expert t
+// (one thread walking the experts and pairs took 21 us of a 72-pair product's 48).
 __device__ void bucket_pairs(const int* s_ids, int P, int E, Buckets* bk, int* s_cnt,
                              int* s_slot) {
-    const int t = threadIdx.x;
-    for (int e = t; e < E; e += blockDim.x) s_cnt[e] = 0;
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    __shared__ int s_tot[4][2];
+    s_cnt[t] = 0;
     __syncthreads();
-    for (int p = t; p < P; p += blockDim.x) {
+    for (int p = t; p < P; p += 256) {
         const int e = s_ids[p];
         if (e >= 0 && e < E) atomicAdd(&s_cnt[e], 1);
     }
     __syncthreads();
-    if (t == 0) {
-        int u = 0, pos = 0;
-        for (int e = 0; e < E; ++e) {
-            if (s_cnt[e] > 0) {
-                bk->expert[u] = e;
-                bk->start[u] = pos;
-                s_slot[e] = pos;
-                pos += s_cnt[e];
-                ++u;
-            }
-        }
-        bk->start[u] = pos;
-        bk->count = u;
-        for (int p = 0; p < P; ++p) {
-            const int e = s_ids[p];
-            if (e >= 0 && e < E) bk->pair[s_slot[e]++] = p;
+    const int cnt = s_cnt[t], on = cnt > 0;
+    int pos = cnt, u = on;  // inclusive sums over the experts up to t
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(pos, o, MJ_WAVE), z = __shfl_up(u, o, MJ_WAVE);
+        if (lane >= o) {
+            pos += y;
+            u += z;
         }
     }
+    if (lane == 63) {
+        s_tot[wv][0] = pos;
+        s_tot[wv][1] = u;
+    }
+    __syncthreads();
+    for (int w = 0; w < wv; ++w) {
+        pos += s_tot[w][0];
+        u += s_tot[w][1];
+    }
+    s_slot[t] = pos - cnt;
+    if (on) {
+        bk->expert[u - 1] = t;
+        bk->start[u - 1] = pos - cnt;
+    }
+    if (t == 255) {
+        bk->start[u] = pos;
+        bk->count = u;
+    }
+    __syncthreads();
+    for (int p = t; p < P; p += 256) {
+        const int e = s_ids[p];
+        if (e >= 0 && e < E) bk->pair[atomicAdd(&s_slot[e], 1)] = p;
+    }
 }
+static_assert(MJ_MAX_EXPERTS == 256, "an expert a thread");
 
 __global__ __launch_bounds__(256) void k_bucket_inds(const int32_t* __restrict__ inds, int P,
                                                      Buckets* bk, const int* abort) {
@@ -369,8 +388,7 @@ hipError_t launch_combine_norm(const uint16_t* down, const float* scores, const 
 //                   qx order with its block sums) and the logits of the group's experts.  The
 //                   router matrix is read in 32 KB pieces by many CUs (a single CU streams only
 //                   a few tens of GB/s).
-//   k_route_topk    one wave per row: top-k of the row's logits, renormalised scores, and the
-//                   row's (row, slot) pairs appended to the experts' lists.
+//   k_route_topk    one wave per row: top-k of the row's logits, renormalised scores.
 // The kernel boundary orders the two: a grid-wide handoff inside one kernel needs a device-
 // scope release (an L2 write-back on this chip), which costs more than the launch.
 // Arithmetic as maple_rms_norm / maple_batched_gemv / maple_route_top8: fp32 sums (the logit
@@ -451,89 +469,32 @@ __global__ __launch_bounds__(256) void k_route_logits(RouteArgs a) {
     if (lane == 0) *(float2*)(a.logits + (size_t)r * E + e0) = make_float2(acc[0], acc[1]);
 }
 
-// inds and scores of every row, and the pair lists of the tile gathers: one 1024-thread block,
-// wave w ranks rows w, w + 16, ... (M <= 64: at most four each, all their logits requested
-// before the first is ranked).  Pairs are grouped by expert with LDS atomics.  With slot records
-// (E <= 64) the routed experts are numbered in increasing id and slot s's record gets expert,
-// count and pairs (count 0 for every slot past the last); otherwise each expert's count and list
-// go to ecnt / eplist.  Every entry a reader uses is rewritten each launch, so nothing needs
-// clearing.  Order inside a list is immaterial: every pair's output is computed the same way
-// wherever it sits.
-#define RT_WAVES 16
+// inds and scores of every row: one wave a row, four rows a block.  (One 16-wave block for the
+// whole pass ranked up to four rows a wave on one CU: 22.7 us for 64 rows of 256 experts, 10.0 us
+// of 64.)
+#define RT_WAVES 4
 template <int NI>
 __global__ __launch_bounds__(64 * RT_WAVES) void k_route_topk(RouteArgs a) {
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, E = a.E, k = a.k, M = a.M;
-    constexpr bool SLOTS_OK = NI == 1;  // slot records: at most 64 experts
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, E = a.E, k = a.k;
     __shared__ __align__(16) float s_row[RT_WAVES][64 * NI];
     __shared__ __align__(16) float s_gate[RT_WAVES][8];
     __shared__ int s_ind[RT_WAVES][8];
-    __shared__ int s_cnt[MJ_MAX_EXPERTS];
-    __shared__ int s_pairs[SLOTS_OK ? 64 : 1][SLOTS_OK ? MJ_ROWS : 1];
-    __shared__ int s_wsum[RT_WAVES];
-    if (aborted(a.abort)) return;
-    const bool slots = SLOTS_OK && a.srec != nullptr;
-    if (tid < E) s_cnt[tid] = 0;
-    // all of the wave's rows (at most four) requested up front, every load unconditional
-    // (clamped row and expert) so no branch waits on one
-    float v[4][NI];
+    const int r = blockIdx.x * RT_WAVES + wv;
+    float v[NI];
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
+    for (int i = 0; i < NI; ++i)
+        v[i] = a.logits[min(r, a.M - 1) * E + min(lane + 64 * i, E - 1)];
+    if (aborted(a.abort) || r >= a.M) return;
 #pragma unroll
-        for (int i = 0; i < NI; ++i)
-            v[s][i] = a.logits[min(wv + RT_WAVES * s, M - 1) * E + min(lane + 64 * i, E - 1)];
-    __syncthreads();  // s_cnt cleared
-#pragma unroll 1
-    for (int s = 0, r = wv; r < M; ++s, r += RT_WAVES) {
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const float t = s == 0 ? v[0][i] : s == 1 ? v[1][i] : s == 2 ? v[2][i] : v[3][i];
-            s_row[wv][lane + 64 * i] = lane + 64 * i < E ? t + 0.0f : -INFINITY;
-        }
-        __builtin_amdgcn_wave_barrier();
-        int e = 0;
-        float gate = 0.0f;
-        row_topk<NI>(s_row[wv], E, k, s_ind[wv], s_gate[wv], e, gate);
-        if (lane < k) {
-            a.inds[r * k + lane] = e;
-            a.scores[r * k + lane] = gate;
-            if (slots) {
-                const int pos = atomicAdd(&s_cnt[e], 1);
-                if constexpr (SLOTS_OK) s_pairs[e][pos] = r * k + lane;
-            } else if (a.ecnt) {
-                const int pos = atomicAdd(&s_cnt[e], 1);
-                a.eplist[e * MJ_ROWS + pos] = r * k + lane;
-            }
-        }
-    }
-    if (!slots && !a.ecnt) return;
-    __syncthreads();
-    if (!slots) {
-        if (tid < E) a.ecnt[tid] = s_cnt[tid];
-        return;
-    }
-    // routed experts numbered in increasing id: slot = routed experts below this one
-    const bool on = tid < E && s_cnt[tid] > 0;
-    const uint64_t bal = __ballot(on);
-    if (lane == 0) s_wsum[wv] = __popcll(bal);
-    __syncthreads();
-    int before = 0, total = 0;
-#pragma unroll
-    for (int w = 0; w < RT_WAVES; ++w) {
-        before += w < wv ? s_wsum[w] : 0;
-        total += s_wsum[w];
-    }
-    if constexpr (SLOTS_OK) {
-        if (on) {
-            const int cnt = s_cnt[tid];
-            int* rec = a.srec + (before + __popcll(bal & ((1ull << lane) - 1))) * MJ_ROWS;
-            for (int j = 0; j < cnt; ++j)
-                rec[j] = s_pairs[tid][j] | (j == 0 ? tid << 16 : j == 1 ? cnt << 16 : 0);
-            if (cnt == 1) rec[1] = 1 << 16;
-        }
-        if (tid >= total && tid < 64) {
-            a.srec[tid * MJ_ROWS] = 0;
-            a.srec[tid * MJ_ROWS + 1] = 0;
-        }
+    for (int i = 0; i < NI; ++i)
+        s_row[wv][lane + 64 * i] = lane + 64 * i < E ? v[i] + 0.0f : -INFINITY;
+    __builtin_amdgcn_wave_barrier();
+    int e = 0;
+    float gate = 0.0f;
+    row_topk<NI>(s_row[wv], E, k, s_ind[wv], s_gate[wv], e, gate);
+    if (lane < k) {
+        a.inds[r * k + lane] = e;
+        a.scores[r * k + lane] = gate;
     }
 }
 
@@ -550,13 +511,13 @@ hipError_t launch_route_logits(const RouteArgs& a, int H, hipStream_t st) {
 }
 
 hipError_t launch_route_topk(const RouteArgs& a, hipStream_t st) {
-    // one block: 16 waves with at most four rows each
     if (a.E < 1 || a.E > MJ_MAX_EXPERTS || a.k < 1 || a.k > 8 || a.k > a.E || a.M < 1 ||
-        a.M > 4 * RT_WAVES || a.M > MJ_ROWS || (a.srec && a.E > 64))
+        a.M > MJ_ROWS)
         return hipErrorInvalidValue;
+    const dim3 grid((a.M + RT_WAVES - 1) / RT_WAVES), block(64 * RT_WAVES);
     if (a.E <= 64)
-        hipLaunchKernelGGL(k_route_topk<1>, dim3(1), dim3(64 * RT_WAVES), 0, st, a);
+        hipLaunchKernelGGL(k_route_topk<1>, grid, block, 0, st, a);
     else
-        hipLaunchKernelGGL(k_route_topk<MJ_MAX_EXPERTS / 64>, dim3(1), dim3(64 * RT_WAVES), 0, st, a);
+        hipLaunchKernelGGL(k_route_topk<MJ_MAX_EXPERTS / 64>, grid, block, 0, st, a);
     return hipGetLastError();
 }

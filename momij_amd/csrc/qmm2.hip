@@ -430,11 +430,12 @@ static hipError_t launch_gather_t(const GatherArgs& a, int n_buckets_max, hipStr
 
 hipError_t launch_gather(const GatherArgs& a, int epi, int max_rows_per_bucket, int n_buckets_max,
                          hipStream_t st) {
-    if (gather3_supported(epi, a.K, a.N, a.gs))
-        return launch_gather3(a, epi, max_rows_per_bucket, n_buckets_max, st);
-    if (a.ecnt != nullptr || a.srec != nullptr)  // expert modes are the tile kernel's
-        return hipErrorInvalidValue;
-    // generic fallback (any K % 256 == 0, N % 16 == 0): K inside each wave, RG row groups
+    // the tile kernel: dense, or over the pairs' expert ids; its SWIGLU is the experts' only
+    const bool per = a.inds != nullptr || a.rlogits != nullptr;
+    if (a.bk == nullptr && (per || epi != EPI_SWIGLU) && gather3_supported(epi, a.K, a.N, a.gs))
+        return launch_gather3(a, epi, max_rows_per_bucket, st);
+    if (per) return hipErrorInvalidValue;
+    // general kernel (any K % 256 == 0, N % 16 == 0): K inside each wave, RG row groups
     const int rows = max_rows_per_bucket;
     const int rg = rows <= 4 ? 1 : (rows <= 8 ? 2 : 4);
 #define MJ_G(R, E)                                      \

@@ -1,0 +1,114 @@
+"""GPU parity of the tile gather's slots, which every block forms from the pairs' expert ids: parts
+of an expert with many pairs, pairs without an expert, column blocks with fewer than four (eight)
+tiles, and the MoE launch over those slots, against the oracle."""
+import numpy as np
+import pytest
+
+from momij_amd import synth
+from tests.gpu_util import assert_close, dev, host
+
+pytestmark = pytest.mark.gpu
+
+# One fp16 rounding of the result, of either sum: 2 * 2^-11 / sqrt(12) of it on average, a third of
+# the bound.
+REL = 1e-3
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from momij_amd.ops import Context
+
+    c = Context(0)
+    yield c
+    c.close()
+
+
+def _ids(rng, kind, P, E):
+    if kind == "one":  # every pair on one expert: more than 64, in parts
+        return np.full(P, E - 1, np.int32)
+    ids = rng.integers(0, E, P).astype(np.int32)
+    if kind == "some":  # pairs that have no expert are left out
+        ids[:: 3] = -1
+        ids[1:: 7] = 256
+    elif kind == "last":  # the last pair alone, after 511 without an expert
+        ids[:-1] = -5
+    return ids
+
+
+@pytest.mark.parametrize("M,ktop,E,K,N,gs,kind,add", [
+    (64, 8, 256, 512, 64, 64, "any", False),     # 512 pairs over every expert a launch takes
+    (64, 8, 3, 1024, 48, 64, "any", False),      # 170 pairs an expert; three tiles of eight
+    (64, 8, 2, 2048, 16, 128, "one", False),     # 512 pairs on one expert, one tile
+    (64, 1, 1, 2048, 80, 64, "one", True),       # dense rows with residual, five tiles
+    (17, 1, 4, 512, 144, 128, "any", True),
+    (9, 1, 1, 1024, 2064, 64, "one", True),
+    (33, 2, 16, 2048, 208, 64, "some", False),
+    (64, 8, 64, 512, 32, 64, "last", False),
+    (2, 1, 4, 2048, 5632, 64, "any", False),     # the fewest pairs that take the tile kernel
+    (16, 4, 8, 1536, 48, 64, "some", False),     # the general kernel (K = 1536), same table rules
+    (5, 8, 256, 4096, 32, 128, "any", False),
+])
+def test_gather_slots(ctx, orc, M, ktop, E, K, N, gs, kind, add):
+    import torch
+
+    print(f"case: slots M={M} ktop={ktop} E={E} K={K} N={N} gs={gs} {kind} add={add}", flush=True)
+    rng = np.random.default_rng(M * 1000 + N)
+    P = M * ktop
+    w, s, b = synth.qweight(rng, (E,), N, K, gs)
+    x = synth.normal_f16(rng, (M, K))
+    ids = _ids(rng, kind, P, E)
+    y0 = synth.normal_f16(rng, (P, N))
+    ok = (ids >= 0) & (ids < 256)
+    ref = orc.qmm2(x, w, s, b, np.where(ok, ids, 0).astype(np.int32), M, ktop, K, N, gs)
+    if add:
+        ref = (y0.astype(np.float32) + ref.astype(np.float32)).astype(np.float16)
+    ref[~ok] = y0[~ok]
+    y, dx, dw, ds, db, di = dev(y0), dev(x), dev(w), dev(s), dev(b), dev(ids)
+    torch.cuda.synchronize()
+    ctx.gather_qmm2(dx, dw, ds, db, di, y, M, ktop, K, N, gs, epilogue=int(add))
+    ctx.sync()
+    got = host(y)
+    assert (got[~ok] == y0[~ok]).all()
+    rel, _ = assert_close(got, ref, what="slots")
+    assert rel < REL
+
+
+@pytest.mark.parametrize("E,I,gs,M,alpha", [
+    (64, 512, 64, 1, False), (64, 512, 64, 16, True), (64, 512, 128, 32, False),  # ranked, I 512
+    (64, 1024, 64, 33, False), (64, 512, 64, 64, True),  # the first rows past the ranked forms
+    (72, 1024, 64, 1, False), (256, 512, 64, 5, True), (256, 1024, 128, 64, False),
+    (8, 1024, 64, 64, False),  # every row on every expert: 64 pairs a slot
+])
+def test_moe_slots(ctx, orc, E, I, gs, M, alpha):
+    import torch
+
+    print(f"case: moe slots E={E} I={I} gs={gs} M={M} alpha={alpha}", flush=True)
+    rng = np.random.default_rng(E + I + M)
+    H = 2048
+    mw = synth.moe_weights(rng, E, H, I, gs)
+    if alpha:
+        for k, n in (("up_gate", 2 * I), ("down", H)):
+            a = rng.uniform(0.005, 0.02, (E, n)).astype(np.float16)
+            mw[k + "_s"] = np.repeat(a[..., None], mw[k + "_s"].shape[-1], -1)
+            mw[k + "_b"] = -mw[k + "_s"]
+            mw[k + "_alpha"] = a
+    x = synth.normal_f16(rng, (M, H))
+    ref, ri, rs = orc.moe_block(mw, x, prenorm=True, residual=True)
+    dmw = {k: (dev(v) if isinstance(v, np.ndarray) else v) for k, v in mw.items()}
+    dx, y = dev(x), torch.empty((M, H), dtype=torch.float16, device="cuda")
+    inds = torch.empty((M, 8), dtype=torch.int32, device="cuda")
+    sc = torch.empty((M, 8), dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    for _ in range(2):  # the second call finds the first one's scratch
+        ctx.moe_block(dmw, dx, y, M, 3, inds, sc)
+    ctx.sync()
+    assert (host(inds) == ri).all()
+    assert_close(host(y), ref, what="moe")
+    # a row's result does not depend on the rows that share its pass: the one-row call, bit for bit
+    y1 = torch.empty((1, H), dtype=torch.float16, device="cuda")
+    for r in {0, M // 2, M - 1}:
+        xr = dx[r:r + 1].contiguous()
+        torch.cuda.synchronize()
+        ctx.moe_block(dmw, xr, y1, 1, 3)
+        ctx.sync()
+        assert torch.equal(y1[0], y[r])
