@@ -245,15 +245,28 @@ struct NucState {
     int need, row, acc;
     float u, Z;
 };
-// Scratch of a nucleus sample over one row of V: the row's keys (e bits), the selection's four
-// rounds of digit histograms (counts [4][256], exact masses [4][256]), the last round's counts
-// per block [blocks][256], and the deferred decision.
+// The selection so far: mass of the keys above the chosen digits, the digits, and whether the
+// target lies within the row's mass at all; and its end, the cut key and id.
+struct NucSel {
+    uint64_t above;
+    uint32_t prefix;
+    int some;
+};
+struct NucCut {
+    uint32_t key;
+    int id;
+};
+// Scratch of a nucleus sample over one row of V: the row's keys (e bits), the selection's three
+// rounds of digit histograms (counts, exact masses), the last round's counts per block, the
+// deferred decision, the selection after the first and second histogram, and the cut.
 struct NucleusBuf {
     uint32_t* keys;
     uint32_t* hcnt;
     uint64_t* hmass;
     uint32_t* hblk;
     NucState* st;
+    NucSel* sel;
+    NucCut* cut;
 };
 size_t nucleus_bytes(int V);
 void nucleus_layout(void* base, int V, NucleusBuf& nb);

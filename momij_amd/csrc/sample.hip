@@ -12,7 +12,7 @@
 // ranked by e descending, the lower id first on ties, kept up to the first ranked prefix whose
 // mass reaches top_p * Z, sampled in id order.  The masses are summed exactly, as integers
 // trunc(e * 2^40), so no order is needed: the cut is found by a radix selection over the e bits
-// (four 8-bit digit rounds of histograms of counts and masses), not by sorting the row.
+// (three digit rounds of histograms of counts and masses), not by sorting the row.
 // Every float operation below happens in a fixed order (chunks of 16 summed sequentially,
 // blocks of 64 chunks summed sequentially, block totals summed sequentially; exp evaluated by
 // canon_expf; IEEE divisions) so the CPU oracle reproduces each decision bit for bit.
@@ -347,16 +347,17 @@ __device__ __forceinline__ void write_result(const SampleArgs& a, int acc, int t
     }
 }
 
-// Walk of row `row` to tgt over its mass -- the residual (resid) or e -- given the running
-// totals of its block sums (pref[b] = ((s_0 + s_1) + ...) + s_b, the totals a sequential walk
+// Walk of a row to tgt over its mass (vals(c, x): chunk c's element values into x, their sum in
+// element order, c clamped by the caller), given the running totals of its block sums (pref[b] = ((s_0 + s_1) + ...) + s_b, the totals a sequential walk
 // forms): the first block whose running total reaches tgt (the last element if none), in it the
 // first chunk (the block's 64 chunk sums recomputed in the same order, running on from the total
 // before the block; the block's last element if none), then the first element of that chunk;
 // writes (fr, token).  Block of 256 threads; the block's chunk sums and element values are
 // computed once, and the running totals of a level are formed redundantly by every lane of
 // wave 0 so that the first lane reaching tgt is found by one ballot.
-__device__ void walk_write(const SampleArgs& a, int row, int fr, bool resid, float tgt,
-                           const float* pref, float mxs, float Zr, float q, int d) {
+template <class F>
+__device__ __forceinline__ void walk_write(const SampleArgs& a, int fr, float tgt,
+                                           const float* pref, F vals) {
     const int t = threadIdx.x;
     const int nch = (a.V + CH - 1) / CH, nb = a.nblocks;
     __shared__ __align__(16) float cs[BLK];
@@ -375,8 +376,7 @@ __device__ void walk_write(const SampleArgs& a, int row, int fr, bool resid, flo
     const float P = blk > 0 ? pref[blk - 1] : 0.0f;
     if (t < BLK) {
         float x[CH];
-        const float s = chunk_vals(a, row, min(c0 + t, nch - 1), resid, mxs, Zr, q, d, x);
-        cs[t] = s;
+        cs[t] = vals(min(c0 + t, nch - 1), x);
         float4* e4 = (float4*)ev[t];
 #pragma unroll
         for (int k = 0; k < CH / 4; ++k)
@@ -468,8 +468,10 @@ __global__ __launch_bounds__(256) void k_sample_decide(SampleArgs a) {
         return;  // block-uniform
     }
     if (t == 0 && a.nb.st) a.nb.st->need = 0;
-    walk_write(a, fr, fr, false, u0 * Z[fr], pref + fr * per, a.rowmax[fr] * a.invT, Z[fr],
-               0.0f, -1);
+    const float mxs = a.rowmax[fr] * a.invT, Zf = Z[fr];
+    walk_write(a, fr, u0 * Zf, pref + fr * per, [&](int c, float x[CH]) {
+        return chunk_vals(a, fr, c, false, mxs, Zf, 0.0f, -1, x);
+    });
 }
 
 // Residual block sums of the rejected row (same chunk / block order as the e sums): one 64-thread
@@ -496,6 +498,16 @@ __global__ __launch_bounds__(64) void k_resid_sums(SampleArgs a) {
     }
 }
 
+// Round r's histogram of the nucleus selection (NUC_HBINS bins kept for each) set empty.
+#define NUC_HBINS 2048
+__device__ __forceinline__ void nuc_clear(const NucleusBuf& nb, int r, int t) {
+#pragma unroll
+    for (int k = 0; k < NUC_HBINS / 256; ++k) {
+        nb.hcnt[NUC_HBINS * r + 256 * k + t] = 0u;
+        nb.hmass[NUC_HBINS * r + 256 * k + t] = 0ull;
+    }
+}
+
 // The rejected row's sample: the residual total S, then a walk to u1 * S over the residual, or,
 // with no residual mass, samplePrepared of the row (nucleus kernels, or a walk to u1 * Z over e
 // with the row's block sums).
@@ -505,10 +517,7 @@ __global__ __launch_bounds__(256) void k_resid_walk(SampleArgs a) {
     const SampleState st = *a.state;
     const int t = threadIdx.x;
     // the nucleus selection's first histogram starts empty (its kernel adds to it next)
-    if (a.nb.st) {
-        a.nb.hcnt[t] = 0u;
-        a.nb.hmass[t] = 0ull;
-    }
+    if (a.nb.st) nuc_clear(a.nb, 0, t);
     if (st.phase != 1) return;
     __shared__ float s_S;
     __shared__ float pref[MAX_CHUNKS / BLK];
@@ -531,117 +540,38 @@ __global__ __launch_bounds__(256) void k_resid_walk(SampleArgs a) {
         if (t == 0) running_totals(pref, a.nblocks);
         __syncthreads();
     }
-    walk_write(a, st.fr, st.fr, walk_resid, walk_resid ? u1 * S : u1 * st.Zr, pref,
-               a.rowmax[st.fr] * a.invT, st.Zr, st.q, st.d);
+    const float mxs = a.rowmax[st.fr] * a.invT;
+    walk_write(a, st.fr, walk_resid ? u1 * S : u1 * st.Zr, pref, [&](int c, float x[CH]) {
+        return chunk_vals(a, st.fr, c, walk_resid, mxs, st.Zr, st.q, st.d, x);
+    });
 }
 
 // ---- nucleus (samplePrepared, LogitsProcessor.swift:137-164) --------------------------------
-// Canonical sum and walk of n values f(i) by a 1024-thread block, in or_canon_sum /
-// or_canon_walk's order: chunks of CH in order, blocks of BLK chunks in order, block totals in
-// order; the walk finds the first block, then chunk, then element whose running total reaches
-// tgt (the last index of the level otherwise).  cs / bs hold the chunk and block sums of f
-// (blk_sum fills them for blk_walk).
-template <class F>
-__device__ float blk_sum(F f, int n, float* cs, float* bs, float* s_out) {
-    const int t = threadIdx.x;
-    const int nch = (n + CH - 1) / CH, nbk = (nch + BLK - 1) / BLK;
-    for (int c = t; c < nch; c += 1024) {
-        float sum = 0.0f;
-        const int e = min(c * CH + CH, n);
-        for (int v = c * CH; v < e; ++v) sum = sum + f(v);
-        cs[c] = sum;
-    }
-    __syncthreads();
-    for (int b = t; b < nbk; b += 1024) {
-        float sum = 0.0f;
-        for (int c = b * BLK; c < min(b * BLK + BLK, nch); ++c) sum = sum + cs[c];
-        bs[b] = sum;
-    }
-    __syncthreads();
-    if (t == 0) {
-        float S = 0.0f;
-        for (int b = 0; b < nbk; ++b) S = S + bs[b];
-        *s_out = S;
-    }
-    __syncthreads();
-    return *s_out;
-}
-
-template <class F>
-__device__ int blk_walk(F f, int n, float tgt, const float* cs, const float* bs, int* s_out) {
-    if (threadIdx.x == 0) {
-        const int nch = (n + CH - 1) / CH, nbk = (nch + BLK - 1) / BLK;
-        int res = n - 1;
-        float P = 0.0f;
-        for (int b = 0; b < nbk; ++b) {
-            const float Pn = P + bs[b];
-            if (tgt <= Pn) {
-                const int c0 = b * BLK, c1 = min(c0 + BLK, nch);
-                res = min(c1 * CH, n) - 1;
-                float Q = P;
-                for (int c = c0; c < c1; ++c) {
-                    const float Qn = Q + cs[c];
-                    if (tgt <= Qn) {
-                        const int e = min(c * CH + CH, n);
-                        res = e - 1;
-                        float R = Q;
-                        for (int v = c * CH; v < e; ++v) {
-                            R = R + f(v);
-                            if (tgt <= R) {
-                                res = v;
-                                break;
-                            }
-                        }
-                        break;
-                    }
-                    Q = Qn;
-                }
-                break;
-            }
-            P = Pn;
-        }
-        *s_out = res;
-    }
-    __syncthreads();
-    return *s_out;
-}
-
-// ---- nucleus cut by radix selection -------------------------------------------------------
-// The e of the nucleus row are non-negative floats, so their bits order as their values.  Round
-// r (0..3) histograms digit r (bits 31 - 8r .. 24 - 8r) of the keys that match the digits
-// already chosen: a count and an exact mass (sum of trunc(e * 2^40)) per digit value.  Scanning a
-// round's digits from the top, the cut lies in the first digit whose mass, added to the mass
-// of the keys above it, reaches the target; after four rounds the cut key is known exactly,
-// and among the keys equal to it (ties, taken in id order) the cut is the j-th, j the fewest
-// that reach the target.  NUC_BLOCKS blocks of 256 threads cover up to NUC_BLOCKS * 2048 ids,
-// block b ids [2048 b, 2048 b + 2048); the last round also keeps each block's digit counts so
-// the j-th tie is found without another pass.
+// The cut, by radix selection.  The e of the nucleus row are non-negative floats, so their bits
+// order as their values.  Round r (0..2) histograms digit r (bits 31..21, 20..10, 9..0) of the keys
+// that match the digits already chosen: a count and an exact mass (sum of trunc(e * 2^40)) per
+// digit value.  Scanning a round's digits from the top, the cut lies in the first digit whose
+// mass, added to the mass of the keys above it, reaches the target; after three rounds the cut
+// key is known exactly, and among the keys equal to it (ties, taken in id order) the cut is the
+// j-th, j the fewest that reach the target.  NUC_BLOCKS blocks of 256 threads cover up to
+// NUC_BLOCKS * 2048 ids, block b ids [2048 b, 2048 b + 2048); the last round also keeps each
+// block's digit counts so the j-th tie is found without another pass.
+// Every kernel scans the histogram before it with its whole block (a thread's digits, then sums
+// across lanes); the state after a scan is left for the next kernel.  (One thread's walk of the
+// digits, three and four histograms a round, took 21, 30 and 37 us; the kept sums and the walk on
+// one CU, element by element, 164 us of a 152k-id row.)
 #define NUC_BLOCKS 96
 #define NUC_PER_BLOCK 2048
 
+template <int R>
+struct NucDigit {  // of round R
+    static constexpr int BITS = R < 2 ? 11 : 10, BINS = 1 << BITS;
+    static constexpr int SHIFT = R == 0 ? 21 : R == 1 ? 10 : 0;
+    static constexpr int OFF = R * NUC_HBINS;  // first bin in hcnt / hmass
+};
+
 __device__ __forceinline__ uint64_t nuc_fixed(float e) {
     return (uint64_t)(e * 0x1p40f);  // exact scaling, then truncation (e <= 1)
-}
-
-// The selection state after rounds 0 .. r - 1: the chosen digits (prefix) and the mass of the
-// keys ranked above them; false when the target exceeds the row's whole mass (every key kept).
-__device__ bool nuc_prefix(const NucleusBuf& nb, int r, uint64_t F, uint32_t& prefix,
-                           uint64_t& above) {
-    prefix = 0u;
-    above = 0ull;
-    for (int rr = 0; rr < r; ++rr) {
-        const uint32_t* cnt = nb.hcnt + 256 * rr;
-        const uint64_t* mass = nb.hmass + 256 * rr;
-        int d = 255;
-        for (; d >= 0; --d) {
-            if (cnt[d] == 0u) continue;
-            if (above + mass[d] >= F) break;
-            above += mass[d];
-        }
-        if (d < 0) return false;
-        prefix = (prefix << 8) | (uint32_t)d;
-    }
-    return true;
 }
 
 __device__ __forceinline__ uint64_t nuc_target(const SampleArgs& a, float Z) {
@@ -649,171 +579,315 @@ __device__ __forceinline__ uint64_t nuc_target(const SampleArgs& a, float Z) {
     return nuc_fixed(tp * Z);
 }
 
+__device__ __forceinline__ uint64_t shfl_up64(uint64_t v, int o) {
+    const uint32_t lo = __shfl_up((uint32_t)v, o, MJ_WAVE);
+    const uint32_t hi = __shfl_up((uint32_t)(v >> 32), o, MJ_WAVE);
+    return ((uint64_t)hi << 32) | lo;
+}
+
+// The selection after round R's histogram, from the state before it: prefix gains the digit, and
+// above the mass of the keys ranked above that digit's; some = false when the target exceeds the
+// row's whole mass (every key is kept).  Block of 256 threads, all of them get the result; thread t
+// holds bins BINS - 1 - t PER .. downwards.
+template <int R>
+__device__ NucSel nuc_scan(const NucleusBuf& nb, NucSel s, uint64_t F) {
+    using Dg = NucDigit<R>;
+    constexpr int PER = Dg::BINS / 256;
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const int lo = Dg::OFF + Dg::BINS - (t + 1) * PER;  // the thread's lowest bin
+    uint32_t cnt[PER];
+    uint64_t mass[PER];
+#pragma unroll
+    for (int k = 0; k < PER; k += 4) {
+        const u4v c = *(const u4v*)(nb.hcnt + lo + k);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) cnt[k + j] = c[j];
+    }
+#pragma unroll
+    for (int k = 0; k < PER; k += 2) {
+        const u4v m = *(const u4v*)(nb.hmass + lo + k);
+        mass[k] = ((uint64_t)m[1] << 32) | m[0];
+        mass[k + 1] = ((uint64_t)m[3] << 32) | m[2];
+    }
+    uint64_t own = 0ull;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) own += mass[k];
+    uint64_t incl = own;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint64_t y = shfl_up64(incl, o);
+        if (lane >= o) incl += y;
+    }
+    __shared__ uint64_t s_w[4];
+    __shared__ uint64_t s_above;
+    __shared__ int s_bin;  // bins below the top
+    if (lane == 63) s_w[wv] = incl;
+    if (t == 0) s_bin = Dg::BINS;
+    __syncthreads();
+    uint64_t above = s.above + incl - own;
+    for (int w = 0; w < wv; ++w) above += s_w[w];
+    // the thread's first bin from the top that reaches the target
+    int hit = Dg::BINS;
+    uint64_t ha = 0ull;
+#pragma unroll
+    for (int k = PER - 1; k >= 0; --k) {
+        if (hit == Dg::BINS && cnt[k] != 0u && above + mass[k] >= F) {
+            hit = t * PER + PER - 1 - k;
+            ha = above;
+        }
+        above += mass[k];
+    }
+    if (hit < Dg::BINS) atomicMin(&s_bin, hit);
+    __syncthreads();
+    if (hit < Dg::BINS && hit == s_bin) s_above = ha;
+    __syncthreads();
+    const int bin = s_bin;
+    if (bin == Dg::BINS) s.some = 0;
+    if (s.some) {
+        s.prefix = (s.prefix << Dg::BITS) | (uint32_t)(Dg::BINS - 1 - bin);
+        s.above = s_above;
+    }
+    return s;
+}
+
 // Round R of the selection; round 0 also computes the row's keys (e bits).
 template <int R>
 __global__ __launch_bounds__(256) void k_nucleus_round(SampleArgs a) {
     if (aborted(a.abort)) return;
     a = resolve(a);
+    using Dg = NucDigit<R>;
     const int t = threadIdx.x, b = blockIdx.x;
     // the next round's histogram starts empty
-    if constexpr (R < 3) {
-        if (b == 0) {
-            a.nb.hcnt[256 * (R + 1) + t] = 0u;
-            a.nb.hmass[256 * (R + 1) + t] = 0ull;
-        }
-    }
+    if constexpr (R < 2)
+        if (b == 0) nuc_clear(a.nb, R + 1, t);
     const NucState st = *a.nb.st;
     if (!st.need) return;
-    __shared__ uint32_t s_cnt[256];
-    __shared__ unsigned long long s_mass[256];
-    s_cnt[t] = 0u;
-    s_mass[t] = 0ull;
-    uint32_t prefix = 0u;
-    uint64_t above = 0ull;
-    bool some = true;
-    if constexpr (R > 0) some = nuc_prefix(a.nb, R, nuc_target(a, st.Z), prefix, above);
+    constexpr int PT = NUC_PER_BLOCK / 256;
+    // the thread's ids' logits (round 0) or keys, requested together ahead of the scan
+    const float* lr = a.logits + (size_t)st.row * a.V;
+    uint32_t key[PT];
+#pragma unroll
+    for (int i = 0; i < PT; ++i) {
+        const int v = min(b * NUC_PER_BLOCK + 256 * i + t, a.V - 1);
+        key[i] = R == 0 ? __float_as_uint(lr[v]) : a.nb.keys[v];
+    }
+    __shared__ uint32_t s_cnt[Dg::BINS];
+    __shared__ unsigned long long s_mass[Dg::BINS];
+#pragma unroll
+    for (int k = 0; k < Dg::BINS / 256; ++k) {
+        s_cnt[256 * k + t] = 0u;
+        s_mass[256 * k + t] = 0ull;
+    }
+    NucSel sel{0ull, 0u, 1};
+    if constexpr (R == 2) sel = a.nb.sel[0];
+    if constexpr (R > 0) {
+        if (sel.some) sel = nuc_scan<(R > 0 ? R - 1 : 0)>(a.nb, sel, nuc_target(a, st.Z));
+        if (b == 0 && t == 0) a.nb.sel[R - 1] = sel;
+    }
     __syncthreads();
-    if (!some) return;  // block-uniform: every key is kept
+    if (!sel.some) return;  // block-uniform: every key is kept
     const float mxs = a.rowmax[st.row] * a.invT;
 #pragma unroll
-    for (int i = 0; i < NUC_PER_BLOCK / 256; ++i) {
+    for (int i = 0; i < PT; ++i) {
         const int v = b * NUC_PER_BLOCK + 256 * i + t;
         if (v >= a.V) break;
-        uint32_t key;
         if constexpr (R == 0) {
-            key = __float_as_uint(e_at(a, st.row, v, mxs));
-            a.nb.keys[v] = key;
+            key[i] = __float_as_uint(e_of(a, __uint_as_float(key[i]), mxs));
+            a.nb.keys[v] = key[i];
         } else {
-            key = a.nb.keys[v];
-            if ((key >> (32 - 8 * R)) != prefix) continue;
+            if ((key[i] >> (Dg::SHIFT + Dg::BITS)) != sel.prefix) continue;
         }
-        const int d = (key >> (24 - 8 * R)) & 255;
+        const int d = (key[i] >> Dg::SHIFT) & (Dg::BINS - 1);
         atomicAdd(&s_cnt[d], 1u);
-        atomicAdd(&s_mass[d], (unsigned long long)nuc_fixed(__uint_as_float(key)));
+        atomicAdd(&s_mass[d], (unsigned long long)nuc_fixed(__uint_as_float(key[i])));
     }
     __syncthreads();
-    if (s_cnt[t] != 0u) {
-        atomicAdd(a.nb.hcnt + 256 * R + t, s_cnt[t]);
-        atomicAdd((unsigned long long*)(a.nb.hmass + 256 * R + t), s_mass[t]);
+#pragma unroll
+    for (int k = 0; k < Dg::BINS / 256; ++k) {
+        const int d = 256 * k + t;
+        if (s_cnt[d] != 0u) {
+            atomicAdd(a.nb.hcnt + Dg::OFF + d, s_cnt[d]);
+            atomicAdd((unsigned long long*)(a.nb.hmass + Dg::OFF + d), s_mass[d]);
+        }
+        if constexpr (R == 2) a.nb.hblk[Dg::BINS * b + d] = s_cnt[d];
     }
-    if constexpr (R == 3) a.nb.hblk[256 * b + t] = s_cnt[t];
 }
 
-// The cut (key and id), the kept mass in id order and the sample.
-__global__ __launch_bounds__(1024) void k_nucleus_pick(SampleArgs a) {
+// e of id v if the nucleus keeps it (a key above the cut, or the cut key up to the cut id), else 0
+__device__ __forceinline__ float nuc_kept(uint32_t k, int v, uint32_t ck, int cid) {
+    return (k > ck || (k == ck && v <= cid)) ? __uint_as_float(k) : 0.0f;
+}
+
+// The cut, and block sums of the kept e in the canonical order: one 256-thread block per 1024 ids
+// (chunks of CH by the first wave).  Every block finds the cut for itself.
+__global__ __launch_bounds__(256) void k_nucleus_sums(SampleArgs a) {
     if (aborted(a.abort)) return;
     a = resolve(a);
     const NucState st = *a.nb.st;
     if (!st.need) return;
-    __shared__ float cs[MAX_CHUNKS];
-    __shared__ float bs[MAX_CHUNKS / BLK];
-    __shared__ float s_f;
-    __shared__ int s_i;
-    __shared__ int s_wsum[16];
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    uint32_t ck = 0u;   // the cut key
-    int cid = a.V - 1;  // the cut id: with every key kept, the last
-    uint64_t above = 0ull;
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6, b = blockIdx.x;
+    const int nch = (a.V + CH - 1) / CH, chunk = b * BLK + t;
+    uint32_t k16[CH];  // the chunk's keys (clamped), requested ahead of the scan
+    if (t < BLK) {
+#pragma unroll
+        for (int k = 0; k < CH; ++k) k16[k] = a.nb.keys[min(chunk * CH + k, a.V - 1)];
+    }
+    using Dg = NucDigit<2>;
     const uint64_t F = nuc_target(a, st.Z);
-    if (nuc_prefix(a.nb, 4, F, ck, above)) {
+    NucSel sel = a.nb.sel[1];
+    if (sel.some) sel = nuc_scan<2>(a.nb, sel, F);  // (block-uniform)
+    uint32_t ck = 0u;   // the cut key
+    int cid = a.V - 1;  // the cut id: with every key (or every tie) kept, the last
+    if (sel.some) {
+        ck = sel.prefix;
         // ties of the cut key, in id order: j of them reach the target (at least one)
         const uint64_t m = nuc_fixed(__uint_as_float(ck));
-        const uint64_t need = F > above ? F - above : 0ull;
+        const uint64_t need = F > sel.above ? F - sel.above : 0ull;
         const int j = need == 0ull ? 1 : (int)((need + m - 1) / m);
-        // the block holding the j-th tie, and its rank there (every thread scans the counts)
-        const int d = ck & 255;
-        int b = 0, before = 0;
-        for (; b < NUC_BLOCKS; ++b) {
-            const int c = (int)a.nb.hblk[256 * b + d];
-            if (before + c >= j) break;
-            before += c;
-        }
-        const int jl = j - before;
-        // two ids a thread of that block's range, counted by a block-wide prefix
-        const int v0 = b * NUC_PER_BLOCK + 2 * t;
-        const bool h0 = v0 < a.V && a.nb.keys[v0] == ck;
-        const bool h1 = v0 + 1 < a.V && a.nb.keys[v0 + 1] == ck;
-        const int c = (int)h0 + (int)h1;
-        int incl = c;
+        const int d = ck & (Dg::BINS - 1);
+        if (j < (int)a.nb.hcnt[Dg::OFF + d]) {  // block-uniform
+            // the block of ids holding the j-th tie: running counts of the NUC_BLOCKS blocks
+            __shared__ int s_b[4], s_blk, s_before, s_id;
+            int c = t < NUC_BLOCKS ? (int)a.nb.hblk[Dg::BINS * t + d] : 0;
+            auto block_incl = [&](int v) {  // inclusive sum over the block's threads
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int y = __shfl_up(incl, o, MJ_WAVE);
-            if (lane >= o) incl += y;
-        }
-        if (lane == 63) s_wsum[wv] = incl;
-        __syncthreads();
-        int off = 0;
-        for (int w = 0; w < wv; ++w) off += s_wsum[w];
-        const int ex = off + incl - c;
-        if (c > 0 && ex < jl && jl <= ex + c) s_i = (h0 && ex + 1 == jl) ? v0 : v0 + 1;
-        __syncthreads();
-        cid = s_i;
-    }
-    const float mxs = a.rowmax[st.row] * a.invT;
-    const uint32_t* keys = a.nb.keys;
-    const auto kept = [&](int v) {
-        const uint32_t k = keys[v];
-        return (k > ck || (k == ck && v <= cid)) ? __uint_as_float(k) : 0.0f;
-    };
-    const float S = blk_sum(kept, a.V, cs, bs, &s_f);
-    int tok;
-    if (S > 0.0f) {
-        tok = blk_walk(kept, a.V, st.u * S, cs, bs, &s_i);
-    } else {  // the top-ranked token: the largest key, the lowest id among equal keys
-        uint32_t bk = 0u;
-        int bi = a.V;
-        for (int v = t; v < a.V; v += 1024) {
-            const uint32_t k = keys[v];
-            if (k > bk || (k == bk && v < bi)) {
-                bk = k;
-                bi = v;
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int y = __shfl_up(v, o, MJ_WAVE);
+                    if (lane >= o) v += y;
+                }
+                __syncthreads();
+                if (lane == 63) s_b[wv] = v;
+                __syncthreads();
+                for (int w = 0; w < wv; ++w) v += s_b[w];
+                return v;
+            };
+            int incl = block_incl(c);
+            if (c > 0 && incl - c < j && j <= incl) {
+                s_blk = t;
+                s_before = incl - c;
             }
-        }
-        if (t == 0) s_i = a.V;
-        __syncthreads();
-        for (int w = 0; w < 16; ++w) {  // fixed order: wave by wave through LDS
             __syncthreads();
-            if (wv == w) {
+            // the j-th tie in it: eight ids a thread
+            const int jl = j - s_before, v0 = s_blk * NUC_PER_BLOCK + 8 * t;
+            uint32_t eq = 0u;
 #pragma unroll
-                for (int o = 32; o > 0; o >>= 1) {
-                    const uint32_t ok = __shfl_xor(bk, o, MJ_WAVE);
-                    const int oi = __shfl_xor(bi, o, MJ_WAVE);
-                    if (ok > bk || (ok == bk && oi < bi)) {
-                        bk = ok;
-                        bi = oi;
-                    }
-                }
-                if (lane == 0) {
-                    const int pi = s_i;
-                    const uint32_t pk = pi < a.V ? keys[pi] : 0u;
-                    if (pi >= a.V || bk > pk || (bk == pk && bi < pi)) s_i = bi;
-                }
+            for (int k = 0; k < 8; ++k)
+                eq |= (uint32_t)(v0 + k < a.V && a.nb.keys[min(v0 + k, a.V - 1)] == ck) << k;
+            c = __popc(eq);
+            incl = block_incl(c);
+            if (c > 0 && incl - c < jl && jl <= incl) {
+                uint32_t e = eq;
+                for (int k = incl - c + 1; k < jl; ++k) e &= e - 1u;
+                s_id = v0 + __ffs(e) - 1;
             }
+            __syncthreads();
+            cid = s_id;
         }
-        __syncthreads();
-        tok = s_i < a.V ? s_i : 0;
     }
-    if (t < 64) write_result(a, st.acc, tok);
+    if (b == 0 && t == 0) *a.nb.cut = NucCut{ck, cid};
+    __shared__ float s[BLK];
+    if (t >= BLK) return;  // the first wave sums
+    float cs = 0.0f;
+#pragma unroll
+    for (int k = 0; k < CH; ++k)
+        if (chunk * CH + k < a.V) cs = cs + nuc_kept(k16[k], chunk * CH + k, ck, cid);
+    s[t] = chunk < nch ? cs : 0.0f;
+    __builtin_amdgcn_wave_barrier();
+    if (t == 0) {
+        float bs = 0.0f;
+        for (int c = 0; c < BLK; ++c)
+            if (b * BLK + c < nch) bs = bs + s[c];
+        a.rbs[b] = bs;
+    }
+}
+
+// The sample: a walk in id order to u * (kept mass), one 256-thread block.
+__global__ __launch_bounds__(256) void k_nucleus_pick(SampleArgs a) {
+    if (aborted(a.abort)) return;
+    a = resolve(a);
+    const NucState st = *a.nb.st;
+    if (!st.need) return;
+    const NucCut cut = *a.nb.cut;
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const uint32_t* keys = a.nb.keys;
+    __shared__ float s_S;
+    __shared__ float pref[MAX_CHUNKS / BLK];
+    stage_lds(pref, a.rbs, a.nblocks, t, 256);
+    __syncthreads();
+    if (t == 0) s_S = running_totals(pref, a.nblocks);
+    __syncthreads();
+    const float S = s_S;
+    if (S > 0.0f) {
+        walk_write(a, st.acc, st.u * S, pref, [&](int c, float x[CH]) {
+            uint32_t k16[CH];
+#pragma unroll
+            for (int k = 0; k < CH; ++k) k16[k] = keys[min(c * CH + k, a.V - 1)];
+            float sum = 0.0f;
+#pragma unroll
+            for (int k = 0; k < CH; ++k) {
+                x[k] = nuc_kept(k16[k], c * CH + k, cut.key, cut.id);
+                if (c * CH + k < a.V) sum = sum + x[k];
+            }
+            return sum;
+        });
+        return;
+    }
+    // no kept mass: the top-ranked token, the largest key, the lowest id among equal keys
+    __shared__ uint32_t s_k[4];
+    __shared__ int s_v[4];
+    uint32_t bk = 0u;
+    int bi = a.V;
+    for (int v = t; v < a.V; v += 256) {
+        const uint32_t k = keys[v];
+        if (k > bk || (k == bk && v < bi)) {
+            bk = k;
+            bi = v;
+        }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const uint32_t ok = __shfl_xor(bk, o, MJ_WAVE);
+        const int oi = __shfl_xor(bi, o, MJ_WAVE);
+        if (ok > bk || (ok == bk && oi < bi)) {
+            bk = ok;
+            bi = oi;
+        }
+    }
+    if (lane == 0) {
+        s_k[wv] = bk;
+        s_v[wv] = bi;
+    }
+    __syncthreads();
+    for (int w = 0; w < 4; ++w)
+        if (s_k[w] > bk || (s_k[w] == bk && s_v[w] < bi)) {
+            bk = s_k[w];
+            bi = s_v[w];
+        }
+    if (t < 64) write_result(a, st.acc, bi < a.V ? bi : 0);
 }
 
 static size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 size_t nucleus_bytes(int V) {
-    return up256((size_t)V * 4) + up256(4 * 256 * 4) + up256(4 * 256 * 8) +
-           up256((size_t)NUC_BLOCKS * 256 * 4) + up256(sizeof(NucState));
+    return up256((size_t)V * 4) + up256(3 * NUC_HBINS * 4) + up256(3 * NUC_HBINS * 8) +
+           up256((size_t)NUC_BLOCKS * NucDigit<2>::BINS * 4) + up256(sizeof(NucState)) +
+           up256(2 * sizeof(NucSel)) + up256(sizeof(NucCut));
 }
 
 void nucleus_layout(void* base, int V, NucleusBuf& nb) {
     char* p = (char*)base;
-    nb.keys = (uint32_t*)p;
-    p += up256((size_t)V * 4);
-    nb.hcnt = (uint32_t*)p;
-    p += up256(4 * 256 * 4);
-    nb.hmass = (uint64_t*)p;
-    p += up256(4 * 256 * 8);
-    nb.hblk = (uint32_t*)p;
-    p += up256((size_t)NUC_BLOCKS * 256 * 4);
-    nb.st = (NucState*)p;
+    auto take = [&](size_t n) {
+        char* q = p;
+        p += up256(n);
+        return (void*)q;
+    };
+    nb.keys = (uint32_t*)take((size_t)V * 4);
+    nb.hcnt = (uint32_t*)take(3 * NUC_HBINS * 4);
+    nb.hmass = (uint64_t*)take(3 * NUC_HBINS * 8);
+    nb.hblk = (uint32_t*)take((size_t)NUC_BLOCKS * NucDigit<2>::BINS * 4);
+    nb.st = (NucState*)take(sizeof(NucState));
+    nb.sel = (NucSel*)take(2 * sizeof(NucSel));
+    nb.cut = (NucCut*)take(sizeof(NucCut));
 }
 
 hipError_t launch_accept_sampled(float* logits, int rows, int V, const int32_t* draft,
@@ -874,10 +948,10 @@ hipError_t launch_accept_sampled(float* logits, int rows, int V, const int32_t* 
     hipLaunchKernelGGL(k_nucleus_round<0>, dim3(NUC_BLOCKS), dim3(256), 0, st, a);
     hipLaunchKernelGGL(k_nucleus_round<1>, dim3(NUC_BLOCKS), dim3(256), 0, st, a);
     hipLaunchKernelGGL(k_nucleus_round<2>, dim3(NUC_BLOCKS), dim3(256), 0, st, a);
-    hipLaunchKernelGGL(k_nucleus_round<3>, dim3(NUC_BLOCKS), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_nucleus_sums, dim3(a.nblocks), dim3(256), 0, st, a);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_nucleus_pick, dim3(1), dim3(1024), 0, st, a);
+    hipLaunchKernelGGL(k_nucleus_pick, dim3(1), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 
