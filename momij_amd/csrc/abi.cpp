@@ -172,6 +172,13 @@ mj_status mj_destroy(mj_ctx* ctx) {
     if (ctx->abort_dev) hipFree(ctx->abort_dev);
     if (ctx->abort_src) hipHostFree(ctx->abort_src);
     if (ctx->fault) hipHostFree(ctx->fault);
+    for (int k = 0; k < 2; ++k) {
+        if (ctx->hist_ev[k]) {
+            hipEventSynchronize(ctx->hist_ev[k]);
+            hipEventDestroy(ctx->hist_ev[k]);
+        }
+        if (ctx->hist_pin[k]) hipHostFree(ctx->hist_pin[k]);
+    }
     if (ctx->own) hipStreamDestroy(ctx->own);
     if (ctx->ctl) hipStreamDestroy(ctx->ctl);
     delete ctx;

@@ -829,6 +829,26 @@ hipError_t launch_accept_greedy(const int32_t* tokens, const int32_t* parents,
     return hipGetLastError();
 }
 
+__global__ __launch_bounds__(64) void k_accept_greedy_tree(const int32_t* tokens,
+                                                           TreeParents parents,
+                                                           const int32_t* argmax, int n,
+                                                           int32_t* out_flat, const int* abort) {
+    if (aborted(abort)) return;
+    const int lane = threadIdx.x;
+    const int tok = lane < n ? tokens[lane] : -1;
+    const int par = lane < n ? parents.p[lane] : -2;
+    const int am = lane < n ? argmax[lane] : -1;
+    accept_greedy_wave(tok, par, am, n, nullptr, out_flat);
+}
+
+hipError_t launch_accept_greedy_tree(const int32_t* tokens, const TreeParents& parents,
+                                     const int32_t* argmax, int n, int32_t* out_flat,
+                                     const int* abort, hipStream_t st) {
+    hipLaunchKernelGGL(k_accept_greedy_tree, dim3(1), dim3(64), 0, st, tokens, parents, argmax, n,
+                       out_flat, abort);
+    return hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------------------
 // KV commit: block per (layer, kv head).  Reads every accepted row first, then writes.
 // ---------------------------------------------------------------------------------------
@@ -938,17 +958,6 @@ hipError_t launch_embed_norm(const uint16_t* table, const StepDesc* sd, int M, i
                              hipStream_t st) {
     if (H != 2048 || rt.half > MJ_ROPE_F || M > MJ_ROWS) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_embed_norm, dim3(M), dim3(256), 0, st, table, sd, h, no, rt, abort);
-    return hipGetLastError();
-}
-
-__global__ __launch_bounds__(64) void k_rope_table(const StepDesc* sd, RopeTab rt) {
-    rope_row(sd, rt, blockIdx.x, threadIdx.x);
-}
-
-hipError_t launch_rope_table(const StepDesc* sd, int M, const RopeTab& rt, hipStream_t st) {
-    if (rt.half > MJ_ROPE_F || M > MJ_ROWS) return hipErrorInvalidValue;
-    if (rt.half == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_rope_table, dim3(M), dim3(64), 0, st, sd, rt);
     return hipGetLastError();
 }
 

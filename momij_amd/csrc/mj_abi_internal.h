@@ -35,6 +35,12 @@ struct mj_ctx {
     int wait_polls = 1 << 17;      // that bound (mj_set_wait_limit)
     void* scratch = nullptr;       // op-level scratch arena
     size_t scratch_bytes = 0;
+    // op-level sampled acceptance: pinned copies of a call's penalty history (at most MJ_MAX_HIST
+    // entries each), taken in turn, each with the event of its last upload
+    int32_t* hist_pin[2] = {};
+    size_t hist_cap[2] = {};
+    hipEvent_t hist_ev[2] = {};
+    int hist_at = 0;
     std::string err;
 };
 

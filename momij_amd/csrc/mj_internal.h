@@ -154,7 +154,7 @@ hipError_t launch_gather3(const GatherArgs& a, int epi, int rows, hipStream_t st
 
 // RoPE angles of a pass: rope_cs[r * MJ_ROPE_F + f] = {cos, sin} of (L + depth[r]) *
 // inv_freq[f] for row r and frequency f < rope_dim / 2, written by the pass's embedding kernel
-// (or k_rope_table) so that no layer evaluates a sine.
+// (or k_attn_front) so that no layer evaluates a sine.
 #define MJ_ROPE_F 64
 struct RopeTab {
     const float* inv_freq;  // [half]
@@ -183,6 +183,17 @@ struct AttnArgs {
 // attn.hip
 hipError_t launch_attn(const AttnArgs& a, hipStream_t st);
 int attn_max_chunks(int window, int64_t L_max, int M);
+
+// What one attention block call's first launch takes by value: the pass descriptor and the RoPE
+// frequencies (half = rope_dim / 2 of them).
+struct AttnFront {
+    StepDesc sd;
+    float inv_freq[MJ_ROPE_F];
+    int half;
+};
+hipError_t launch_attn_front(const AttnFront& f, const uint16_t* x, const uint16_t* w, float eps,
+                             uint16_t* xperm, float2* xsum, int rows, int H, StepDesc* sd,
+                             float2* cs, const int* abort, hipStream_t st);
 
 // head.hip
 // Optional per-row log-sum-exp of logits / T: k = log2(e) / T, block partials pm / ps
@@ -216,6 +227,13 @@ int head_blocks();
 hipError_t launch_accept_greedy(const int32_t* tokens, const int32_t* parents,
                                 const int32_t* argmax, int n, StepResult* res, int32_t* out_flat,
                                 const int* abort, hipStream_t st);
+// the same with the tree by value (nothing to upload)
+struct TreeParents {
+    int32_t p[MJ_ROWS];
+};
+hipError_t launch_accept_greedy_tree(const int32_t* tokens, const TreeParents& parents,
+                                     const int32_t* argmax, int n, int32_t* out_flat,
+                                     const int* abort, hipStream_t st);
 hipError_t launch_kv_commit(uint16_t* kv, int64_t layer_stride, int n_layers, int64_t C, int nKV,
                             const StepDesc* sd, const StepResult* res, const int* abort,
                             hipStream_t st);
@@ -227,7 +245,6 @@ hipError_t launch_embed(const uint16_t* table, const StepDesc* sd, int M, int H,
 hipError_t launch_embed_norm(const uint16_t* table, const StepDesc* sd, int M, int H, uint16_t* h,
                              const NormOut& no, const RopeTab& rt, const int* abort,
                              hipStream_t st);  // H = 2048
-hipError_t launch_rope_table(const StepDesc* sd, int M, const RopeTab& rt, hipStream_t st);
 // One wave that waits `us` microseconds of wall-clock time (bounded), so that the host can
 // queue the launches that follow it before the GPU reaches them.
 hipError_t launch_hold(unsigned us, hipStream_t st);

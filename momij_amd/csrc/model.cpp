@@ -826,18 +826,18 @@ mj_status mj_attn_block(mj_ctx* ctx, const mj_attn_config* cfg, const mj_attn_we
     hipSetDevice(ctx->device);
     mj_status s = mj_hip(ctx, set_kernel_attributes(), "kernel attributes");
     if (s != MJ_OK) return s;
-    StepDesc sd{};
-    sd.L = L;
-    sd.M = M;
-    s = fill_tree(ctx, &sd, parents_host, M);
+    AttnFront front{};
+    front.sd.L = L;
+    front.sd.M = M;
+    s = fill_tree(ctx, &front.sd, parents_host, M);
     if (s != MJ_OK) return s;
+    front.half = c.rope_dim / 2;
+    for (int i = 0; i < front.half; ++i)
+        front.inv_freq[i] = powf(c.rope_base, -(float)i / (float)front.half);
     const int H = c.H, nQ = c.n_heads, nKV = c.n_kv_heads;
     const int qkvN = (nQ + 2 * nKV) * 128;
     const int maxc = attn_max_chunks(c.window, L, M);
     const int nqt16 = ((M * (nQ / nKV) + 15) / 16) * 16;
-    std::vector<float> inv(c.rope_dim > 0 ? c.rope_dim / 2 : 1, 1.0f);
-    for (int i = 0; c.rope_dim > 0 && i < c.rope_dim / 2; ++i)
-        inv[i] = powf(c.rope_base, -(float)i / (float)(c.rope_dim / 2));
     auto layout = [&](Arena& a, void** p) {
         p[0] = a.take((size_t)M * H * 2);                 // xperm
         p[1] = a.take((size_t)M * (H / 64) * 8);          // xsum
@@ -848,9 +848,8 @@ mj_status mj_attn_block(mj_ctx* ctx, const mj_attn_config* cfg, const mj_attn_we
         p[6] = a.take((size_t)M * nQ * 128 * 2);          // aperm
         p[7] = a.take((size_t)M * nQ * 2 * 8);            // asum
         p[8] = a.take(sizeof(StepDesc));
-        p[9] = a.take(inv.size() * 4);
     };
-    void* p[10];
+    void* p[9];
     Arena count;
     layout(count, p);
     s = mj_scratch_reserve(ctx, count.off);
@@ -858,15 +857,10 @@ mj_status mj_attn_block(mj_ctx* ctx, const mj_attn_config* cfg, const mj_attn_we
     Arena real{ctx->scratch, 0};
     layout(real, p);
     hipStream_t st = ctx->stream;
-    s = mj_hip(ctx, hipMemcpyAsync(p[8], &sd, sizeof sd, hipMemcpyHostToDevice, st), "sd upload");
-    if (s == MJ_OK)
-        s = mj_hip(ctx, hipMemcpyAsync(p[9], inv.data(), inv.size() * 4, hipMemcpyHostToDevice, st),
-                   "inv_freq upload");
-    if (s == MJ_OK) s = mj_hip(ctx, hipStreamSynchronize(st), "upload sync");
-    if (s != MJ_OK) return s;
     const int* ab = ctx->abort_dev;
-    s = mj_hip(ctx, launch_rmsnorm_qx((const uint16_t*)h, (const uint16_t*)w->norm_w, c.eps,
-                                      nullptr, (uint16_t*)p[0], (float2*)p[1], M, H, ab, st),
+    s = mj_hip(ctx, launch_attn_front(front, (const uint16_t*)h, (const uint16_t*)w->norm_w, c.eps,
+                                      (uint16_t*)p[0], (float2*)p[1], M, H, (StepDesc*)p[8],
+                                      (float2*)p[3], ab, st),
                "attn norm");
     if (s != MJ_OK) return s;
     GatherArgs q{};
@@ -882,9 +876,6 @@ mj_status mj_attn_block(mj_ctx* ctx, const mj_attn_config* cfg, const mj_attn_we
     q.gs = c.gs;
     q.x_div = 1;
     q.abort = ab;
-    const RopeTab rt{(const float*)p[9], (float2*)p[3], c.rope_dim / 2};
-    s = mj_hip(ctx, launch_rope_table((const StepDesc*)p[8], M, rt, st), "rope table");
-    if (s != MJ_OK) return s;
     s = mj_hip(ctx, launch_gather(q, EPI_STORE, M, 1, st), "qkv");
     if (s != MJ_OK) return s;
     AttnArgs a{};
@@ -1027,16 +1018,40 @@ mj_status mj_accept_greedy(mj_ctx* ctx, const int32_t* tokens, const int32_t* pa
     StepDesc sd{};
     mj_status s = fill_tree(ctx, &sd, parents_host, n_rows);
     if (s != MJ_OK) return s;
-    s = mj_scratch_reserve(ctx, MJ_MAX_ROWS * 4 + 256);
-    if (s != MJ_OK) return s;
     hipSetDevice(ctx->device);
-    int32_t* pdev = (int32_t*)ctx->scratch;
-    s = mj_hip(ctx, hipMemcpyAsync(pdev, sd.parents, n_rows * 4, hipMemcpyHostToDevice,
-                                   ctx->stream), "parents upload");
-    if (s == MJ_OK) s = mj_hip(ctx, hipStreamSynchronize(ctx->stream), "upload sync");
+    TreeParents tp;
+    std::memcpy(tp.p, sd.parents, sizeof tp.p);
+    return mj_hip(ctx, launch_accept_greedy_tree(tokens, tp, argmax, n_rows, out, ctx->abort_dev,
+                                                 ctx->stream), "accept greedy");
+}
+
+// Pinned room for n words of a call's penalty history, free to write: two buffers in turn, each
+// behind the event of its last copy, so a call does not wait for its own upload (the copy, its wait
+// and the gap it left took 12 us of a 9-row acceptance).
+static mj_status mj_hist_stage(mj_ctx* ctx, size_t n, int32_t** out) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    mj_status s = mj_hip(ctx, hipStreamIsCapturing(ctx->stream, &cs), "history");
     if (s != MJ_OK) return s;
-    return mj_hip(ctx, launch_accept_greedy(tokens, pdev, argmax, n_rows, nullptr, out,
-                                            ctx->abort_dev, ctx->stream), "accept greedy");
+    if (cs != hipStreamCaptureStatusNone)  // a replay would upload whatever the buffer holds then
+        return mj_fail(ctx, MJ_HIP_ERROR, "accept_sampled: a penalty history cannot be captured");
+    const int k = ctx->hist_at = 1 - ctx->hist_at;
+    if (!ctx->hist_ev[k]) {
+        s = mj_hip(ctx, hipEventCreateWithFlags(&ctx->hist_ev[k], hipEventDisableTiming), "history");
+        if (s != MJ_OK) return s;
+    } else {
+        s = mj_hip(ctx, hipEventSynchronize(ctx->hist_ev[k]), "history");
+        if (s != MJ_OK) return s;
+    }
+    if (ctx->hist_cap[k] < n) {
+        if (ctx->hist_pin[k]) hipHostFree(ctx->hist_pin[k]);
+        ctx->hist_pin[k] = nullptr;
+        ctx->hist_cap[k] = 0;
+        s = mj_hip(ctx, hipHostMalloc(&ctx->hist_pin[k], n * 4, hipHostMallocDefault), "history");
+        if (s != MJ_OK) return s;
+        ctx->hist_cap[k] = n;
+    }
+    *out = ctx->hist_pin[k];
+    return MJ_OK;
 }
 
 mj_status mj_accept_sampled_ex(mj_ctx* ctx, const float* logits, int rows, int V,
@@ -1061,8 +1076,8 @@ mj_status mj_accept_sampled_ex(mj_ctx* ctx, const float* logits, int rows, int V
         *rowmax = (float*)a.take((size_t)rows * 4);
         *bsum = (float*)a.take(sample_scratch_floats(rows, V) * 4);
         *lcopy = pen ? (float*)a.take((size_t)rows * V * 4) : nullptr;
-        *dt = (int32_t*)a.take((size_t)ht.size() * 4 + 4);
-        *dc = (int32_t*)a.take((size_t)hc.size() * 4 + 4);
+        *dt = (int32_t*)a.take(2 * ht.size() * 4 + 4);  // the tokens, then their counts
+        *dc = *dt ? *dt + ht.size() : nullptr;
         *nbase = nucleus ? a.take(nucleus_bytes(V)) : nullptr;
     };
     float *rowmax, *bsum, *lcopy;
@@ -1084,12 +1099,14 @@ mj_status mj_accept_sampled_ex(mj_ctx* ctx, const float* logits, int rows, int V
         lg = lcopy;
     }
     if (!ht.empty()) {
-        s = mj_hip(ctx, hipMemcpyAsync(dt, ht.data(), ht.size() * 4, hipMemcpyHostToDevice, st),
+        int32_t* stage = nullptr;
+        s = mj_hist_stage(ctx, 2 * ht.size(), &stage);
+        if (s != MJ_OK) return s;
+        std::memcpy(stage, ht.data(), ht.size() * 4);
+        std::memcpy(stage + ht.size(), hc.data(), hc.size() * 4);
+        s = mj_hip(ctx, hipMemcpyAsync(dt, stage, 2 * ht.size() * 4, hipMemcpyHostToDevice, st),
                    "history");
-        if (s == MJ_OK)
-            s = mj_hip(ctx, hipMemcpyAsync(dc, hc.data(), hc.size() * 4, hipMemcpyHostToDevice,
-                                           st), "history");
-        if (s == MJ_OK) s = mj_hip(ctx, hipStreamSynchronize(st), "history upload");
+        if (s == MJ_OK) s = mj_hip(ctx, hipEventRecord(ctx->hist_ev[ctx->hist_at], st), "history");
         if (s != MJ_OK) return s;
     }
     o.hist_tok = dt;

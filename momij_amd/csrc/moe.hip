@@ -15,11 +15,10 @@
 #include "moe_topk.h"
 
 // One 256-thread block per row; H % 2048 == 0, H <= 8192.
-__global__ __launch_bounds__(256) void k_rmsnorm_qx(const uint16_t* __restrict__ x,
-                                                    const uint16_t* __restrict__ w, float eps,
-                                                    uint16_t* out_plain, uint16_t* xperm,
-                                                    float2* xsum, int H, const int* abort) {
-    if (aborted(abort)) return;
+__device__ __forceinline__ void rmsnorm_qx_row(const uint16_t* __restrict__ x,
+                                               const uint16_t* __restrict__ w, float eps,
+                                               uint16_t* out_plain, uint16_t* xperm,
+                                               float2* xsum, int H) {
     const int row = blockIdx.x, t = threadIdx.x, lane = t & 63;
     const uint16_t* xr = x + (size_t)row * H;
     const int nch = H / 2048;
@@ -57,6 +56,44 @@ __global__ __launch_bounds__(256) void k_rmsnorm_qx(const uint16_t* __restrict__
         if (out_plain) *(u4v*)(out_plain + (size_t)row * H + k0) = o;
         if (xperm) emit_qx(o, lane, xperm + (size_t)row * H, xsum + (size_t)row * (H / 64), k0);
     }
+}
+
+__global__ __launch_bounds__(256) void k_rmsnorm_qx(const uint16_t* __restrict__ x,
+                                                    const uint16_t* __restrict__ w, float eps,
+                                                    uint16_t* out_plain, uint16_t* xperm,
+                                                    float2* xsum, int H, const int* abort) {
+    if (aborted(abort)) return;
+    rmsnorm_qx_row(x, w, eps, out_plain, xperm, xsum, H);
+}
+
+// The front of one attention block call: the input norm of its rows, their RoPE angles, and the
+// pass descriptor, which comes as a kernel argument.  One launch, with nothing to upload: two
+// copies, the wait for them, the norm and the table as launches of their own took 30 us of a
+// 9-row block's 56.
+__global__ __launch_bounds__(256) void k_attn_front(AttnFront f, const uint16_t* __restrict__ x,
+                                                    const uint16_t* __restrict__ w, float eps,
+                                                    uint16_t* xperm, float2* xsum, int H,
+                                                    StepDesc* sd, float2* cs, const int* abort) {
+    const int r = blockIdx.x, t = threadIdx.x;
+    static_assert(sizeof(StepDesc) % 8 == 0, "copied in 8-byte words");
+    if (r == 0)
+        for (int i = t; i < (int)(sizeof(StepDesc) / 8); i += 256)
+            ((uint64_t*)sd)[i] = ((const uint64_t*)&f.sd)[i];
+    if (t < f.half) {
+        const float th = (float)(f.sd.L + f.sd.depth[r]) * f.inv_freq[t];
+        cs[r * MJ_ROPE_F + t] = make_float2(cosf(th), sinf(th));
+    }
+    if (aborted(abort)) return;
+    rmsnorm_qx_row(x, w, eps, nullptr, xperm, xsum, H);
+}
+
+hipError_t launch_attn_front(const AttnFront& f, const uint16_t* x, const uint16_t* w, float eps,
+                             uint16_t* xperm, float2* xsum, int rows, int H, StepDesc* sd,
+                             float2* cs, const int* abort, hipStream_t st) {
+    if (rows < 1 || rows > MJ_ROWS || f.half > MJ_ROPE_F) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_attn_front, dim3(rows), dim3(256), 0, st, f, x, w, eps, xperm, xsum, H, sd,
+                       cs, abort);
+    return hipGetLastError();
 }
 
 hipError_t launch_rmsnorm_qx(const uint16_t* x, const uint16_t* w, float eps, uint16_t* out_plain,
