@@ -17,6 +17,8 @@
 //                   (K finished, V as projected) at slot (L + r) % C.
 // k_attn_combine    merges the chunk partials per (row, head) and writes the output in the qx
 //                   format consumed by the o-projection.
+#include <algorithm>
+
 #include "mj_device.h"
 #include "mj_internal.h"
 
@@ -52,6 +54,36 @@ int attn_max_chunks(int window, int64_t L_max, int M) {
     // position-aligned chunks: one more than the keys span, one for a tree's own rows
     const int64_t keys = (window > 0 ? (int64_t)window - 1 : L_max) + M;
     return (int)((keys + AK - 1) / AK) + 2;
+}
+
+// Groups of AG chunks, by absolute chunk index (a tree's own chunks are a group after them).  A
+// group's partial is its chunks merged in increasing order (merge_part), whether one block
+// computed them all or the combine merges the chunks of several: a row's result does not depend on
+// which.
+#define AG 4
+__host__ __device__ inline int group_count(const ChunkGeom& g) {
+    return (g.n_abs > 0 ? (int)((g.c0 + g.n_abs - 1) / AG - g.c0 / AG + 1) : 0) +
+           (g.nch > g.n_abs ? 1 : 0);
+}
+// chunks cb .. ce - 1 of group j (none past the last group)
+__device__ __forceinline__ void group_chunks(const ChunkGeom& g, int j, int& cb, int& ce) {
+    const int64_t a0 = (g.c0 / AG + j) * AG - g.c0;  // first chunk of the group, may be < 0
+    cb = a0 < 0 ? 0 : (int)a0;
+    ce = (int)(a0 + AG < g.n_abs ? a0 + AG : g.n_abs);
+    if (a0 >= g.n_abs) {  // past the chunks placed by position
+        const bool own = j == group_count(g) - 1 && g.nch > g.n_abs;
+        cb = own ? g.n_abs : g.nch;
+        ce = g.nch;
+    }
+}
+// Weights of the merge of a further part (maximum m) into a running one (mg): the new maximum
+// replaces mg, the running sums scale by fa, the part's by fb.  Empty parts (-inf) leave exact
+// values alone.
+__device__ __forceinline__ void merge_part(float& mg, float m, float& fa, float& fb) {
+    const float mn = fmaxf(mg, m);
+    fa = mg == mn ? 1.0f : __builtin_amdgcn_exp2f(mg - mn);
+    fb = m == mn ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+    mg = mn;
 }
 
 // DPP lane moves (no LDS round trip): quad_perm [1,0,3,2] (xor 1) 0xB1, [2,3,0,1] (xor 2)
@@ -160,51 +192,55 @@ __host__ __device__ inline int tab_floats2(int M, int half) {
 }
 // HALF: rope_dim / 2 (0: no RoPE).  JR: finishing jobs (8 a vector) a thread requests before the
 // first barrier; jobs past 256 JR go in further rounds, each a dependent load round trip, so
-// passes with more vectors (a 17-row tree: 680 jobs) take JR = 3 and one round.
-// NT: threads of a block, 256 or 512.  The K / V staging takes threads 0 .. 255; a pass of more
-// than four query tiles (a 17-row tree: five) runs 512 threads, so that no wave takes two tiles
-// and the finishing jobs spread over twice the threads.
-template <int HALF, int JR, int NT>
-__global__ __launch_bounds__(NT) void k_attn_chunk(AttnArgs a) {
-    static_assert(NT == 256 || NT == 512, "block size");
-    constexpr int NW = NT / 64;  // waves
+// passes with more of them take JR = 3.
+// CG: chunks a block takes, 1, or AG (the chunks of a group in turn, the next one's K and V
+// requested before the current one's products; the block's tiles are then at most one a wave).
+template <int HALF, int JR, int CG>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_attn_chunk(AttnArgs a) {
+    constexpr int NT = 256;
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    const bool kvt = NT == 256 || t < 256;  // stages K / V (wave-uniform)
-    const int tk = t & 255;
-    const int g = blockIdx.x / a.max_chunks, c = blockIdx.x % a.max_chunks;
+    const int g = blockIdx.x / a.parts, part = blockIdx.x % a.parts;
     const StepDesc* sd = a.sd;
     const int64_t L = sd->L;
     const int M = a.M;
     const int gqa = a.nQ / a.nKV;
-    const int nqv = M * gqa, nqt = (nqv + 15) / 16;
+    // the block's query vectors qv0 .. qv0 + nqv - 1: tpp tiles of 16 a block
+    const int qv0 = 16 * a.tpp * blockIdx.y, nqt_all = (M * gqa + 15) / 16;
+    const int nqt = min(a.tpp, nqt_all - a.tpp * (int)blockIdx.y);
+    const int nqv = min(16 * nqt, M * gqa - qv0);
     const int qkvN = (a.nQ + 2 * a.nKV) * HD;
     constexpr int half = HALF;
     const ChunkGeom cg = chunk_geom(a.window, L, M, sd->chain != 0);
-    // ring slot of position p (p - L is within the cache: |p - L| < C)
-    const int64_t Lm = L % a.C;
-    auto slot_of = [&](int64_t p) -> int64_t {
-        int64_t sl = Lm + (p - L);
-        sl += sl < 0 ? a.C : 0;
-        sl -= sl >= a.C ? a.C : 0;
+    int c = part, ce = part + 1;
+    if constexpr (CG > 1) group_chunks(cg, part, c, ce);
+    if (c >= cg.nch) return;  // whole block
+    // Positions are taken relative to L, in 32 bits (|p - L| < C < 2^23).  Key lane k of the
+    // current chunk sits at rel = crel + k (chunks placed by position) and is of class -2 none,
+    // -1 committed, else own row (its index); all by selects, no branches.
+    const int C = (int)a.C, lo = (int)(cg.lo - L), hi = (int)(cg.hi - L);
+    const int Lm = (int)((uint64_t)L >> 32 ? L % a.C : (int64_t)((uint32_t)L % (uint32_t)C));
+    bool by_pos = true, own_chunk = false;
+    int crel = 0, arow = 0;  // rel of lane 0; own row of lane 0 (a tree's chunks)
+    auto set_chunk = [&]() {
+        by_pos = c < cg.n_abs;
+        crel = by_pos ? (int)((cg.c0 + c) * AK - L) : 0;
+        arow = (c - cg.n_abs) * AK;
+        // the pass's own rows fall in the current chunk
+        own_chunk = by_pos ? crel + AK - 1 >= 0 && crel <= hi : true;
+    };
+    set_chunk();
+    auto slot_of = [&](int rel) -> int {  // ring slot
+        int sl = Lm + rel;
+        sl += sl < 0 ? C : 0;
+        sl -= sl >= C ? C : 0;
         return sl;
     };
-    if (c >= cg.nch) return;  // whole block
-    const bool by_pos = c < cg.n_abs;
-    const int64_t cpos = (cg.c0 + c) * AK;  // position of key lane 0 (chunks placed by position)
-    // key lane k of this chunk: -2 none, -1 committed (at position p), else own row (its
-    // index; its position is L + depth[row])
-    auto key_of = [&](int k, int64_t& p) -> int {
-        if (by_pos) {
-            p = cpos + k;
-            if (p < cg.lo || p > cg.hi) return -2;
-            return p < L ? -1 : (int)(p - L);
-        }
-        p = 0;
-        const int ar = (c - cg.n_abs) * AK + k;
-        return ar < M ? ar : -2;
+    auto key_of = [&](int k) -> int {
+        const int rel = crel + k, ar = arow + k;
+        const int cp = (rel < lo) | (rel > hi) ? -2 : rel < 0 ? -1 : rel;
+        const int ct = ar < M ? ar : -2;
+        return by_pos ? cp : ct;
     };
-    // the pass's own rows fall in this block's chunk
-    const bool own_chunk = by_pos ? cpos + AK - 1 >= L && cpos <= cg.hi : true;
 
     extern __shared__ uint16_t lds[];
     uint16_t* Qs = lds;                          // [nqt*16][QSTR]
@@ -218,65 +254,67 @@ __global__ __launch_bounds__(NT) void k_attn_chunk(AttnArgs a) {
     uint16_t* knw_s = qnw_s + HD;                  // [HD] k norm weights
     int* s_abort = (int*)(knw_s + HD);
 
-    // ---- K: key kk = tk / 4, dims 32 dq ..
-    const int kk = tk >> 2, dq = tk & 3;
-    int64_t kp;
-    const int kcls = key_of(kk, kp);
-    const bool kvalid = kcls != -2;
-    const bool kown = kcls >= 0;
-    const int ar = kown ? kcls : 0;  // pass row of an own key
-    u4v kv[4];
-    if (kvt) {
-        const int64_t slot = kvalid && !kown ? slot_of(kp) : 0;
-        const uint16_t* ks = kown ? a.qkv + (size_t)ar * qkvN + (a.nQ + g) * HD + 32 * dq
-                                  : a.kc + ((size_t)g * a.C + slot) * HD + 32 * dq;
+    // ---- K: key kk = t / 4, dims 32 dq ..;  V: keys 4 vg .. 4 vg + 3, dims 8 vd ..
+    const int kk = t >> 2, dq = t & 3;
+    const int vg = t & 15, vd = t >> 4;
+    u4v kv[4], vv[4];
+    int kcls = -2, vcls[4];
+    // each 8-dim part from the projection (own rows) or the cache, at clamped slots
+    auto src_of = [&](int cls, int k, const uint16_t* own, const uint16_t* cache) {
+        const int sl = cls == -1 ? slot_of(crel + k) : 0;
+        const uint32_t off = cls >= 0 ? (uint32_t)(cls * qkvN) : (uint32_t)(sl * HD);
+        return (cls >= 0 ? own : cache) + off;
+    };
+    const uint16_t* const kown = a.qkv + (a.nQ + g) * HD;
+    const uint16_t* const vown = kown + a.nKV * HD;
+    const uint16_t* const kcg = a.kc + (size_t)g * a.C * HD;
+    const uint16_t* const vcg = a.vc + (size_t)g * a.C * HD;
+    auto request_kv = [&]() {
+        kcls = key_of(kk);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) vcls[j] = key_of(4 * vg + j);
+        const uint16_t* ks = src_of(kcls, kk, kown, kcg) + 32 * dq;
 #pragma unroll
         for (int q = 0; q < 4; ++q) kv[q] = *(const u4v*)(ks + 8 * q);
-    }
-    // ---- V: keys 4 vg .. 4 vg + 3, dims 8 vd ..
-    const int vg = tk & 15, vd = tk >> 4;
-    u4v vv[4];
-    int vcls[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        int64_t p;
-        vcls[j] = key_of(4 * vg + j, p);
-        const int64_t slot = vcls[j] == -1 ? slot_of(p) : 0;
-        const uint16_t* vs =
-            vcls[j] >= 0 ? a.qkv + (size_t)vcls[j] * qkvN + (a.nQ + a.nKV + g) * HD + 8 * vd
-                         : a.vc + ((size_t)g * a.C + slot) * HD + 8 * vd;
-        if (kvt) vv[j] = *(const u4v*)vs;
-    }
+        for (int j = 0; j < 4; ++j)
+            vv[j] = *(const u4v*)(src_of(vcls[j], 4 * vg + j, vown, vcg) + 8 * vd);
+    };
+    request_kv();
     // ---- vectors to finish (RMSNorm + RoPE): the block's queries (vector qv = r * gqa + j is
     // head g * gqa + j of row r) and the pass's own keys in this chunk (lanes ko0 .. ko1 - 1).
     // Job jb of a vector holds its parts pa and pa + X (8 dims each; X = half / 8 parts apart,
     // so a rotated pair of dims sits in one thread), 8 jobs a vector in 8 consecutive threads.
     constexpr int X = HALF >= 16 ? HALF / 8 : 8;
-    int ko0 = 0, ko1 = 0;
-    if (own_chunk) {
-        ko0 = by_pos ? (int)(L - cpos > 0 ? L - cpos : 0) : 0;
-        ko1 = by_pos ? (int)(cg.hi - cpos + 1 < AK ? cg.hi - cpos + 1 : AK)
-                     : (M - (c - cg.n_abs) * AK < AK ? M - (c - cg.n_abs) * AK : AK);
-    }
-    const int njobs = 8 * (nqv + ko1 - ko0);
+    // (nqj: queries among the jobs -- all of the block's with its first chunk, none later)
+    int ko0 = 0, ko1 = 0, njobs = 0, nqj = nqv;
     u4v jxa[JR], jxb[JR];
     auto job_src = [&](int j, int& pa) -> const uint16_t* {
         const int vi = j >> 3, jb = j & 7;
         pa = (jb & (X - 1)) | ((jb & ~(X - 1)) << 1);
-        if (vi < nqv)
-            return a.qkv + (size_t)(vi / gqa) * qkvN + (g * gqa + vi % gqa) * HD;
-        int64_t p;
-        const int r2 = key_of(ko0 + vi - nqv, p);
-        return a.qkv + (size_t)(r2 >= 0 ? r2 : 0) * qkvN + (a.nQ + g) * HD;
+        const bool isq = vi < nqj;
+        const int r2 = max(key_of(ko0 + vi - nqj), 0);
+        const int qr = (qv0 + vi) / gqa, qh = g * gqa + (qv0 + vi) - qr * gqa;
+        return a.qkv + (uint32_t)((isq ? qr : r2) * qkvN + (isq ? qh : a.nQ + g) * HD);
     };
+    auto request_jobs = [&]() {
+        ko0 = ko1 = 0;
+        if (own_chunk) {
+            ko0 = by_pos ? max(-crel, 0) : 0;
+            ko1 = min(by_pos ? hi - crel + 1 : M - arow, AK);
+        }
+        njobs = 8 * (nqj + ko1 - ko0);
+        if (CG > 1 && njobs == 0) return;
 #pragma unroll
-    for (int jj = 0; jj < JR; ++jj) {
-        const int j = t + NT * jj;
-        int pa;
-        const uint16_t* src = job_src(j < njobs ? j : njobs - 1, pa);
-        jxa[jj] = *(const u4v*)(src + 8 * pa);
-        jxb[jj] = *(const u4v*)(src + 8 * (pa + X));
-    }
+        for (int jj = 0; jj < JR; ++jj) {
+            const int j = t + NT * jj;
+            int pa;
+            const uint16_t* src = job_src(j < njobs ? j : njobs - 1, pa);
+            jxa[jj] = *(const u4v*)(src + 8 * pa);
+            jxb[jj] = *(const u4v*)(src + 8 * (pa + X));
+        }
+    };
+    request_jobs();
     // the norm weights into LDS (16 lanes each of wave 0)
     if (wv == 0 && lane < HD / 8) {
         __builtin_amdgcn_global_load_lds(a.q_norm_w + 8 * lane,
@@ -295,8 +333,6 @@ __global__ __launch_bounds__(NT) void k_attn_chunk(AttnArgs a) {
                                              (__attribute__((address_space(3))) void*)(tab + 2 * e0),
                                              16, 0, 0);
     }
-    int64_t mpos;
-    const int mcls = key_of(t & (AK - 1), mpos);  // -2 invalid, -1 committed, >= 0 own row
     const int rdep = sd->depth[t < M ? t : M - 1];
     const uint64_t ranc_t = sd->anc[t < M ? t : M - 1];
     const int abort_v = a.abort ? *a.abort : 0;  // thread 0's copy decides for the block
@@ -305,32 +341,54 @@ __global__ __launch_bounds__(NT) void k_attn_chunk(AttnArgs a) {
     // rows of the last tile (read by the MFMAs, masked after) are cleared
     for (int i = nqv * 16 + t; i < nqt * 16 * 16; i += NT)
         *(u4v*)(Qs + (i >> 4) * QSTR + 8 * (i & 15)) = (u4v){0u, 0u, 0u, 0u};
-    if (kvt) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            *(u4v*)(Ks + kk * QSTR + 32 * dq + 8 * q) = kvalid ? kv[q] : (u4v){0u, 0u, 0u, 0u};
-        u4v w[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) w[j] = vcls[j] != -2 ? vv[j] : (u4v){0u, 0u, 0u, 0u};
-        // dim 8 vd + i of keys 4 vg .. + 3: halves i of the four key vectors
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int sh = 16 * (i & 1);
-            const uint32_t a0 = (w[0][i >> 1] >> sh) & 0xFFFFu, a1 = (w[1][i >> 1] >> sh) & 0xFFFFu;
-            const uint32_t a2 = (w[2][i >> 1] >> sh) & 0xFFFFu, a3 = (w[3][i >> 1] >> sh) & 0xFFFFu;
-            *(uint2*)(Vt + (8 * vd + i) * VSTR + 4 * vg) = make_uint2(a0 | (a1 << 16), a2 | (a3 << 16));
-        }
-    }
-    if (t < AK) {
-        // position - L: p - L in chunks placed by position, depth[row] for a tree's own rows
-        const int64_t rel = by_pos ? mpos - L : (int64_t)sd->depth[mcls >= 0 ? mcls : 0];
-        kmeta[t] = mcls == -2 ? (int)0x80000000 : (int)rel * 128 + (mcls + 2);
-    }
     if (t < M) {
         rlo[t] = a.window > 0 ? rdep - a.window + 1 : INT32_MIN / 2;
         ranc[t] = ranc_t;
     }
     if (t == 0) *s_abort = abort_v;
+    const float sc2 = a.scale * LOG2E;
+    const int ln = lane & 15, lq = lane >> 4;
+    // the group's partial so far (CG > 1): maximum and sum of query vector ln, outputs as O below
+    float mg = -INFINITY, lg = 0.0f;
+    f4 og[CG > 1 ? 8 : 1];
+#pragma unroll
+    for (int dt = 0; dt < (CG > 1 ? 8 : 1); ++dt) og[dt] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+    // partial `part` of query vector tile qt: lane (d, lq) holds query vectors 16 qt + 4 lq + r,
+    // dim 16 dt + d
+    auto write_part = [&](int qt, const f4* O, float m, float l) {
+        const size_t pbase =
+            ((size_t)g * a.max_chunks + part) * (size_t)(nqt_all * 16) + qv0 + qt * 16;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float* op = a.opart + (pbase + 4 * lq + r) * HD;
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt) op[16 * dt + ln] = O[dt][r];
+        }
+        if (lq == 0) a.mlpart[pbase + ln] = make_float2(m, l);
+    };
+
+  for (;;) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        *(u4v*)(Ks + kk * QSTR + 32 * dq + 8 * q) = kcls != -2 ? kv[q] : (u4v){0u, 0u, 0u, 0u};
+    u4v w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = vcls[j] != -2 ? vv[j] : (u4v){0u, 0u, 0u, 0u};
+    // dim 8 vd + i of keys 4 vg .. + 3: halves i of the four key vectors
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int sh = 16 * (i & 1);
+        const uint32_t a0 = (w[0][i >> 1] >> sh) & 0xFFFFu, a1 = (w[1][i >> 1] >> sh) & 0xFFFFu;
+        const uint32_t a2 = (w[2][i >> 1] >> sh) & 0xFFFFu, a3 = (w[3][i >> 1] >> sh) & 0xFFFFu;
+        *(uint2*)(Vt + (8 * vd + i) * VSTR + 4 * vg) = make_uint2(a0 | (a1 << 16), a2 | (a3 << 16));
+    }
+    if (t < AK) {
+        const int mcls = key_of(t);
+        // position - L: p - L in chunks placed by position, depth[row] for a tree's own rows
+        int rel = crel + t;
+        if (!by_pos) rel = sd->depth[mcls >= 0 ? mcls : 0];
+        kmeta[t] = mcls == -2 ? (int)0x80000000 : rel * 128 + (mcls + 2);
+    }
     __syncthreads();
     if (*s_abort) return;  // block-uniform
 
@@ -350,11 +408,10 @@ __global__ __launch_bounds__(NT) void k_attn_chunk(AttnArgs a) {
             }
             const int vi = j >> 3, jb = j & 7;
             const int pa = (jb & (X - 1)) | ((jb & ~(X - 1)) << 1), pb = pa + X;
-            const bool isq = vi < nqv;
-            int64_t kpos2;
-            const int kl = ko0 + vi - nqv;  // own key lane
-            const int kr2 = isq ? 0 : key_of(kl & (AK - 1), kpos2);
-            const int row = isq ? (vi < nqv ? vi / gqa : 0) : (kr2 >= 0 ? kr2 : 0);
+            const bool isq = vi < nqj;
+            const int kl = ko0 + vi - nqj;  // own key lane
+            const int kr2 = max(key_of(kl), 0);
+            const int row = min(isq ? (qv0 + vi) / gqa : kr2, M - 1);
             float xa[8], xb[8], wa[8], wb[8];
             unpack8(jxa[jj], xa);
             unpack8(jxb[jj], xb);
@@ -394,55 +451,84 @@ __global__ __launch_bounds__(NT) void k_attn_chunk(AttnArgs a) {
                 } else {
                     *(u4v*)(Ks + kl * QSTR + 8 * pa) = oa;
                     *(u4v*)(Ks + kl * QSTR + 8 * pb) = ob;
-                    const size_t dst = ((size_t)g * a.C + slot_of(L + kr2)) * HD;
-                    *(u4v*)(a.kc + dst + 8 * pa) = oa;
-                    *(u4v*)(a.kc + dst + 8 * pb) = ob;
+                    if (blockIdx.y == 0) {
+                        const size_t dst = ((size_t)g * a.C + slot_of(kr2)) * HD;
+                        *(u4v*)(a.kc + dst + 8 * pa) = oa;
+                        *(u4v*)(a.kc + dst + 8 * pb) = ob;
+                    }
                 }
             }
         }
     }
-    if (own_chunk && kvt) {
+    if (own_chunk && blockIdx.y == 0) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             if (vcls[j] >= 0)
-                *(u4v*)(a.vc + ((size_t)g * a.C + slot_of(L + vcls[j])) * HD + 8 * vd) = vv[j];
+                *(u4v*)(a.vc + ((size_t)g * a.C + slot_of(vcls[j])) * HD + 8 * vd) = vv[j];
     }
     // LDS-only barrier: the K / V appends above are read by later launches, not by this block
     // (it holds the finished keys in LDS), so they complete behind the attention work instead of
     // before it (__syncthreads would wait for the stores too)
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
-    const float sc2 = a.scale * LOG2E;
-    const int ln = lane & 15, lq = lane >> 4;
-    const int iters = (nqt + NW - 1) / NW;
-    for (int it = 0; it < iters; ++it) {
-        const int qt = wv + NW * it;
-        if (qt >= nqt) break;  // wave-uniform; no block barrier follows
+    // the group's next chunk: its K and V (and own keys) requested ahead of this one's products
+    const bool more = CG > 1 && c + 1 < ce;
+    if (more) {
+        ++c;
+        set_chunk();
+        nqj = 0;
+        request_kv();
+        request_jobs();
+    }
+
+    const int qt = wv;  // a tile a wave
+    if (qt < nqt) {
         // S^T tiles: keys 16 kt + 4 lq + r against query vector 16 qt + ln
         u4v qb[4];
 #pragma unroll
         for (int s4 = 0; s4 < 4; ++s4) qb[s4] = *(const u4v*)(Qs + (qt * 16 + ln) * QSTR + 32 * s4 + 8 * lq);
+        // all of the tile's K operands requested before its first product, and the V operands
+        // before the mask and softmax (left to itself the compiler waits for each LDS read in
+        // turn)
         f4 S[4];
+        u4v av[4][4];
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
-            S[kt] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+        for (int s4 = 0; s4 < 4; ++s4)
 #pragma unroll
-            for (int s4 = 0; s4 < 4; ++s4) {
-                const u4v av = *(const u4v*)(Ks + (16 * kt + ln) * QSTR + 32 * s4 + 8 * lq);
-                S[kt] = mfma16x16x32(as_h8(av), as_h8(qb[s4]), S[kt]);
-            }
-        }
+            for (int kt = 0; kt < 4; ++kt)
+                av[kt][s4] = *(const u4v*)(Ks + (16 * kt + ln) * QSTR + 32 * s4 + 8 * lq);
+        int4 km[4];
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) km[kt] = *(const int4*)(kmeta + 16 * kt + 4 * lq);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) S[kt] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s4 = 0; s4 < 4; ++s4)
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt)
+                S[kt] = mfma16x16x32(as_h8(av[kt][s4]), as_h8(qb[s4]), S[kt]);
         const int qv = qt * 16 + ln;
-        const int row = qv < nqv ? qv / gqa : 0;
+        const int row = qv < nqv ? (qv0 + qv) / gqa : 0;
         const int lo_r = rlo[row];
         const uint64_t anc = ranc[row];
+        // B lane (d, lq) of the PV products = V^T[d][32 j + 4 lq .. + 3] and [32 j + 16 + 4 lq ..]
+        uint2 bl[2][8], bh[2][8];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt) {
+                const uint16_t* vr = Vt + (16 * dt + ln) * VSTR + 32 * j + 4 * lq;
+                bl[j][dt] = *(const uint2*)vr;
+                bh[j][dt] = *(const uint2*)(vr + 16);
+            }
+        __builtin_amdgcn_sched_barrier(0);
         float m = -INFINITY;
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
-            const int4 km = *(const int4*)(kmeta + 16 * kt + 4 * lq);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int e = r == 0 ? km.x : r == 1 ? km.y : r == 2 ? km.z : km.w;
+                const int e = r == 0 ? km[kt].x : r == 1 ? km[kt].y : r == 2 ? km[kt].z : km[kt].w;
                 const int cls = (e & 127) - 2;  // -2 invalid, -1 committed, >= 0 own row
                 const bool ok = (qv < nqv) & (e != (int)0x80000000) & ((e >> 7) >= lo_r) &
                                 ((cls < 0) | (((anc >> (cls & 63)) & 1ull) != 0));
@@ -466,7 +552,7 @@ __global__ __launch_bounds__(NT) void k_attn_chunk(AttnArgs a) {
             pa[kt >> 1][2 * (kt & 1) + 1] = (uint32_t)f2h(p[2]) | ((uint32_t)f2h(p[3]) << 16);
         }
         l = xrow_sum(l);
-        // O = P V: B lane (d, lq) = V^T[d][32 j + 4 lq .. + 3] and [32 j + 16 + 4 lq .. + 3]
+        // O = P V
         f4 O[8];
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) O[dt] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
@@ -474,29 +560,41 @@ __global__ __launch_bounds__(NT) void k_attn_chunk(AttnArgs a) {
         for (int j = 0; j < 2; ++j) {
 #pragma unroll
             for (int dt = 0; dt < 8; ++dt) {
-                const uint16_t* vr = Vt + (16 * dt + ln) * VSTR + 32 * j + 4 * lq;
-                const uint2 lo4 = *(const uint2*)vr, hi4 = *(const uint2*)(vr + 16);
-                const u4v bv = {lo4.x, lo4.y, hi4.x, hi4.y};
+                const u4v bv = {bl[j][dt].x, bl[j][dt].y, bh[j][dt].x, bh[j][dt].y};
                 O[dt] = mfma16x16x32(as_h8(pa[j]), as_h8(bv), O[dt]);
             }
         }
-        // lane (d, lq) holds O of query vectors 16 qt + 4 lq + r, dim 16 dt + ln
-        const size_t pbase = ((size_t)g * a.max_chunks + c) * (size_t)(nqt * 16);
+        if constexpr (CG == 1) {
+            write_part(qt, O, m, l);
+        } else {
+            float fa, fb;
+            merge_part(mg, m, fa, fb);
+            lg = fmaf(fb, l, lg * fa);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            float* op = a.opart + (pbase + qt * 16 + 4 * lq + r) * HD;
+            for (int r = 0; r < 4; ++r) {
+                // weights of query vector 4 lq + r
+                const float far = __shfl(fa, 4 * lq + r, MJ_WAVE);
+                const float fbr = __shfl(fb, 4 * lq + r, MJ_WAVE);
 #pragma unroll
-            for (int dt = 0; dt < 8; ++dt) op[16 * dt + ln] = O[dt][r];
+                for (int dt = 0; dt < 8; ++dt) og[dt][r] = fmaf(fbr, O[dt][r], og[dt][r] * far);
+            }
         }
-        if (lq == 0) a.mlpart[pbase + qv] = make_float2(m, l);
+    }
+    if (!more) break;
+    // every wave is done with this chunk's K, V and metadata
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  }
+    if constexpr (CG > 1) {
+        if (wv < nqt) write_part(wv, og, mg, lg);
     }
 }
 
-// One 256-thread block per (row, query head): wave w merges, in increasing order, the chunks
+// One 256-thread block per (row, query head): wave w merges, in increasing order, the groups
 // whose absolute index is w mod 4 (lane = two dims), then the four wave sums are added in wave
-// order and the row is written in qx order.  Every chunk of the pass holds a partial (a fully
-// masked one has max -inf, sum 0, output 0 and adds exact zeros), so a row's merge depends only
-// on the chunks that hold its keys.
+// order and the row is written in qx order.  A group is merged from its chunks first (CG 1), or
+// came merged (CG 4).  Every part of the pass is there (a fully masked one has max -inf, sum 0,
+// output 0 and adds exact zeros), so a row's merge depends only on the chunks that hold its keys.
+template <int CG>
 __global__ __launch_bounds__(256) void k_attn_combine(AttnArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int r = blockIdx.x / a.nQ, hq = blockIdx.x % a.nQ;
@@ -504,42 +602,63 @@ __global__ __launch_bounds__(256) void k_attn_combine(AttnArgs a) {
     const int g = hq / gqa, qv = r * gqa + (hq % gqa);
     const size_t nq16 = (size_t)((a.M * gqa + 15) / 16) * 16;
     const ChunkGeom cg = chunk_geom(a.window, a.sd->L, a.M, a.sd->chain != 0);
-    const int nch = cg.nch;
-    const int cs = (int)(((int64_t)wv - cg.c0) & 3);  // this wave's first chunk
+    const int ng = group_count(cg), nparts = CG == 1 ? cg.nch : ng;
+    const int gs = (int)(((int64_t)wv - cg.c0 / AG) & 3);  // this wave's first group
     const float2* ml = a.mlpart + (size_t)g * a.max_chunks * nq16 + qv;
     const float* op = a.opart + ((size_t)g * a.max_chunks * nq16 + qv) * HD + 2 * lane;
-    // this wave's chunks cb + 4j, j < 4, requested at clamped indices (every lane loads; chunks
-    // past the end are skipped below); two rounds (32 chunks) at once
+    // a round: four parts, requested at clamped indices (parts past the end are skipped below) --
+    // the chunks of one group, or four of the wave's groups; two rounds at once
+    constexpr int GR = CG == 1 ? 1 : 4;  // groups a round
     float2 m4[2][4], p4[2][4];
-    const int clast = nch > 0 ? nch - 1 : 0;
-    auto request = [&](int cb, float2* mm, float2* pp) {
+    const int plast = nparts > 0 ? nparts - 1 : 0;
+    auto request = [&](int gb, float2* mm, float2* pp) {
+        int cb = 0, ce = 0;
+        if constexpr (CG == 1) group_chunks(cg, gb, cb, ce);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int c = min(cb + 4 * j, clast);
+            const int c = min(CG == 1 ? cb + j : gb + 4 * j, plast);
             mm[j] = ml[(size_t)c * nq16];
             pp[j] = *(const float2*)(op + (size_t)c * nq16 * HD);
         }
     };
-    // the first two rounds, together with the chunk maxima (they do not need them)
-    request(cs, m4[0], p4[0]);
-    request(cs + 16, m4[1], p4[1]);
-    // the maximum over the chunks (clamped indices: a repeated chunk leaves it unchanged)
-    float mx = ml[(size_t)min(lane, clast) * nq16].x;
-    for (int c = lane + 64; c < nch; c += 64) mx = fmaxf(mx, ml[(size_t)c * nq16].x);
+    // the first two rounds, together with the maxima (they do not need them)
+    request(gs, m4[0], p4[0]);
+    request(gs + 4 * GR, m4[1], p4[1]);
+    // the maximum over the parts (clamped indices: a repeated part leaves it unchanged)
+    float mx = ml[(size_t)min(lane, plast) * nq16].x;
+    for (int c = lane + 64; c < nparts; c += 64) mx = fmaxf(mx, ml[(size_t)c * nq16].x);
     mx = wave_max(mx);
     float o0 = 0.0f, o1 = 0.0f, ls = 0.0f;
-    for (int cb = cs, rd = 0; cb < nch; cb += 16, ++rd) {
-        if (rd >= 2) request(cb, m4[0], p4[0]);
+    auto add_group = [&](float m, float l, float v0, float v1) {
+        const float w = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mx);  // log2 units
+        ls = fmaf(l, w, ls);
+        o0 = fmaf(w, v0, o0);
+        o1 = fmaf(w, v1, o1);
+    };
+    for (int gb = gs, rd = 0; gb < ng; gb += 4 * GR, ++rd) {
+        if (rd >= 2) request(gb, m4[0], p4[0]);
         const float2* mm = rd == 1 ? m4[1] : m4[0];
         const float2* pp = rd == 1 ? p4[1] : p4[0];
+        if constexpr (CG == 1) {
+            int cb, ce;
+            group_chunks(cg, gb, cb, ce);
+            float mg = -INFINITY, lg = 0.0f, g0 = 0.0f, g1 = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if (cb + 4 * j >= nch) break;
-            // log2 units
-            const float w = mm[j].x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mm[j].x - mx);
-            ls += mm[j].y * w;
-            o0 += w * pp[j].x;
-            o1 += w * pp[j].y;
+            for (int j = 0; j < 4; ++j) {
+                if (cb + j >= ce) break;
+                float fa, fb;
+                merge_part(mg, mm[j].x, fa, fb);
+                lg = fmaf(fb, mm[j].y, lg * fa);
+                g0 = fmaf(fb, pp[j].x, g0 * fa);
+                g1 = fmaf(fb, pp[j].y, g1 * fa);
+            }
+            add_group(mg, lg, g0, g1);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (gb + 4 * j >= ng) break;
+                add_group(mm[j].x, mm[j].y, pp[j].x, pp[j].y);
+            }
         }
     }
     __shared__ float s_o[4][HD];
@@ -569,7 +688,8 @@ __global__ __launch_bounds__(256) void k_attn_combine(AttnArgs a) {
     }
 }
 
-hipError_t launch_attn(const AttnArgs& a, hipStream_t st) {
+hipError_t launch_attn(const AttnArgs& args, hipStream_t st) {
+    AttnArgs a = args;
     if (a.M < 1 || a.M > MJ_ROWS) return hipErrorInvalidValue;  // row metadata is staged per row
     // RoPE partners are found by lane moves: half = rope_dim / 2 in {16, 32, 64}
     if (a.rope_dim != 0 && a.rope_dim != 32 && a.rope_dim != 64 && a.rope_dim != 128)
@@ -578,43 +698,61 @@ hipError_t launch_attn(const AttnArgs& a, hipStream_t st) {
     if (a.C < 1 || a.C >= ((int64_t)1 << 23)) return hipErrorInvalidValue;
     const int gqa = a.nQ / a.nKV;
     const int nqt = (a.M * gqa + 15) / 16;
-    const size_t lds = (size_t)(nqt * 16 * QSTR + AK * QSTR + HD * VSTR) * 2 +
+    // Groups of chunks a block where the keys run deep: the partials are the launch's traffic (64
+    // rows at 6000 keys write and read 51 MB of them, 13 MB in groups: block 56 -> 48 us), but a
+    // further chunk in turn costs a block 2.4 us (64 rows: at 3000 keys 45 -> 43 us, at 1500 39 ->
+    // 42; one row at 6000 29 -> 30).  Query tiles: two a block until the blocks pass 400, then four
+    // (64 rows at 130 keys 40 -> 34 us, at 1024 43 -> 39, where two a block take 42; 17 rows at
+    // 1024 28.1 -> 27.4; before, one block took all of the pass's tiles).
+    const int nch = std::min(a.nch, a.max_chunks);
+    const bool groups = nch >= MJ_ATTN_DEEP && nqt >= 3;
+    a.parts = groups ? (nch + 1) / AG + 2 : nch;
+    a.tpp = a.nKV * a.parts * ((nqt + 1) / 2) <= 400 ? 2 : 4;
+    if (a.tpp > nqt) a.tpp = nqt;
+    const int qparts = (nqt + a.tpp - 1) / a.tpp;
+    const size_t lds = (size_t)(a.tpp * 16 * QSTR + AK * QSTR + HD * VSTR) * 2 +
                        (size_t)tab_floats2(a.M, a.rope_dim / 2) * 8 + AK * 4 + MJ_ROWS * (4 + 8) +
                        2 * HD * 2 + 16;
-    // finishing jobs of the block that also holds the pass's own keys; more than four query
-    // tiles take 512-thread blocks (two jobs a thread then cover up to 1024)
-    const int jobs = 8 * (a.M * gqa + (a.M < AK ? a.M : AK));
-    const bool wide = nqt > 4;
+    // finishing jobs of a block that also holds the pass's own keys
+    const int jobs = 8 * (std::min(a.M * gqa, 16 * a.tpp) + (a.M < AK ? a.M : AK));
     const bool jr3 = jobs > 256 * 2;
-    auto go = [&](auto k2, auto k3, auto w2) {
-        const dim3 grid(a.nKV * a.max_chunks);
-        if (wide)
-            launch_timed(w2, grid, dim3(512), lds, st, a);
-        else
-            launch_timed(jr3 ? k3 : k2, grid, dim3(256), lds, st, a);
+    const dim3 grid(a.nKV * a.parts, qparts);
+    auto go = [&](auto k2, auto k3, auto kg) {
+        launch_timed(groups ? kg : jr3 ? k3 : k2, grid, dim3(256), lds, st, a);
     };
+#define MJ_AT(H) go(k_attn_chunk<H, 2, 1>, k_attn_chunk<H, 3, 1>, k_attn_chunk<H, 2, AG>)
     switch (a.rope_dim) {
-        case 0: go(k_attn_chunk<0, 2, 256>, k_attn_chunk<0, 3, 256>, k_attn_chunk<0, 2, 512>); break;
-        case 32: go(k_attn_chunk<16, 2, 256>, k_attn_chunk<16, 3, 256>, k_attn_chunk<16, 2, 512>); break;
-        case 64: go(k_attn_chunk<32, 2, 256>, k_attn_chunk<32, 3, 256>, k_attn_chunk<32, 2, 512>); break;
-        default: go(k_attn_chunk<64, 2, 256>, k_attn_chunk<64, 3, 256>, k_attn_chunk<64, 2, 512>); break;
+        case 0: MJ_AT(0); break;
+        case 32: MJ_AT(16); break;
+        case 64: MJ_AT(32); break;
+        default: MJ_AT(64); break;
     }
+#undef MJ_AT
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_attn_combine, dim3(a.M * a.nQ), dim3(256), 0, st, a);
+    const dim3 rows(a.M * a.nQ);
+    if (groups)
+        hipLaunchKernelGGL(k_attn_combine<AG>, rows, dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL(k_attn_combine<1>, rows, dim3(256), 0, st, a);
     return hipGetLastError();
 }
 
-hipError_t set_attn_attributes() {
+template <int HALF>
+static hipError_t attn_attr() {
     hipError_t e = hipSuccess;
-    const void* ks[] = {(const void*)k_attn_chunk<0, 2, 256>,  (const void*)k_attn_chunk<16, 2, 256>,
-                        (const void*)k_attn_chunk<32, 2, 256>, (const void*)k_attn_chunk<64, 2, 256>,
-                        (const void*)k_attn_chunk<0, 3, 256>,  (const void*)k_attn_chunk<16, 3, 256>,
-                        (const void*)k_attn_chunk<32, 3, 256>, (const void*)k_attn_chunk<64, 3, 256>,
-                        (const void*)k_attn_chunk<0, 2, 512>,  (const void*)k_attn_chunk<16, 2, 512>,
-                        (const void*)k_attn_chunk<32, 2, 512>, (const void*)k_attn_chunk<64, 2, 512>};
+    const void* ks[] = {(const void*)k_attn_chunk<HALF, 2, 1>, (const void*)k_attn_chunk<HALF, 3, 1>,
+                        (const void*)k_attn_chunk<HALF, 2, AG>};
     for (const void* k : ks)
         if (e == hipSuccess)
             e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    return e;
+}
+
+hipError_t set_attn_attributes() {
+    hipError_t e = attn_attr<0>();
+    if (e == hipSuccess) e = attn_attr<16>();
+    if (e == hipSuccess) e = attn_attr<32>();
+    if (e == hipSuccess) e = attn_attr<64>();
     return e;
 }

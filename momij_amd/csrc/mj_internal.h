@@ -175,6 +175,8 @@ struct AttnArgs {
     uint16_t* out_perm;      // attention output, qx [M][nQ*128]
     float2* out_sum;         // [M][nQ*2]
     int M, nQ, nKV, rope_dim, window, max_chunks;
+    int nch;                 // bound on the pass's chunks (at most max_chunks)
+    int parts, tpp;          // set by launch_attn: parts (chunks, or groups) and query tiles a block
     int64_t C;
     float eps, scale;
     const int* abort;
@@ -183,6 +185,8 @@ struct AttnArgs {
 // attn.hip
 hipError_t launch_attn(const AttnArgs& a, hipStream_t st);
 int attn_max_chunks(int window, int64_t L_max, int M);
+// Chunks from which a launch takes its keys in groups (launch_attn)
+#define MJ_ATTN_DEEP 40
 
 // What one attention block call's first launch takes by value: the pass descriptor and the RoPE
 // frequencies (half = rope_dim / 2 of them).

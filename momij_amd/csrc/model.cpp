@@ -70,6 +70,7 @@ struct mj_model {
     StepResult* res_dev = nullptr;
     StepResult* res_host = nullptr;
     int64_t offset = 0;
+    bool deep = false;  // this pass's full-attention layers may span MJ_ATTN_DEEP chunks or more
     bool graphs = true;
     std::map<int, hipGraphExec_t> graph_cache;
     mj_capture cap{};  // debug capture (device pointers; all null: off)
@@ -152,6 +153,8 @@ static mj_status enqueue_layer(mj_model* m, int l, int M, int kind, hipStream_t 
     a.rope_dim = m->lrope[l];
     a.window = m->lwin[l];
     a.max_chunks = m->max_chunks;
+    a.nch = m->lwin[l] > 0 ? attn_max_chunks(m->lwin[l], 0, M)
+                           : (m->deep ? m->max_chunks : MJ_ATTN_DEEP - 1);
     a.C = c.kv_capacity;
     a.eps = c.eps;
     a.scale = (float)std::pow((double)D, -0.5);
@@ -328,6 +331,9 @@ static mj_status run_pass(mj_model* m, int kind, int M) {
     s = mj_hip(ctx, hipMemcpyAsync(m->sd_dev, m->sd_host, sizeof(StepDesc),
                                    hipMemcpyHostToDevice, st), "descriptor upload");
     if (s != MJ_OK) return s;
+    bool any_full = false;
+    for (int w : m->lwin) any_full = any_full || w <= 0;
+    m->deep = any_full && attn_max_chunks(0, m->offset, M) >= MJ_ATTN_DEEP;
     const mj_capture& cp = m->cap;
     const bool capturing = cp.h || cp.inds || cp.logits || cp.attn_out || cp.moe_in ||
                            cp.router_logits || cp.head_in || cp.kv_rows;
@@ -348,7 +354,7 @@ static mj_status run_pass(mj_model* m, int kind, int M) {
     }
     hipEventRecord(m->ev0, st);
     if (capture_ok) {
-        const int key = kind * 1000 + M;
+        const int key = (m->deep ? 100000 : 0) + kind * 1000 + M;
         auto it = m->graph_cache.find(key);
         if (it == m->graph_cache.end()) {
             hipGraph_t g = nullptr;
@@ -895,7 +901,7 @@ mj_status mj_attn_block(mj_ctx* ctx, const mj_attn_config* cfg, const mj_attn_we
     a.nKV = nKV;
     a.rope_dim = c.rope_dim;
     a.window = c.window;
-    a.max_chunks = maxc;
+    a.max_chunks = a.nch = maxc;
     a.C = c.kv_capacity;
     a.eps = c.eps;
     a.scale = (float)std::pow(128.0, -0.5);
