@@ -465,6 +465,11 @@ mj_status moe_scratch(mj_ctx* ctx, int H, int I, int E, int k, int M, MoeScratch
 #define MJ_TILE_MIN_ROWS 1
 #endif
 
+bool moe_wide_supported(int H, int I, int E, int k, int gs) {
+    return route_supported(H, E, k) && gather3_supported(EPI_SWIGLU, H, 2 * I, gs) &&
+           gather3_supported(EPI_STORE, I, H, gs) && I <= 1024;
+}
+
 mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint16_t* y, int M,
                   int flags, const MoeScratch& ms, int32_t* inds, float* scores, hipStream_t st,
                   Prof* prof, const NormOut* next) {
@@ -477,7 +482,10 @@ mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint1
     const bool dn_tile = gather3_supported(EPI_STORE, I, H, w->gs);
     // tile path: one row takes it too, so a row's result does not depend on how many rows share
     // its pass (a verify row equals the one-row decode step at its position, bit for bit)
-    const bool tile = fused && M >= MJ_TILE_MIN_ROWS && M <= MJ_MAX_ROWS && up_tile && dn_tile;
+    const bool wide = M > MJ_MAX_ROWS;  // a wide prefill pass: the products take slot tables
+    const bool tile = fused && M >= MJ_TILE_MIN_ROWS && up_tile && dn_tile;
+    if (wide && (!moe_wide_supported(H, I, E, k, w->gs) || !ms.up_tab.rec))
+        return mj_fail(ctx, MJ_INVALID_ARG, "MoE block of %d rows", M);
     // the common expert shape, up to 32 rows over at most 64 experts: one launch ranks the
     // logits (its blocks form the slot records themselves) and runs both products
     const bool moe_fused =
@@ -509,6 +517,13 @@ mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint1
         if (s != MJ_OK) return s;
         if (!topk_in_up) {
             s = mj_hip(ctx, launch_route_topk(ra, st), "route top-k");
+            if (s != MJ_OK) return s;
+        }
+        if (wide) {
+            SlotTab ut = ms.up_tab, dt = ms.dn_tab;
+            ut.ps = gather3_part_rows(EPI_SWIGLU, H, w->gs, w->up_gate_alpha != nullptr);
+            dt.ps = gather3_part_rows(EPI_STORE, I, w->gs, w->down_alpha != nullptr);
+            s = mj_hip(ctx, launch_wide_slots(inds, M * k, ut, dt, ab, st), "slots");
             if (s != MJ_OK) return s;
         }
         if (M == 1 && !tile && (flags & MJ_MOE_PRENORM)) xn = ms.xn;
@@ -584,6 +599,9 @@ mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint1
         up.b = (const uint16_t*)w->up_gate_b;
         if (!tile) {
             up.bk = ms.bk;
+        } else if (wide) {
+            up.tab = ms.up_tab.rec;
+            up.tab_slots = ms.up_tab.n;
         } else if (!topk_in_up) {
             up.inds = inds;
             up.npairs = M * k;
@@ -612,18 +630,22 @@ mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint1
         }
         // the tile kernel's SwiGLU epilogue writes act without block sums: the tile down
         // kernel forms them from its staged rows, any other down kernel gets them here
-        if (up_tile && !dn_tile) {
+        // (a wide pass too: each act row is staged by many items)
+        if (up_tile && (!dn_tile || wide)) {
             s = mj_hip(ctx, launch_qx_sums(ms.act, ms.act_sum, M * k, I, ab, st), "act sums");
             if (s != MJ_OK) return s;
         }
         GatherArgs dn = up;
         dn.rlogits = nullptr;  // the down product takes the ids the routing wrote
-        if (tile) {
+        if (wide) {
+            dn.tab = ms.dn_tab.rec;
+            dn.tab_slots = ms.dn_tab.n;
+        } else if (tile) {
             dn.inds = inds;
             dn.npairs = M * k;
         }
         dn.xperm = ms.act;
-        dn.xsum = dn_tile ? nullptr : ms.act_sum;
+        dn.xsum = dn_tile && !wide ? nullptr : ms.act_sum;
         dn.w = w->down_w;
         dn.s = (const uint16_t*)w->down_s;
         dn.b = (const uint16_t*)w->down_b;

@@ -45,7 +45,7 @@ __device__ __forceinline__ void load_lds4(const void* g, void* lds) {
 // staged in LDS per pass (a bucket with more rows takes several passes; `multi` says whether
 // any can), K = 256 * KPL.  A block has WPB waves = TPB tiles of 16
 // weight rows x KS K-slices: wave w owns tile w % TPB and K-slice w / TPB.
-template <int KPL, int GS, int EPI, int WPB, int KS>
+template <int KPL, int GS, int EPI, int WPB, int KS, bool ROWA = false>
 struct G5Shape {
     static constexpr int R = 16;
     static constexpr int K = KPL * 256;
@@ -59,7 +59,8 @@ struct G5Shape {
     static constexpr bool HSC = SCH == 0;
     static constexpr int SCW = HSC ? 1 : SCH / KS;  // ... per K-slice
     static constexpr int WCODE = 16 * KBW * 16;  // bytes of one wave's code tile
-    static constexpr int WSB = 16 * SCW * 16;    // bytes of one wave's scales (and of its biases)
+    // bytes of one wave's scales (and of its biases); row-alpha tiles hold one alpha a row
+    static constexpr int WSB = ROWA ? 32 : 16 * SCW * 16;
     static constexpr int WAVE_BYTES = WCODE + 2 * WSB;
     static constexpr int SS = KB + 2;          // LDS row stride of block sums (float2)
     static_assert(WAVE_BYTES >= 64 * 16, "a K-slice partial fits in its wave's tile area");
@@ -152,7 +153,9 @@ struct FuseIO {
 // Where a persistent launch's slot records come from.  REC_RANK: the launch ranks the router
 // logits itself (passes of at most FR rows over at most 64 experts).  REC_IDS: from the expert id
 // of every (row, slot) pair in global memory (any rows and experts a pass may have).
-enum { REC_NONE = 0, REC_RANK = 1, REC_IDS = 2 };
+// REC_TAB (wide passes): from a slot table in global memory; the next item's record is requested
+// behind the current one's weights.
+enum { REC_NONE = 0, REC_RANK = 1, REC_IDS = 2, REC_TAB = 3 };
 
 // FR: rows the fused routing ranks at most (16: two a wave, ranks in er; 32: four a wave, rows
 // 16 .. 31's ranks in er1)
@@ -162,7 +165,8 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
     constexpr bool PER = REC != REC_NONE;
     constexpr bool FUS = REC == REC_RANK && MODE != 2;  // ranks the logits in its prologue
     static_assert(FR == 16 || FR == 32, "fused routing rows");
-    using S = G5Shape<KPL, GS, EPI, WPB, KS>;
+    using S = G5Shape<KPL, GS, EPI, WPB, KS, ROWA>;
+    constexpr bool LIST = REC == REC_IDS || REC == REC_TAB;  // slots of any number
     constexpr int R = S::R, K = S::K, KB = S::KB, KBW = S::KBW, TPB = S::TPB, XS = S::XS;
     constexpr int SCW = S::SCW;
     constexpr int NT = WPB * 64;
@@ -216,7 +220,9 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
     // record of slot sl: pair j in lane j, expert id and pair count in the high halves of lanes 0
     // and 1 (count 0 past the last slot)
     auto slot_rec = [&](int sl) -> int {
-      if constexpr (REC == REC_IDS) {
+      if constexpr (REC == REC_TAB) {
+        return a.tab[16 * min(sl, a.tab_slots - 1) + (lane & 15)];
+      } else if constexpr (REC == REC_IDS) {
         // lane l holds the ids of pairs l + 64 i; the pairs of the slot's expert are numbered
         // in increasing index by ballots and sent to the lane of their number in the part.
         // Lanes with nothing to send, in round i, send to the lane below the round's first
@@ -410,9 +416,11 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
                 const int G = (int)gridDim.x, rem = (nS * a.fup_ncb) % G;
                 item = (int)blockIdx.x >= rem ? (int)blockIdx.x - rem : (int)blockIdx.x + (G - rem);
             }
-            const int rec = slot_rec(REC == REC_IDS ? item / ncb : min(item / ncb, 63));
+            const int rec = slot_rec(LIST ? item / ncb : min(item / ncb, 63));
+            if constexpr (REC == REC_TAB)
+                if (aborted(a.abort)) return;
             e = __builtin_amdgcn_readlane(rec, 0) >> 16;
-            np = REC == REC_IDS || item / ncb < 64 ? __builtin_amdgcn_readlane(rec, 1) >> 16 : 0;
+            np = LIST || item / ncb < 64 ? __builtin_amdgcn_readlane(rec, 1) >> 16 : 0;
             lpair = rec & 0xFFFF;
             cb = item % ncb;
         }
@@ -635,9 +643,12 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
         }
         // ranked routing's up product: a stand-in load behind this item's weights (PF: one vector
         // load younger than them), whose value is consumed (times zero) so that it stays
-        constexpr int PF = FUS ? 1 : 0;
+        // a slot table's next record: requested there for good
+        constexpr int PF = FUS || REC == REC_TAB ? 1 : 0;
         if constexpr (FUS) {
             if (pb == 0) rec_n = *(const int*)a.rlogits;
+        } else if constexpr (REC == REC_TAB) {
+            rec_n = slot_rec((item + (int)gridDim.x) / ncb);
         }
         wait_vmcnt<G + PF>();      // scales and biases have landed
         u4v sv[SCW], bv[SCW];
@@ -707,14 +718,15 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
         // scales and first half of the code groups are requested once this item's first half
         // is done (its scales are in registers, its first half's codes read), the rest after
         // its MFMAs; the item waits for its own groups first, so later waits count nothing new
-        constexpr bool SPLIT = PER && (MODE != 0 || REC == REC_IDS) && G >= 2;
+        constexpr bool SPLIT = PER && (MODE != 0 || LIST) && G >= 2;
         constexpr int GP = G / 2;  // code groups a part (four parts measured slower)
         bool stage_next = false;
         int np_next = 0;
         auto next_item = [&]() {
             if constexpr (PER) {
                 const int nx = item + (int)gridDim.x;
-                if constexpr (REC == REC_IDS) {
+                if constexpr (REC == REC_TAB) {
+                } else if constexpr (REC == REC_IDS) {
                     rec_n = slot_rec(nx / ncb);
                 } else if constexpr (MODE == 2) {
                     rec_n = slot_rec(min(nx / ncb, 63));
@@ -722,7 +734,7 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
                     rec_n = slot_rec(min(nx / ncb, 63)) | (rec_n & (int)opaque(0u));
                 }
                 np_next = __builtin_amdgcn_readlane(rec_n, 1) >> 16;
-                stage_next = pb + RA >= np && (REC == REC_IDS || nx / ncb < 64) && np_next > 0;
+                stage_next = pb + RA >= np && (LIST || nx / ncb < 64) && np_next > 0;
             }
         };
         // sum_B s_B * (sum q x)_B: per 64-block f16 MFMA sums, scaled in fp32, one column group
@@ -912,7 +924,7 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
     }
     if constexpr (!PER) break;
     item += gridDim.x;
-    if (REC != REC_IDS && item / ncb >= 64) break;
+    if (!LIST && item / ncb >= 64) break;
     np = __builtin_amdgcn_readlane(rec_n, 1) >> 16;
     if (np <= 0) break;
     e = __builtin_amdgcn_readlane(rec_n, 0) >> 16;
@@ -951,7 +963,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
 
 // static LDS of a persistent kernel: its pair lists and what its records are formed from
 constexpr size_t g5_stat(int rec, int FR) {
-    return 256 + (rec == REC_IDS ? sizeof(IdsLds) : g5_fused_rec_bytes(FR));
+    return 256 + (rec == REC_IDS ? sizeof(IdsLds) : rec == REC_TAB ? 0 : g5_fused_rec_bytes(FR));
 }
 
 // dynamic LDS a tile-gather launch may take (the device has 160 KB per workgroup)
@@ -970,17 +982,25 @@ static int persistent_blocks() {
     return 2 * cus;
 }
 
+// staged rows per pass: for the persistent products as many as keep two blocks per CU (more
+// rows on one expert take extra passes, or slots); dense projections take up to 16
 template <int KPL, int GS, int EPI, int WPB, int KS, int REC = REC_NONE, bool ROWA = false>
-static hipError_t launch_g5(const GatherArgs& a, int rows, int slots, hipStream_t st) {
-    using S = G5Shape<KPL, GS, EPI, WPB, KS>;
+static int g5_rows(int want) {
+    using S = G5Shape<KPL, GS, EPI, WPB, KS, ROWA>;
     constexpr bool PER = REC != REC_NONE;
-    const int ncb = (a.N + 16 * S::TPB - 1) / (16 * S::TPB);
-    // staged rows per pass: for the persistent products as many as keep two blocks per CU (more
-    // rows on one expert take extra passes); dense projections take up to 16
-    const int want = rows < 1 ? 1 : rows;
     int RA = want < S::R ? want : S::R;
     const size_t limit = PER ? 80 * 1024 - g5_stat(REC, MJ_G5_FUSED_ROWS) : G5_LDS_MAX;
     while (RA > 1 && S::lds(RA, want > RA || PER) > limit) --RA;
+    return RA;
+}
+
+template <int KPL, int GS, int EPI, int WPB, int KS, int REC = REC_NONE, bool ROWA = false>
+static hipError_t launch_g5(const GatherArgs& a, int rows, int slots, hipStream_t st) {
+    using S = G5Shape<KPL, GS, EPI, WPB, KS, ROWA>;
+    constexpr bool PER = REC != REC_NONE;
+    const int ncb = (a.N + 16 * S::TPB - 1) / (16 * S::TPB);
+    const int want = rows < 1 ? 1 : rows;
+    const int RA = g5_rows<KPL, GS, EPI, WPB, KS, REC, ROWA>(want);
     const bool multi = want > RA;
     int grid = slots * ncb;
     if (PER && grid > persistent_blocks()) grid = persistent_blocks();
@@ -1003,7 +1023,23 @@ bool gather3_supported(int epi, int K, int N, int gs) {
 
 hipError_t launch_gather3(const GatherArgs& a, int epi, int rows, hipStream_t st) {
     if (!gather3_supported(epi, a.K, a.N, a.gs)) return hipErrorInvalidValue;
-    const bool rank = a.rlogits != nullptr, per = rank || a.inds != nullptr;
+    const bool rank = a.rlogits != nullptr, per = rank || a.inds != nullptr || a.tab != nullptr;
+    if (a.tab != nullptr) {
+        // wide passes: the experts' two products, their slots listed in the table
+        const bool al = a.alpha != nullptr;
+        const int slots = a.tab_slots;
+        if (slots < 1) return hipErrorInvalidValue;
+#define MJ_G5T(KPL, E, KS64, KS128)                                                          \
+    return a.gs == 64 ? (al ? launch_g5<KPL, 64, E, 8, KS64, REC_TAB, true>(a, 16, slots, st)   \
+                            : launch_g5<KPL, 64, E, 8, KS64, REC_TAB, false>(a, 16, slots, st)) \
+                      : (al ? launch_g5<KPL, 128, E, 8, KS128, REC_TAB, true>(a, 16, slots, st) \
+                            : launch_g5<KPL, 128, E, 8, KS128, REC_TAB, false>(a, 16, slots, st));
+        if (epi == EPI_SWIGLU) { MJ_G5T(8, EPI_SWIGLU, 2, 2) }
+        if (epi != EPI_STORE || a.K > 1024) return hipErrorInvalidValue;
+        if (a.K == 512) { MJ_G5T(2, EPI_STORE, 1, 1) }
+        MJ_G5T(4, EPI_STORE, 1, 1)
+#undef MJ_G5T
+    }
     // ranked routing: the up || gate product ranks the router logits itself
     if (rank && (epi != EPI_SWIGLU || a.rM < 1 || a.rM > MJ_G5_FUSED_ROWS || a.rE < 1 ||
                  a.rE > 64 || a.rk < 1 || a.rk > 8 || a.rk > a.rE || a.x_div != a.rk ||
@@ -1060,6 +1096,18 @@ hipError_t launch_gather3(const GatherArgs& a, int epi, int rows, hipStream_t st
     if (a.K == 1024) { MJ_G5D(4, EPI_STORE, 8, 1, 1) }
     MJ_G5D(8, EPI_STORE, 4, 4, 2)
 #undef MJ_G5D
+}
+
+int gather3_part_rows(int epi, int K, int gs, bool alpha) {
+#define MJ_R(KPL, E, KS)                                                                     \
+    return gs == 64 ? (alpha ? g5_rows<KPL, 64, E, 8, KS, REC_TAB, true>(16)                    \
+                             : g5_rows<KPL, 64, E, 8, KS, REC_TAB, false>(16))                  \
+                    : (alpha ? g5_rows<KPL, 128, E, 8, KS, REC_TAB, true>(16)                   \
+                             : g5_rows<KPL, 128, E, 8, KS, REC_TAB, false>(16));
+    if (epi == EPI_SWIGLU) { MJ_R(8, EPI_SWIGLU, 2) }
+    if (K == 512) { MJ_R(2, EPI_STORE, 1) }
+    MJ_R(4, EPI_STORE, 1)
+#undef MJ_R
 }
 
 // static LDS of the fused MoE kernel: both phases' pair lists and the routing words
@@ -1138,7 +1186,7 @@ template <int KPL, int GS, int EPI, int WPB, int KS, int REC = REC_NONE, bool RO
 static hipError_t g5_attr() {
     return hipFuncSetAttribute((const void*)k_gather5<KPL, GS, EPI, WPB, KS, REC, ROWA>,
                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)std::min(G5Shape<KPL, GS, EPI, WPB, KS>::lds(16, true),
+                               (int)std::min(G5Shape<KPL, GS, EPI, WPB, KS, ROWA>::lds(16, true),
                                              G5_LDS_MAX));
 }
 
@@ -1166,6 +1214,12 @@ hipError_t set_gather3_attributes() {
     MJ_A(2, EPI_ADD, 8, 1, 1, REC_IDS, false)
     MJ_A(4, EPI_ADD, 8, 1, 1, REC_IDS, false)
     MJ_A(8, EPI_ADD, 8, 2, 2, REC_IDS, false)
+    MJ_A(8, EPI_SWIGLU, 8, 2, 2, REC_TAB, false)
+    MJ_A(8, EPI_SWIGLU, 8, 2, 2, REC_TAB, true)
+    MJ_A(2, EPI_STORE, 8, 1, 1, REC_TAB, false)
+    MJ_A(2, EPI_STORE, 8, 1, 1, REC_TAB, true)
+    MJ_A(4, EPI_STORE, 8, 1, 1, REC_TAB, false)
+    MJ_A(4, EPI_STORE, 8, 1, 1, REC_TAB, true)
 #undef MJ_A
     // the fused MoE kernels
     {

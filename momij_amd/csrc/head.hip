@@ -964,7 +964,8 @@ hipError_t launch_kv_commit(uint16_t* kv, int64_t layer_stride, int n_layers, in
 // maple_qk_norm_rope's angle (SeedlessMetal.swift:2832-2846), evaluated once per pass.
 __device__ __forceinline__ void rope_row(const StepDesc* sd, const RopeTab& rt, int r, int t) {
     if (t < rt.half) {
-        const float pos = (float)(sd->L + sd->depth[r]);
+        const StepDesc* d = sd + r / MJ_ROWS;
+        const float pos = (float)(d->L + d->depth[r % MJ_ROWS]);
         const float th = pos * rt.inv_freq[t];
         rt.cs[r * MJ_ROPE_F + t] = make_float2(cosf(th), sinf(th));
     }
@@ -996,7 +997,7 @@ __global__ __launch_bounds__(256) void k_embed_norm(const uint16_t* table, const
     if (aborted(abort)) return;
     const int r = blockIdx.x, t = threadIdx.x;
     rope_row(sd, rt, r, t);
-    const int tok = sd->tokens[r];
+    const int tok = sd[r / MJ_ROWS].tokens[r % MJ_ROWS];
     const u4v v = *(const u4v*)(table + (size_t)tok * 2048 + 8 * t);
     *(u4v*)(h + (size_t)r * 2048 + 8 * t) = v;
     norm_row_2048(v, no, r);
@@ -1005,7 +1006,7 @@ __global__ __launch_bounds__(256) void k_embed_norm(const uint16_t* table, const
 hipError_t launch_embed_norm(const uint16_t* table, const StepDesc* sd, int M, int H, uint16_t* h,
                              const NormOut& no, const RopeTab& rt, const int* abort,
                              hipStream_t st) {
-    if (H != 2048 || rt.half > MJ_ROPE_F || M > MJ_ROWS) return hipErrorInvalidValue;
+    if (H != 2048 || rt.half > MJ_ROPE_F || M > MJ_WIDE_ROWS) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_embed_norm, dim3(M), dim3(256), 0, st, table, sd, h, no, rt, abort);
     return hipGetLastError();
 }

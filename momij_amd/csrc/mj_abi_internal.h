@@ -62,6 +62,7 @@ struct MoeScratch {
     uint16_t* act;       // [M*k][I] (qx for M > 1, plain for M == 1)
     float2* act_sum;     // [M*k][I/64]
     uint16_t* down;      // [M*k][H]
+    SlotTab up_tab{}, dn_tab{};  // passes past MJ_MAX_ROWS rows (wide prefill; else unset)
     bool want_plain = false;  // also write the normed rows plain into xn (debug capture)
 };
 
@@ -103,6 +104,8 @@ mj_status mj_abort_end(mj_ctx* ctx, unsigned gen);
 // Scratch of an MoE block call laid out over an arena (base nullptr: size counting only).
 void moe_scratch_layout(Arena& a, int H, int I, int E, int k, int M, MoeScratch& ms);
 mj_status moe_scratch(mj_ctx* ctx, int H, int I, int E, int k, int M, MoeScratch& ms);
+// Whether passes of up to MJ_WIDE_ROWS rows can take the block (the tile kernels' shapes).
+bool moe_wide_supported(int H, int I, int E, int k, int gs);
 // next: also normalise the block's output y into these outputs (the following RMSNorm).
 mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint16_t* y, int M,
                   int flags, const MoeScratch& ms, int32_t* inds, float* scores, hipStream_t st,

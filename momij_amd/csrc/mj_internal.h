@@ -28,6 +28,10 @@ inline void launch_timed(K kernel, dim3 grid, dim3 block, size_t lds, hipStream_
 
 #define MJ_MAX_EXPERTS 256
 #define MJ_MAX_PAIRS 512  // rows * top_k per pass
+// Rows of a wide prefill pass (whole 64-row chunks of a prompt sharing every launch but
+// attention's)
+#define MJ_WIDE_ROWS 256
+#define MJ_WIDE_PAIRS (MJ_WIDE_ROWS * 8)
 
 // Rows of one pass grouped by expert (filled on the device by the router, or implied for a
 // dense projection).  pair[start[u] .. start[u+1]) lists the (row * top_k + slot) indices
@@ -56,6 +60,7 @@ struct NormOut {
 // Per-pass parameters read by the kernels from device memory, so one captured graph serves
 // every step with the same row count.  Row r of a pass sits at position L + depth[r]; anc[r]
 // has bit a set iff row a is row r or one of its ancestors; tokens[r] is the token fed there.
+// A wide prefill pass has one for each 64 rows.
 struct StepDesc {
     int64_t L;
     int32_t M;
@@ -98,6 +103,8 @@ struct GatherArgs {
     const Buckets* bk;      // general kernel: rows grouped by expert (nullptr: dense)
     const int32_t* inds;    // tile kernel, persistent: expert of every pair [npairs] (pairs whose
     int npairs;             // id is outside [0, MJ_MAX_EXPERTS) are left out)
+    const int32_t* tab;     // tile kernel, persistent, wide passes: the slot table (SlotTab)
+    int tab_slots;
     int dense_rows;         // dense: rows 0 .. dense_rows-1 of expert 0
     const uint16_t* alpha;  // row-alpha weights [E][N] fp16 (scale alpha, bias -alpha in
                             // every group): the tile expert kernels read it instead of s / b
@@ -144,6 +151,22 @@ hipError_t launch_gather(const GatherArgs& a, int epi, int max_rows_per_bucket, 
                          hipStream_t st);
 hipError_t launch_selftest_mfma(const uint16_t* A, const uint16_t* B, float* D, hipStream_t st);
 
+// Slot table of a wide pass's product: rec[16 s + j], j < 16: pair j of slot s in the low 16 bits,
+// the expert and the pair count in the high halves of entries 0 and 1; at most ps (<= 16) pairs a
+// slot, an expert's pairs spread evenly over its slots; slots past the last have count 0, the last
+// record (n - 1) always.
+struct SlotTab {
+    int32_t* rec;  // [n][16]
+    int n, ps;
+};
+#define MJ_SLOT_PS_MIN 8  // pairs a slot the tables are sized for, at least
+constexpr int slot_tab_size(int E, int ps) { return E + MJ_WIDE_PAIRS / ps + 1; }
+hipError_t launch_wide_slots(const int32_t* inds, int P, const SlotTab& up, const SlotTab& dn,
+                             const int* abort, hipStream_t st);
+
+// gather.hip: pairs a slot of a wide pass's product takes (its launch's rows a pass)
+int gather3_part_rows(int epi, int K, int gs, bool alpha);
+
 // gather.hip: the tile gather (one 16-row weight tile over the whole K per wave)
 bool gather3_supported(int epi, int K, int N, int gs);
 // the fused MoE launch: up || gate with its routing, then down, in one persistent kernel
@@ -158,7 +181,7 @@ hipError_t launch_gather3(const GatherArgs& a, int epi, int rows, hipStream_t st
 #define MJ_ROPE_F 64
 struct RopeTab {
     const float* inv_freq;  // [half]
-    float2* cs;             // [MJ_ROWS][MJ_ROPE_F]
+    float2* cs;             // [rows][MJ_ROPE_F]
     int half;               // rope_dim / 2 (0: no RoPE layer in the model)
 };
 
@@ -334,7 +357,7 @@ struct RouteArgs {
     int act_n16;             // 16-byte chunk of them set to the marker 0xFFFF here, before it
 };
 bool route_supported(int H, int E, int k);
-hipError_t launch_route_logits(const RouteArgs& a, int H, hipStream_t st);
+hipError_t launch_route_logits(const RouteArgs& a, int H, hipStream_t st);  // up to MJ_WIDE_ROWS
 // inds and scores of every row from the logits
 hipError_t launch_route_topk(const RouteArgs& a, hipStream_t st);
 // y = [x_resid +] combine of the k expert rows (as launch_score_combine), then the norm of y

@@ -6,7 +6,8 @@
 // MJ_MAX_ROWS rows, an absolute offset (committed tokens).  A verify pass is one stream of
 // kernels (embed -> layers -> final norm -> lm_head (+ greedy acceptance in its final launch)
 // -> sampled acceptance -> KV commit for a tree -> result copy) with a single host wait.  Per-pass parameters live in a device StepDesc so the pass can be
-// captured once per (kind, rows) into a HIP graph and replayed.
+// captured once per (kind, rows, key depth) into a HIP graph and replayed; up to four 64-row chunks
+// of a prompt share a wide pass, launched eagerly.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -65,7 +66,8 @@ struct mj_model {
     int32_t *inds_all;
     float* scores_all;
     MoeScratch ms{};
-    StepDesc* sd_dev = nullptr;
+    int wide_rows = 0;            // rows a prefill pass may have (MJ_MAX_ROWS: no wide passes)
+    StepDesc* sd_dev = nullptr;   // one for each 64 rows of a pass
     StepDesc* sd_host = nullptr;
     StepResult* res_dev = nullptr;
     StepResult* res_host = nullptr;
@@ -136,33 +138,39 @@ static mj_status enqueue_layer(mj_model* m, int l, int M, int kind, hipStream_t 
     if (pf) pf->end(st);
     if (s != MJ_OK) return s;
     AttnArgs a{};
-    a.qkv = m->qkv;
     a.q_norm_w = (const uint16_t*)w.attn.q_norm_w;
     a.k_norm_w = (const uint16_t*)w.attn.k_norm_w;
-    a.rope_cs = m->rope_cs;
-    a.sd = m->sd_dev;
     a.kc = m->kv + (int64_t)l * m->layer_stride;
     a.vc = a.kc + (int64_t)nKV * c.kv_capacity * 128;
     a.opart = m->opart;
     a.mlpart = m->mlpart;
-    a.out_perm = m->aperm;
-    a.out_sum = m->asum;
-    a.M = M;
     a.nQ = nQ;
     a.nKV = nKV;
     a.rope_dim = m->lrope[l];
     a.window = m->lwin[l];
     a.max_chunks = m->max_chunks;
-    a.nch = m->lwin[l] > 0 ? attn_max_chunks(m->lwin[l], 0, M)
-                           : (m->deep ? m->max_chunks : MJ_ATTN_DEEP - 1);
     a.C = c.kv_capacity;
     a.eps = c.eps;
     a.scale = (float)std::pow((double)D, -0.5);
     a.abort = ab;
-    if (pf) pf->begin(PROF_ATTN, st);
-    s = mj_hip(ctx, launch_attn(a, st), "attention");
-    if (pf) pf->end(st);
-    if (s != MJ_OK) return s;
+    // a wide pass attends 64 rows at a time, each 64 after the keys of those before it are appended
+    for (int r0 = 0; r0 < M; r0 += MJ_MAX_ROWS) {
+        const int rows = std::min(M - r0, MJ_MAX_ROWS);
+        a.qkv = m->qkv + (size_t)r0 * qkvN;
+        a.rope_cs = m->rope_cs + (size_t)r0 * MJ_ROPE_F;
+        a.sd = m->sd_dev + r0 / MJ_MAX_ROWS;
+        a.out_perm = m->aperm + (size_t)r0 * nQ * 128;
+        a.out_sum = m->asum + (size_t)r0 * nQ * 2;
+        a.M = rows;
+        a.nch = m->lwin[l] > 0 ? attn_max_chunks(m->lwin[l], 0, rows)
+                : M > MJ_MAX_ROWS ? attn_max_chunks(0, m->offset + r0, rows)
+                : m->deep         ? m->max_chunks
+                                  : MJ_ATTN_DEEP - 1;
+        if (pf) pf->begin(PROF_ATTN, st);
+        s = mj_hip(ctx, launch_attn(a, st), "attention");
+        if (pf) pf->end(st);
+        if (s != MJ_OK) return s;
+    }
     GatherArgs o{};
     o.xperm = m->aperm;
     o.xsum = m->asum;
@@ -187,8 +195,9 @@ static mj_status enqueue_layer(mj_model* m, int l, int M, int kind, hipStream_t 
                                        hipMemcpyDeviceToDevice, st), "capture");
         if (s != MJ_OK) return s;
     }
-    int32_t* inds = m->inds_all + (size_t)l * MJ_MAX_ROWS * c.top_k;
-    float* scores = m->scores_all + (size_t)l * MJ_MAX_ROWS * c.top_k;
+    const bool wide = M > MJ_MAX_ROWS;
+    int32_t* inds = wide ? m->ms.inds : m->inds_all + (size_t)l * MJ_MAX_ROWS * c.top_k;
+    float* scores = wide ? m->ms.scores : m->scores_all + (size_t)l * MJ_MAX_ROWS * c.top_k;
     NormOut next{};
     const bool last = l + 1 == c.n_layers;
     if (!last)
@@ -212,6 +221,12 @@ static mj_status enqueue_layer(mj_model* m, int l, int M, int kind, hipStream_t 
         if (s != MJ_OK) return s;
     }
     return MJ_OK;
+}
+
+// Rows of a wide pass that go through the head: the last 64-row chunk's, as where the chunks are
+// passes of their own; the last row alone where no logits are captured (only its argmax is read).
+static int wide_head_rows(const mj_model* m, int M) {
+    return m->cap.logits ? (M - 1) % MJ_MAX_ROWS + 1 : 1;
 }
 
 static mj_status enqueue_pass(mj_model* m, int kind, int M, hipStream_t st) {
@@ -270,29 +285,33 @@ static mj_status enqueue_pass(mj_model* m, int kind, int M, hipStream_t st) {
         }
         float* logits =
             (sampled_pass(kind) || m->cap.logits) ? m->logits : nullptr;
+        const bool wide = M > MJ_MAX_ROWS;
+        const int hm = wide ? wide_head_rows(m, M) : M;
+        const uint16_t* xf = m->xf + (size_t)(M - hm) * H;
         // a greedy pass's acceptance runs in the head's final launch
         const int32_t* toks = (const int32_t*)((char*)m->sd_dev + offsetof(StepDesc, tokens));
         const int32_t* pars = (const int32_t*)((char*)m->sd_dev + offsetof(StepDesc, parents));
+        // (a wide pass's acceptance serves its argmax rows only: its chunk's tree is a chain)
         const GreedyAccept ga{toks, pars, m->res_dev};
         const GreedyAccept* gap = sampled_pass(kind) ? nullptr : &ga;
         if (m->profiling) m->prof.begin(PROF_HEAD, st);
         if (c.head_bits == 4)
             s = mj_hip(ctx,
-                       launch_lm_head_q4(m->xf, (const uint32_t*)m->lm_head,
+                       launch_lm_head_q4(xf, (const uint32_t*)m->lm_head,
                                          (const uint16_t*)c.lm_head_scales,
-                                         (const uint16_t*)c.lm_head_biases, M, H, c.vocab, nullptr,
+                                         (const uint16_t*)c.lm_head_biases, hm, H, c.vocab, nullptr,
                                          0, logits, m->pval, m->pidx, m->argmax, m->maxv,
                                          HeadLse{}, ab, st, gap),
                        "lm_head q4");
         else
-            s = mj_hip(ctx, launch_lm_head(m->xf, m->lm_head, M, H, c.vocab, nullptr, 0, logits,
+            s = mj_hip(ctx, launch_lm_head(xf, m->lm_head, hm, H, c.vocab, nullptr, 0, logits,
                                            m->pval, m->pidx, m->argmax, m->maxv, HeadLse{}, ab,
                                            st, gap),
                        "lm_head");
         if (m->profiling) m->prof.end(st);
         if (s != MJ_OK) return s;
         if (m->cap.logits) {
-            s = mj_hip(ctx, hipMemcpyAsync(m->cap.logits, m->logits, (size_t)M * c.vocab * 4,
+            s = mj_hip(ctx, hipMemcpyAsync(m->cap.logits, m->logits, (size_t)hm * c.vocab * 4,
                                            hipMemcpyDeviceToDevice, st), "capture");
             if (s != MJ_OK) return s;
         }
@@ -328,7 +347,8 @@ static mj_status run_pass(mj_model* m, int kind, int M) {
     mj_status s = mj_abort_begin(ctx, &gen);  // set: nothing is queued
     if (s != MJ_OK) return s;
     hipSetDevice(ctx->device);
-    s = mj_hip(ctx, hipMemcpyAsync(m->sd_dev, m->sd_host, sizeof(StepDesc),
+    s = mj_hip(ctx, hipMemcpyAsync(m->sd_dev, m->sd_host,
+                                   sizeof(StepDesc) * ((M + MJ_MAX_ROWS - 1) / MJ_MAX_ROWS),
                                    hipMemcpyHostToDevice, st), "descriptor upload");
     if (s != MJ_OK) return s;
     bool any_full = false;
@@ -337,7 +357,9 @@ static mj_status run_pass(mj_model* m, int kind, int M) {
     const mj_capture& cp = m->cap;
     const bool capturing = cp.h || cp.inds || cp.logits || cp.attn_out || cp.moe_in ||
                            cp.router_logits || cp.head_in || cp.kv_rows;
-    const bool capture_ok = m->graphs && !capturing && !m->profiling;
+    // (wide passes are launched one by one: a graph a prompt length would be built for each, and
+    // their kernels are long enough to cover the launches)
+    const bool capture_ok = m->graphs && !capturing && !m->profiling && M <= MJ_MAX_ROWS;
     m->prof.used = 0;
     // A profiled pass is queued behind a hold, so every kernel starts as soon as its
     // predecessor ends: its event pair then brackets the kernel, not the host's launch gap.
@@ -478,22 +500,26 @@ mj_status mj_model_create(mj_ctx* ctx, const mj_model_config* cfg, const mj_laye
     m->lm_head = (const uint16_t*)lm_head;
     const int H = c.H, nQ = c.n_heads, nKV = c.n_kv_heads, R = MJ_MAX_ROWS;
     const int qkvN = (nQ + 2 * nKV) * 128;
+    const bool wide_ok = moe_wide_supported(H, c.I, c.E, c.top_k, c.gs) &&
+                         gather3_supported(EPI_STORE, H, qkvN, c.gs) &&
+                         gather3_supported(EPI_ADD, nQ * 128, H, c.gs);
+    const int RW = m->wide_rows = wide_ok ? MJ_WIDE_ROWS : MJ_MAX_ROWS;
     m->layer_stride = 2LL * nKV * c.kv_capacity * 128;
     m->max_chunks = 0;
     for (int w : lwin) m->max_chunks = std::max(m->max_chunks, attn_max_chunks(w, c.kv_capacity, R));
     const int gqa = nQ / nKV;
     const int nqt16 = ((R * gqa + 15) / 16) * 16;
     auto layout = [&](Arena& a) {
-        m->h = (uint16_t*)a.take((size_t)R * H * 2);
-        m->xperm = (uint16_t*)a.take((size_t)R * H * 2);
-        m->xsum = (float2*)a.take((size_t)R * (H / 64) * 8);
-        m->qkv = (uint16_t*)a.take((size_t)R * qkvN * 2);
-        m->rope_cs = (float2*)a.take((size_t)R * MJ_ROPE_F * sizeof(float2));
+        m->h = (uint16_t*)a.take((size_t)RW * H * 2);
+        m->xperm = (uint16_t*)a.take((size_t)RW * H * 2);
+        m->xsum = (float2*)a.take((size_t)RW * (H / 64) * 8);
+        m->qkv = (uint16_t*)a.take((size_t)RW * qkvN * 2);
+        m->rope_cs = (float2*)a.take((size_t)RW * MJ_ROPE_F * sizeof(float2));
         m->opart = (float*)a.take((size_t)nKV * m->max_chunks * nqt16 * 128 * 4);
         m->mlpart = (float2*)a.take((size_t)nKV * m->max_chunks * nqt16 * 8);
-        m->aperm = (uint16_t*)a.take((size_t)R * nQ * 128 * 2);
-        m->asum = (float2*)a.take((size_t)R * nQ * 2 * 8);
-        m->xf = (uint16_t*)a.take((size_t)R * H * 2);
+        m->aperm = (uint16_t*)a.take((size_t)RW * nQ * 128 * 2);
+        m->asum = (float2*)a.take((size_t)RW * nQ * 2 * 8);
+        m->xf = (uint16_t*)a.take((size_t)RW * H * 2);
         m->pval = (float*)a.take((size_t)head_blocks() * 32 * 4);
         m->pidx = (int*)a.take((size_t)head_blocks() * 32 * 4);
         m->argmax = (int32_t*)a.take((size_t)R * 4);
@@ -506,19 +532,25 @@ mj_status mj_model_create(mj_ctx* ctx, const mj_model_config* cfg, const mj_laye
         nucleus_layout(a.take(nucleus_bytes(c.vocab)), c.vocab, m->nuc);
         m->inds_all = (int32_t*)a.take((size_t)c.n_layers * R * c.top_k * 4);
         m->scores_all = (float*)a.take((size_t)c.n_layers * R * c.top_k * 4);
-        m->sd_dev = (StepDesc*)a.take(sizeof(StepDesc));
+        m->sd_dev = (StepDesc*)a.take(sizeof(StepDesc) * (RW / MJ_MAX_ROWS));
         m->res_dev = (StepResult*)a.take(sizeof(StepResult));
         MoeScratch& ms = m->ms;
-        ms.xn = (uint16_t*)a.take((size_t)R * H * 2);
-        ms.xperm = (uint16_t*)a.take((size_t)R * H * 2);
-        ms.xsum = (float2*)a.take((size_t)R * (H / 64) * 8);
-        ms.logits = (float*)a.take((size_t)R * c.E * 4);
-        ms.inds = (int32_t*)a.take((size_t)R * c.top_k * 4);
-        ms.scores = (float*)a.take((size_t)R * c.top_k * 4);
+        ms.xn = (uint16_t*)a.take((size_t)RW * H * 2);
+        ms.xperm = (uint16_t*)a.take((size_t)RW * H * 2);
+        ms.xsum = (float2*)a.take((size_t)RW * (H / 64) * 8);
+        ms.logits = (float*)a.take((size_t)RW * c.E * 4);
+        ms.inds = (int32_t*)a.take((size_t)RW * c.top_k * 4);
+        ms.scores = (float*)a.take((size_t)RW * c.top_k * 4);
         ms.bk = (Buckets*)a.take(sizeof(Buckets));
-        ms.act = (uint16_t*)a.take((size_t)R * c.top_k * c.I * 2);
-        ms.act_sum = (float2*)a.take((size_t)R * c.top_k * (c.I / 64) * 8);
-        ms.down = (uint16_t*)a.take((size_t)R * c.top_k * H * 2);
+        ms.act = (uint16_t*)a.take((size_t)RW * c.top_k * c.I * 2);
+        ms.act_sum = (float2*)a.take((size_t)RW * c.top_k * (c.I / 64) * 8);
+        ms.down = (uint16_t*)a.take((size_t)RW * c.top_k * H * 2);
+        if (RW > R) {
+            for (SlotTab* tab : {&ms.up_tab, &ms.dn_tab}) {
+                tab->n = slot_tab_size(MJ_MAX_EXPERTS, MJ_SLOT_PS_MIN);
+                tab->rec = (int32_t*)a.take((size_t)tab->n * 16 * 4);
+            }
+        }
     };
     Arena count;
     layout(count);
@@ -528,7 +560,7 @@ mj_status mj_model_create(mj_ctx* ctx, const mj_model_config* cfg, const mj_laye
     if (hipMalloc(&m->arena, count.off) != hipSuccess ||
         hipMalloc(&m->kv, (size_t)c.n_layers * m->layer_stride * 2) != hipSuccess ||
         hipMalloc(&m->inv_freq, inv.size() * 4) != hipSuccess ||
-        hipHostMalloc(&m->sd_host, sizeof(StepDesc), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc(&m->sd_host, sizeof(StepDesc) * (RW / MJ_MAX_ROWS), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc(&m->res_host, sizeof(StepResult), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc(&m->hist_host, (size_t)2 * MJ_MAX_HIST * 4, hipHostMallocDefault) !=
             hipSuccess ||
@@ -538,7 +570,7 @@ mj_status mj_model_create(mj_ctx* ctx, const mj_model_config* cfg, const mj_laye
     }
     Arena real{m->arena, 0};
     layout(real);
-    std::memset(m->sd_host, 0, sizeof(StepDesc));
+    std::memset(m->sd_host, 0, sizeof(StepDesc) * (RW / MJ_MAX_ROWS));
     std::memset(m->res_host, 0, sizeof(StepResult));
     s = mj_hip(ctx, hipMemcpy(m->inv_freq, inv.data(), inv.size() * 4, hipMemcpyHostToDevice),
                "inv_freq upload");
@@ -661,16 +693,56 @@ static mj_status feed_rows(mj_model* m, const int32_t* tokens, const int32_t* pa
     return run_pass(m, kind, M);
 }
 
+// Rows of the next pass of a prompt of n more tokens in 64-row chunks: whole chunks together where
+// the wide pass can take them, up to the first chunk that would be refused (a pass of its own then
+// refuses it, with the chunks before it committed).
+static int wide_span(mj_model* m, const int32_t* tokens, int n) {
+    const mj_capture& cp = m->cap;
+    const int most = std::min(n, m->wide_rows);
+    if (most <= MJ_MAX_ROWS || m->profiling || cp.h || cp.inds || cp.attn_out || cp.moe_in ||
+        cp.router_logits || cp.head_in || cp.kv_rows)
+        return std::min(n, MJ_MAX_ROWS);
+    bool any_full = false;
+    for (int w : m->lwin) any_full = any_full || w <= 0;
+    int rows = 0;
+    while (rows < most) {
+        const int M = std::min(most - rows, MJ_MAX_ROWS);
+        bool ok = !any_full || m->offset + rows + M <= m->cfg.kv_capacity;
+        for (int r = 0; r < M; ++r)
+            ok = ok && tokens[rows + r] >= 0 && tokens[rows + r] < m->cfg.vocab;
+        if (!ok) break;
+        rows += M;
+    }
+    return rows > 0 ? rows : std::min(n, MJ_MAX_ROWS);
+}
+
+// A wide pass over rows that wide_span() found good: one descriptor for each 64 rows.
+static mj_status feed_wide(mj_model* m, const int32_t* tokens, int M, int kind) {
+    for (int r0 = 0; r0 < M; r0 += MJ_MAX_ROWS) {
+        StepDesc* sd = m->sd_host + r0 / MJ_MAX_ROWS;
+        sd->L = m->offset + r0;
+        sd->M = std::min(M - r0, MJ_MAX_ROWS);
+        std::copy(tokens + r0, tokens + r0 + sd->M, sd->tokens);
+        mj_status s = fill_tree(m->ctx, sd, nullptr, sd->M);
+        if (s != MJ_OK) return s;
+    }
+    return run_pass(m, kind, M);
+}
+
 mj_status mj_prefill(mj_model* m, const int32_t* tokens, int n, int chunk, int32_t* out_next) {
     if (!m || !tokens || n < 1) return MJ_INVALID_ARG;
     if (chunk < 1 || chunk > MJ_MAX_ROWS) chunk = MJ_MAX_ROWS;
-    for (int i = 0; i < n; i += chunk) {
-        const int M = n - i < chunk ? n - i : chunk;
-        const bool last = i + M >= n;
-        mj_status s = feed_rows(m, tokens + i, nullptr, M, last ? PASS_CHAIN : PASS_PREFILL);
+    for (int i = 0; i < n;) {
+        const int M = chunk < MJ_MAX_ROWS ? std::min(n - i, chunk) : wide_span(m, tokens + i, n - i);
+        const bool last = i + M >= n, wide = M > MJ_MAX_ROWS;
+        const int kind = last ? PASS_CHAIN : PASS_PREFILL;
+        mj_status s = wide ? feed_wide(m, tokens + i, M, kind)
+                           : feed_rows(m, tokens + i, nullptr, M, kind);
         if (s != MJ_OK) return s;
         m->offset += M;
-        if (last && out_next) *out_next = m->res_host->argmax[M - 1];
+        i += M;
+        if (last && out_next)
+            *out_next = m->res_host->argmax[(wide ? wide_head_rows(m, M) : M) - 1];
     }
     return MJ_OK;
 }

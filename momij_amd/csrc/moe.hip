@@ -10,6 +10,8 @@
 //            grouped by expert so every routed expert is streamed once for all its rows.
 // Combine    maple_score_reduce / maple_score_resid (2452-2493):
 //            y = [x +] half(sum_j half(down_j) * score_j), j in slot order.
+#include <initializer_list>
+
 #include "mj_device.h"
 #include "mj_internal.h"
 #include "moe_topk.h"
@@ -436,15 +438,19 @@ hipError_t launch_combine_norm(const uint16_t* down, const float* scores, const 
 // ---------------------------------------------------------------------------------------
 #define RS_EPB 8  // router rows (experts) per block: two per wave
 
+// RPB: rows a block takes (its experts' router rows are read once for them): one, so that few rows
+// still fill the chip, four in passes past 64 rows (200 rows
+// of 256 experts: 17 us, as passes of 64 rows 26).
+template <int RPB>
 __global__ __launch_bounds__(256) void k_route_logits(RouteArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int E = a.E, S = E / RS_EPB;
-    const int r = blockIdx.x / S, grp = blockIdx.x - r * S;
-    __shared__ __align__(16) uint16_t xn[RT_H];
-    __shared__ float s_ss[4];
+    const int r0 = blockIdx.x / S * RPB, grp = blockIdx.x % S;
+    __shared__ __align__(16) uint16_t xn[RPB][RT_H];
+    __shared__ float s_ss[RPB][4];
     if (aborted(a.abort)) return;
 
-    // router rows of this wave first (k = 512 c + 8 lane .. +7), then the row
+    // router rows of this wave first (k = 512 c + 8 lane .. +7), then the rows (clamped past M)
     const int e0 = grp * RS_EPB + 2 * wv;
     u4v wr[2][4];
 #pragma unroll
@@ -452,58 +458,78 @@ __global__ __launch_bounds__(256) void k_route_logits(RouteArgs a) {
 #pragma unroll
         for (int c = 0; c < 4; ++c)
             wr[j][c] = *(const u4v*)(a.W + (size_t)(e0 + j) * RT_H + 512 * c + 8 * lane);
-    u4v xv = *(const u4v*)(a.x + (size_t)r * RT_H + 8 * tid);
+    u4v xv[RPB];
+#pragma unroll
+    for (int i = 0; i < RPB; ++i)
+        xv[i] = *(const u4v*)(a.x + (size_t)min(r0 + i, a.M - 1) * RT_H + 8 * tid);
     u4v nw = {0u, 0u, 0u, 0u};
     if (a.norm_w) nw = *(const u4v*)(a.norm_w + 8 * tid);
 
     if (a.norm_w) {
-        float ss = 0.0f;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float x0 = h2f(xv[q] & 0xFFFFu), x1 = h2f(xv[q] >> 16);
-            ss += x0 * x0;
-            ss += x1 * x1;
+        for (int i = 0; i < RPB; ++i) {
+            float ss = 0.0f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float x0 = h2f(xv[i][q] & 0xFFFFu), x1 = h2f(xv[i][q] >> 16);
+                ss += x0 * x0;
+                ss += x1 * x1;
+            }
+            ss = wave_sum(ss);
+            if (lane == 0) s_ss[i][wv] = ss;
         }
-        ss = wave_sum(ss);
-        if (lane == 0) s_ss[wv] = ss;
         __syncthreads();
-        const float tot = (s_ss[0] + s_ss[1]) + (s_ss[2] + s_ss[3]);
-        const float inv = 1.0f / sqrtf(tot / (float)RT_H + a.eps);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float x0 = h2f(xv[q] & 0xFFFFu) * inv * h2f(nw[q] & 0xFFFFu);
-            const float x1 = h2f(xv[q] >> 16) * inv * h2f(nw[q] >> 16);
-            xv[q] = (uint32_t)f2h(x0) | ((uint32_t)f2h(x1) << 16);
+        for (int i = 0; i < RPB; ++i) {
+            const float tot = (s_ss[i][0] + s_ss[i][1]) + (s_ss[i][2] + s_ss[i][3]);
+            const float inv = 1.0f / sqrtf(tot / (float)RT_H + a.eps);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float x0 = h2f(xv[i][q] & 0xFFFFu) * inv * h2f(nw[q] & 0xFFFFu);
+                const float x1 = h2f(xv[i][q] >> 16) * inv * h2f(nw[q] >> 16);
+                xv[i][q] = (uint32_t)f2h(x0) | ((uint32_t)f2h(x1) << 16);
+            }
         }
     }
-    *(u4v*)(xn + 8 * tid) = xv;
+#pragma unroll
+    for (int i = 0; i < RPB; ++i) *(u4v*)(xn[i] + 8 * tid) = xv[i];
     // the fused MoE launch's act rows: the "not yet written" marker, before that launch starts
     for (int i = blockIdx.x * 256 + tid; i < a.act_n16; i += gridDim.x * 256)
         ((u4v*)a.act_mark)[i] = (u4v){~0u, ~0u, ~0u, ~0u};
     if (grp == 0) {
-        if (a.xn) *(u4v*)(a.xn + (size_t)r * RT_H + 8 * tid) = xv;
-        if (a.xperm)
-            emit_qx(xv, lane, a.xperm + (size_t)r * RT_H, a.xsum + (size_t)r * (RT_H / 64), 8 * tid);
+#pragma unroll
+        for (int i = 0; i < RPB; ++i) {
+            const int r = r0 + i;
+            if (r >= a.M) break;
+            if (a.xn) *(u4v*)(a.xn + (size_t)r * RT_H + 8 * tid) = xv[i];
+            if (a.xperm)
+                emit_qx(xv[i], lane, a.xperm + (size_t)r * RT_H, a.xsum + (size_t)r * (RT_H / 64),
+                        8 * tid);
+        }
     }
     __syncthreads();
 
-    u4v xa[4];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) xa[c] = *(const u4v*)(xn + 512 * c + 8 * lane);
-    float acc[2];
+    for (int i = 0; i < RPB; ++i) {
+        u4v xa[4];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        acc[j] = 0.0f;
+        for (int c = 0; c < 4; ++c) xa[c] = *(const u4v*)(xn[i] + 512 * c + 8 * lane);
+        float acc[2];
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
+        for (int j = 0; j < 2; ++j) {
+            acc[j] = 0.0f;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) acc[j] = dot2(wr[j][c][q], xa[c][q], acc[j]);
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc[j] = dot2(wr[j][c][q], xa[c][q], acc[j]);
+        }
+#pragma unroll
+        for (int m = 32; m > 0; m >>= 1)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[j] += __shfl_xor(acc[j], m, MJ_WAVE);
+        if (lane == 0 && r0 + i < a.M)
+            *(float2*)(a.logits + (size_t)(r0 + i) * E + e0) = make_float2(acc[0], acc[1]);
     }
-#pragma unroll
-    for (int m = 32; m > 0; m >>= 1)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[j] += __shfl_xor(acc[j], m, MJ_WAVE);
-    if (lane == 0) *(float2*)(a.logits + (size_t)r * E + e0) = make_float2(acc[0], acc[1]);
 }
 
 // inds and scores of every row: one wave a row, four rows a block.  (One 16-wave block for the
@@ -541,20 +567,106 @@ bool route_supported(int H, int E, int k) {
 }
 
 hipError_t launch_route_logits(const RouteArgs& a, int H, hipStream_t st) {
-    if (!route_supported(H, a.E, a.k) || a.M < 1 || a.M > MJ_ROWS) return hipErrorInvalidValue;
+    if (!route_supported(H, a.E, a.k) || a.M < 1 || a.M > MJ_WIDE_ROWS) return hipErrorInvalidValue;
     if (!a.logits) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_route_logits, dim3(a.M * (a.E / RS_EPB)), dim3(256), 0, st, a);
+    if (a.M <= MJ_ROWS)
+        hipLaunchKernelGGL(k_route_logits<1>, dim3(a.M * (a.E / RS_EPB)), dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL(k_route_logits<4>, dim3((a.M + 3) / 4 * (a.E / RS_EPB)), dim3(256), 0, st,
+                           a);
     return hipGetLastError();
 }
 
 hipError_t launch_route_topk(const RouteArgs& a, hipStream_t st) {
     if (a.E < 1 || a.E > MJ_MAX_EXPERTS || a.k < 1 || a.k > 8 || a.k > a.E || a.M < 1 ||
-        a.M > MJ_ROWS)
+        a.M > MJ_WIDE_ROWS)
         return hipErrorInvalidValue;
     const dim3 grid((a.M + RT_WAVES - 1) / RT_WAVES), block(64 * RT_WAVES);
     if (a.E <= 64)
         hipLaunchKernelGGL(k_route_topk<1>, grid, block, 0, st, a);
     else
         hipLaunchKernelGGL(k_route_topk<MJ_MAX_EXPERTS / 64>, grid, block, 0, st, a);
+    return hipGetLastError();
+}
+
+// The slot tables of a wide pass's two expert products, from its pairs' expert ids: one block,
+// thread t < 256 numbering expert t's slots by sums across the experts, then a pair a thread
+// taking the next place of its expert.  The places' order varies from run to run, which moves rows
+// within a slot and changes no value.
+__global__ __launch_bounds__(1024) void k_wide_slots(const int32_t* __restrict__ inds, int P,
+                                                     SlotTab up, SlotTab dn, const int* abort) {
+    __shared__ int s_cnt[MJ_MAX_EXPERTS], s_at[MJ_MAX_EXPERTS], s_first[2][MJ_MAX_EXPERTS];
+    __shared__ int s_tot[2][4];
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    constexpr int PT = MJ_WIDE_PAIRS / 1024;
+    int id[PT];
+#pragma unroll
+    for (int i = 0; i < PT; ++i) id[i] = t + 1024 * i < P ? inds[t + 1024 * i] : -1;
+    if (aborted(abort)) return;
+    if (t < MJ_MAX_EXPERTS) s_cnt[t] = s_at[t] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PT; ++i)
+        if ((unsigned)id[i] < (unsigned)MJ_MAX_EXPERTS) atomicAdd(&s_cnt[id[i]], 1);
+    __syncthreads();
+    int incl[2] = {0, 0}, parts[2] = {0, 0};
+    if (t < MJ_MAX_EXPERTS) {
+        const int c = s_cnt[t];
+        parts[0] = (c + up.ps - 1) / up.ps;
+        parts[1] = (c + dn.ps - 1) / dn.ps;
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            incl[x] = parts[x];
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(incl[x], o, MJ_WAVE);
+                if (lane >= o) incl[x] += y;
+            }
+            if (lane == 63) s_tot[x][wv] = incl[x];
+        }
+    }
+    __syncthreads();
+    if (t < MJ_MAX_EXPERTS) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            for (int w = 0; w < wv; ++w) incl[x] += s_tot[x][w];
+            s_first[x][t] = incl[x] - parts[x];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+        const SlotTab& tab = x ? dn : up;
+        const int n = ((s_tot[x][0] + s_tot[x][1]) + s_tot[x][2]) + s_tot[x][3];
+        for (int sl = n + t; sl < tab.n; sl += 1024) *(int2*)(tab.rec + 16 * sl) = make_int2(0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < PT; ++i) {
+        const int e = id[i], p = t + 1024 * i;
+        if ((unsigned)e >= (unsigned)MJ_MAX_EXPERTS) continue;
+        const int c = s_cnt[e], at = atomicAdd(&s_at[e], 1);
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            // the first `more` slots take one pair more than the others
+            const SlotTab& tab = x ? dn : up;
+            const int np = (c + tab.ps - 1) / tab.ps, base = c / np, more = c - base * np;
+            const int lead = more * (base + 1);
+            const int sl = at < lead ? at / (base + 1) : more + (at - lead) / base;
+            const int off = at < lead ? at - sl * (base + 1) : (at - lead) - (sl - more) * base;
+            const int cnt = base + (sl < more ? 1 : 0);
+            int32_t* rec = tab.rec + 16 * (s_first[x][e] + sl);
+            rec[off] = p | (off == 0 ? e << 16 : off == 1 ? cnt << 16 : 0);
+            if (cnt == 1) rec[1] = 1 << 16;
+        }
+    }
+}
+
+hipError_t launch_wide_slots(const int32_t* inds, int P, const SlotTab& up, const SlotTab& dn,
+                             const int* abort, hipStream_t st) {
+    for (const SlotTab* tab : {&up, &dn})
+        if (tab->ps < 1 || tab->ps > 16 || tab->n < slot_tab_size(MJ_MAX_EXPERTS, tab->ps))
+            return hipErrorInvalidValue;
+    if (P < 1 || P > MJ_WIDE_PAIRS) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_wide_slots, dim3(1), dim3(1024), 0, st, inds, P, up, dn, abort);
     return hipGetLastError();
 }

@@ -431,7 +431,7 @@ static hipError_t launch_gather_t(const GatherArgs& a, int n_buckets_max, hipStr
 hipError_t launch_gather(const GatherArgs& a, int epi, int max_rows_per_bucket, int n_buckets_max,
                          hipStream_t st) {
     // the tile kernel: dense, or over the pairs' expert ids; its SWIGLU is the experts' only
-    const bool per = a.inds != nullptr || a.rlogits != nullptr;
+    const bool per = a.inds != nullptr || a.rlogits != nullptr || a.tab != nullptr;
     if (a.bk == nullptr && (per || epi != EPI_SWIGLU) && gather3_supported(epi, a.K, a.N, a.gs))
         return launch_gather3(a, epi, max_rows_per_bucket, st);
     if (per) return hipErrorInvalidValue;

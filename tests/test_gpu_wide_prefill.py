@@ -1,0 +1,100 @@
+"""GPU: a prompt's 64-row chunks sharing a wide pass give the same bits as passes of their own."""
+import numpy as np
+import pytest
+
+from momij_amd import _lib
+from momij_amd._lib import MomijError
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from momij_amd.ops import Context
+
+    c = Context(0)
+    yield c
+    c.close()
+
+
+def _engine(ctx, E, I, gs, alpha, top_k, capacity):
+    import torch
+
+    from momij_amd.engine import MapleLikeConfig, VerifyEngine, random_model
+
+    wins, ropes = MapleLikeConfig.maple_layer_mix(2, 96, 64, ["sliding_attention", "full"])
+    cfg = MapleLikeConfig(n_layers=2, E=E, I=I, gs=gs, top_k=top_k, vocab=2048, window=96,
+                          kv_capacity=capacity, layer_window=wins, layer_rope_dim=ropes)
+    layers, *rest = random_model(cfg, seed=E + I)
+    if alpha:  # scale alpha, bias -alpha in every group of a row
+        for lw in layers:
+            for nm in ("up_gate", "down"):
+                m = lw["moe"]
+                al = m[nm + "_s"][..., 0].contiguous()
+                m[nm + "_s"] = al[..., None].expand_as(m[nm + "_s"]).contiguous()
+                m[nm + "_b"] = -m[nm + "_s"]
+                m[nm + "_alpha"] = al
+    torch.cuda.synchronize()
+    return VerifyEngine(ctx, cfg, layers, *rest), cfg
+
+
+def _cache(eng, cfg):
+    import torch
+
+    class View:
+        def __init__(self, p):
+            self.__cuda_array_interface__ = dict(
+                data=(p, False), shape=(cfg.n_kv_heads, cfg.kv_capacity, cfg.head_dim),
+                typestr="<f2", version=2)
+
+    return [torch.as_tensor(View(p), device="cuda").cpu().numpy().view(np.uint16)
+            for l in range(cfg.n_layers) for p in eng.kv(l)]
+
+
+# experts with one slot and with many (8 experts, all routed by every row), each group size, rows
+# with and without one alpha, both down widths
+@pytest.mark.parametrize("E,I,gs,alpha,top_k", [
+    (64, 1024, 64, False, 8), (256, 512, 128, True, 8), (8, 1024, 128, False, 8),
+    (40, 512, 64, True, 3), (16, 1024, 64, True, 4), (24, 512, 128, False, 1)])
+def test_wide_equals_chunk_passes(ctx, E, I, gs, alpha, top_k):
+    import torch
+
+    print(f"case: wide prefill E={E} I={I} gs={gs} alpha={alpha} top_k={top_k}", flush=True)
+    eng, cfg = _engine(ctx, E, I, gs, alpha, top_k, 640)
+    rng = np.random.default_rng(E)
+    logits = torch.zeros((_lib.MJ_MAX_ROWS, cfg.vocab), device="cuda")
+    for n in (65, 200, 256, 257, 500):
+        prompt = rng.integers(0, cfg.vocab, n).tolist()
+        eng.rewind(0)
+        for i in range(0, n, 64):  # passes of their own
+            last = eng.step_chain_feeds(prompt[i:i + 64])
+        ref = _cache(eng, cfg)
+        eng.set_capture(logits=logits)
+        eng.rewind(n - len(last))
+        eng.step_chain_feeds(prompt[n - len(last):])
+        ref_logits = logits[:len(last)].clone()
+        for capture in (True, False):
+            eng.set_capture(logits=logits if capture else None)
+            eng.rewind(0)
+            logits.zero_()
+            torch.cuda.synchronize()
+            assert eng.prefill(prompt) == last[-1] and eng.offset == n
+            for a, b in zip(_cache(eng, cfg), ref):
+                assert (a == b).all(), n
+            if capture:
+                assert torch.equal(logits[:len(last)], ref_logits), n
+    eng.close()
+
+
+def test_wide_refusals(ctx):
+    """A bad token, or a prompt past the capacity, is refused at its chunk, the chunks before it
+    committed."""
+    eng, cfg = _engine(ctx, 16, 512, 64, False, 4, 320)
+    prompt = [int(t) for t in np.random.default_rng(1).integers(0, cfg.vocab, 400)]
+    for bad, at, status in ((prompt[:150] + [cfg.vocab] + prompt[150:200], 128, 4),
+                            ([-1] + prompt[:100], 0, 4), (prompt, 320, 7)):
+        eng.rewind(0)
+        with pytest.raises(MomijError) as e:
+            eng.prefill(bad)
+        assert e.value.status == status and eng.offset == at, (e.value, eng.offset)
+    eng.close()
