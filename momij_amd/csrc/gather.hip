@@ -1084,6 +1084,12 @@ hipError_t launch_gather3(const GatherArgs& a, int epi, int rows, hipStream_t st
     // one block unpacking its tile again for every further 16 rows.
     const int groups = (a.dense_rows + 15) / 16;
     rows = rows < 16 ? rows : 16;
+    // Past 16 rows at group 128 (two K-slices): 16 staged rows leave LDS for one block a CU, of four
+    // waves or of eight; eight: qkv of 64 rows 9.4 -> 6.3 us, of 200 19.6 -> 13.7, o-proj of 200
+    // 16.6 -> 11.3.  (Group 64's four slices of a tile fit two blocks.)
+    if (a.K == 2048 && a.gs == 128 && a.dense_rows > 16)
+        return epi == EPI_ADD ? launch_g5<8, 128, EPI_ADD, 8, 2>(a, rows, groups, st)
+                              : launch_g5<8, 128, EPI_STORE, 8, 2>(a, rows, groups, st);
 #define MJ_G5D(KPL, E, W, KS64, KS128)                                                    \
     return a.gs == 64 ? launch_g5<KPL, 64, E, W, KS64>(a, rows, groups, st)               \
                       : launch_g5<KPL, 128, E, W, KS128>(a, rows, groups, st);
@@ -1201,6 +1207,8 @@ hipError_t set_gather3_attributes() {
     MJ_A(2, EPI_STORE, 8, 1, 1, REC_NONE, false)
     MJ_A(4, EPI_STORE, 8, 1, 1, REC_NONE, false)
     MJ_A(8, EPI_STORE, 4, 4, 2, REC_NONE, false)
+    MJ_A(8, EPI_STORE, 8, 4, 2, REC_NONE, false)
+    MJ_A(8, EPI_ADD, 8, 4, 2, REC_NONE, false)
     MJ_A(8, EPI_SWIGLU, 8, 2, 2, REC_RANK, false)
     MJ_A(8, EPI_SWIGLU, 8, 2, 2, REC_RANK, true)
     MJ_A(8, EPI_SWIGLU, 8, 2, 2, REC_IDS, false)

@@ -438,19 +438,15 @@ hipError_t launch_combine_norm(const uint16_t* down, const float* scores, const 
 // ---------------------------------------------------------------------------------------
 #define RS_EPB 8  // router rows (experts) per block: two per wave
 
-// RPB: rows a block takes (its experts' router rows are read once for them): one, so that few rows
-// still fill the chip, four in passes past 64 rows (200 rows
-// of 256 experts: 17 us, as passes of 64 rows 26).
-template <int RPB>
 __global__ __launch_bounds__(256) void k_route_logits(RouteArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int E = a.E, S = E / RS_EPB;
-    const int r0 = blockIdx.x / S * RPB, grp = blockIdx.x % S;
-    __shared__ __align__(16) uint16_t xn[RPB][RT_H];
-    __shared__ float s_ss[RPB][4];
+    const int r = blockIdx.x / S, grp = blockIdx.x - r * S;
+    __shared__ __align__(16) uint16_t xn[RT_H];
+    __shared__ float s_ss[4];
     if (aborted(a.abort)) return;
 
-    // router rows of this wave first (k = 512 c + 8 lane .. +7), then the rows (clamped past M)
+    // router rows of this wave first (k = 512 c + 8 lane .. +7), then the row
     const int e0 = grp * RS_EPB + 2 * wv;
     u4v wr[2][4];
 #pragma unroll
@@ -458,77 +454,118 @@ __global__ __launch_bounds__(256) void k_route_logits(RouteArgs a) {
 #pragma unroll
         for (int c = 0; c < 4; ++c)
             wr[j][c] = *(const u4v*)(a.W + (size_t)(e0 + j) * RT_H + 512 * c + 8 * lane);
-    u4v xv[RPB];
-#pragma unroll
-    for (int i = 0; i < RPB; ++i)
-        xv[i] = *(const u4v*)(a.x + (size_t)min(r0 + i, a.M - 1) * RT_H + 8 * tid);
+    u4v xv = *(const u4v*)(a.x + (size_t)r * RT_H + 8 * tid);
     u4v nw = {0u, 0u, 0u, 0u};
     if (a.norm_w) nw = *(const u4v*)(a.norm_w + 8 * tid);
 
     if (a.norm_w) {
+        float ss = 0.0f;
 #pragma unroll
-        for (int i = 0; i < RPB; ++i) {
-            float ss = 0.0f;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float x0 = h2f(xv[i][q] & 0xFFFFu), x1 = h2f(xv[i][q] >> 16);
-                ss += x0 * x0;
-                ss += x1 * x1;
-            }
-            ss = wave_sum(ss);
-            if (lane == 0) s_ss[i][wv] = ss;
+        for (int q = 0; q < 4; ++q) {
+            const float x0 = h2f(xv[q] & 0xFFFFu), x1 = h2f(xv[q] >> 16);
+            ss += x0 * x0;
+            ss += x1 * x1;
         }
+        ss = wave_sum(ss);
+        if (lane == 0) s_ss[wv] = ss;
         __syncthreads();
+        const float tot = (s_ss[0] + s_ss[1]) + (s_ss[2] + s_ss[3]);
+        const float inv = 1.0f / sqrtf(tot / (float)RT_H + a.eps);
 #pragma unroll
-        for (int i = 0; i < RPB; ++i) {
-            const float tot = (s_ss[i][0] + s_ss[i][1]) + (s_ss[i][2] + s_ss[i][3]);
-            const float inv = 1.0f / sqrtf(tot / (float)RT_H + a.eps);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float x0 = h2f(xv[i][q] & 0xFFFFu) * inv * h2f(nw[q] & 0xFFFFu);
-                const float x1 = h2f(xv[i][q] >> 16) * inv * h2f(nw[q] >> 16);
-                xv[i][q] = (uint32_t)f2h(x0) | ((uint32_t)f2h(x1) << 16);
-            }
+        for (int q = 0; q < 4; ++q) {
+            const float x0 = h2f(xv[q] & 0xFFFFu) * inv * h2f(nw[q] & 0xFFFFu);
+            const float x1 = h2f(xv[q] >> 16) * inv * h2f(nw[q] >> 16);
+            xv[q] = (uint32_t)f2h(x0) | ((uint32_t)f2h(x1) << 16);
         }
     }
-#pragma unroll
-    for (int i = 0; i < RPB; ++i) *(u4v*)(xn[i] + 8 * tid) = xv[i];
+    *(u4v*)(xn + 8 * tid) = xv;
     // the fused MoE launch's act rows: the "not yet written" marker, before that launch starts
     for (int i = blockIdx.x * 256 + tid; i < a.act_n16; i += gridDim.x * 256)
         ((u4v*)a.act_mark)[i] = (u4v){~0u, ~0u, ~0u, ~0u};
     if (grp == 0) {
-#pragma unroll
-        for (int i = 0; i < RPB; ++i) {
-            const int r = r0 + i;
-            if (r >= a.M) break;
-            if (a.xn) *(u4v*)(a.xn + (size_t)r * RT_H + 8 * tid) = xv[i];
-            if (a.xperm)
-                emit_qx(xv[i], lane, a.xperm + (size_t)r * RT_H, a.xsum + (size_t)r * (RT_H / 64),
-                        8 * tid);
-        }
+        if (a.xn) *(u4v*)(a.xn + (size_t)r * RT_H + 8 * tid) = xv;
+        if (a.xperm)
+            emit_qx(xv, lane, a.xperm + (size_t)r * RT_H, a.xsum + (size_t)r * (RT_H / 64), 8 * tid);
     }
     __syncthreads();
 
+    u4v xa[4];
 #pragma unroll
-    for (int i = 0; i < RPB; ++i) {
-        u4v xa[4];
+    for (int c = 0; c < 4; ++c) xa[c] = *(const u4v*)(xn + 512 * c + 8 * lane);
+    float acc[2];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) xa[c] = *(const u4v*)(xn[i] + 512 * c + 8 * lane);
-        float acc[2];
+    for (int j = 0; j < 2; ++j) {
+        acc[j] = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            acc[j] = 0.0f;
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc[j] = dot2(wr[j][c][q], xa[c][q], acc[j]);
+    }
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[j] += __shfl_xor(acc[j], m, MJ_WAVE);
+    if (lane == 0) *(float2*)(a.logits + (size_t)r * E + e0) = make_float2(acc[0], acc[1]);
+}
+
+// The logits of a wide pass, from rows already normed: a wave keeps four experts' router rows in
+// registers over RW_ROWS rows, two at a time.  Its eight sums meet by halves: at each of the first
+// three lane distances a lane keeps half of its sums and takes the other lane's part of them, so the
+// additions are those of k_route_logits' tree with 10 lane moves for eight sums instead of 48.
+// Norming again in each of 32 blocks a row, with an LDS copy of it, took 17 us for 200 rows of 256
+// experts; the norm launch and this one 14.4.
+#define RW_ROWS 8
+__global__ __launch_bounds__(256) void k_route_wide(RouteArgs a) {
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int E = a.E, G = (E + 15) / 16;
+    const int r0 = blockIdx.x / G * RW_ROWS, e0 = blockIdx.x % G * 16 + 4 * wv;
+    if (aborted(a.abort) || e0 >= E) return;
+    u4v wr[4][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            wr[j][c] = *(const u4v*)(a.W + (size_t)min(e0 + j, E - 1) * RT_H + 512 * c + 8 * lane);
+    u4v xa[2][2][4];
+    auto request = [&](int r, u4v (&x)[2][4]) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int c = 0; c < 4; ++c)
+                x[i][c] = *(const u4v*)(a.x + (size_t)min(r + i, a.M - 1) * RT_H + 512 * c + 8 * lane);
+    };
+    request(r0, xa[0]);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) acc[j] = dot2(wr[j][c][q], xa[c][q], acc[j]);
+    for (int it = 0; it < RW_ROWS / 2; ++it) {
+        const int r = r0 + 2 * it;
+        if (r >= a.M) break;
+        if (it + 1 < RW_ROWS / 2) request(r + 2, xa[(it + 1) & 1]);
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                float acc = 0.0f;
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) acc = dot2(wr[j][c][q], xa[it & 1][i][c][q], acc);
+                v[4 * i + j] = acc;
+            }
+#pragma unroll
+        for (int m = 32, n = 4; m > 4; m >>= 1, n >>= 1) {
+            const bool up = (lane & m) != 0;
+#pragma unroll
+            for (int i = 0; i < n; ++i) {
+                const float keep = up ? v[i + n] : v[i], send = up ? v[i] : v[i + n];
+                v[i] = keep + __shfl_xor(send, m, MJ_WAVE);
+            }
         }
 #pragma unroll
-        for (int m = 32; m > 0; m >>= 1)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[j] += __shfl_xor(acc[j], m, MJ_WAVE);
-        if (lane == 0 && r0 + i < a.M)
-            *(float2*)(a.logits + (size_t)(r0 + i) * E + e0) = make_float2(acc[0], acc[1]);
+        for (int m = 4; m > 0; m >>= 1) v[0] += __shfl_xor(v[0], m, MJ_WAVE);
+        // lane 8 s: sum s = 4 i + j (bit 5 of the lane chose i, bits 4 and 3 j)
+        const int row = r + (lane >> 5), e = e0 + ((lane >> 3) & 3);
+        if ((lane & 7) == 0 && row < a.M && e < E) a.logits[(size_t)row * E + e] = v[0];
     }
 }
 
@@ -569,11 +606,18 @@ bool route_supported(int H, int E, int k) {
 hipError_t launch_route_logits(const RouteArgs& a, int H, hipStream_t st) {
     if (!route_supported(H, a.E, a.k) || a.M < 1 || a.M > MJ_WIDE_ROWS) return hipErrorInvalidValue;
     if (!a.logits) return hipErrorInvalidValue;
-    if (a.M <= MJ_ROWS)
-        hipLaunchKernelGGL(k_route_logits<1>, dim3(a.M * (a.E / RS_EPB)), dim3(256), 0, st, a);
-    else
-        hipLaunchKernelGGL(k_route_logits<4>, dim3((a.M + 3) / 4 * (a.E / RS_EPB)), dim3(256), 0, st,
-                           a);
+    if (a.M <= MJ_ROWS) {
+        hipLaunchKernelGGL(k_route_logits, dim3(a.M * (a.E / RS_EPB)), dim3(256), 0, st, a);
+        return hipGetLastError();
+    }
+    // a wide pass: the rows normed by a launch of their own (into xn, and in qx order)
+    if (!a.norm_w || !a.xn || !a.xperm || a.act_n16 != 0) return hipErrorInvalidValue;
+    hipError_t e = launch_rmsnorm_qx(a.x, a.norm_w, a.eps, a.xn, a.xperm, a.xsum, a.M, H, a.abort, st);
+    if (e != hipSuccess) return e;
+    RouteArgs w = a;
+    w.x = a.xn;
+    hipLaunchKernelGGL(k_route_wide,
+                       dim3((a.M + RW_ROWS - 1) / RW_ROWS * ((a.E + 15) / 16)), dim3(256), 0, st, w);
     return hipGetLastError();
 }
 
