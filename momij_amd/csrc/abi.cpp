@@ -521,8 +521,9 @@ mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint1
         }
         if (wide) {
             SlotTab ut = ms.up_tab, dt = ms.dn_tab;
-            ut.ps = gather3_part_rows(EPI_SWIGLU, H, w->gs, w->up_gate_alpha != nullptr);
-            dt.ps = gather3_part_rows(EPI_STORE, I, w->gs, w->down_alpha != nullptr);
+            ut.ps = gather3_part_rows(EPI_SWIGLU, H, 2 * I, w->gs, w->up_gate_alpha != nullptr,
+                                      M * k, E);
+            dt.ps = gather3_part_rows(EPI_STORE, I, H, w->gs, w->down_alpha != nullptr, M * k, E);
             s = mj_hip(ctx, launch_wide_slots(inds, M * k, ut, dt, ab, st), "slots");
             if (s != MJ_OK) return s;
         }
@@ -602,10 +603,12 @@ mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint1
         } else if (wide) {
             up.tab = ms.up_tab.rec;
             up.tab_slots = ms.up_tab.n;
+            up.npairs = M * k;
         } else if (!topk_in_up) {
             up.inds = inds;
             up.npairs = M * k;
         }
+        up.experts = E;
         up.alpha = tile ? (const uint16_t*)w->up_gate_alpha : nullptr;
         up.y = ms.act;
         up.ysum = ms.act_sum;

@@ -967,7 +967,7 @@ constexpr size_t g5_stat(int rec, int FR) {
 }
 
 // dynamic LDS a tile-gather launch may take (the device has 160 KB per workgroup)
-constexpr size_t G5_LDS_MAX = 159 * 1024;
+constexpr size_t G5_LDS_MAX = 160 * 1024 - 256;
 
 // blocks of a persistent launch: two per CU (the LDS footprint allows two)
 static int persistent_blocks() {
@@ -982,14 +982,16 @@ static int persistent_blocks() {
     return 2 * cus;
 }
 
-// staged rows per pass: for the persistent products as many as keep two blocks per CU (more
+// staged rows per pass: for the persistent products as many as keep two blocks per CU, or one of
+// 16 waves (more
 // rows on one expert take extra passes, or slots); dense projections take up to 16
 template <int KPL, int GS, int EPI, int WPB, int KS, int REC = REC_NONE, bool ROWA = false>
 static int g5_rows(int want) {
     using S = G5Shape<KPL, GS, EPI, WPB, KS, ROWA>;
     constexpr bool PER = REC != REC_NONE;
     int RA = want < S::R ? want : S::R;
-    const size_t limit = PER ? 80 * 1024 - g5_stat(REC, MJ_G5_FUSED_ROWS) : G5_LDS_MAX;
+    const size_t limit =
+        PER ? (WPB == 16 ? 160 : 80) * 1024 - g5_stat(REC, MJ_G5_FUSED_ROWS) : G5_LDS_MAX;
     while (RA > 1 && S::lds(RA, want > RA || PER) > limit) --RA;
     return RA;
 }
@@ -1003,7 +1005,8 @@ static hipError_t launch_g5(const GatherArgs& a, int rows, int slots, hipStream_
     const int RA = g5_rows<KPL, GS, EPI, WPB, KS, REC, ROWA>(want);
     const bool multi = want > RA;
     int grid = slots * ncb;
-    if (PER && grid > persistent_blocks()) grid = persistent_blocks();
+    const int most = WPB == 16 ? persistent_blocks() / 2 : persistent_blocks();
+    if (PER && grid > most) grid = most;
     launch_timed(k_gather5<KPL, GS, EPI, WPB, KS, REC, ROWA>, dim3(grid), dim3(WPB * 64),
                  S::lds(RA, multi || PER), st, a, RA, (int)multi);
     return hipGetLastError();
@@ -1021,6 +1024,17 @@ bool gather3_supported(int epi, int K, int N, int gs) {
     return false;
 }
 
+// Whether an up || gate product over listed slots takes 16-wave blocks, one a CU, rather than two of
+// eight waves: a block then stages 16 rows, not 8, so an expert with 9 to 16 rows is unpacked once
+// (the unpacking is what bounds such passes: two thirds of the VALU's time), and each staged row
+// serves twice the columns.  Where most experts have fewer rows the barriers over 16 waves only
+// cost.  MoE of 64 rows over 64 experts (8 an expert) 64.9 -> 56.5 us, 40 rows (5) 54.8 -> 53.7, 20
+// rows over 128 (1.25) 62.8 -> 66.4; 200-token prefill of two layers, 64 experts 604 -> 554, 256
+// experts (6) 485 -> 464.
+static bool g5_many(int npairs, int experts, int N) {
+    return experts > 0 && npairs >= 5 * experts && N % 128 == 0;
+}
+
 hipError_t launch_gather3(const GatherArgs& a, int epi, int rows, hipStream_t st) {
     if (!gather3_supported(epi, a.K, a.N, a.gs)) return hipErrorInvalidValue;
     const bool rank = a.rlogits != nullptr, per = rank || a.inds != nullptr || a.tab != nullptr;
@@ -1029,15 +1043,18 @@ hipError_t launch_gather3(const GatherArgs& a, int epi, int rows, hipStream_t st
         const bool al = a.alpha != nullptr;
         const int slots = a.tab_slots;
         if (slots < 1) return hipErrorInvalidValue;
-#define MJ_G5T(KPL, E, KS64, KS128)                                                          \
-    return a.gs == 64 ? (al ? launch_g5<KPL, 64, E, 8, KS64, REC_TAB, true>(a, 16, slots, st)   \
-                            : launch_g5<KPL, 64, E, 8, KS64, REC_TAB, false>(a, 16, slots, st)) \
-                      : (al ? launch_g5<KPL, 128, E, 8, KS128, REC_TAB, true>(a, 16, slots, st) \
-                            : launch_g5<KPL, 128, E, 8, KS128, REC_TAB, false>(a, 16, slots, st));
-        if (epi == EPI_SWIGLU) { MJ_G5T(8, EPI_SWIGLU, 2, 2) }
+#define MJ_G5T(KPL, E, W, KS)                                                              \
+    return a.gs == 64 ? (al ? launch_g5<KPL, 64, E, W, KS, REC_TAB, true>(a, 16, slots, st)   \
+                            : launch_g5<KPL, 64, E, W, KS, REC_TAB, false>(a, 16, slots, st)) \
+                      : (al ? launch_g5<KPL, 128, E, W, KS, REC_TAB, true>(a, 16, slots, st)  \
+                            : launch_g5<KPL, 128, E, W, KS, REC_TAB, false>(a, 16, slots, st));
+        if (epi == EPI_SWIGLU && g5_many(a.npairs, a.experts, a.N)) {
+            MJ_G5T(8, EPI_SWIGLU, 16, 2)
+        }
+        if (epi == EPI_SWIGLU) { MJ_G5T(8, EPI_SWIGLU, 8, 2) }
         if (epi != EPI_STORE || a.K > 1024) return hipErrorInvalidValue;
-        if (a.K == 512) { MJ_G5T(2, EPI_STORE, 1, 1) }
-        MJ_G5T(4, EPI_STORE, 1, 1)
+        if (a.K == 512) { MJ_G5T(2, EPI_STORE, 8, 1) }
+        MJ_G5T(4, EPI_STORE, 8, 1)
 #undef MJ_G5T
     }
     // ranked routing: the up || gate product ranks the router logits itself
@@ -1058,6 +1075,10 @@ hipError_t launch_gather3(const GatherArgs& a, int epi, int rows, hipStream_t st
     if (epi == EPI_SWIGLU) {
         if (rank && al) { MJ_G5(8, EPI_SWIGLU, 8, 2, 2, REC_RANK, true) }
         if (rank) { MJ_G5(8, EPI_SWIGLU, 8, 2, 2, REC_RANK, false) }
+        if (g5_many(a.npairs, a.experts, a.N)) {
+            if (al) { MJ_G5(8, EPI_SWIGLU, 16, 2, 2, REC_IDS, true) }
+            MJ_G5(8, EPI_SWIGLU, 16, 2, 2, REC_IDS, false)
+        }
         if (al) { MJ_G5(8, EPI_SWIGLU, 8, 2, 2, REC_IDS, true) }
         MJ_G5(8, EPI_SWIGLU, 8, 2, 2, REC_IDS, false)
     }
@@ -1104,15 +1125,16 @@ hipError_t launch_gather3(const GatherArgs& a, int epi, int rows, hipStream_t st
 #undef MJ_G5D
 }
 
-int gather3_part_rows(int epi, int K, int gs, bool alpha) {
-#define MJ_R(KPL, E, KS)                                                                     \
-    return gs == 64 ? (alpha ? g5_rows<KPL, 64, E, 8, KS, REC_TAB, true>(16)                    \
-                             : g5_rows<KPL, 64, E, 8, KS, REC_TAB, false>(16))                  \
-                    : (alpha ? g5_rows<KPL, 128, E, 8, KS, REC_TAB, true>(16)                   \
-                             : g5_rows<KPL, 128, E, 8, KS, REC_TAB, false>(16));
-    if (epi == EPI_SWIGLU) { MJ_R(8, EPI_SWIGLU, 2) }
-    if (K == 512) { MJ_R(2, EPI_STORE, 1) }
-    MJ_R(4, EPI_STORE, 1)
+int gather3_part_rows(int epi, int K, int N, int gs, bool alpha, int npairs, int experts) {
+#define MJ_R(KPL, E, W, KS)                                                                  \
+    return gs == 64 ? (alpha ? g5_rows<KPL, 64, E, W, KS, REC_TAB, true>(16)                    \
+                             : g5_rows<KPL, 64, E, W, KS, REC_TAB, false>(16))                  \
+                    : (alpha ? g5_rows<KPL, 128, E, W, KS, REC_TAB, true>(16)                   \
+                             : g5_rows<KPL, 128, E, W, KS, REC_TAB, false>(16));
+    if (epi == EPI_SWIGLU && g5_many(npairs, experts, N)) { MJ_R(8, EPI_SWIGLU, 16, 2) }
+    if (epi == EPI_SWIGLU) { MJ_R(8, EPI_SWIGLU, 8, 2) }
+    if (K == 512) { MJ_R(2, EPI_STORE, 8, 1) }
+    MJ_R(4, EPI_STORE, 8, 1)
 #undef MJ_R
 }
 
@@ -1224,6 +1246,10 @@ hipError_t set_gather3_attributes() {
     MJ_A(8, EPI_ADD, 8, 2, 2, REC_IDS, false)
     MJ_A(8, EPI_SWIGLU, 8, 2, 2, REC_TAB, false)
     MJ_A(8, EPI_SWIGLU, 8, 2, 2, REC_TAB, true)
+    MJ_A(8, EPI_SWIGLU, 16, 2, 2, REC_TAB, false)
+    MJ_A(8, EPI_SWIGLU, 16, 2, 2, REC_TAB, true)
+    MJ_A(8, EPI_SWIGLU, 16, 2, 2, REC_IDS, false)
+    MJ_A(8, EPI_SWIGLU, 16, 2, 2, REC_IDS, true)
     MJ_A(2, EPI_STORE, 8, 1, 1, REC_TAB, false)
     MJ_A(2, EPI_STORE, 8, 1, 1, REC_TAB, true)
     MJ_A(4, EPI_STORE, 8, 1, 1, REC_TAB, false)

@@ -103,8 +103,9 @@ struct GatherArgs {
     const Buckets* bk;      // general kernel: rows grouped by expert (nullptr: dense)
     const int32_t* inds;    // tile kernel, persistent: expert of every pair [npairs] (pairs whose
     int npairs;             // id is outside [0, MJ_MAX_EXPERTS) are left out)
-    const int32_t* tab;     // tile kernel, persistent, wide passes: the slot table (SlotTab)
-    int tab_slots;
+    int experts;            // experts the pairs are spread over (0: not known)
+    const int32_t* tab;     // tile kernel, persistent, wide passes: the slot table (SlotTab) of the
+    int tab_slots;          // npairs pairs
     int dense_rows;         // dense: rows 0 .. dense_rows-1 of expert 0
     const uint16_t* alpha;  // row-alpha weights [E][N] fp16 (scale alpha, bias -alpha in
                             // every group): the tile expert kernels read it instead of s / b
@@ -165,7 +166,7 @@ hipError_t launch_wide_slots(const int32_t* inds, int P, const SlotTab& up, cons
                              const int* abort, hipStream_t st);
 
 // gather.hip: pairs a slot of a wide pass's product takes (its launch's rows a pass)
-int gather3_part_rows(int epi, int K, int gs, bool alpha);
+int gather3_part_rows(int epi, int K, int N, int gs, bool alpha, int npairs, int experts);
 
 // gather.hip: the tile gather (one 16-row weight tile over the whole K per wave)
 bool gather3_supported(int epi, int K, int N, int gs);

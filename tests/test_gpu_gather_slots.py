@@ -77,7 +77,9 @@ def test_gather_slots(ctx, orc, M, ktop, E, K, N, gs, kind, add):
     (64, 512, 64, 1, False), (64, 512, 64, 16, True), (64, 512, 128, 32, False),  # ranked, I 512
     (64, 1024, 64, 33, False), (64, 512, 64, 64, True),  # the first rows past the ranked forms
     (72, 1024, 64, 1, False), (256, 512, 64, 5, True), (256, 1024, 128, 64, False),
-    (8, 1024, 64, 64, False),  # every row on every expert: 64 pairs a slot
+    (8, 1024, 64, 64, False),  # every row on every expert: 64 pairs of each
+    # five pairs an expert and just fewer: 16-wave blocks, and two of eight
+    (40, 512, 128, 25, True), (40, 1024, 128, 25, False), (40, 512, 64, 24, False),
 ])
 def test_moe_slots(ctx, orc, E, I, gs, M, alpha):
     import torch
