@@ -1168,14 +1168,8 @@ mj_status mj_accept_sampled_ex(mj_ctx* ctx, const float* logits, int rows, int V
     Arena real{ctx->scratch, 0};
     layout(real, &rowmax, &bsum, &lcopy, &dt, &dc, &nbase);
     hipStream_t st = ctx->stream;
-    // the penalties rewrite the logits: on a copy, the caller's buffer is read-only here
-    float* lg = const_cast<float*>(logits);
-    if (pen) {
-        s = mj_hip(ctx, hipMemcpyAsync(lcopy, logits, (size_t)rows * V * 4,
-                                       hipMemcpyDeviceToDevice, st), "logits copy");
-        if (s != MJ_OK) return s;
-        lg = lcopy;
-    }
+    // the penalised rows go to a copy: the caller's buffer is read-only here
+    float* lg = pen ? lcopy : const_cast<float*>(logits);
     if (!ht.empty()) {
         int32_t* stage = nullptr;
         s = mj_hist_stage(ctx, 2 * ht.size(), &stage);
@@ -1193,7 +1187,8 @@ mj_status mj_accept_sampled_ex(mj_ctx* ctx, const float* logits, int rows, int V
     if (nucleus) nucleus_layout(nbase, V, nb);
     return mj_hip(ctx, launch_accept_sampled(lg, rows, V, draft, sp->temperature, q_mode, q_point,
                                              seed, counter, o, nucleus ? &nb : nullptr, rowmax,
-                                             bsum, out, nullptr, nullptr, ctx->abort_dev, st),
+                                             bsum, out, nullptr, nullptr, ctx->abort_dev, st,
+                                             nullptr, pen ? logits : nullptr),
                   "accept sampled");
 }
 
