@@ -307,7 +307,7 @@ __global__ __launch_bounds__(512) void k_lm_head(HeadArgs a) {
 //
 // Work unit: one K half of a strip, as k_lm_head: wave (slot, h) takes half h of strips
 // blockIdx.x * 4 + slot + round * gridDim.x * 4, the h = 1 partial meets the h = 0 one in
-// LDS.  A half streams as pieces of PL group pairs (16 rows x PL x 128 k codes plus their
+// LDS (four slots; eight where a block has 16 waves).  A half streams as pieces of PL group pairs (16 rows x PL x 128 k codes plus their
 // scales and biases), the next requested before the current one is multiplied.
 struct HeadQ4Args {
     const uint16_t* x;   // [M][K] fp16
@@ -330,8 +330,14 @@ struct Q4Piece {
     uint32_t sc[PL], bs[PL];            // scales / biases of groups 2 j, 2 j + 1 (lo, hi)
 };
 
-template <int NT, int PL>
-__global__ __launch_bounds__(512) void k_lm_head_q4(HeadQ4Args a) {
+// NW: waves of a block.  One tile of hidden rows leaves room for two eight-wave blocks a CU; two
+// tiles (132 KB) for one, of 16 waves (17 rows 56.8 -> 51.6 us, 64 rows with logits 115.7 -> 110.8);
+// with the log-sum-exp's state (LSE) 16 waves would spill, and take eight.  (The fp16 head, bound by
+// its weight stream, is slower so: 17 rows 115 -> 123.)
+template <int NT, int PL, int NW, bool LSE>
+__global__ __launch_bounds__(NW * 64) void k_lm_head_q4(HeadQ4Args a) {
+    constexpr int NS = NW / 2;  // strips a block takes at a time
+
     if (aborted(a.abort)) return;
     extern __shared__ __align__(16) char q4lds[];
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
@@ -341,10 +347,10 @@ __global__ __launch_bounds__(512) void k_lm_head_q4(HeadQ4Args a) {
     __shared__ int s_ban[MJ_HEAD_MAX_BANNED];  // banned ids (read with LDS, not vector, loads)
     const int n = lane & 15, q = lane >> 4;
     const int nstrips = (a.V + 15) / 16;
-    const int slot = wv & 3, h = wv >> 2;
+    const int slot = wv % NS, h = wv / NS;
     const int NH = G / 2 / (2 * PL);   // pieces per half strip
-    const int SW = gridDim.x * 4;
-    const int rounds = (nstrips - (int)blockIdx.x * 4 + SW - 1) / SW;
+    const int SW = gridDim.x * NS;
+    const int rounds = (nstrips - (int)blockIdx.x * NS + SW - 1) / SW;
     // the code offset 0x4C00 (fp16 16) kept in a VGPR so each nibble pair is one mask-or
     uint32_t c16 = 0x4C004C00u;
     asm("" : "+v"(c16));
@@ -352,15 +358,17 @@ __global__ __launch_bounds__(512) void k_lm_head_q4(HeadQ4Args a) {
     const int hsh = 16 * (q & 1);      // this lane's half of a scale word in the remainder chain
     float bv[NT][4];
     int bi[NT][4];
-    float lm[NT][4], ls[NT][4];  // running log-sum-exp of logits / T (log2 units)
+    float lm[LSE ? NT : 1][4], ls[LSE ? NT : 1][4];  // running log-sum-exp of logits / T (log2 units)
 #pragma unroll
     for (int tl = 0; tl < NT; ++tl)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             bv[tl][r] = -INFINITY;
             bi[tl][r] = 0x7fffffff;
-            lm[tl][r] = -INFINITY;
-            ls[tl][r] = 0.0f;
+            if constexpr (LSE) {
+                lm[tl][r] = -INFINITY;
+                ls[tl][r] = 0.0f;
+            }
         }
     auto load_piece = [&](int strip, int pc, Q4Piece<PL>& pz) {
         const int vr = min(strip * 16 + n, a.V - 1);
@@ -386,13 +394,13 @@ __global__ __launch_bounds__(512) void k_lm_head_q4(HeadQ4Args a) {
         }
     };
     constexpr int NPB = NT == 1 ? 2 : 1;
-    __shared__ f4 s_part[NPB][4][NT][64];
+    __shared__ f4 s_part[NPB][NS][NT][64];
     // The wave's pieces form one stream (rounds x NH) through two register sets taken in
     // turn: a set is refilled with the piece two ahead as soon as it has been multiplied, so
     // one piece is always in flight behind the one in use and no set is copied.  Every load is
     // issued -- past the stream's end at the clamped last row, a cached line -- which keeps the
     // wait before a set's use from covering the other set's requests.
-    const int strip0 = blockIdx.x * 4 + slot, TP = rounds * NH;
+    const int strip0 = blockIdx.x * NS + slot, TP = rounds * NH;
     int ld_strip = strip0, ld_pc = 0;
     auto issue = [&](Q4Piece<PL>& pz) {
         load_piece(ld_strip, ld_pc, pz);
@@ -487,11 +495,13 @@ __global__ __launch_bounds__(512) void k_lm_head_q4(HeadQ4Args a) {
                             bv[tl][r] = val;
                             bi[tl][r] = v;
                         }
-                        if (keep && a.lse.pm) {
-                            const float xk = val * a.lse.k, mn = fmaxf(lm[tl][r], xk);
-                            ls[tl][r] = ls[tl][r] * __builtin_amdgcn_exp2f(lm[tl][r] - mn) +
-                                        __builtin_amdgcn_exp2f(xk - mn);
-                            lm[tl][r] = mn;
+                        if constexpr (LSE) {
+                            if (keep) {
+                                const float xk = val * a.lse.k, mn = fmaxf(lm[tl][r], xk);
+                                ls[tl][r] = ls[tl][r] * __builtin_amdgcn_exp2f(lm[tl][r] - mn) +
+                                            __builtin_amdgcn_exp2f(xk - mn);
+                                lm[tl][r] = mn;
+                            }
                         }
                         if (a.logits && m < a.M && v < a.V) a.logits[(size_t)m * a.V + v] = val;
                     }
@@ -504,9 +514,9 @@ __global__ __launch_bounds__(512) void k_lm_head_q4(HeadQ4Args a) {
         for (int tl = 0; tl < NT; ++tl) acc[tl] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
     };
     Q4Piece<PL> pa, pb;
-    for (int idx = t; idx < a.n_banned; idx += 512) s_ban[idx] = a.banned[idx];
+    for (int idx = t; idx < a.n_banned; idx += NW * 64) s_ban[idx] = a.banned[idx];
     // group sums: a row's 64-groups over the threads, each read whole before it is summed in order
-    for (int idx = t; idx < NT * 16 * G; idx += 512) {
+    for (int idx = t; idx < NT * 16 * G; idx += NW * 64) {
         const int m = idx / G, g = idx - m * G;
         u4v v[8];
 #pragma unroll
@@ -519,7 +529,7 @@ __global__ __launch_bounds__(512) void k_lm_head_q4(HeadQ4Args a) {
             for (int j = 0; j < 4; ++j) sum += h2f(v[c][j] & 0xFFFFu) + h2f(v[c][j] >> 16);
         xg[m * GS1 + g] = m < a.M ? sum : 0.0f;
     }
-    stage_hidden<NT * 16, 8>(
+    stage_hidden<NT * 16, NW>(
         a.x, a.M, K, wv, lane,
         [&](int m, int c, u4v v) {
             u4v o;
@@ -555,10 +565,10 @@ __global__ __launch_bounds__(512) void k_lm_head_q4(HeadQ4Args a) {
                     bi[tl][r] = oi;
                 }
             }
-    __shared__ float sv[4][32];
-    __shared__ int si[4][32];
-    __shared__ float slm[4][32], sls[4][32];
-    if (a.lse.pm) {
+    __shared__ float sv[NS][32];
+    __shared__ int si[NS][32];
+    __shared__ float slm[NS][32], sls[NS][32];
+    if constexpr (LSE) {
 #pragma unroll
         for (int tl = 0; tl < NT; ++tl)
 #pragma unroll
@@ -575,24 +585,26 @@ __global__ __launch_bounds__(512) void k_lm_head_q4(HeadQ4Args a) {
             for (int r = 0; r < 4; ++r) {
                 sv[slot][tl * 16 + 4 * q + r] = bv[tl][r];
                 si[slot][tl * 16 + 4 * q + r] = bi[tl][r];
-                slm[slot][tl * 16 + 4 * q + r] = lm[tl][r];
-                sls[slot][tl * 16 + 4 * q + r] = ls[tl][r];
+                if constexpr (LSE) {
+                    slm[slot][tl * 16 + 4 * q + r] = lm[tl][r];
+                    sls[slot][tl * 16 + 4 * q + r] = ls[tl][r];
+                }
             }
     }
     __syncthreads();
     if (t < NT * 16 && t < a.M) {
         float bb = sv[0][t];
         int ii = si[0][t];
-        for (int w2 = 1; w2 < 4; ++w2)
+        for (int w2 = 1; w2 < NS; ++w2)
             if (sv[w2][t] > bb || (sv[w2][t] == bb && si[w2][t] < ii)) {
                 bb = sv[w2][t];
                 ii = si[w2][t];
             }
         a.pval[(size_t)blockIdx.x * 32 + t] = bb;
         a.pidx[(size_t)blockIdx.x * 32 + t] = ii;
-        if (a.lse.pm) {
+        if constexpr (LSE) {
             float m = slm[0][t], sm = sls[0][t];
-            for (int w2 = 1; w2 < 4; ++w2) lse_merge(m, sm, slm[w2][t], sls[w2][t]);
+            for (int w2 = 1; w2 < NS; ++w2) lse_merge(m, sm, slm[w2][t], sls[w2][t]);
             a.lse.pm[(size_t)blockIdx.x * 32 + t] = m;
             a.lse.ps[(size_t)blockIdx.x * 32 + t] = sm;
         }
@@ -609,28 +621,28 @@ __device__ __forceinline__ int head_fold_row(const float* pval, const int* pidx,
     int i = 0x7fffffff;
     float lm = -INFINITY, ls = 0.0f;
     for (int k0 = 0; k0 < nblk; k0 += 8 * 64) {
-        float v[8];
+        // (everything at clamped indices, so that all of it is in flight together: waiting for the
+        // maxima before the log-sum-exp pairs were requested made the fold of 9 rows 8.4 us, 7.7 so)
+        float v[8], pm[8], ps[8];
         int j[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            const int k = k0 + 64 * u + lane;
-            v[u] = k < nblk ? pval[(size_t)k * 32 + m] : -INFINITY;
-            j[u] = k < nblk ? pidx[(size_t)k * 32 + m] : 0x7fffffff;
+            const size_t at = (size_t)min(k0 + 64 * u + lane, nblk - 1) * 32 + m;
+            v[u] = pval[at];
+            j[u] = pidx[at];
+            if (lse.out) {
+                pm[u] = lse.pm[at];
+                ps[u] = lse.ps[at];
+            }
         }
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < 8; ++u)
             if (v[u] > b || (v[u] == b && j[u] < i)) {
                 b = v[u];
                 i = j[u];
             }
-        if (lse.out) {  // requested together as well (one at a time: the fold 4.6 -> 13.5 us)
-            float pm[8], ps[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int k = min(k0 + 64 * u + lane, nblk - 1);
-                pm[u] = lse.pm[(size_t)k * 32 + m];
-                ps[u] = lse.ps[(size_t)k * 32 + m];
-            }
+        if (lse.out) {
 #pragma unroll
             for (int u = 0; u < 8; ++u)
                 if (k0 + 64 * u + lane < nblk) lse_merge(lm, ls, pm[u], ps[u]);
@@ -839,7 +851,7 @@ hipError_t launch_lm_head(const uint16_t* x, const uint16_t* w, int M, int K, in
                 launch_timed(k_lm_head<1, 4>, dim3(nb), dim3(512), lds, st, a);
         } else {
             const size_t lds = (size_t)32 * (K + 8) * 2;
-            if (lds > 140 * 1024) return hipErrorInvalidValue;  // K <= 2232 for 17..32 rows
+            if (lds > 136 * 1024) return hipErrorInvalidValue;  // K <= 2168 for 17..32 rows
             if (pl8)
                 launch_timed(k_lm_head<2, 8>, dim3(nb), dim3(512), lds, st, a);
             else
@@ -1044,21 +1056,25 @@ hipError_t launch_lm_head_q4(const uint16_t* x, const uint32_t* w, const uint16_
         const int mg = M - m0 < 32 ? M - m0 : 32;
         const int nt = mg <= 16 ? 1 : 2;
         const size_t lds = (size_t)nt * 16 * (K + 8) * 2 + (size_t)nt * 16 * (K / 64 + 1) * 4;
-        if (lds > 140 * 1024) return hipErrorInvalidValue;
+        if (lds > 136 * 1024) return hipErrorInvalidValue;
         const int nb = nt == 1 ? head_blocks() : head_blocks() / 2;
         HeadLse gl = lse;
         if (!gl.out) gl.pm = gl.ps = nullptr;
         else gl.out += m0;
         HeadQ4Args qa{x + (size_t)m0 * K, w, s, b, mg, K, V, banned, n_banned,
                       logits ? logits + (size_t)m0 * V : nullptr, pval, pidx, abort, gl};
+        const bool ls = gl.out != nullptr;
+        auto go = [&](auto plain, auto with_lse, int nw, int nw_lse) {
+            launch_timed(ls ? with_lse : plain, dim3(nb), dim3(64 * (ls ? nw_lse : nw)), lds, st, qa);
+        };
         if (nt == 1 && pl4)
-            launch_timed(k_lm_head_q4<1, 4>, dim3(nb), dim3(512), lds, st, qa);
+            go(k_lm_head_q4<1, 4, 8, false>, k_lm_head_q4<1, 4, 8, true>, 8, 8);
         else if (nt == 1)
-            launch_timed(k_lm_head_q4<1, 2>, dim3(nb), dim3(512), lds, st, qa);
+            go(k_lm_head_q4<1, 2, 8, false>, k_lm_head_q4<1, 2, 8, true>, 8, 8);
         else if (pl4)
-            launch_timed(k_lm_head_q4<2, 4>, dim3(nb), dim3(512), lds, st, qa);
+            go(k_lm_head_q4<2, 4, 16, false>, k_lm_head_q4<2, 4, 8, true>, 16, 8);
         else
-            launch_timed(k_lm_head_q4<2, 2>, dim3(nb), dim3(512), lds, st, qa);
+            go(k_lm_head_q4<2, 2, 16, false>, k_lm_head_q4<2, 2, 8, true>, 16, 8);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         e = launch_head_final(pval, pidx, nb, M, m0, mg, out_idx, out_max, gl, abort, st, ga);
@@ -1070,13 +1086,23 @@ hipError_t launch_lm_head_q4(const uint16_t* x, const uint32_t* w, const uint16_
 hipError_t set_kernel_attributes() {
     static bool done = false;
     if (done) return hipSuccess;
-    const void* hk[8] = {(const void*)k_lm_head<1, 8>,    (const void*)k_lm_head<1, 4>,
-                         (const void*)k_lm_head<2, 8>,    (const void*)k_lm_head<2, 4>,
-                         (const void*)k_lm_head_q4<1, 4>, (const void*)k_lm_head_q4<1, 2>,
-                         (const void*)k_lm_head_q4<2, 4>, (const void*)k_lm_head_q4<2, 2>};
+    // (two tiles: 136 KB of hidden rows beside 21 KB of partials)
+    const void* hk[] = {(const void*)k_lm_head<1, 8>,
+                        (const void*)k_lm_head<1, 4>,
+                        (const void*)k_lm_head<2, 8>,
+                        (const void*)k_lm_head<2, 4>,
+                        (const void*)k_lm_head_q4<1, 4, 8, false>,
+                        (const void*)k_lm_head_q4<1, 4, 8, true>,
+                        (const void*)k_lm_head_q4<1, 2, 8, false>,
+                        (const void*)k_lm_head_q4<1, 2, 8, true>,
+                        (const void*)k_lm_head_q4<2, 4, 16, false>,
+                        (const void*)k_lm_head_q4<2, 4, 8, true>,
+                        (const void*)k_lm_head_q4<2, 2, 16, false>,
+                        (const void*)k_lm_head_q4<2, 2, 8, true>};
     hipError_t e = hipSuccess;
-    for (int i = 0; i < 8 && e == hipSuccess; ++i)
-        e = hipFuncSetAttribute(hk[i], hipFuncAttributeMaxDynamicSharedMemorySize, 140 * 1024);
+    for (const void* k : hk)
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 136 * 1024);
     if (e == hipSuccess) e = set_attn_attributes();
     if (e == hipSuccess) e = set_gather3_attributes();
     if (e == hipSuccess) done = true;

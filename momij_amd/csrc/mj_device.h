@@ -94,6 +94,34 @@ __device__ __forceinline__ UnpackK unpack_consts() {
                    {opaque(0x5C005C00u), opaque(0x54005400u), opaque(0x4C004C00u), opaque(0x44004400u)}};
 }
 
+// {sum x, sum base*x} of one 64-block in qx order, over eight consecutive lanes: lane c (= its index
+// in the group) holds halves 8c .. 8c + 7, sums its pairs in turn, and the eight partial sums meet
+// in lane moves.  Every lane of the group returns the sums.
+__device__ __forceinline__ float2 block_sum8(const u4v v, int c) {
+    float X = 0.0f, Bx = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        // qx pair (x_i, x_{i+8}) of a 16-block, i = (4c + j) % 8: base of code i
+        const float base = (float)(256 >> (2 * j));
+        const float p = h2f((uint16_t)v[j]) + h2f((uint16_t)(v[j] >> 16));
+        X += p;
+        Bx = fmaf(base, p, Bx);
+    }
+    auto move = [](float f, int ctrl) {
+        const int x = __float_as_int(f);
+        const int r = ctrl == 0   ? __builtin_amdgcn_update_dpp(x, x, 0xB1, 0xF, 0xF, false)
+                      : ctrl == 1 ? __builtin_amdgcn_update_dpp(x, x, 0x4E, 0xF, 0xF, false)
+                                  : __builtin_amdgcn_update_dpp(x, x, 0x141, 0xF, 0xF, false);
+        return __int_as_float(r);
+    };
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {  // quad xor 1, xor 2, then the half row mirrored
+        X += move(X, m);
+        Bx += move(Bx, m);
+    }
+    return make_float2(X, Bx);
+}
+
 // fp16 pair (lo, hi) from two raw fp16 bit patterns
 __device__ __forceinline__ uint32_t pack2(uint32_t lo16, uint32_t hi16) {
     return (lo16 & 0xFFFFu) | (hi16 << 16);

@@ -1067,7 +1067,7 @@ mj_status mj_lm_head_verify_q4(mj_ctx* ctx, const void* x, const void* w, const 
                        (double)temperature);
     if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)scales | (uintptr_t)biases) & 15)
         return mj_fail(ctx, MJ_INVALID_ARG, "lm_head_verify_q4: operands need 16-byte alignment");
-    const int kmax = M > 16 ? 2048 : 4096;  // staged hidden rows fit 140 KB of LDS
+    const int kmax = M > 16 ? 2048 : 4096;  // staged hidden rows fit 136 KB of LDS
     if (group_size != 64 || K % 512 != 0 || K > kmax)
         return mj_fail(ctx, MJ_UNSUPPORTED_SHAPE,
                        "lm_head_verify_q4: K=%d gs=%d (need gs 64, K%%512==0, K<=%d)", K,

@@ -66,30 +66,20 @@ __global__ __launch_bounds__(256) void k_qx_prep(const uint16_t* __restrict__ x,
     if ((lane & 7) == 0) xsum[(size_t)row * (K / 64) + 8 * c + (lane >> 3)] = make_float2(X, Bx);
 }
 
-// Block sums {sum x, sum base*x} of rows already in qx order (one thread per 64-block).
+// Block sums {sum x, sum base*x} of rows already in qx order, eight lanes a 64-block.
 __global__ __launch_bounds__(256) void k_qx_sums(const uint16_t* __restrict__ xperm,
                                                  float2* __restrict__ xsum, int rows, int K,
                                                  const int* abort) {
-    if (aborted(abort)) return;
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= rows * (K / 64)) return;
-    const uint16_t* xr = xperm + (size_t)i * 64;
-    float X = 0.0f, Bx = 0.0f;
-    for (int c = 0; c < 8; ++c) {
-        const u4v v = *(const u4v*)(xr + 8 * c);
-        for (int j = 0; j < 4; ++j) {
-            const float base = code_base(4 * c + j);  // pair (x_i, x_{i+8}), i = (4c+j)%8
-            const float lo = h2f((uint16_t)v[j]), hi = h2f((uint16_t)(v[j] >> 16));
-            X += lo + hi;
-            Bx += base * (lo + hi);
-        }
-    }
-    xsum[i] = make_float2(X, Bx);
+    const int i = blockIdx.x * 256 + threadIdx.x, n = rows * (K / 8);
+    const u4v v = *(const u4v*)(xperm + 8 * (size_t)min(i, n - 1));
+    if (aborted(abort) || i >= n) return;  // (whole groups: n is a multiple of 8)
+    const float2 sums = block_sum8(v, i & 7);
+    if ((i & 7) == 0) xsum[i >> 3] = sums;
 }
 
 hipError_t launch_qx_sums(const uint16_t* xperm, float2* xsum, int rows, int K, const int* abort,
                           hipStream_t st) {
-    const int n = rows * (K / 64);
+    const int n = rows * (K / 8);
     hipLaunchKernelGGL(k_qx_sums, dim3((n + 255) / 256), dim3(256), 0, st, xperm, xsum, rows, K,
                        abort);
     return hipGetLastError();
