@@ -312,7 +312,8 @@ mj_status mj_model_kv(mj_model* model, int layer, void** kcache, void** vcache);
 
 /* prefillPrompt (SeedlessDecodeEngine.swift:516-545): feed tokens in chunks of <= chunk rows
  * (<= MJ_MAX_ROWS), commit them, return the argmax after the last token.  Synchronises.  With
- * chunk = MJ_MAX_ROWS up to four chunks share a pass (the same results; an abort voids the pass). */
+ * chunk = MJ_MAX_ROWS up to four chunks share a pass (the same results; an abort voids the pass,
+ * and the model goes on from its start). */
 mj_status mj_prefill(mj_model* model, const int32_t* tokens, int n, int chunk,
                      int32_t* out_next);
 

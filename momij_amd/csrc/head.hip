@@ -963,6 +963,32 @@ hipError_t launch_kv_rows(const uint16_t* kv, int64_t layer_stride, int n_layers
     return hipGetLastError();
 }
 
+// Rows r0 .. r0 + n - 1 of a pass at L: every layer's K and V at their ring slots into `save`
+// ([layer][row][2][nKV][128]), or back out of it.  One wave a (layer, row), no abort word: a pass
+// that is being aborted is what it serves.
+__global__ __launch_bounds__(64) void k_kv_save(uint16_t* kv, int64_t layer_stride, int64_t C,
+                                                int nKV, int64_t L, int r0, int n, uint16_t* save,
+                                                int restore) {
+    const int l = blockIdx.x / n, i = blockIdx.x % n;
+    const int64_t slot = (L + r0 + i) % C;
+    u4v* s = (u4v*)(save + (size_t)blockIdx.x * 2 * nKV * 128);
+    for (int p = threadIdx.x; p < 2 * nKV * 16; p += 64) {
+        u4v* k = (u4v*)(kv + l * layer_stride + ((int64_t)(p >> 4) * C + slot) * 128) + (p & 15);
+        if (restore)
+            *k = s[p];
+        else
+            s[p] = *k;
+    }
+}
+
+hipError_t launch_kv_save(uint16_t* kv, int64_t layer_stride, int n_layers, int64_t C, int nKV,
+                          int64_t L, int r0, int n, uint16_t* save, bool restore, hipStream_t st) {
+    if (n < 1 || C < 1) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_kv_save, dim3(n_layers * n), dim3(64), 0, st, kv, layer_stride, C, nKV, L,
+                       r0, n, save, (int)restore);
+    return hipGetLastError();
+}
+
 hipError_t launch_kv_commit(uint16_t* kv, int64_t layer_stride, int n_layers, int64_t C, int nKV,
                             const StepDesc* sd, const StepResult* res, const int* abort,
                             hipStream_t st) {

@@ -267,6 +267,8 @@ hipError_t launch_kv_commit(uint16_t* kv, int64_t layer_stride, int n_layers, in
                             hipStream_t st);
 hipError_t launch_kv_rows(const uint16_t* kv, int64_t layer_stride, int n_layers, int64_t C,
                           int nKV, const StepDesc* sd, uint16_t* dst, hipStream_t st);
+hipError_t launch_kv_save(uint16_t* kv, int64_t layer_stride, int n_layers, int64_t C, int nKV,
+                          int64_t L, int r0, int n, uint16_t* save, bool restore, hipStream_t st);
 // The embedding kernels also write the pass's RoPE table (rt.half == 0: none).
 hipError_t launch_embed(const uint16_t* table, const StepDesc* sd, int M, int H, uint16_t* h,
                         const RopeTab& rt, const int* abort, hipStream_t st);

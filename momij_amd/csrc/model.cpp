@@ -67,6 +67,10 @@ struct mj_model {
     float* scores_all;
     MoeScratch ms{};
     int wide_rows = 0;            // rows a prefill pass may have (MJ_MAX_ROWS: no wide passes)
+    // what the rows of a wide pass past the ring's slack of 64 overwrite, kept until the pass is
+    // through: an aborted pass puts it back, so that its start stays a position to go on from
+    uint16_t* kv_save = nullptr;
+    bool kv_saved = false;        // taken by the pass now queued
     StepDesc* sd_dev = nullptr;   // one for each 64 rows of a pass
     StepDesc* sd_host = nullptr;
     StepResult* res_dev = nullptr;
@@ -235,6 +239,13 @@ static mj_status enqueue_pass(mj_model* m, int kind, int M, hipStream_t st) {
     const int H = c.H;
     const int* ab = ctx->abort_dev;
     mj_status s;
+    if (M > MJ_MAX_ROWS && m->offset + M > c.kv_capacity) {  // (else no slot is taken twice)
+        s = mj_hip(ctx, launch_kv_save(m->kv, m->layer_stride, c.n_layers, c.kv_capacity,
+                                       c.n_kv_heads, m->offset, MJ_MAX_ROWS, M - MJ_MAX_ROWS,
+                                       m->kv_save, false, st), "kv save");
+        if (s != MJ_OK) return s;
+        m->kv_saved = true;
+    }
     const NormOut first{(const uint16_t*)m->layers[0].attn.norm_w, c.eps, nullptr, m->xperm,
                         m->xsum};
     const RopeTab rt{m->inv_freq, m->rope_cs, c.rope_dim / 2};
@@ -546,6 +557,7 @@ mj_status mj_model_create(mj_ctx* ctx, const mj_model_config* cfg, const mj_laye
         ms.act_sum = (float2*)a.take((size_t)RW * c.top_k * (c.I / 64) * 8);
         ms.down = (uint16_t*)a.take((size_t)RW * c.top_k * H * 2);
         if (RW > R) {
+            m->kv_save = (uint16_t*)a.take((size_t)c.n_layers * (RW - R) * 2 * nKV * 128 * 2);
             for (SlotTab* tab : {&ms.up_tab, &ms.dn_tab}) {
                 tab->n = slot_tab_size(MJ_MAX_EXPERTS, MJ_SLOT_PS_MIN);
                 tab->rec = (int32_t*)a.take((size_t)tab->n * 16 * 4);
@@ -726,7 +738,18 @@ static mj_status feed_wide(mj_model* m, const int32_t* tokens, int M, int kind) 
         mj_status s = fill_tree(m->ctx, sd, nullptr, sd->M);
         if (s != MJ_OK) return s;
     }
-    return run_pass(m, kind, M);
+    m->kv_saved = false;
+    mj_status s = run_pass(m, kind, M);
+    if (s == MJ_ABORTED && m->kv_saved) {
+        const mj_model_config& c = m->cfg;
+        mj_status r = mj_hip(m->ctx, launch_kv_save(m->kv, m->layer_stride, c.n_layers,
+                                                    c.kv_capacity, c.n_kv_heads, m->offset,
+                                                    MJ_MAX_ROWS, M - MJ_MAX_ROWS, m->kv_save, true,
+                                                    m->ctx->stream), "kv restore");
+        if (r == MJ_OK) r = mj_hip(m->ctx, hipStreamSynchronize(m->ctx->stream), "kv restore");
+        if (r != MJ_OK) return r;
+    }
+    return s;
 }
 
 mj_status mj_prefill(mj_model* m, const int32_t* tokens, int n, int chunk, int32_t* out_next) {

@@ -17,13 +17,14 @@ def ctx():
     c.close()
 
 
-def _engine(ctx, E, I, gs, alpha, top_k, capacity):
+def _engine(ctx, E, I, gs, alpha, top_k, capacity, n_layers=2, full=True):
     import torch
 
     from momij_amd.engine import MapleLikeConfig, VerifyEngine, random_model
 
-    wins, ropes = MapleLikeConfig.maple_layer_mix(2, 96, 64, ["sliding_attention", "full"])
-    cfg = MapleLikeConfig(n_layers=2, E=E, I=I, gs=gs, top_k=top_k, vocab=2048, window=96,
+    kinds = ["sliding_attention", "full" if full else "sliding_attention"] * n_layers
+    wins, ropes = MapleLikeConfig.maple_layer_mix(n_layers, 96, 64, kinds)
+    cfg = MapleLikeConfig(n_layers=n_layers, E=E, I=I, gs=gs, top_k=top_k, vocab=2048, window=96,
                           kv_capacity=capacity, layer_window=wins, layer_rope_dim=ropes)
     layers, *rest = random_model(cfg, seed=E + I)
     if alpha:  # scale alpha, bias -alpha in every group of a row
@@ -97,4 +98,57 @@ def test_wide_refusals(ctx):
         with pytest.raises(MomijError) as e:
             eng.prefill(bad)
         assert e.value.status == status and eng.offset == at, (e.value, eng.offset)
+    eng.close()
+
+
+def test_wide_in_a_wrapped_ring(ctx):
+    """Passes of more rows than the ring has slots past the window, from offsets all around it."""
+    eng, cfg = _engine(ctx, 16, 512, 64, False, 4, 160, full=False)
+    rng = np.random.default_rng(5)
+    prompt = rng.integers(0, cfg.vocab, 700).tolist()
+    for i in range(0, 700, 50):
+        last = eng.step_chain_feeds(prompt[i:i + 50])
+    ref = _cache(eng, cfg)
+    for at in (0, 64, 150, 299, 444):
+        eng.rewind(0)
+        for i in range(0, at, 64):
+            eng.step_chain_feeds(prompt[i:min(i + 64, at)])
+        assert eng.prefill(prompt[at:]) == last[-1]
+        for a, b in zip(_cache(eng, cfg), ref):
+            assert (a == b).all(), at
+    eng.close()
+
+
+def test_wide_abort_leaves_its_start_valid(ctx):
+    """A prefill cut off in a wide pass goes on from the model's offset to the uninterrupted state:
+    what the pass had overwritten of the window before it is back."""
+    import threading
+    import time
+
+    eng, cfg = _engine(ctx, 64, 1024, 64, False, 8, 160, n_layers=6, full=False)
+    prompt = np.random.default_rng(6).integers(0, cfg.vocab, 3000).tolist()
+    want = eng.prefill(prompt)
+    ref = _cache(eng, cfg)
+    eng.rewind(0)
+    t0 = time.perf_counter()
+    eng.prefill(prompt)
+    t_full = time.perf_counter() - t0
+    cut = 0
+    for k in range(8):
+        eng.rewind(0)
+        timer = threading.Timer(t_full * (0.15 + 0.08 * k), lambda: ctx.set_abort(True))
+        timer.start()
+        try:
+            eng.prefill(prompt)
+        except MomijError as e:
+            assert e.status == 5
+            cut += 1
+        timer.join()
+        ctx.set_abort(False)
+        print(f"cut at offset {eng.offset}", flush=True)
+        if eng.offset < len(prompt):
+            assert eng.prefill(prompt[eng.offset:]) == want
+            for a, b in zip(_cache(eng, cfg), ref):
+                assert (a == b).all()
+    assert cut > 0
     eng.close()
