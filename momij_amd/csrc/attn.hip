@@ -172,6 +172,40 @@ __device__ __forceinline__ int rope_f0(int d0) {
     return d0 < 2 * HALF ? (d0 < HALF ? d0 : d0 - HALF) : 0;
 }
 
+// One vector's RMSNorm and RoPE over eight lanes: a lane holds dims 8 pa + i (xa) and, X parts above,
+// the dims they rotate with (xb), with their norm weights; cs: the row's angles.
+template <int HALF>
+__device__ __forceinline__ void finish_vec(float xa[8], float xb[8], const float wa[8],
+                                           const float wb[8], const float2* cs_row, int pa,
+                                           float eps) {
+    float ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ss = fmaf(xa[i], xa[i], ss);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ss = fmaf(xb[i], xb[i], ss);
+    ss = lane8_sum(ss);
+    const float scl = 1.0f / sqrtf(ss / (float)HD + eps);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        xa[i] = xa[i] * scl * wa[i];
+        xb[i] = xb[i] * scl * wb[i];
+    }
+    if constexpr (HALF > 0) {
+        // dims 8 pa + i < half pair with 8 pa + i + half
+        const bool rot = 8 * pa < HALF;
+        const float2* cs = cs_row + (rot ? 8 * pa : 0);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float2 c2 = cs[i];
+            const float cx = rot ? c2.x : 1.0f, sy = rot ? c2.y : 0.0f;
+            // (the fused products spelled out: the same wherever this is inlined)
+            const float ra = fmaf(xa[i], cx, -(xb[i] * sy)), rb = fmaf(xb[i], cx, xa[i] * sy);
+            xa[i] = ra;
+            xb[i] = rb;
+        }
+    }
+}
+
 // Work of one block (kv head g, chunk c), 256 threads:
 //   loads, every one issued before the first wait (all unconditional, at clamped addresses):
 //     K: key t / 4, dims 32 (t % 4) ..      (the layout the own-key norm reduces over)
@@ -195,19 +229,28 @@ __host__ __device__ inline int tab_floats2(int M, int half) {
 // passes with more of them take JR = 3.
 // CG: chunks a block takes, 1, or AG (the chunks of a group in turn, the next one's K and V
 // requested before the current one's products; the block's tiles are then at most one a wave).
-template <int HALF, int JR, int CG>
+// WIDE: the 64-row parts of a wide prefill pass in one launch, part z = blockIdx.z.  Queries and own
+// keys are finished in place in the projection rows before it (k_attn_finish), so the keys of every
+// pass row come from there, the older ones from the cache, and nothing is appended (k_attn_combine
+// does, once nobody reads what the append overwrites).
+template <int HALF, int JR, int CG, bool WIDE = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_attn_chunk(AttnArgs a) {
     constexpr int NT = 256;
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     const int g = blockIdx.x / a.parts, part = blockIdx.x % a.parts;
-    const StepDesc* sd = a.sd;
+    const int z = WIDE ? blockIdx.z : 0;
+    const StepDesc* sd = a.sd + z;
     const int64_t L = sd->L;
-    const int M = a.M;
+    const int M = WIDE ? sd->M : a.M;
+    const int row0 = MJ_ROWS * z;  // the pass's rows before this part
     const int gqa = a.nQ / a.nKV;
     // the block's query vectors qv0 .. qv0 + nqv - 1: tpp tiles of 16 a block
     const int qv0 = 16 * a.tpp * blockIdx.y, nqt_all = (M * gqa + 15) / 16;
     const int nqt = min(a.tpp, nqt_all - a.tpp * (int)blockIdx.y);
+    if (WIDE && nqt <= 0) return;  // whole block (a shorter last part)
     const int nqv = min(16 * nqt, M * gqa - qv0);
+    // partials are laid out over the tiles of a whole part
+    const int nqt_part = WIDE ? (MJ_ROWS * gqa + 15) / 16 : nqt_all;
     const int qkvN = (a.nQ + 2 * a.nKV) * HD;
     constexpr int half = HALF;
     const ChunkGeom cg = chunk_geom(a.window, L, M, sd->chain != 0);
@@ -261,9 +304,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     int kcls = -2, vcls[4];
     // each 8-dim part from the projection (own rows) or the cache, at clamped slots
     auto src_of = [&](int cls, int k, const uint16_t* own, const uint16_t* cache) {
-        const int sl = cls == -1 ? slot_of(crel + k) : 0;
-        const uint32_t off = cls >= 0 ? (uint32_t)(cls * qkvN) : (uint32_t)(sl * HD);
-        return (cls >= 0 ? own : cache) + off;
+        const int pr = WIDE ? row0 + crel + k : cls;  // pass row
+        const bool inp = WIDE ? cls != -2 && pr >= 0 : cls >= 0;
+        const int sl = cls == -1 && !inp ? slot_of(crel + k) : 0;
+        const uint32_t off = inp ? (uint32_t)(pr * qkvN) : (uint32_t)(sl * HD);
+        return (inp ? own : cache) + off;
     };
     const uint16_t* const kown = a.qkv + (a.nQ + g) * HD;
     const uint16_t* const vown = kown + a.nKV * HD;
@@ -314,9 +359,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             jxb[jj] = *(const u4v*)(src + 8 * (pa + X));
         }
     };
-    request_jobs();
+    u4v qf[4];  // WIDE: 16-byte parts of the block's finished queries
+    if constexpr (WIDE) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int e = t + NT * j, v = qv0 + min(e >> 4, nqv - 1), r = v / gqa;
+            qf[j] = *(const u4v*)(a.qkv + (uint32_t)((row0 + r) * qkvN +
+                                                     (g * gqa + v - r * gqa) * HD + 8 * (e & 15)));
+        }
+    } else {
+        request_jobs();
+    }
     // the norm weights into LDS (16 lanes each of wave 0)
-    if (wv == 0 && lane < HD / 8) {
+    if (!WIDE && wv == 0 && lane < HD / 8) {
         __builtin_amdgcn_global_load_lds(a.q_norm_w + 8 * lane,
                                          (__attribute__((address_space(3))) void*)qnw_s, 16, 0, 0);
         __builtin_amdgcn_global_load_lds(a.k_norm_w + 8 * lane,
@@ -325,7 +380,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     // ---- RoPE table rows (float4 = two angles), key and row metadata
     // the table goes straight into LDS (16 bytes a lane): pairs 2e, 2e + 1 of the [M][half]
     // angles, wave w taking pairs 64 w + lane, 64 (w + 4) + lane, ...
-    const int ntab4 = M * half / 2, hd = half > 0 ? half : 1;
+    const int ntab4 = WIDE ? 0 : M * half / 2, hd = half > 0 ? half : 1;
     for (int e0 = 64 * wv; e0 < ntab4; e0 += NT) {
         const int e = e0 + lane;
         if (e < ntab4)
@@ -346,6 +401,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         ranc[t] = ranc_t;
     }
     if (t == 0) *s_abort = abort_v;
+    if constexpr (WIDE) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int e = t + NT * j;
+            if (e < 16 * nqv) *(u4v*)(Qs + (e >> 4) * QSTR + 8 * (e & 15)) = qf[j];
+        }
+    }
     const float sc2 = a.scale * LOG2E;
     const int ln = lane & 15, lq = lane >> 4;
     // the group's partial so far (CG > 1): maximum and sum of query vector ln, outputs as O below
@@ -357,7 +419,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     // dim 16 dt + d
     auto write_part = [&](int qt, const f4* O, float m, float l) {
         const size_t pbase =
-            ((size_t)g * a.max_chunks + part) * (size_t)(nqt_all * 16) + qv0 + qt * 16;
+            ((size_t)(z * a.nKV + g) * a.max_chunks + part) * (size_t)(nqt_part * 16) + qv0 + qt * 16;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             float* op = a.opart + (pbase + 4 * lq + r) * HD;
@@ -396,6 +458,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     // d + half (maple_qk_norm_rope); queries into Qs, own keys into Ks and appended at slot
     // (L + r) % C with their V rows (maple_write_kv_pair).  No other block of this launch
     // reads those slots (the committed window never reaches them).
+    if constexpr (!WIDE)
     for (int j0 = 0; j0 < njobs; j0 += NT * JR) {
 #pragma unroll
         for (int jj = 0; jj < JR; ++jj) {
@@ -418,31 +481,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             const uint16_t* nw = isq ? qnw_s : knw_s;
             unpack8(*(const u4v*)(nw + 8 * pa), wa);
             unpack8(*(const u4v*)(nw + 8 * pb), wb);
-            float ss = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) ss += xa[i] * xa[i];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) ss += xb[i] * xb[i];
-            ss = lane8_sum(ss);
-            const float scl = 1.0f / sqrtf(ss / (float)HD + a.eps);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                xa[i] = xa[i] * scl * wa[i];
-                xb[i] = xb[i] * scl * wb[i];
-            }
-            if constexpr (HALF > 0) {
-                // dims 8 pa + i < half pair with 8 pa + i + half = 8 pb + i
-                const bool rot = 8 * pa < half;
-                const float2* cs = tab + row * half + (rot ? 8 * pa : 0);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const float2 c2 = cs[i];
-                    const float cx = rot ? c2.x : 1.0f, sy = rot ? c2.y : 0.0f;
-                    const float ra = xa[i] * cx - xb[i] * sy, rb = xb[i] * cx + xa[i] * sy;
-                    xa[i] = ra;
-                    xb[i] = rb;
-                }
-            }
+            finish_vec<HALF>(xa, xb, wa, wb, tab + row * half, pa, a.eps);
             const u4v oa = pack8(xa), ob = pack8(xb);
             if (j < njobs) {
                 if (isq) {
@@ -460,7 +499,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             }
         }
     }
-    if (own_chunk && blockIdx.y == 0) {
+    if (!WIDE && own_chunk && blockIdx.y == 0) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             if (vcls[j] >= 0)
@@ -594,14 +633,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // order and the row is written in qx order.  A group is merged from its chunks first (CG 1), or
 // came merged (CG 4).  Every part of the pass is there (a fully masked one has max -inf, sum 0,
 // output 0 and adds exact zeros), so a row's merge depends only on the chunks that hold its keys.
-template <int CG>
+// WIDE: of all parts of a wide pass; the blocks past its rows append the pass's keys and values to
+// the cache, two rows a block (of rows that share a slot, the last).
+template <int CG, bool WIDE = false>
 __global__ __launch_bounds__(256) void k_attn_combine(AttnArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int r = blockIdx.x / a.nQ, hq = blockIdx.x % a.nQ;
+    if constexpr (WIDE) {
+        if ((int)blockIdx.x >= a.M * a.nQ) {
+            const int row = 2 * (blockIdx.x - a.M * a.nQ) + (tid >> 7);
+            if (aborted(a.abort) || row >= a.M || row + a.C < a.M) return;
+            const int64_t slot = (a.sd->L + row) % a.C;
+            const uint16_t* src = a.qkv + (size_t)row * (a.nQ + 2 * a.nKV) * HD + a.nQ * HD;
+            for (int p = tid & 127; p < 2 * a.nKV * 16; p += 128) {
+                const int h = p >> 4;  // K heads, then V heads
+                uint16_t* dst = (h < a.nKV ? a.kc : a.vc) +
+                                ((size_t)(h < a.nKV ? h : h - a.nKV) * a.C + slot) * HD;
+                *(u4v*)(dst + 8 * (p & 15)) = *(const u4v*)(src + 8 * p);
+            }
+            return;
+        }
+    }
+    const int r = blockIdx.x / a.nQ, hq = blockIdx.x % a.nQ;  // row of the pass
+    const int z = WIDE ? r / MJ_ROWS : 0;
+    const StepDesc* sd = a.sd + z;
+    const int M = WIDE ? sd->M : a.M;
     const int gqa = a.nQ / a.nKV;
-    const int g = hq / gqa, qv = r * gqa + (hq % gqa);
-    const size_t nq16 = (size_t)((a.M * gqa + 15) / 16) * 16;
-    const ChunkGeom cg = chunk_geom(a.window, a.sd->L, a.M, a.sd->chain != 0);
+    const int g = z * a.nKV + hq / gqa, qv = (r - MJ_ROWS * z) * gqa + (hq % gqa);
+    const size_t nq16 = (size_t)(((WIDE ? MJ_ROWS : M) * gqa + 15) / 16) * 16;
+    const ChunkGeom cg = chunk_geom(a.window, sd->L, M, sd->chain != 0);
     const int ng = group_count(cg), nparts = CG == 1 ? cg.nch : ng;
     const int gs = (int)(((int64_t)wv - cg.c0 / AG) & 3);  // this wave's first group
     const float2* ml = a.mlpart + (size_t)g * a.max_chunks * nq16 + qv;
@@ -738,6 +797,62 @@ hipError_t launch_attn(const AttnArgs& args, hipStream_t st) {
     return hipGetLastError();
 }
 
+// The queries and keys of a wide pass's projection rows finished in place (RMSNorm, RoPE), the
+// arithmetic of k_attn_chunk's jobs: eight lanes a vector.
+template <int HALF>
+__global__ __launch_bounds__(256) void k_attn_finish(AttnArgs a) {
+    constexpr int X = HALF >= 16 ? HALF / 8 : 8;
+    const int heads = a.nQ + a.nKV, vi = (blockIdx.x * 256 + threadIdx.x) >> 3, jb = threadIdx.x & 7;
+    const int row = vi / heads, head = vi - row * heads;
+    if (row >= a.M || aborted(a.abort)) return;  // (whole groups of eight)
+    const int pa = (jb & (X - 1)) | ((jb & ~(X - 1)) << 1), pb = pa + X;
+    uint16_t* v = const_cast<uint16_t*>(a.qkv) + (size_t)row * (a.nQ + 2 * a.nKV) * HD + head * HD;
+    const uint16_t* nw = head < a.nQ ? a.q_norm_w : a.k_norm_w;
+    float xa[8], xb[8], wa[8], wb[8];
+    unpack8(*(const u4v*)(v + 8 * pa), xa);
+    unpack8(*(const u4v*)(v + 8 * pb), xb);
+    unpack8(*(const u4v*)(nw + 8 * pa), wa);
+    unpack8(*(const u4v*)(nw + 8 * pb), wb);
+    finish_vec<HALF>(xa, xb, wa, wb, a.rope_cs + (size_t)row * MJ_ROPE_F, pa, a.eps);
+    *(u4v*)(v + 8 * pa) = pack8(xa);
+    *(u4v*)(v + 8 * pb) = pack8(xb);
+}
+
+// Attention of a wide pass (a.M rows, a descriptor for each 64 at a.sd) with at most MJ_ATTN_DEEP - 1
+// chunks a part: three launches for all parts.  (A part after another, each with a launch for its
+// partials, took 13.7 us a part: 200-token prefill of four layers 865 us, 735 so.)  The cases past that
+// keep the parts in turn: there a part's launch fills the chip, and partials for all parts at once
+// would take hundreds of MB.
+hipError_t launch_attn_wide(const AttnArgs& args, hipStream_t st) {
+    AttnArgs a = args;
+    if (a.M <= MJ_ROWS || a.M > MJ_WIDE_ROWS || a.nch >= MJ_ATTN_DEEP || a.nch > a.max_chunks)
+        return hipErrorInvalidValue;
+    if (a.C < 1 || a.C >= ((int64_t)1 << 23)) return hipErrorInvalidValue;
+    const int gqa = a.nQ / a.nKV, nz = (a.M + MJ_ROWS - 1) / MJ_ROWS;
+    const int nqt = (MJ_ROWS * gqa + 15) / 16;
+    a.max_chunks = a.parts = a.nch;
+    a.tpp = std::min(4, nqt);
+    const int jobs = a.M * (a.nQ + a.nKV) * 8;
+    const dim3 fg((jobs + 255) / 256), blk(256);
+    switch (a.rope_dim) {
+        case 0: hipLaunchKernelGGL(k_attn_finish<0>, fg, blk, 0, st, a); break;
+        case 32: hipLaunchKernelGGL(k_attn_finish<16>, fg, blk, 0, st, a); break;
+        case 64: hipLaunchKernelGGL(k_attn_finish<32>, fg, blk, 0, st, a); break;
+        case 128: hipLaunchKernelGGL(k_attn_finish<64>, fg, blk, 0, st, a); break;
+        default: return hipErrorInvalidValue;
+    }
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const size_t lds = (size_t)(a.tpp * 16 * QSTR + AK * QSTR + HD * VSTR) * 2 + AK * 4 +
+                       MJ_ROWS * (4 + 8) + 2 * HD * 2 + 16;
+    launch_timed(k_attn_chunk<0, 1, 1, true>, dim3(a.nKV * a.parts, (nqt + a.tpp - 1) / a.tpp, nz), blk,
+                 lds, st, a);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((k_attn_combine<1, true>), dim3(a.M * a.nQ + (a.M + 1) / 2), blk, 0, st, a);
+    return hipGetLastError();
+}
+
 template <int HALF>
 static hipError_t attn_attr() {
     hipError_t e = hipSuccess;
@@ -751,6 +866,9 @@ static hipError_t attn_attr() {
 
 hipError_t set_attn_attributes() {
     hipError_t e = attn_attr<0>();
+    if (e == hipSuccess)
+        e = hipFuncSetAttribute((const void*)k_attn_chunk<0, 1, 1, true>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (e == hipSuccess) e = attn_attr<16>();
     if (e == hipSuccess) e = attn_attr<32>();
     if (e == hipSuccess) e = attn_attr<64>();

@@ -208,6 +208,7 @@ struct AttnArgs {
 
 // attn.hip
 hipError_t launch_attn(const AttnArgs& a, hipStream_t st);
+hipError_t launch_attn_wide(const AttnArgs& a, hipStream_t st);
 int attn_max_chunks(int window, int64_t L_max, int M);
 // Chunks from which a launch takes its keys in groups (launch_attn)
 #define MJ_ATTN_DEEP 40

@@ -157,8 +157,25 @@ static mj_status enqueue_layer(mj_model* m, int l, int M, int kind, hipStream_t 
     a.eps = c.eps;
     a.scale = (float)std::pow((double)D, -0.5);
     a.abort = ab;
-    // a wide pass attends 64 rows at a time, each 64 after the keys of those before it are appended
-    for (int r0 = 0; r0 < M; r0 += MJ_MAX_ROWS) {
+    // a wide pass: all of its 64-row parts together while the keys are few, else one part after
+    // another, each after the keys of those before it are appended
+    const int rl = (M - 1) / MJ_MAX_ROWS * MJ_MAX_ROWS;  // first row of the last part
+    a.nch = m->lwin[l] > 0 ? attn_max_chunks(m->lwin[l], 0, std::min(M, MJ_MAX_ROWS))
+                           : attn_max_chunks(0, m->offset + rl, M - rl);
+    const bool together = M > MJ_MAX_ROWS && a.nch < MJ_ATTN_DEEP;
+    if (together) {
+        a.qkv = m->qkv;
+        a.rope_cs = m->rope_cs;
+        a.sd = m->sd_dev;
+        a.out_perm = m->aperm;
+        a.out_sum = m->asum;
+        a.M = M;
+        a.max_chunks = std::min(m->max_chunks, MJ_ATTN_DEEP - 1);
+        a.nch = std::min(a.nch, a.max_chunks);
+        s = mj_hip(ctx, launch_attn_wide(a, st), "attention");
+        if (s != MJ_OK) return s;
+    }
+    for (int r0 = 0; r0 < M && !together; r0 += MJ_MAX_ROWS) {
         const int rows = std::min(M - r0, MJ_MAX_ROWS);
         a.qkv = m->qkv + (size_t)r0 * qkvN;
         a.rope_cs = m->rope_cs + (size_t)r0 * MJ_ROPE_F;
@@ -526,8 +543,10 @@ mj_status mj_model_create(mj_ctx* ctx, const mj_model_config* cfg, const mj_laye
         m->xsum = (float2*)a.take((size_t)RW * (H / 64) * 8);
         m->qkv = (uint16_t*)a.take((size_t)RW * qkvN * 2);
         m->rope_cs = (float2*)a.take((size_t)RW * MJ_ROPE_F * sizeof(float2));
-        m->opart = (float*)a.take((size_t)nKV * m->max_chunks * nqt16 * 128 * 4);
-        m->mlpart = (float2*)a.take((size_t)nKV * m->max_chunks * nqt16 * 8);
+        // (a wide pass whose parts attend together: fewer chunks, for each of them)
+        const size_t parts = std::max(m->max_chunks, RW / R * std::min(m->max_chunks, MJ_ATTN_DEEP - 1));
+        m->opart = (float*)a.take(nKV * parts * nqt16 * 128 * 4);
+        m->mlpart = (float2*)a.take(nKV * parts * nqt16 * 8);
         m->aperm = (uint16_t*)a.take((size_t)RW * nQ * 128 * 2);
         m->asum = (float2*)a.take((size_t)RW * nQ * 2 * 8);
         m->xf = (uint16_t*)a.take((size_t)RW * H * 2);

@@ -119,6 +119,23 @@ def test_wide_in_a_wrapped_ring(ctx):
     eng.close()
 
 
+def test_wide_past_the_deep_line(ctx):
+    """Full attention from passes whose parts attend together to passes whose keys are too many."""
+    eng, cfg = _engine(ctx, 16, 512, 64, False, 4, 2944)
+    prompt = np.random.default_rng(8).integers(0, cfg.vocab, 2900).tolist()
+    for i in range(0, 2900, 64):
+        last = eng.step_chain_feeds(prompt[i:i + 64])
+    ref = _cache(eng, cfg)
+    for at in (0, 2200):
+        eng.rewind(0)
+        for i in range(0, at, 64):
+            eng.step_chain_feeds(prompt[i:min(i + 64, at)])
+        assert eng.prefill(prompt[at:]) == last[-1]
+        for a, b in zip(_cache(eng, cfg), ref):
+            assert (a == b).all(), at
+    eng.close()
+
+
 def test_wide_abort_leaves_its_start_valid(ctx):
     """A prefill cut off in a wide pass goes on from the model's offset to the uninterrupted state:
     what the pass had overwritten of the window before it is back."""
