@@ -12,6 +12,8 @@
 // k_kv_commit    keeps the accepted rows: the KV written at slot L + path[i] moves to L + i
 //                (SeedlessAttn.swift:219-270 rewinds the offset for append-only writes; a tree
 //                also needs the accepted path compacted into consecutive positions).
+#include <algorithm>
+
 #include "mj_device.h"
 #include "mj_internal.h"
 
@@ -31,6 +33,9 @@ struct HeadArgs {
     int* pidx;           // [blocks][32]
     const int* abort;
     HeadLse lse;
+    // rows 32 .. M - 1 by every other set of eight blocks (M > 32): both halves of the blocks go
+    // through the strips side by side, on the same XCD, so the weights come from memory once
+    int pair;
 };
 
 // The hidden rows of a head block into LDS: wave w of WAVES takes rows w, w + WAVES, ..., a row's
@@ -54,7 +59,9 @@ __device__ __forceinline__ void stage_hidden(const uint16_t* x, int M, int K, in
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int m = wv + WAVES * (r0 + r), part = p0 + 64 * i + lane;
-                    v[r][i] = *(const u4v*)(x + (size_t)min(m, M - 1) * K + 8 * min(part, parts - 1));
+                    v[r][i] = (u4v){0u, 0u, 0u, 0u};
+                    if (m < M)  // (wave-uniform)
+                        v[r][i] = *(const u4v*)(x + (size_t)m * K + 8 * min(part, parts - 1));
                 }
             if (r0 + RB >= RPW && p0 + 256 >= parts) {
                 __builtin_amdgcn_sched_barrier(0);
@@ -65,7 +72,7 @@ __device__ __forceinline__ void stage_hidden(const uint16_t* x, int M, int K, in
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int m = wv + WAVES * (r0 + r), part = p0 + 64 * i + lane;
-                    if (part < parts) put(m, part, m < M ? v[r][i] : (u4v){0u, 0u, 0u, 0u});
+                    if (part < parts) put(m, part, v[r][i]);
                 }
         }
     }
@@ -74,6 +81,23 @@ __device__ __forceinline__ void stage_hidden(const uint16_t* x, int M, int K, in
 template <int NT, int PL>
 __global__ __launch_bounds__(512) void k_lm_head(HeadArgs a) {
     if (aborted(a.abort)) return;
+    // block bid of nb, over the rows of its group (pair: blocks 16 i + 8 .. 16 i + 15 are group 1's)
+    int bid = blockIdx.x, nb = gridDim.x;
+    if (NT == 2 && a.pair) {
+        const int grp = (bid >> 3) & 1;
+        bid = (bid >> 4) << 3 | (bid & 7);
+        nb >>= 1;
+        a.M = grp ? a.M - 32 : 32;
+        a.x += (size_t)grp * 32 * a.K;
+        if (a.logits) a.logits += (size_t)grp * 32 * a.V;
+        const size_t at = (size_t)grp * nb * 32;
+        a.pval += at;
+        a.pidx += at;
+        if (a.lse.pm) {
+            a.lse.pm += at;
+            a.lse.ps += at;
+        }
+    }
     extern __shared__ uint16_t xs[];  // [NT*16][K + 8]
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     const int K = a.K, XS = K + 8;
@@ -91,7 +115,7 @@ __global__ __launch_bounds__(512) void k_lm_head(HeadArgs a) {
         ls[tl] = 0.0f;
     }
     // Work unit: one K half of a 16-row strip.  Wave (slot, h) of a block takes half h of
-    // strips blockIdx.x * 4 + slot + round * gridDim.x * 4; the h = 1 partial meets the h = 0
+    // strips bid * 4 + slot + round * nb * 4; the h = 1 partial meets the h = 0
     // one in LDS (two slot sets by round parity), so twice as many units as strips keep the
     // waves' loads even.  A wave's halves are one stream of pieces of PL 32-k chunks (16 rows x
     // 256 k, 8 KB, when K / 2 allows) through two register sets taken in turn: a set is
@@ -101,9 +125,9 @@ __global__ __launch_bounds__(512) void k_lm_head(HeadArgs a) {
     // before a set's use from covering the other set's requests.
     const int slot = wv & 3, h = wv >> 2;
     const int NH = K / 64 / PL;                // pieces per half strip
-    const int SW = gridDim.x * 4;
-    const int rounds = (nstrips - (int)blockIdx.x * 4 + SW - 1) / SW;  // of this block's slot 0
-    const int strip0 = blockIdx.x * 4 + slot, TP = rounds * NH;
+    const int SW = nb * 4;
+    const int rounds = (nstrips - bid * 4 + SW - 1) / SW;  // of this block's slot 0
+    const int strip0 = bid * 4 + slot, TP = rounds * NH;
     struct Piece {
         u4v c[PL];
     };
@@ -274,13 +298,13 @@ __global__ __launch_bounds__(512) void k_lm_head(HeadArgs a) {
                 b = sv[w][t];
                 i = si[w][t];
             }
-        a.pval[(size_t)blockIdx.x * 32 + t] = b;
-        a.pidx[(size_t)blockIdx.x * 32 + t] = i;
+        a.pval[(size_t)bid * 32 + t] = b;
+        a.pidx[(size_t)bid * 32 + t] = i;
         if (a.lse.pm) {
             float m = slm[0][t], sm = sls[0][t];
             for (int w = 1; w < 4; ++w) lse_merge(m, sm, slm[w][t], sls[w][t]);
-            a.lse.pm[(size_t)blockIdx.x * 32 + t] = m;
-            a.lse.ps[(size_t)blockIdx.x * 32 + t] = sm;
+            a.lse.pm[(size_t)bid * 32 + t] = m;
+            a.lse.ps[(size_t)bid * 32 + t] = sm;
         }
     }
 }
@@ -307,7 +331,7 @@ __global__ __launch_bounds__(512) void k_lm_head(HeadArgs a) {
 //
 // Work unit: one K half of a strip, as k_lm_head: wave (slot, h) takes half h of strips
 // blockIdx.x * 4 + slot + round * gridDim.x * 4, the h = 1 partial meets the h = 0 one in
-// LDS (four slots; eight where a block has 16 waves).  A half streams as pieces of PL group pairs (16 rows x PL x 128 k codes plus their
+// LDS.  A half streams as pieces of PL group pairs (16 rows x PL x 128 k codes plus their
 // scales and biases), the next requested before the current one is multiplied.
 struct HeadQ4Args {
     const uint16_t* x;   // [M][K] fp16
@@ -330,13 +354,11 @@ struct Q4Piece {
     uint32_t sc[PL], bs[PL];            // scales / biases of groups 2 j, 2 j + 1 (lo, hi)
 };
 
-// NW: waves of a block.  One tile of hidden rows leaves room for two eight-wave blocks a CU; two
-// tiles (132 KB) for one, of 16 waves (17 rows 56.8 -> 51.6 us, 64 rows with logits 115.7 -> 110.8);
-// with the log-sum-exp's state (LSE) 16 waves would spill, and take eight.  (The fp16 head, bound by
-// its weight stream, is slower so: 17 rows 115 -> 123.)
-template <int NT, int PL, int NW, bool LSE>
-__global__ __launch_bounds__(NW * 64) void k_lm_head_q4(HeadQ4Args a) {
-    constexpr int NS = NW / 2;  // strips a block takes at a time
+// LSE: with the log-sum-exp's state (32 registers less without it, two tiles).  One tile of hidden
+// rows leaves room for two blocks a CU, two tiles (132 KB) for one.  (One of 16 waves: faster on
+// weights in the last-level cache, 58 -> 54 us for 17 rows, slower from HBM, 62.4 -> 64.1 for 24.)
+template <int NT, int PL, bool LSE>
+__global__ __launch_bounds__(512) void k_lm_head_q4(HeadQ4Args a) {
 
     if (aborted(a.abort)) return;
     extern __shared__ __align__(16) char q4lds[];
@@ -347,10 +369,10 @@ __global__ __launch_bounds__(NW * 64) void k_lm_head_q4(HeadQ4Args a) {
     __shared__ int s_ban[MJ_HEAD_MAX_BANNED];  // banned ids (read with LDS, not vector, loads)
     const int n = lane & 15, q = lane >> 4;
     const int nstrips = (a.V + 15) / 16;
-    const int slot = wv % NS, h = wv / NS;
+    const int slot = wv & 3, h = wv >> 2;
     const int NH = G / 2 / (2 * PL);   // pieces per half strip
-    const int SW = gridDim.x * NS;
-    const int rounds = (nstrips - (int)blockIdx.x * NS + SW - 1) / SW;
+    const int SW = gridDim.x * 4;
+    const int rounds = (nstrips - (int)blockIdx.x * 4 + SW - 1) / SW;
     // the code offset 0x4C00 (fp16 16) kept in a VGPR so each nibble pair is one mask-or
     uint32_t c16 = 0x4C004C00u;
     asm("" : "+v"(c16));
@@ -394,13 +416,13 @@ __global__ __launch_bounds__(NW * 64) void k_lm_head_q4(HeadQ4Args a) {
         }
     };
     constexpr int NPB = NT == 1 ? 2 : 1;
-    __shared__ f4 s_part[NPB][NS][NT][64];
+    __shared__ f4 s_part[NPB][4][NT][64];
     // The wave's pieces form one stream (rounds x NH) through two register sets taken in
     // turn: a set is refilled with the piece two ahead as soon as it has been multiplied, so
     // one piece is always in flight behind the one in use and no set is copied.  Every load is
     // issued -- past the stream's end at the clamped last row, a cached line -- which keeps the
     // wait before a set's use from covering the other set's requests.
-    const int strip0 = blockIdx.x * NS + slot, TP = rounds * NH;
+    const int strip0 = blockIdx.x * 4 + slot, TP = rounds * NH;
     int ld_strip = strip0, ld_pc = 0;
     auto issue = [&](Q4Piece<PL>& pz) {
         load_piece(ld_strip, ld_pc, pz);
@@ -514,22 +536,26 @@ __global__ __launch_bounds__(NW * 64) void k_lm_head_q4(HeadQ4Args a) {
         for (int tl = 0; tl < NT; ++tl) acc[tl] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
     };
     Q4Piece<PL> pa, pb;
-    for (int idx = t; idx < a.n_banned; idx += NW * 64) s_ban[idx] = a.banned[idx];
+    for (int idx = t; idx < a.n_banned; idx += 512) s_ban[idx] = a.banned[idx];
     // group sums: a row's 64-groups over the threads, each read whole before it is summed in order
-    for (int idx = t; idx < NT * 16 * G; idx += NW * 64) {
+    for (int idx = t; idx < NT * 16 * G; idx += 512) {
         const int m = idx / G, g = idx - m * G;
+        if (m >= a.M) {
+            xg[m * GS1 + g] = 0.0f;
+            continue;
+        }
         u4v v[8];
 #pragma unroll
         for (int c = 0; c < 8; ++c)
-            v[c] = *(const u4v*)(a.x + (size_t)min(m, a.M - 1) * K + 64 * g + 8 * c);
+            v[c] = *(const u4v*)(a.x + (size_t)m * K + 64 * g + 8 * c);
         float sum = 0.0f;
 #pragma unroll
         for (int c = 0; c < 8; ++c)
 #pragma unroll
             for (int j = 0; j < 4; ++j) sum += h2f(v[c][j] & 0xFFFFu) + h2f(v[c][j] >> 16);
-        xg[m * GS1 + g] = m < a.M ? sum : 0.0f;
+        xg[m * GS1 + g] = sum;
     }
-    stage_hidden<NT * 16, NW>(
+    stage_hidden<NT * 16, 8>(
         a.x, a.M, K, wv, lane,
         [&](int m, int c, u4v v) {
             u4v o;
@@ -565,9 +591,9 @@ __global__ __launch_bounds__(NW * 64) void k_lm_head_q4(HeadQ4Args a) {
                     bi[tl][r] = oi;
                 }
             }
-    __shared__ float sv[NS][32];
-    __shared__ int si[NS][32];
-    __shared__ float slm[NS][32], sls[NS][32];
+    __shared__ float sv[4][32];
+    __shared__ int si[4][32];
+    __shared__ float slm[4][32], sls[4][32];
     if constexpr (LSE) {
 #pragma unroll
         for (int tl = 0; tl < NT; ++tl)
@@ -595,7 +621,7 @@ __global__ __launch_bounds__(NW * 64) void k_lm_head_q4(HeadQ4Args a) {
     if (t < NT * 16 && t < a.M) {
         float bb = sv[0][t];
         int ii = si[0][t];
-        for (int w2 = 1; w2 < NS; ++w2)
+        for (int w2 = 1; w2 < 4; ++w2)
             if (sv[w2][t] > bb || (sv[w2][t] == bb && si[w2][t] < ii)) {
                 bb = sv[w2][t];
                 ii = si[w2][t];
@@ -604,7 +630,7 @@ __global__ __launch_bounds__(NW * 64) void k_lm_head_q4(HeadQ4Args a) {
         a.pidx[(size_t)blockIdx.x * 32 + t] = ii;
         if constexpr (LSE) {
             float m = slm[0][t], sm = sls[0][t];
-            for (int w2 = 1; w2 < NS; ++w2) lse_merge(m, sm, slm[w2][t], sls[w2][t]);
+            for (int w2 = 1; w2 < 4; ++w2) lse_merge(m, sm, slm[w2][t], sls[w2][t]);
             a.lse.pm[(size_t)blockIdx.x * 32 + t] = m;
             a.lse.ps[(size_t)blockIdx.x * 32 + t] = sm;
         }
@@ -833,6 +859,33 @@ hipError_t launch_lm_head(const uint16_t* x, const uint16_t* w, int M, int K, in
                           const int* abort, hipStream_t st, const GreedyAccept* ga) {
     if (K % 256 != 0 || M < 1 || n_banned > MJ_HEAD_MAX_BANNED)  // halves of 128-k multiples
         return hipErrorInvalidValue;
+    // Past 32 rows (the most a block stages): both groups of rows in one launch, half of the blocks
+    // each (64 rows 267 -> 169 us as one launch after another; V 151936, logits kept)
+    const int nb2 = head_blocks() / 2;
+    if (M > 32 && M <= 64 && nb2 % 16 == 0) {
+        const size_t lds = (size_t)32 * (K + 8) * 2;
+        if (lds > 136 * 1024) return hipErrorInvalidValue;
+        HeadLse gl = lse;
+        if (!gl.out) gl.pm = gl.ps = nullptr;
+        HeadArgs a{x, w, M, K, V, banned, n_banned, logits, pval, pidx, abort, gl, 1};
+        if ((K / 64) % 8 == 0)
+            launch_timed(k_lm_head<2, 8>, dim3(nb2), dim3(512), lds, st, a);
+        else
+            launch_timed(k_lm_head<2, 4>, dim3(nb2), dim3(512), lds, st, a);
+        hipError_t e = hipGetLastError();
+        for (int m0 = 0; m0 < M && e == hipSuccess; m0 += 32) {
+            HeadLse fl = gl;
+            const size_t at = (size_t)m0 * (nb2 / 2);
+            if (fl.out) {
+                fl.out += m0;
+                fl.pm += at;
+                fl.ps += at;
+            }
+            e = launch_head_final(pval + at, pidx + at, nb2 / 2, M, m0, std::min(M - m0, 32), out_idx,
+                                  out_max, fl, abort, st, ga);
+        }
+        return e;
+    }
     for (int m0 = 0; m0 < M; m0 += 32) {
         const int mg = M - m0 < 32 ? M - m0 : 32;
         // two blocks per CU for one 16-row tile; a 32-row group's LDS allows one
@@ -841,7 +894,7 @@ hipError_t launch_lm_head(const uint16_t* x, const uint16_t* w, int M, int K, in
         if (!gl.out) gl.pm = gl.ps = nullptr;
         else gl.out += m0;
         HeadArgs a{x + (size_t)m0 * K, w, mg, K, V, banned, n_banned,
-                   logits ? logits + (size_t)m0 * V : nullptr, pval, pidx, abort, gl};
+                   logits ? logits + (size_t)m0 * V : nullptr, pval, pidx, abort, gl, 0};
         const bool pl8 = (K / 64) % 8 == 0;  // 8-chunk pieces when the half strip allows
         if (mg <= 16) {
             const size_t lds = (size_t)16 * (K + 8) * 2;
@@ -1090,17 +1143,17 @@ hipError_t launch_lm_head_q4(const uint16_t* x, const uint32_t* w, const uint16_
         HeadQ4Args qa{x + (size_t)m0 * K, w, s, b, mg, K, V, banned, n_banned,
                       logits ? logits + (size_t)m0 * V : nullptr, pval, pidx, abort, gl};
         const bool ls = gl.out != nullptr;
-        auto go = [&](auto plain, auto with_lse, int nw, int nw_lse) {
-            launch_timed(ls ? with_lse : plain, dim3(nb), dim3(64 * (ls ? nw_lse : nw)), lds, st, qa);
+        auto go = [&](auto plain, auto with_lse) {
+            launch_timed(ls ? with_lse : plain, dim3(nb), dim3(512), lds, st, qa);
         };
         if (nt == 1 && pl4)
-            go(k_lm_head_q4<1, 4, 8, false>, k_lm_head_q4<1, 4, 8, true>, 8, 8);
+            go(k_lm_head_q4<1, 4, false>, k_lm_head_q4<1, 4, true>);
         else if (nt == 1)
-            go(k_lm_head_q4<1, 2, 8, false>, k_lm_head_q4<1, 2, 8, true>, 8, 8);
+            go(k_lm_head_q4<1, 2, false>, k_lm_head_q4<1, 2, true>);
         else if (pl4)
-            go(k_lm_head_q4<2, 4, 16, false>, k_lm_head_q4<2, 4, 8, true>, 16, 8);
+            go(k_lm_head_q4<2, 4, false>, k_lm_head_q4<2, 4, true>);
         else
-            go(k_lm_head_q4<2, 2, 16, false>, k_lm_head_q4<2, 2, 8, true>, 16, 8);
+            go(k_lm_head_q4<2, 2, false>, k_lm_head_q4<2, 2, true>);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         e = launch_head_final(pval, pidx, nb, M, m0, mg, out_idx, out_max, gl, abort, st, ga);
@@ -1112,19 +1165,18 @@ hipError_t launch_lm_head_q4(const uint16_t* x, const uint32_t* w, const uint16_
 hipError_t set_kernel_attributes() {
     static bool done = false;
     if (done) return hipSuccess;
-    // (two tiles: 136 KB of hidden rows beside 21 KB of partials)
     const void* hk[] = {(const void*)k_lm_head<1, 8>,
                         (const void*)k_lm_head<1, 4>,
                         (const void*)k_lm_head<2, 8>,
                         (const void*)k_lm_head<2, 4>,
-                        (const void*)k_lm_head_q4<1, 4, 8, false>,
-                        (const void*)k_lm_head_q4<1, 4, 8, true>,
-                        (const void*)k_lm_head_q4<1, 2, 8, false>,
-                        (const void*)k_lm_head_q4<1, 2, 8, true>,
-                        (const void*)k_lm_head_q4<2, 4, 16, false>,
-                        (const void*)k_lm_head_q4<2, 4, 8, true>,
-                        (const void*)k_lm_head_q4<2, 2, 16, false>,
-                        (const void*)k_lm_head_q4<2, 2, 8, true>};
+                        (const void*)k_lm_head_q4<1, 4, false>,
+                        (const void*)k_lm_head_q4<1, 4, true>,
+                        (const void*)k_lm_head_q4<1, 2, false>,
+                        (const void*)k_lm_head_q4<1, 2, true>,
+                        (const void*)k_lm_head_q4<2, 4, false>,
+                        (const void*)k_lm_head_q4<2, 4, true>,
+                        (const void*)k_lm_head_q4<2, 2, false>,
+                        (const void*)k_lm_head_q4<2, 2, true>};
     hipError_t e = hipSuccess;
     for (const void* k : hk)
         if (e == hipSuccess)
