@@ -484,6 +484,8 @@ mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint1
     // its pass (a verify row equals the one-row decode step at its position, bit for bit)
     const bool wide = M > MJ_MAX_ROWS;  // a wide prefill pass: the products take slot tables
     const bool tile = fused && M >= MJ_TILE_MIN_ROWS && up_tile && dn_tile;
+    // other shapes (experts not a multiple of 8, H 4096, an I one product has no tile kernel for):
+    // each product takes the tile kernel where it has one, the general kernel over buckets else
     if (wide && (!moe_wide_supported(H, I, E, k, w->gs) || !ms.up_tab.rec))
         return mj_fail(ctx, MJ_INVALID_ARG, "MoE block of %d rows", M);
     // the common expert shape, up to 32 rows over at most 64 experts: one launch ranks the
@@ -584,10 +586,11 @@ mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint1
             s = mj_hip(ctx, launch_router((const uint16_t*)w->router_w, xn, ms.logits, M, E, H,
                                           ab, st), "router");
             if (s != MJ_OK) return s;
-            s = mj_hip(ctx, launch_topk_bucket(ms.logits, M, E, k, inds, scores, ms.bk, ab, st),
+            s = mj_hip(ctx, launch_topk_bucket(ms.logits, M, E, k, inds, scores,
+                                               up_tile && dn_tile ? nullptr : ms.bk, ab, st),
                        "topk");
             if (s != MJ_OK) return s;
-        } else if (!tile) {
+        } else if (!up_tile || !dn_tile) {
             s = mj_hip(ctx, launch_bucket_inds(inds, M * k, ms.bk, ab, st), "bucket");
             if (s != MJ_OK) return s;
         }
@@ -598,7 +601,7 @@ mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint1
         up.w = w->up_gate_w;
         up.s = (const uint16_t*)w->up_gate_s;
         up.b = (const uint16_t*)w->up_gate_b;
-        if (!tile) {
+        if (!up_tile) {
             up.bk = ms.bk;
         } else if (wide) {
             up.tab = ms.up_tab.rec;
@@ -631,21 +634,22 @@ mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint1
             if (prof) prof->end(st);
             if (s != MJ_OK) return s;
         }
-        // the tile kernel's SwiGLU epilogue writes act without block sums: the tile down
-        // kernel forms them from its staged rows, any other down kernel gets them here
-        // (a wide pass too: each act row is staged by many items)
+        // act's block sums: the general kernel's SwiGLU epilogue writes them, the tile kernel's
+        // does not.  The tile down kernel forms them from its staged rows, any other down kernel
+        // gets them here (a wide pass too: each act row is staged by many items)
         if (up_tile && (!dn_tile || wide)) {
             s = mj_hip(ctx, launch_qx_sums(ms.act, ms.act_sum, M * k, I, ab, st), "act sums");
             if (s != MJ_OK) return s;
         }
         GatherArgs dn = up;
         dn.rlogits = nullptr;  // the down product takes the ids the routing wrote
+        dn.bk = dn_tile ? nullptr : ms.bk;
         if (wide) {
             dn.tab = ms.dn_tab.rec;
             dn.tab_slots = ms.dn_tab.n;
-        } else if (tile) {
-            dn.inds = inds;
-            dn.npairs = M * k;
+        } else {
+            dn.inds = dn_tile ? inds : nullptr;
+            dn.npairs = dn_tile ? M * k : 0;
         }
         dn.xperm = ms.act;
         dn.xsum = dn_tile && !wide ? nullptr : ms.act_sum;
