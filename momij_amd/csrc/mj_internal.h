@@ -321,7 +321,8 @@ void nucleus_layout(void* base, int V, NucleusBuf& nb);
 // Full-vocabulary sampled acceptance.  With sd the temperature, q, uniforms' seed / counter,
 // the drafts and the options' scalars come from the step descriptor (hist arrays from o).
 // head_max: the exact maxima of the rows as given (the lm_head's), for a call without
-// penalties only (the caller knows): the launch that makes the rows ready is then left out.
+// penalties only (the caller knows): the launch that makes the rows ready, or finds their maxima
+// where nothing is to be made ready, is then left out.
 // src: the logits given, where `logits` is the buffer their penalised rows go to (nullptr: in place).
 hipError_t launch_accept_sampled(float* logits, int rows, int V, const int32_t* draft,
                                  float temperature, int q_mode, const float* q_point,

@@ -55,3 +55,32 @@ def test_penalties(ctx, orc, V, n_hist):
         ref = orc.accept_sampled_ex(lg, draft, 0.9, 1, u, hist_tok=tok, hist_cnt=cnt, **kw)
         assert tuple(int(v) for v in host(out)) == ref, (trial, V, n_hist)
     assert (host(dl).view(np.uint32) == lg.view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("V", [1, 31, 33, 4096, 40001, 196608])
+@pytest.mark.parametrize("rows", [1, 9, 64])
+def test_without_penalties(ctx, orc, V, rows):
+    """The row maxima alone: fewer ids than slices, rows of no multiple of 4 and rows that start
+    off a 16-byte line, the maximum in the first and the last id."""
+    import torch
+
+    print(f"case: no penalties V={V} rows={rows}", flush=True)
+    rng = np.random.default_rng(V + rows)
+    lg = (rng.standard_normal((rows, V)) * 2).astype(np.float32)
+    draft = rng.integers(0, V, rows - 1).astype(np.int32)
+    for r in range(rows - 1):
+        lg[r, draft[r]] += 12.0
+    lg[0, 0] = 30.0
+    lg[-1, V - 1] = 40.0
+    buf = torch.zeros(rows * V + 4, dtype=torch.float32, device="cuda")
+    dd = dev(draft) if rows > 1 else torch.zeros(1, dtype=torch.int32, device="cuda")
+    for off, top_p in ((0, 1.0), (0, 0.8), (1, 1.0)):
+        dl = buf[off:off + rows * V]
+        dl.copy_(dev(lg).reshape(-1))
+        out = torch.empty(2, dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        ctx.accept_sampled_ex(dl, rows, V, dd, 1, 5, off, out, 0.9, top_p=top_p)
+        ctx.sync()
+        u = orc.verify_uniforms(5, off, rows)
+        ref = orc.accept_sampled_ex(lg, draft, 0.9, 1, u, top_p=top_p)
+        assert tuple(int(v) for v in host(out)) == ref, (off, top_p)
