@@ -526,7 +526,7 @@ mj_status run_moe(mj_ctx* ctx, const mj_moe_weights* w, const uint16_t* x, uint1
             ut.ps = gather3_part_rows(EPI_SWIGLU, H, 2 * I, w->gs, w->up_gate_alpha != nullptr,
                                       M * k, E);
             dt.ps = gather3_part_rows(EPI_STORE, I, H, w->gs, w->down_alpha != nullptr, M * k, E);
-            s = mj_hip(ctx, launch_wide_slots(inds, M * k, ut, dt, ab, st), "slots");
+            s = mj_hip(ctx, launch_wide_slots(inds, M * k, E, ut, dt, ab, st), "slots");
             if (s != MJ_OK) return s;
         }
         if (M == 1 && !tile && (flags & MJ_MOE_PRENORM)) xn = ms.xn;

@@ -284,7 +284,7 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
         if (tid == 0) t.nslot = aborted(a.abort) ? -1 : 0;
         __syncthreads();
         if (t.nslot < 0) return;
-        const bool ok = (unsigned)idv < (unsigned)MJ_MAX_EXPERTS;
+        const bool ok = (unsigned)idv < (unsigned)(a.experts > 0 ? a.experts : MJ_MAX_EXPERTS);
         if (tid < MJ_MAX_PAIRS) ((uint8_t*)t.id)[8 * (tid & 63) + (tid >> 6)] = (uint8_t)idv;
         if (ok) atomicAdd(&s_cnt[idv], 1u);
         // (pairs without an expert: their bits of the lanes' bytes go through the scratch)

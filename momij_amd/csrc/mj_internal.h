@@ -102,8 +102,8 @@ struct GatherArgs {
     const uint16_t* b;
     const Buckets* bk;      // general kernel: rows grouped by expert (nullptr: dense)
     const int32_t* inds;    // tile kernel, persistent: expert of every pair [npairs] (pairs whose
-    int npairs;             // id is outside [0, MJ_MAX_EXPERTS) are left out)
-    int experts;            // experts the pairs are spread over (0: not known)
+    int npairs;             // id is outside [0, experts) are left out)
+    int experts;            // experts the pairs are spread over (0: not known, MJ_MAX_EXPERTS at most)
     const int32_t* tab;     // tile kernel, persistent, wide passes: the slot table (SlotTab) of the
     int tab_slots;          // npairs pairs
     int dense_rows;         // dense: rows 0 .. dense_rows-1 of expert 0
@@ -162,8 +162,8 @@ struct SlotTab {
 };
 #define MJ_SLOT_PS_MIN 8  // pairs a slot the tables are sized for, at least
 constexpr int slot_tab_size(int E, int ps) { return E + MJ_WIDE_PAIRS / ps + 1; }
-hipError_t launch_wide_slots(const int32_t* inds, int P, const SlotTab& up, const SlotTab& dn,
-                             const int* abort, hipStream_t st);
+hipError_t launch_wide_slots(const int32_t* inds, int P, int E, const SlotTab& up,
+                             const SlotTab& dn, const int* abort, hipStream_t st);
 
 // gather.hip: pairs a slot of a wide pass's product takes (its launch's rows a pass)
 int gather3_part_rows(int epi, int K, int N, int gs, bool alpha, int npairs, int experts);

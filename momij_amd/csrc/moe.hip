@@ -635,10 +635,11 @@ hipError_t launch_route_topk(const RouteArgs& a, hipStream_t st) {
 
 // The slot tables of a wide pass's two expert products, from its pairs' expert ids: one block,
 // thread t < 256 numbering expert t's slots by sums across the experts, then a pair a thread
-// taking the next place of its expert.  The places' order varies from run to run, which moves rows
+// taking the next place of its expert (a pair whose id is outside [0, E) has none).  The places' order varies from run to run, which moves rows
 // within a slot and changes no value.
 __global__ __launch_bounds__(1024) void k_wide_slots(const int32_t* __restrict__ inds, int P,
-                                                     SlotTab up, SlotTab dn, const int* abort) {
+                                                     int E, SlotTab up, SlotTab dn,
+                                                     const int* abort) {
     __shared__ int s_cnt[MJ_MAX_EXPERTS], s_at[MJ_MAX_EXPERTS], s_first[2][MJ_MAX_EXPERTS];
     __shared__ int s_tot[2][4];
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
@@ -651,7 +652,7 @@ __global__ __launch_bounds__(1024) void k_wide_slots(const int32_t* __restrict__
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < PT; ++i)
-        if ((unsigned)id[i] < (unsigned)MJ_MAX_EXPERTS) atomicAdd(&s_cnt[id[i]], 1);
+        if ((unsigned)id[i] < (unsigned)E) atomicAdd(&s_cnt[id[i]], 1);
     __syncthreads();
     int incl[2] = {0, 0}, parts[2] = {0, 0};
     if (t < MJ_MAX_EXPERTS) {
@@ -687,7 +688,7 @@ __global__ __launch_bounds__(1024) void k_wide_slots(const int32_t* __restrict__
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
         const int e = id[i], p = t + 1024 * i;
-        if ((unsigned)e >= (unsigned)MJ_MAX_EXPERTS) continue;
+        if ((unsigned)e >= (unsigned)E) continue;
         const int c = s_cnt[e], at = atomicAdd(&s_at[e], 1);
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
@@ -705,12 +706,12 @@ __global__ __launch_bounds__(1024) void k_wide_slots(const int32_t* __restrict__
     }
 }
 
-hipError_t launch_wide_slots(const int32_t* inds, int P, const SlotTab& up, const SlotTab& dn,
-                             const int* abort, hipStream_t st) {
+hipError_t launch_wide_slots(const int32_t* inds, int P, int E, const SlotTab& up,
+                             const SlotTab& dn, const int* abort, hipStream_t st) {
     for (const SlotTab* tab : {&up, &dn})
         if (tab->ps < 1 || tab->ps > 16 || tab->n < slot_tab_size(MJ_MAX_EXPERTS, tab->ps))
             return hipErrorInvalidValue;
-    if (P < 1 || P > MJ_WIDE_PAIRS) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_wide_slots, dim3(1), dim3(1024), 0, st, inds, P, up, dn, abort);
+    if (P < 1 || P > MJ_WIDE_PAIRS || E < 1 || E > MJ_MAX_EXPERTS) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_wide_slots, dim3(1), dim3(1024), 0, st, inds, P, E, up, dn, abort);
     return hipGetLastError();
 }

@@ -68,8 +68,10 @@ __device__ __forceinline__ T wave_reduce_dpp(T v, Op op) {
 // 64): experts ahead of it -- a larger logit, or an equal logit at a lower index.  The row is
 // read as broadcast float4s issued together and "larger" counted from the sign of l - o (exact
 // for distinct finite values, +0 for equal ones; -0 was folded into +0 when the row was
-// staged).  Without ties the counts of the E experts are a permutation of 0..E-1; any other sum
-// sends the row through the exact comparison rule.  Padding is -inf, which no real logit is
+// staged).  Without ties the counts of the E experts are a permutation of 0..E-1; any other sum,
+// and a NaN, sends the row through the exact comparison rule.  That compares the bits as integers in
+// the values' order, in which NaN has a place too: the ranks are a permutation of 0..E-1 whatever the
+// row holds, so every row picks k experts that exist.  Padding is -inf, which no real logit is
 // below.
 __device__ __forceinline__ int row_rank64(const float* s_row, int E) {
     const int lane = threadIdx.x & 63;
@@ -86,11 +88,16 @@ __device__ __forceinline__ int row_rank64(const float* s_row, int E) {
             gt += (__float_as_uint(l - o[j4][c]) >> 31) + (__float_as_uint(l - o[j4][c + 1]) >> 31);
     int rank = (int)gt;
     const float rsum = wave_reduce_dpp(lane < E ? (float)gt : 0.0f, add_op);
-    if (rsum != 0.5f * (float)(E * (E - 1))) {
+    if (rsum != 0.5f * (float)(E * (E - 1)) || __ballot(l != l) != 0ull) {
+        const auto key = [](float v) {
+            const int b = __float_as_int(v);
+            return b ^ ((b >> 31) & 0x7FFFFFFF);
+        };
+        const int lk = key(l);
         rank = 0;
         for (int jj = 0; jj < E; ++jj) {
-            const float oj = s_row[jj];
-            rank += (int)(oj > l) + (int)(oj == l && jj < lane);
+            const int oj = key(s_row[jj]);
+            rank += (int)(oj > lk) + (int)(oj == lk && jj < lane);
         }
     }
     return rank;

@@ -143,3 +143,38 @@ def test_moe_shapes_without_the_routed_launch(ctx, orc, H, E, I, gs, k, M):
     assert (host(inds) == ri).all()
     rel, _ = assert_close(host(y), ref, what="moe")
     assert rel < 5e-3  # fp16 between the stages, as the block's other shapes
+
+
+@pytest.mark.parametrize("E,I,gs,M", [
+    (16, 512, 64, 40), (40, 1024, 64, 64), (256, 512, 128, 17), (12, 1024, 64, 20),  # from ids
+    (64, 1024, 64, 9), (64, 1024, 64, 24), (64, 512, 64, 12),  # ranked in the product's launch
+])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_a_row_that_overflowed_keeps_to_itself(ctx, E, I, gs, M, bad):
+    """A row whose router logits are NaN still picks experts that exist (and, by the fused router,
+    distinct ones), and the rows that share its pass come out as without it, bit for bit."""
+    import torch
+
+    print(f"case: overflowed row E={E} I={I} gs={gs} M={M} {bad}", flush=True)
+    rng = np.random.default_rng(E + I + M)
+    H, k = 2048, 8
+    mw = synth.moe_weights(rng, E, H, I, gs, top_k=k)
+    dmw = {n: (dev(v) if isinstance(v, np.ndarray) else v) for n, v in mw.items()}
+    x = synth.normal_f16(rng, (M, H))
+    r = M // 2
+    outs = []
+    for v in (None, bad):
+        xv = x.copy()
+        if v is not None:
+            xv[r, 5] = v
+        dx, y = dev(xv), torch.empty((M, H), dtype=torch.float16, device="cuda")
+        inds = torch.full((M, k), -1, dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        ctx.moe_block(dmw, dx, y, M, 3, inds)
+        ctx.sync()
+        outs.append((host(y).view(np.uint16), host(inds)))
+    (y0, i0), (y1, i1) = outs
+    rest = np.arange(M) != r
+    assert (y0[rest] == y1[rest]).all() and (i0[rest] == i1[rest]).all()
+    assert i1[r].min() >= 0 and i1[r].max() < E
+    assert E % 8 or len(set(i1[r].tolist())) == k
