@@ -68,7 +68,7 @@ struct mj_model {
     MoeScratch ms{};
     int wide_rows = 0;            // rows a prefill pass may have (MJ_MAX_ROWS: no wide passes)
     // what the rows of a wide pass past the ring's slack of 64 overwrite, kept until the pass is
-    // through: an aborted pass puts it back, so that its start stays a position to go on from
+    // through: a pass that fails puts it back, so that its start stays a position to go on from
     uint16_t* kv_save = nullptr;
     bool kv_saved = false;        // taken by the pass now queued
     StepDesc* sd_dev = nullptr;   // one for each 64 rows of a pass
@@ -759,7 +759,9 @@ static mj_status feed_wide(mj_model* m, const int32_t* tokens, int M, int kind) 
     }
     m->kv_saved = false;
     mj_status s = run_pass(m, kind, M);
-    if (s == MJ_ABORTED && m->kv_saved) {
+    // whatever ended the pass (an abort, a fault left by an earlier call, a launch refused half way):
+    // the rows go back, on the stream, behind what was queued of it
+    if (s != MJ_OK && m->kv_saved) {
         const mj_model_config& c = m->cfg;
         mj_status r = mj_hip(m->ctx, launch_kv_save(m->kv, m->layer_stride, c.n_layers,
                                                     c.kv_capacity, c.n_kv_heads, m->offset,

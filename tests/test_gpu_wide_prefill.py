@@ -169,3 +169,46 @@ def test_wide_abort_leaves_its_start_valid(ctx):
                 assert (a == b).all()
     assert cut > 0
     eng.close()
+
+
+def test_wide_failure_leaves_its_start_valid(ctx):
+    """The same where the pass ends with an error: a wait that ran out its bound in an earlier call
+    (forced by a bound of 0) is reported by the prefill that follows it."""
+    import torch
+
+    from momij_amd import synth
+
+    eng, cfg = _engine(ctx, 16, 512, 64, False, 4, 160, full=False)
+    rng = np.random.default_rng(9)
+    # 100 rows from 150: the last 36 take the slots of keys that the first ones need, and every row
+    # is still in the cache at the end
+    prompt = rng.integers(0, cfg.vocab, 250).tolist()
+    want = eng.prefill(prompt)
+    ref = _cache(eng, cfg)
+    mw = synth.moe_weights(rng, 64, 2048, 1024, 64)
+    dmw = {n: (torch.from_numpy(v.view(np.int32) if v.dtype == np.uint32 else v).cuda()
+               if isinstance(v, np.ndarray) else v) for n, v in mw.items()}
+    x = torch.from_numpy(synth.normal_f16(rng, (1, 2048))).cuda()
+    y = torch.empty_like(x)
+    torch.cuda.synchronize()
+    reported = 0
+    for _ in range(4):
+        eng.rewind(0)
+        eng.prefill(prompt[:150])
+        ctx.set_wait_limit(0)
+        try:
+            # one row: half of the blocks have no up item and check down items' rows at once
+            ctx.moe_block(dmw, x, y, 1, 3)
+        finally:
+            ctx.set_wait_limit(1 << 17)
+        try:
+            got = eng.prefill(prompt[150:])
+        except MomijError as e:
+            assert e.status == 6 and eng.offset == 150, e
+            reported += 1
+            got = eng.prefill(prompt[150:])
+        assert got == want
+        for a, b in zip(_cache(eng, cfg), ref):
+            assert (a == b).all()
+    assert reported > 0
+    eng.close()
