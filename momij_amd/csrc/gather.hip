@@ -211,6 +211,7 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
     constexpr bool FUSABLE = FUS;
     static_assert(!FUS || EPI == EPI_SWIGLU, "fused routing: persistent up || gate");
     __shared__ __align__(16) std::conditional_t<FUSABLE, FusedRoute, char> s_fr;
+    __shared__ int s_stop;
     constexpr bool fused = FUS;
     static_assert(MODE == 0 || (MODE == 1 && FUS) || (MODE == 2 && REC == REC_RANK && EPI == EPI_STORE),
                   "fused MoE phases: up || gate with routing, then down");
@@ -358,13 +359,15 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
 #pragma unroll
             for (int sr = 0; sr < RPW; ++sr)
                 v[sr] = a.rlogits[min(wv + WPB * sr, M - 1) * E + min(lane, E - 1)];
-            if (aborted(a.abort)) return;
+            const bool ab = aborted(a.abort);
+            if (tid == 0) s_stop = ab ? 1 : 0;  // one reading decides for the block, as block_aborted
             if (wv == 0) {
                 s_fr.em[lane] = 0u;
                 s_fr.er[lane] = 0ull;
                 if constexpr (FR > 16) s_fr.er1[lane] = 0ull;
             }
             __syncthreads();  // (LDS only: the logits stay in flight)
+            if (s_stop) return;
             // expert t picked by row r at rank rk: its bits, ORed in from any wave
             auto mark = [&](int t, int r, int rk) {
                 __hip_atomic_fetch_or(&s_fr.em[t], 1u << r, __ATOMIC_RELAXED,
@@ -408,7 +411,9 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
         }
     }
     {
-        const int ab = !PER && a.abort ? *a.abort : 0;  // persistent: checked with the routing
+        // (persistent: decided with the routing, for the block; dense: a wave by itself, since the
+        // rows it writes follow from the block's index alone)
+        const int ab = !PER && a.abort ? *a.abort : 0;
         if constexpr (PER) {
             if constexpr (MODE == 2) {
                 // blocks with one up item fewer come free first: they take the first down items
@@ -419,7 +424,7 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
             }
             const int rec = slot_rec(LIST ? item / ncb : min(item / ncb, 63));
             if constexpr (REC == REC_TAB)
-                if (aborted(a.abort)) return;
+                if (block_aborted(a.abort)) return;
             e = __builtin_amdgcn_readlane(rec, 0) >> 16;
             np = LIST || item / ncb < 64 ? __builtin_amdgcn_readlane(rec, 1) >> 16 : 0;
             lpair = rec & 0xFFFF;
@@ -441,6 +446,8 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
     char* red = (char*)(xsl0 + RA * S::SS);  // [KS-1][TPB][64] f4
     __shared__ int s_pair[NBUF][R];
     int buf = 0;
+    // pair of row i of the pass from pb
+    auto pair_of = [&](int pb, int i) { return PER ? s_pair[buf][i] : rbase + pb + i; };
     auto xs_of = [&](int) { return xs0; };
     auto xsl_of = [&](int) { return xsl0; };
 
@@ -474,7 +481,7 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
         for (int j = 0; j < R / WPB; ++j) {
             const int r = wv + WPB * j;
             const int pr = __builtin_amdgcn_readlane(prl, r);
-            if (lane == 0) s_pair[b][r] = pr;
+            if (PER && lane == 0) s_pair[b][r] = pr;
             if (r < npass) {
                 const char* src = (const char*)(a.xperm + (size_t)(pr / a.x_div) * K);
 #pragma unroll
@@ -559,8 +566,9 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
     // block is resident, two a CU, and then every up item completes; a wait that runs out its
     // bound sets the fault word, which the host reports, and goes on, so the launch always ends.
     __shared__ int s_mark[WPB];
-    // a half of the pass's staged rows still holds the marker (the same answer in every thread)
-    auto rows_marked = [&](int npass) -> bool {
+    // bit 0: a half of the pass's staged rows still holds the marker; bit 1, where it is looked at:
+    // the abort word is set (thread 0's reading).  The same answer in every thread
+    auto rows_marked = [&](int npass, bool look) -> int {
         const uint16_t* xs = xs_of(buf);
         bool bad = false;
         for (int idx = tid; idx < npass * (K / 8); idx += NT) {
@@ -571,12 +579,14 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
                 bad |= (v[w] & 0xFFFFu) == 0xFFFFu || (v[w] >> 16) == 0xFFFFu;
         }
         const bool wbad = __ballot(bad) != 0ull;
-        if (lane == 0) s_mark[wv] = wbad ? 1 : 0;
+        int mine = wbad ? 1 : 0;
+        if (look && wv == 0) mine |= aborted(a.abort) ? 2 : 0;
+        if (lane == 0) s_mark[wv] = mine;
         lds_only_barrier();
         int any = 0;
 #pragma unroll
         for (int w = 0; w < WPB; ++w) any |= s_mark[w];
-        return any != 0;
+        return any;
     };
 
   for (;;) {
@@ -615,13 +625,14 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
             lds_barrier<0>();
         if constexpr (MODE == 2) {
             // act rows an up item has not finished yet: staged again until they have
-            for (int it = 0; rows_marked(npass); ++it) {
+            for (int it = 0;; ++it) {
+                const int marks = rows_marked(npass, (it & 63) == 63);
+                if (marks != 1) break;
                 if (it >= a.fpolls) {
                     if (a.ffault != nullptr && tid == 0)
                         __hip_atomic_store(a.ffault, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                     break;
                 }
-                if ((it & 63) == 63 && aborted(a.abort)) break;
                 lds_only_barrier();  // every wave has read the marks before they are rewritten
                 __builtin_amdgcn_s_sleep(8);
                 stage_load(pb, npass, buf, lpair, np);
@@ -865,7 +876,7 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
                 up = fminf(fmaxf(up, -7.0f), 7.0f);
                 const float act = hround(g / (1.0f + expf(-g)) * up);
                 const int j = (cb * TPB + tt) * 8 + (n & 7);
-                uint16_t* dst = a.y + (size_t)s_pair[buf][i] * I + (j & ~15) + perm_pos(j & 15);
+                uint16_t* dst = a.y + (size_t)pair_of(pb, i) * I + (j & ~15) + perm_pos(j & 15);
                 if constexpr (MODE == 1)
                     __hip_atomic_store(dst, f2h(act), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 else
@@ -890,7 +901,7 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
             for (int r = 0; r < NR; ++r) {
                 const int i = NR == 1 ? q : 4 * q + r;
                 if (kh == 0 && i < npass && col < a.N) {
-                    uint16_t* yp = a.y + (size_t)s_pair[buf][i] * a.N + col;
+                    uint16_t* yp = a.y + (size_t)pair_of(pb, i) * a.N + col;
                     if constexpr (EPI == EPI_ADD) {
                         const uint16_t res = res_pf && pb == 0 ? (uint16_t)resv[r] : *yp;
                         *yp = f2h(h2f(res) + hround(acc[r]));

@@ -969,7 +969,7 @@ hipError_t launch_accept_greedy_tree(const int32_t* tokens, const TreeParents& p
 __global__ __launch_bounds__(256) void k_kv_commit(uint16_t* kv, int64_t layer_stride,
                                                    int64_t C, int nKV, const StepDesc* sd,
                                                    const StepResult* res, const int* abort) {
-    if (aborted(abort)) return;
+    if (block_aborted(abort)) return;
     const int t = threadIdx.x;
     // the accepted count and path (one entry a thread) requested together
     const int acc = res->accepted;

@@ -228,6 +228,18 @@ __device__ __forceinline__ h8 as_h8(u4v v) { return __builtin_bit_cast(h8, v); }
 
 __device__ __forceinline__ bool aborted(const int* flag) { return flag != nullptr && *flag != 0; }
 
+// The abort word for a block whose waves form global addresses from LDS words that other waves
+// wrote: one reading, thread 0's, decides for all of them.  The word may be set at any time; of
+// waves that each went by their own reading some would leave, and the others go on with words that
+// nobody set.  Whole block, once a kernel.
+__device__ __forceinline__ bool block_aborted(const int* flag) {
+    __shared__ int s_abort;
+    const bool ab = aborted(flag);
+    if (threadIdx.x == 0) s_abort = ab ? 1 : 0;
+    __syncthreads();
+    return s_abort != 0;
+}
+
 // ------------------------------------------------------------------------------------------
 // Canonical arithmetic for sampled acceptance.  The CPU oracle evaluates the identical IEEE
 // operation sequence, so both produce the same bits: exp by Cody-Waite reduction and a

@@ -194,7 +194,7 @@ static_assert(MJ_MAX_EXPERTS == 256, "an expert a thread");
 
 __global__ __launch_bounds__(256) void k_bucket_inds(const int32_t* __restrict__ inds, int P,
                                                      Buckets* bk, const int* abort) {
-    if (aborted(abort)) return;
+    if (block_aborted(abort)) return;
     __shared__ int s_ids[MJ_MAX_PAIRS];
     __shared__ int s_cnt[MJ_MAX_EXPERTS];
     __shared__ int s_slot[MJ_MAX_EXPERTS];
@@ -213,7 +213,7 @@ hipError_t launch_bucket_inds(const int32_t* inds, int P, Buckets* bk, const int
 __global__ __launch_bounds__(256) void k_topk_bucket(const float* __restrict__ logits, int M,
                                                      int E, int k, int32_t* inds, float* scores,
                                                      Buckets* bk, const int* abort) {
-    if (aborted(abort)) return;
+    if (block_aborted(abort)) return;
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     __shared__ int s_inds[MJ_MAX_PAIRS];
     __shared__ int s_cnt[MJ_MAX_EXPERTS];
@@ -647,7 +647,7 @@ __global__ __launch_bounds__(1024) void k_wide_slots(const int32_t* __restrict__
     int id[PT];
 #pragma unroll
     for (int i = 0; i < PT; ++i) id[i] = t + 1024 * i < P ? inds[t + 1024 * i] : -1;
-    if (aborted(abort)) return;
+    if (block_aborted(abort)) return;
     if (t < MJ_MAX_EXPERTS) s_cnt[t] = s_at[t] = 0;
     __syncthreads();
 #pragma unroll

@@ -480,7 +480,7 @@ __device__ __forceinline__ void walk_write(const SampleArgs& a, int fr, float tg
 // bonus here (or leaves it to the nucleus kernels); a reject hands row fr to k_resid_sums /
 // k_resid_walk through the state.
 __global__ __launch_bounds__(256) void k_sample_decide(SampleArgs a) {
-    if (aborted(a.abort)) return;
+    if (block_aborted(a.abort)) return;
     a = resolve(a);
     const int t = threadIdx.x;
     const int D = a.rows - 1;
@@ -786,7 +786,7 @@ __device__ __forceinline__ float nuc_kept(uint32_t k, int v, uint32_t ck, int ci
 // The cut, and block sums of the kept e in the canonical order: one 256-thread block per 1024 ids
 // (chunks of CH by the first wave).  Every block finds the cut for itself.
 __global__ __launch_bounds__(256) void k_nucleus_sums(SampleArgs a) {
-    if (aborted(a.abort)) return;
+    if (block_aborted(a.abort)) return;
     a = resolve(a);
     const NucState st = *a.nb.st;
     if (!st.need) return;
