@@ -317,7 +317,7 @@ mj_status mj_gather_qmm2(mj_ctx* ctx, const void* x, const uint32_t* w, const vo
     if (s != MJ_OK) return s;
     const int epi = epilogue == MJ_EPI_ADD ? EPI_ADD : EPI_STORE;
     // the tile kernel forms its row sets from the ids itself
-    const bool tile = gather3_supported(epi, K, N, gs);
+    const bool tile = gather3_takes(epi, K, N, gs, w, scales, biases);
     if (!tile) {
         s = mj_hip(ctx, launch_bucket_inds(inds, P, bk, ctx->abort_dev, ctx->stream), "bucket");
         if (s != MJ_OK) return s;

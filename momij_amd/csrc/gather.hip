@@ -1026,6 +1026,16 @@ bool gather3_supported(int epi, int K, int N, int gs) {
     return false;
 }
 
+// The tile kernel fetches codes, scales and biases in 16-byte parts straight into LDS, the general
+// kernel a scale at a time.  Arrays that start off a 16-byte line (views into a larger buffer) stay
+// with the general kernel in the shapes it is made for: N in steps of 16, and residual products of
+// K = 512 or 1024.  (Steps of 64 otherwise are the tile kernel's whatever the arrays' start.)
+bool gather3_takes(int epi, int K, int N, int gs, const void* w, const void* s, const void* b) {
+    const bool whole = N % 64 == 0 && (epi != EPI_ADD || K == 2048);
+    return gather3_supported(epi, K, N, gs) &&
+           (whole || (((uintptr_t)w | (uintptr_t)s | (uintptr_t)b) & 15) == 0);
+}
+
 // Whether an up || gate product over listed slots takes 16-wave blocks, one a CU, rather than two of
 // eight waves: a block then stages 16 rows, not 8, so an expert with 9 to 16 rows is unpacked once
 // (the unpacking is what bounds such passes: two thirds of the VALU's time), and each staged row

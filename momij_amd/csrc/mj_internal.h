@@ -170,6 +170,8 @@ int gather3_part_rows(int epi, int K, int N, int gs, bool alpha, int npairs, int
 
 // gather.hip: the tile gather (one 16-row weight tile over the whole K per wave)
 bool gather3_supported(int epi, int K, int N, int gs);
+// whether a product of a caller's own operands goes to it
+bool gather3_takes(int epi, int K, int N, int gs, const void* w, const void* s, const void* b);
 // the fused MoE launch: up || gate with its routing, then down, in one persistent kernel
 // (the shapes, and two blocks of the launch resident a CU: its waits assume every block runs)
 bool moe_fused_supported(int H, int I, int E, int gs, int M, bool rowa);

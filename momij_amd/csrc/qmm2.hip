@@ -422,7 +422,8 @@ hipError_t launch_gather(const GatherArgs& a, int epi, int max_rows_per_bucket, 
                          hipStream_t st) {
     // the tile kernel: dense, or over the pairs' expert ids; its SWIGLU is the experts' only
     const bool per = a.inds != nullptr || a.rlogits != nullptr || a.tab != nullptr;
-    if (a.bk == nullptr && (per || epi != EPI_SWIGLU) && gather3_supported(epi, a.K, a.N, a.gs))
+    if (a.bk == nullptr && (per ? gather3_supported(epi, a.K, a.N, a.gs)
+                                : epi != EPI_SWIGLU && gather3_takes(epi, a.K, a.N, a.gs, a.w, a.s, a.b)))
         return launch_gather3(a, epi, max_rows_per_bucket, st);
     if (per) return hipErrorInvalidValue;
     // general kernel (any K % 256 == 0, N % 16 == 0): K inside each wave, RG row groups

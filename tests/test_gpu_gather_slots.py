@@ -73,6 +73,44 @@ def test_gather_slots(ctx, orc, M, ktop, E, K, N, gs, kind, add):
     assert rel < REL
 
 
+def _off(a, by):
+    """a on the device, `by` elements past the start of a buffer of its own."""
+    import torch
+
+    t = dev(a)
+    buf = torch.empty(t.numel() + by, dtype=t.dtype, device="cuda")
+    buf[by:].copy_(t.reshape(-1))
+    return buf[by:]
+
+
+@pytest.mark.parametrize("M,ktop,E,K,N,gs,add", [
+    (5, 4, 8, 2048, 48, 64, False), (33, 2, 4, 512, 80, 128, False),
+    (17, 1, 2, 512, 128, 128, True), (9, 1, 1, 1024, 2048, 64, True),
+])
+@pytest.mark.parametrize("woff,soff", [(1, 0), (0, 1), (2, 4)])
+def test_gather_operands_off_a_line(ctx, orc, M, ktop, E, K, N, gs, add, woff, soff):
+    """Codes, scales and biases that start off a 16-byte line (views into a larger buffer)."""
+    import torch
+
+    print(f"case: off a line M={M} K={K} N={N} gs={gs} add={add} {woff} {soff}", flush=True)
+    rng = np.random.default_rng(M + K + N)
+    P = M * ktop
+    w, s, b = synth.qweight(rng, (E,), N, K, gs)
+    x = synth.normal_f16(rng, (M, K))
+    ids = rng.integers(0, E, P).astype(np.int32)
+    y0 = synth.normal_f16(rng, (P, N))
+    ref = orc.qmm2(x, w, s, b, ids, M, ktop, K, N, gs)
+    if add:
+        ref = (y0.astype(np.float32) + ref.astype(np.float32)).astype(np.float16)
+    y, dx, di = dev(y0), dev(x), dev(ids)
+    dw, ds, db = _off(w, woff), _off(s, soff), _off(b, soff)
+    torch.cuda.synchronize()
+    ctx.gather_qmm2(dx, dw, ds, db, di, y, M, ktop, K, N, gs, epilogue=int(add))
+    ctx.sync()
+    rel, _ = assert_close(host(y), ref, what="off a line")
+    assert rel < REL
+
+
 @pytest.mark.parametrize("E,I,gs,M,alpha", [
     (64, 512, 64, 1, False), (64, 512, 64, 16, True), (64, 512, 128, 32, False),  # ranked, I 512
     (64, 1024, 64, 33, False), (64, 512, 64, 64, True),  # the first rows past the ranked forms
