@@ -17,7 +17,7 @@ def ctx():
     c.close()
 
 
-def _engine(ctx, E, I, gs, alpha, top_k, capacity, n_layers=2, full=True):
+def _engine(ctx, E, I, gs, alpha, top_k, capacity, n_layers=2, full=True, heads=(16, 4)):
     import torch
 
     from momij_amd.engine import MapleLikeConfig, VerifyEngine, random_model
@@ -25,7 +25,8 @@ def _engine(ctx, E, I, gs, alpha, top_k, capacity, n_layers=2, full=True):
     kinds = ["sliding_attention", "full" if full else "sliding_attention"] * n_layers
     wins, ropes = MapleLikeConfig.maple_layer_mix(n_layers, 96, 64, kinds)
     cfg = MapleLikeConfig(n_layers=n_layers, E=E, I=I, gs=gs, top_k=top_k, vocab=2048, window=96,
-                          kv_capacity=capacity, layer_window=wins, layer_rope_dim=ropes)
+                          kv_capacity=capacity, layer_window=wins, layer_rope_dim=ropes,
+                          n_heads=heads[0], n_kv_heads=heads[1])
     layers, *rest = random_model(cfg, seed=E + I)
     if alpha:  # scale alpha, bias -alpha in every group of a row
         for lw in layers:
@@ -84,6 +85,23 @@ def test_wide_equals_chunk_passes(ctx, E, I, gs, alpha, top_k):
                 assert (a == b).all(), n
             if capture:
                 assert torch.equal(logits[:len(last)], ref_logits), n
+    eng.close()
+
+
+@pytest.mark.parametrize("heads", [(4, 4), (8, 1), (8, 4), (16, 16), (4, 2)])
+def test_wide_head_shapes(ctx, heads):
+    eng, cfg = _engine(ctx, 16, 512, 128, False, 4, 320, heads=heads)
+    rng = np.random.default_rng(sum(heads))
+    for n in (65, 250, 300):
+        prompt = rng.integers(0, cfg.vocab, n).tolist()
+        eng.rewind(0)
+        for i in range(0, n, 64):
+            last = eng.step_chain_feeds(prompt[i:i + 64])
+        ref = _cache(eng, cfg)
+        eng.rewind(0)
+        assert eng.prefill(prompt) == last[-1]
+        for a, b in zip(_cache(eng, cfg), ref):
+            assert (a == b).all(), n
     eng.close()
 
 
