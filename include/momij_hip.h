@@ -382,8 +382,9 @@ float mj_model_last_pass_ms(const mj_model* model);
  * every call).  A profiled pass waits behind a 15 ms hold kernel, so its launches are queued
  * before the GPU reaches them, and starts with 8 brackets around a kernel that waits 20 us of
  * wall-clock time: each bracketed time is the kernel's duration plus the timer's own cost, and
- * MJ_KERNEL_TIMER minus 20 us per launch is that cost.  mj_model_kernel_ms returns the summed
- * milliseconds and the launch count. */
+ * MJ_KERNEL_TIMER minus 20 us per launch is that cost.  A profiled prefill runs its 64-row chunks
+ * as passes of their own: the classes are those passes' kernels, not a shared pass's.
+ * mj_model_kernel_ms returns the summed milliseconds and the launch count. */
 #define MJ_KERNEL_EXPERT_UP 0   /* bucketed up||gate gather + SwiGLU */
 #define MJ_KERNEL_EXPERT_DOWN 1 /* bucketed down gather */
 #define MJ_KERNEL_LM_HEAD 2     /* fp16 lm_head + argmax partials */

@@ -3,8 +3,9 @@
 //
 // k_attn_chunk      maple_sdpa_d128 math (SeedlessMetal.swift:2919-2997): softmax(q k^T /
 //                   sqrt(128)) v in fp32, GQA.  Split-K over 64-key chunks ("flash decoding");
-//                   one 256-thread block per (kv head, chunk) stages Q (all rows x heads of the
-//                   group), K and V^T in LDS and runs QK^T and PV on v_mfma_f32_16x16x32_f16.
+//                   one 256-thread block per (kv head, chunk or group of four, two or four of the
+//                   pass's 16-vector query tiles) stages its Q (row x head of the kv group), K and
+//                   V^T in LDS and runs QK^T and PV on v_mfma_f32_16x16x32_f16.
 //                   Mask: committed positions inside the row's window [P-W+1, L-1]
 //                   (AttentionMasks.swift:10-27) plus the row's ancestors and itself; a chain is
 //                   the causal M-row pass.
@@ -12,9 +13,10 @@
 //                   maple_qk_norm_rope + maple_write_kv_pair do (2794-2901): per-head RMSNorm(eps)
 //                   * w, non-traditional half-split RoPE on the first rope_dim dims at the row's
 //                   position L + depth(r) (angles from the pass's RoPE table).  Queries are
-//                   finished by every block of the group (they are small); the pass's own keys
-//                   are finished by the block whose chunk holds them, which also appends them
-//                   (K finished, V as projected) at slot (L + r) % C.
+//                   finished by every block that takes them (they are small); the pass's own keys
+//                   by the blocks whose chunk holds them, the first of which also appends them
+//                   (K finished, V as projected) at slot (L + r) % C.  Of a wide prefill pass
+//                   k_attn_finish does both in place before, and k_attn_combine appends.
 // k_attn_combine    merges the chunk partials per (row, head) and writes the output in the qx
 //                   format consumed by the o-projection.
 #include <algorithm>
@@ -87,23 +89,11 @@ __device__ __forceinline__ void merge_part(float& mg, float m, float& fa, float&
 }
 
 // DPP lane moves (no LDS round trip): quad_perm [1,0,3,2] (xor 1) 0xB1, [2,3,0,1] (xor 2)
-// 0x4E; row_half_mirror 0x141, row_mirror 0x140; row_ror:n 0x120 + n (lane i of a row of 16
-// takes lane i - n mod 16)
+// 0x4E; row_half_mirror 0x141
 template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
     return __int_as_float(
         __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, 0xF, 0xF, false));
-}
-__device__ __forceinline__ float quad_xor1(float v) { return dpp<0xB1>(v); }
-__device__ __forceinline__ float quad_xor2(float v) { return dpp<0x4E>(v); }
-// sum over each row of 16 lanes, every lane of the row gets it (the same bits in every lane:
-// each step adds the same two values in either order)
-__device__ __forceinline__ float row16_sum(float v) {
-    v += dpp<0xB1>(v);
-    v += dpp<0x4E>(v);
-    v += dpp<0x141>(v);
-    v += dpp<0x140>(v);
-    return v;
 }
 // sum over each group of 8 lanes (the same bits in every lane of the group)
 __device__ __forceinline__ float lane8_sum(float v) {
@@ -128,16 +118,6 @@ __device__ __forceinline__ float xrow_sum(float v) {
     const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
-// lane i ^ X of a row of 16, X in {2, 4, 8}
-template <int X>
-__device__ __forceinline__ float row16_xor(float v, int lane) {
-    static_assert(X == 2 || X == 4 || X == 8, "lane distance");
-    if constexpr (X == 2) return dpp<0x4E>(v);
-    if constexpr (X == 8) return dpp<0x128>(v);
-    const float up = dpp<0x12C>(v), dn = dpp<0x124>(v);  // lanes i + 4, i - 4
-    return (lane & 4) ? dn : up;
-}
-
 __device__ __forceinline__ void unpack8(const u4v v, float x[8]) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -150,26 +130,6 @@ __device__ __forceinline__ u4v pack8(const float x[8]) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) o[j] = (uint32_t)f2h(x[2 * j]) | ((uint32_t)f2h(x[2 * j + 1]) << 16);
     return o;
-}
-
-// RoPE of 8 dims d0 .. d0 + 7 (d0 a multiple of 8: the run lies on one side of half and of
-// 2 half): dims below half take v cos - u sin, dims in [half, 2 half) v cos + u sin (u the
-// partner dim d +/- half, angles cs[i]), later dims pass through (cos 1, sin 0).  Branch-free.
-template <int HALF>
-__device__ __forceinline__ void rope8(float v[8], const float u[8], const float2* cs, int d0) {
-    const bool rot = d0 < 2 * HALF;
-    const float sg = d0 < HALF ? -1.0f : 1.0f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const float2 c = cs[i];
-        const float cx = rot ? c.x : 1.0f, sy = rot ? sg * c.y : 0.0f;
-        v[i] = v[i] * cx + u[i] * sy;
-    }
-}
-// first angle of dims d0 .. (frequency d0 or d0 - half; 0 past 2 half, where nothing is read)
-template <int HALF>
-__device__ __forceinline__ int rope_f0(int d0) {
-    return d0 < 2 * HALF ? (d0 < HALF ? d0 : d0 - HALF) : 0;
 }
 
 // One vector's RMSNorm and RoPE over eight lanes: a lane holds dims 8 pa + i (xa) and, X parts above,

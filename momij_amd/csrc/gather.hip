@@ -5,7 +5,8 @@
 //
 // Layout of the work: a block serves one expert (or the dense projection) and a strip of
 // its output rows.  It stages the activation rows routed to that expert (qx order, up to 16
-// per pass, read from the expert's pair list) in LDS once for all its waves.  Each wave owns
+// per pass) in LDS once for all its waves; which rows those are it forms itself, from the router
+// logits or the pairs' expert ids, or reads from a slot table.  Each wave owns
 // a tile of 16 weight rows over one K-slice (KS slices per tile, summed through LDS at the
 // end).  It issues every load of its weight tile (scales, biases, then the codes in 1 KB
 // column groups, global -> LDS directly) before its first wait, and runs the MFMAs of a
@@ -68,10 +69,8 @@ struct G5Shape {
     // K-slice partials: in a wave's own tile area when every bucket is one pass, else in their
     // own region (later passes reuse the tiles)
     static constexpr int RED = (KS - 1) * TPB * 64 * 16;
-    // dbl: two sets of staged rows (persistent mode stages the next item's while this one
-    // finishes)
-    __host__ __device__ static size_t lds(int RA, bool multi, bool dbl = false) {
-        return (size_t)WPB * WAVE_BYTES + (dbl ? 2 : 1) * ((size_t)RA * XS * 2 + (size_t)RA * SS * 8) +
+    __host__ __device__ static size_t lds(int RA, bool multi) {
+        return (size_t)WPB * WAVE_BYTES + (size_t)RA * XS * 2 + (size_t)RA * SS * 8 +
                (multi ? RED : 0);
     }
 };
@@ -123,7 +122,6 @@ __device__ __forceinline__ void lds_only_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// static LDS of the fused routing's slot records (persistent up || gate kernels)
 // static LDS of the routing words of a launch that ranks up to FR rows itself
 constexpr size_t g5_fused_rec_bytes(int FR) { return 64 * (4 + 8 + (FR > 16 ? 8 : 0)); }
 
@@ -377,7 +375,7 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
                 __hip_atomic_fetch_or(w, (uint64_t)rk << (3 * (r & 15)), __ATOMIC_RELAXED,
                                       __HIP_MEMORY_SCOPE_WORKGROUP);
             };
-            const bool wr = blockIdx.x == gridDim.x - 1;  // writes inds / scores / records
+            const bool wr = blockIdx.x == gridDim.x - 1;  // writes inds / scores
 #pragma unroll
             for (int sr = 0; sr < RPW; ++sr) {
                 const int r = wv + WPB * sr;
@@ -437,19 +435,16 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
     char* wcode = wreg;
     uint16_t* wsc = (uint16_t*)(wreg + S::WCODE);          // [16][K/GS/KS] this K-slice
     uint16_t* wbi = (uint16_t*)(wreg + S::WCODE + S::WSB);
-    // staged rows: one set, two in persistent mode (set buf serves the current item)
-    // one row set; persistent mode keeps two pair lists (the next item's rows are staged once
+    // one set of staged rows; persistent mode keeps two pair lists (the next item's rows are staged once
     // every wave is done with the current ones, while the current epilogue still needs its pairs)
     constexpr int NBUF = PER ? 2 : 1;
-    uint16_t* const xs0 = (uint16_t*)(g5lds + (size_t)WPB * S::WAVE_BYTES);  // [RA][XS] qx rows
-    float2* const xsl0 = (float2*)(xs0 + RA * XS);  // [RA][SS] {sum x, sum base*x}
-    char* red = (char*)(xsl0 + RA * S::SS);  // [KS-1][TPB][64] f4
+    uint16_t* const xs = (uint16_t*)(g5lds + (size_t)WPB * S::WAVE_BYTES);  // [RA][XS] qx rows
+    float2* const xsl = (float2*)(xs + RA * XS);  // [RA][SS] {sum x, sum base*x}
+    char* red = (char*)(xsl + RA * S::SS);  // [KS-1][TPB][64] f4
     __shared__ int s_pair[NBUF][R];
     int buf = 0;
     // pair of row i of the pass from pb
     auto pair_of = [&](int pb, int i) { return PER ? s_pair[buf][i] : rbase + pb + i; };
-    auto xs_of = [&](int) { return xs0; };
-    auto xsl_of = [&](int) { return xsl0; };
 
     // ---- activation rows of a pass, straight into LDS: rows < npass only (the rest feed
     // MFMA output rows that are discarded).  Wave w stages rows w, w + WPB, ...
@@ -461,8 +456,6 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
     const bool res_pf = RES_PF && kh == 0;
     uint32_t resv[4] = {0u, 0u, 0u, 0u};
     auto stage_load = [&](int pb, int npass, int b, int lp, int npp, bool first = false) {
-        uint16_t* xs = xs_of(b);
-        float2* xsl = xsl_of(b);
         const int myr = min(pb + (lane < R ? lane : 0), npp - 1);
         const int prl = PER ? __shfl(lp, myr, MJ_WAVE) : rbase + myr;
         if constexpr (RES_PF) {
@@ -499,11 +492,9 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
     // down product of 17 rows over 256 experts took 16.4 us (14.3 so), the fused launch of 9 rows
     // 31.2 (30.4)
     auto own_block_sums = [&](int npass) {
-        const uint16_t* xs = xs_of(buf);
-        float2* xsl = xsl_of(buf);
         for (int idx = tid; idx < npass * KB * 8; idx += NT) {
             const int rb = idx >> 3, c = idx & 7, r = rb % npass, b = rb / npass;
-            const float2 sums = block_sum8(*(const u4v*)(xs + r * XS + 64 * b + 8 * c), c);
+            const float2 sums = block_sum8(*(const u4v*)(xs + r * XS + 64 * b + 8 * c));
             if (c == 0) lds_store_f2(xsl + r * S::SS + b, sums);
         }
     };
@@ -569,7 +560,6 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
     // bit 0: a half of the pass's staged rows still holds the marker; bit 1, where it is looked at:
     // the abort word is set (thread 0's reading).  The same answer in every thread
     auto rows_marked = [&](int npass, bool look) -> int {
-        const uint16_t* xs = xs_of(buf);
         bool bad = false;
         for (int idx = tid; idx < npass * (K / 8); idx += NT) {
             const int r = idx / (K / 8), c = idx - r * (K / 8);
@@ -675,7 +665,7 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
 #pragma unroll
         for (int c = 0; c < 4; ++c) corr[c] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
         const float* xcs =
-            (const float*)(xsl_of(buf) + xr * S::SS + kh * KBW + (q >> 1)) + (q & 1);
+            (const float*)(xsl + xr * S::SS + kh * KBW + (q >> 1)) + (q & 1);
         // this lane's B values: the biases (term 0) or the negated scales (term 1), taken from
         // the fp16 half of block 2i + q/2's group (the sign flipped in the fp16 bits)
         const uint32_t sgn = (q & 1) ? 0x8000u : 0u;
@@ -706,7 +696,7 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
         }
         __builtin_amdgcn_sched_barrier(0);
         // A: activation row xr, quarter q, of this K-slice
-        const uint16_t* xak = xs_of(buf) + xr * XS + 16 * q + 64 * kh * KBW;
+        const uint16_t* xak = xs + xr * XS + 16 * q + 64 * kh * KBW;
         // the correction chain's sum starts the accumulator (its four partial chains are
         // then free); outputs r >= NR stay unused
         float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -985,8 +975,7 @@ static int persistent_blocks() {
 }
 
 // staged rows per pass: for the persistent products as many as keep two blocks per CU, or one of
-// 16 waves (more
-// rows on one expert take extra passes, or slots); dense projections take up to 16
+// 16 waves (more rows on one expert take extra passes, or slots); dense projections take up to 16
 template <int KPL, int GS, int EPI, int WPB, int KS, int REC = REC_NONE, bool ROWA = false>
 static int g5_rows(int want) {
     using S = G5Shape<KPL, GS, EPI, WPB, KS, ROWA>;
@@ -1241,8 +1230,9 @@ hipError_t set_gather3_attributes() {
     MJ_A(2, EPI_STORE, 8, 1, 1, REC_NONE, false)
     MJ_A(4, EPI_STORE, 8, 1, 1, REC_NONE, false)
     MJ_A(8, EPI_STORE, 4, 4, 2, REC_NONE, false)
-    MJ_A(8, EPI_STORE, 8, 4, 2, REC_NONE, false)
-    MJ_A(8, EPI_ADD, 8, 4, 2, REC_NONE, false)
+    // (past 16 rows, group 128 alone)
+    if (e == hipSuccess) e = g5_attr<8, 128, EPI_STORE, 8, 2>();
+    if (e == hipSuccess) e = g5_attr<8, 128, EPI_ADD, 8, 2>();
     MJ_A(8, EPI_SWIGLU, 8, 2, 2, REC_RANK, false)
     MJ_A(8, EPI_SWIGLU, 8, 2, 2, REC_RANK, true)
     MJ_A(8, EPI_SWIGLU, 8, 2, 2, REC_IDS, false)

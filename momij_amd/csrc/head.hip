@@ -835,7 +835,7 @@ static hipError_t launch_head_final(const float* pval, const int* pidx, int nb, 
                        out_max ? out_max + m0 : nullptr, gl, abort);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !ga || m0 + mg < M) return e;
-    return launch_accept_greedy(ga->tokens, ga->parents, out_idx, M, ga->res, nullptr, abort, st);
+    return launch_accept_greedy(ga->tokens, ga->parents, out_idx, M, ga->res, abort, st);
 }
 
 // two 512-thread blocks per CU (the staged rows take at most 66 KB of LDS each)
@@ -925,21 +925,20 @@ hipError_t launch_lm_head(const uint16_t* x, const uint16_t* w, int M, int K, in
 __global__ __launch_bounds__(64) void k_accept_greedy(const int32_t* tokens,
                                                       const int32_t* parents,
                                                       const int32_t* argmax, int n,
-                                                      StepResult* res, int32_t* out_flat,
-                                                      const int* abort) {
+                                                      StepResult* res, const int* abort) {
     if (aborted(abort)) return;
     const int lane = threadIdx.x;
     const int tok = lane < n ? tokens[lane] : -1;
     const int par = lane < n ? parents[lane] : -2;
     const int am = lane < n ? argmax[lane] : -1;
-    accept_greedy_wave(tok, par, am, n, res, out_flat);
+    accept_greedy_wave(tok, par, am, n, res, nullptr);
 }
 
 hipError_t launch_accept_greedy(const int32_t* tokens, const int32_t* parents,
-                                const int32_t* argmax, int n, StepResult* res, int32_t* out_flat,
-                                const int* abort, hipStream_t st) {
+                                const int32_t* argmax, int n, StepResult* res, const int* abort,
+                                hipStream_t st) {
     hipLaunchKernelGGL(k_accept_greedy, dim3(1), dim3(64), 0, st, tokens, parents, argmax, n, res,
-                       out_flat, abort);
+                       abort);
     return hipGetLastError();
 }
 

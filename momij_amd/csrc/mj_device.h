@@ -94,10 +94,10 @@ __device__ __forceinline__ UnpackK unpack_consts() {
                    {opaque(0x5C005C00u), opaque(0x54005400u), opaque(0x4C004C00u), opaque(0x44004400u)}};
 }
 
-// {sum x, sum base*x} of one 64-block in qx order, over eight consecutive lanes: lane c (= its index
-// in the group) holds halves 8c .. 8c + 7, sums its pairs in turn, and the eight partial sums meet
+// {sum x, sum base*x} of one 64-block in qx order, over eight consecutive lanes: lane c of the group
+// holds halves 8c .. 8c + 7, sums its pairs in turn, and the eight partial sums meet
 // in lane moves.  Every lane of the group returns the sums.
-__device__ __forceinline__ float2 block_sum8(const u4v v, int c) {
+__device__ __forceinline__ float2 block_sum8(const u4v v) {
     float X = 0.0f, Bx = 0.0f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {

@@ -256,9 +256,9 @@ hipError_t launch_lm_head_q4(const uint16_t* x, const uint32_t* w, const uint16_
                              hipStream_t st, const GreedyAccept* ga = nullptr);
 int head_blocks();
 hipError_t launch_accept_greedy(const int32_t* tokens, const int32_t* parents,
-                                const int32_t* argmax, int n, StepResult* res, int32_t* out_flat,
-                                const int* abort, hipStream_t st);
-// the same with the tree by value (nothing to upload)
+                                const int32_t* argmax, int n, StepResult* res, const int* abort,
+                                hipStream_t st);
+// the same with the tree by value (nothing to upload), the result flat in the caller's array
 struct TreeParents {
     int32_t p[MJ_ROWS];
 };

@@ -73,7 +73,7 @@ __global__ __launch_bounds__(256) void k_qx_sums(const uint16_t* __restrict__ xp
     const int i = blockIdx.x * 256 + threadIdx.x, n = rows * (K / 8);
     const u4v v = *(const u4v*)(xperm + 8 * (size_t)min(i, n - 1));
     if (aborted(abort) || i >= n) return;  // (whole groups: n is a multiple of 8)
-    const float2 sums = block_sum8(v, i & 7);
+    const float2 sums = block_sum8(v);
     if ((i & 7) == 0) xsum[i >> 3] = sums;
 }
 
