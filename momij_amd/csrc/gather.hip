@@ -490,10 +490,12 @@ __device__ __forceinline__ void g5_body(GatherArgs a, int RA, int multi, FuseIO&
     // {sum x, sum base*x} of each (row, 64-block) from the staged rows: a block over eight lanes
     // (block_sum8).  With a block a lane, 64 elements in turn by one wave while the others waited, the
     // down product of 17 rows over 256 experts took 16.4 us (14.3 so), the fused launch of 9 rows
-    // 31.2 (30.4)
+    // 31.2 (30.4).  Row and block by constants: with a division by the pass's rows, blocks of 9 rows
+    // over 64 experts of 512 took 26.6 us (25.9 so; 25.5 before the slots came from ids), of 16 over 8
+    // of 1024 25.4 (25.1; 24.6)
     auto own_block_sums = [&](int npass) {
         for (int idx = tid; idx < npass * KB * 8; idx += NT) {
-            const int rb = idx >> 3, c = idx & 7, r = rb % npass, b = rb / npass;
+            const int rb = idx >> 3, c = idx & 7, r = rb / KB, b = rb % KB;
             const float2 sums = block_sum8(*(const u4v*)(xs + r * XS + 64 * b + 8 * c));
             if (c == 0) lds_store_f2(xsl + r * S::SS + b, sums);
         }
