@@ -73,7 +73,10 @@ mj_status mj_scratch_reserve(mj_ctx* ctx, size_t bytes) {
     const size_t want = bytes + (bytes >> 2) + 4096;
     s = mj_hip(ctx, hipMalloc(&ctx->scratch, want), "scratch alloc");
     if (s != MJ_OK) return s;
-    s = mj_hip(ctx, hipMemset(ctx->scratch, 0, want), "scratch clear");
+    // on the context's stream and waited for: hipMemset returns before it is done, and its stream (the
+    // default one) is ordered with none of ours, so it could clear what the call's kernels had written
+    s = mj_hip(ctx, hipMemsetAsync(ctx->scratch, 0, want, ctx->stream), "scratch clear");
+    if (s == MJ_OK) s = mj_hip(ctx, hipStreamSynchronize(ctx->stream), "scratch clear");
     if (s != MJ_OK) return s;
     ctx->scratch_bytes = want;
     return MJ_OK;
