@@ -13,6 +13,7 @@
 //                (SeedlessAttn.swift:219-270 rewinds the offset for append-only writes; a tree
 //                also needs the accepted path compacted into consecutive positions).
 #include <algorithm>
+#include <type_traits>
 
 #include "mj_device.h"
 #include "mj_internal.h"
@@ -76,6 +77,75 @@ __device__ __forceinline__ void stage_hidden(const uint16_t* x, int M, int K, in
                 }
         }
     }
+}
+
+// The same with every request counted: nothing is left out by a branch of a lane's or row's own (what
+// lies past a row's end goes into its padding, part K / 8; a row past M repeats the last and is stored
+// as zeros), so neither the rows' stores nor the compute behind them wait for the weight stream's
+// first two pieces, as they do where a branch makes the count unknown.  Heads of 1024 x 32000: 9 rows
+// 21.1 us, 19.3 so (20.1 with the rows ahead of any weight); of 256 x 8000: 17 rows 11.1, 10.6 (10.4).
+// The fp16 head's, unless two groups of rows go side by side (they fall out of step: 33 rows of 2048 x
+// 32000 46.5 -> 48.7); the 4-bit head's loop loses 1 to 2% by it.
+template <int ROWS, int WAVES, class Put, class Last>
+__device__ __forceinline__ void stage_counted(const uint16_t* x, int M, int K, int wave, int lane,
+                                              Put put, Last before_last) {
+    constexpr int RPW = ROWS / WAVES, RB = RPW < 2 ? RPW : 2;
+    static_assert(ROWS % WAVES == 0 && RPW % RB == 0, "rows spread evenly");
+    const int wv = __builtin_amdgcn_readfirstlane(wave), parts = K / 8;
+    const u4v zero = {0u, 0u, 0u, 0u};
+    auto batch = [&](int p0, int r0, auto ni, auto last) {
+        constexpr int NI = decltype(ni)::value;
+        if (wv + WAVES * r0 < M) {
+            u4v v[RB][NI];
+#pragma unroll
+            for (int r = 0; r < RB; ++r)
+#pragma unroll
+                for (int i = 0; i < NI; ++i) {
+                    const int m = min(wv + WAVES * (r0 + r), M - 1);
+                    v[r][i] = *(const u4v*)(x + (size_t)m * K + 8 * min(p0 + 64 * i + lane, parts - 1));
+                }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (decltype(last)::value) before_last();
+#pragma unroll
+            for (int r = 0; r < RB; ++r)
+#pragma unroll
+                for (int i = 0; i < NI; ++i) {
+                    const int m = wv + WAVES * (r0 + r);
+                    put(m, min(p0 + 64 * i + lane, parts), m < M ? v[r][i] : zero);
+                }
+        } else {
+            if constexpr (decltype(last)::value) before_last();
+#pragma unroll
+            for (int r = 0; r < RB; ++r)
+#pragma unroll
+                for (int i = 0; i < NI; ++i)
+                    put(wv + WAVES * (r0 + r), min(p0 + 64 * i + lane, parts), zero);
+        }
+    };
+    int p0 = 0;
+    for (; p0 + 256 < parts; p0 += 256)
+#pragma unroll
+        for (int r0 = 0; r0 < RPW; r0 += RB)
+            batch(p0, r0, std::integral_constant<int, 4>{}, std::false_type{});
+    auto end = [&](auto ni) {
+#pragma unroll
+        for (int r0 = 0; r0 + RB < RPW; r0 += RB) batch(p0, r0, ni, std::false_type{});
+        batch(p0, RPW - RB, ni, std::true_type{});
+    };
+    if (parts - p0 > 128)
+        end(std::integral_constant<int, 4>{});
+    else if (parts - p0 > 64)
+        end(std::integral_constant<int, 2>{});
+    else
+        end(std::integral_constant<int, 1>{});
+}
+
+// Thread t's banned id (of no use past n), requested ahead of the hidden rows and put into LDS behind
+// them (a load into LDS before them is a memory round trip more).  Always a load, so that no wait
+// falls where paths meet; x stands in for no ids.
+__device__ __forceinline__ int banned_id(const int32_t* banned, int n, const uint16_t* x, int t) {
+    const int32_t* p = n > 0 ? banned : (const int32_t*)x;
+    return p[min(t, max(n - 1, 0))];
 }
 
 template <int NT, int PL>
@@ -237,15 +307,19 @@ __global__ __launch_bounds__(512) void k_lm_head(HeadArgs a) {
         for (int tl = 0; tl < NT; ++tl) acc[tl] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
     };
     Piece pa, pb;
-    for (int idx = t; idx < a.n_banned; idx += 512) s_ban[idx] = a.banned[idx];
-    stage_hidden<NT * 16, 8>(
-        a.x, a.M, K, wv, lane, [&](int m, int part, u4v v) { *(u4v*)(xs + m * XS + 8 * part) = v; },
-        [&]() {
-            issue(pa);
-            __builtin_amdgcn_sched_barrier(0);  // all of pa's requests before pb's
-            issue(pb);
-            __builtin_amdgcn_sched_barrier(0);
-        });
+    const int ban = banned_id(a.banned, a.n_banned, a.x, t);
+    const auto put = [&](int m, int part, u4v v) { *(u4v*)(xs + m * XS + 8 * part) = v; };
+    const auto stream = [&]() {
+        issue(pa);
+        __builtin_amdgcn_sched_barrier(0);  // all of pa's requests before pb's
+        issue(pb);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (NT == 2 && a.pair)
+        stage_hidden<NT * 16, 8>(a.x, a.M, K, wv, lane, put, stream);
+    else
+        stage_counted<NT * 16, 8>(a.x, a.M, K, wv, lane, put, stream);
+    if (t < MJ_HEAD_MAX_BANNED) s_ban[t] = ban;
     lds_only_sync();
     for (int i = 0; i < TP; i += 2) {
         step(pa, i);
@@ -536,7 +610,7 @@ __global__ __launch_bounds__(512) void k_lm_head_q4(HeadQ4Args a) {
         for (int tl = 0; tl < NT; ++tl) acc[tl] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
     };
     Q4Piece<PL> pa, pb;
-    for (int idx = t; idx < a.n_banned; idx += 512) s_ban[idx] = a.banned[idx];
+    const int ban = banned_id(a.banned, a.n_banned, a.x, t);
     // group sums: a row's 64-groups over the threads, each read whole before it is summed in order
     for (int idx = t; idx < NT * 16 * G; idx += 512) {
         const int m = idx / G, g = idx - m * G;
@@ -572,6 +646,7 @@ __global__ __launch_bounds__(512) void k_lm_head_q4(HeadQ4Args a) {
             issue(pb);
             __builtin_amdgcn_sched_barrier(0);
         });
+    if (t < MJ_HEAD_MAX_BANNED) s_ban[t] = ban;
     lds_only_sync();
     for (int i = 0; i < TP; i += 2) {
         step(pa, i);
