@@ -5,6 +5,9 @@
  * cross this boundary.  Every call is asynchronous on the context's stream unless it says it
  * synchronises; a context is not re-entrant (the reference engine is single-request too,
  * README.md:32, Server.swift:677-700); distinct contexts may be driven from distinct threads.
+ * Calls that take host arrays (an attention block, greedy acceptance, a penalty history) are refused
+ * with MJ_HIP_ERROR while their stream is being captured into a graph: a replay would run on the
+ * captured call's.
  * The caller owns every tensor it allocates (weights, activations, outputs); the library owns
  * only its scratch and, for a model, the KV cache.
  *

@@ -931,6 +931,17 @@ mj_status mj_verify_sampled(mj_model* m, int32_t y, const int32_t* draft, int n_
 }
 
 // ------------------------------------------------------------------ op-level entries
+// Calls whose host arrays go with the launch are refused while their stream is captured, as when they
+// were uploaded and waited for: a replay would run on those of the captured call (and an attention
+// block's on scratch that a larger call may have replaced).
+static mj_status mj_refuse_capture(mj_ctx* ctx, const char* what) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    mj_status s = mj_hip(ctx, hipStreamIsCapturing(ctx->stream, &cs), what);
+    if (s == MJ_OK && cs != hipStreamCaptureStatusNone)
+        s = mj_fail(ctx, MJ_HIP_ERROR, "%s cannot be captured", what);
+    return s;
+}
+
 mj_status mj_attn_block(mj_ctx* ctx, const mj_attn_config* cfg, const mj_attn_weights* w,
                         void* h, void* kcache, void* vcache, int64_t L,
                         const int32_t* parents_host, int M) {
@@ -947,6 +958,8 @@ mj_status mj_attn_block(mj_ctx* ctx, const mj_attn_config* cfg, const mj_attn_we
                        (long long)c.kv_capacity);
     hipSetDevice(ctx->device);
     mj_status s = mj_hip(ctx, set_kernel_attributes(), "kernel attributes");
+    if (s != MJ_OK) return s;
+    s = mj_refuse_capture(ctx, "attn_block");
     if (s != MJ_OK) return s;
     AttnFront front{};
     front.sd.L = L;
@@ -1141,6 +1154,8 @@ mj_status mj_accept_greedy(mj_ctx* ctx, const int32_t* tokens, const int32_t* pa
     mj_status s = fill_tree(ctx, &sd, parents_host, n_rows);
     if (s != MJ_OK) return s;
     hipSetDevice(ctx->device);
+    s = mj_refuse_capture(ctx, "accept_greedy");
+    if (s != MJ_OK) return s;
     TreeParents tp;
     std::memcpy(tp.p, sd.parents, sizeof tp.p);
     return mj_hip(ctx, launch_accept_greedy_tree(tokens, tp, argmax, n_rows, out, ctx->abort_dev,
@@ -1151,11 +1166,8 @@ mj_status mj_accept_greedy(mj_ctx* ctx, const int32_t* tokens, const int32_t* pa
 // behind the event of its last copy, so a call does not wait for its own upload (the copy, its wait
 // and the gap it left took 12 us of a 9-row acceptance).
 static mj_status mj_hist_stage(mj_ctx* ctx, size_t n, int32_t** out) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    mj_status s = mj_hip(ctx, hipStreamIsCapturing(ctx->stream, &cs), "history");
+    mj_status s = mj_refuse_capture(ctx, "accept_sampled: a penalty history");
     if (s != MJ_OK) return s;
-    if (cs != hipStreamCaptureStatusNone)  // a replay would upload whatever the buffer holds then
-        return mj_fail(ctx, MJ_HIP_ERROR, "accept_sampled: a penalty history cannot be captured");
     const int k = ctx->hist_at = 1 - ctx->hist_at;
     if (!ctx->hist_ev[k]) {
         s = mj_hip(ctx, hipEventCreateWithFlags(&ctx->hist_ev[k], hipEventDisableTiming), "history");

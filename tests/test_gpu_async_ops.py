@@ -128,3 +128,44 @@ def test_history_under_capture_is_refused(ctx):
     torch.cuda.synchronize()
     ctx.accept_sampled_ex(lg, 1, 64, d, 0, 1, 2, out, 1.0, **call)
     ctx.sync()
+
+
+@pytest.mark.parametrize("op", ["attn_block", "accept_greedy"])
+def test_host_trees_under_capture_are_refused(ctx, op):
+    """The draft tree (and an attention block's position) is host data of the call too."""
+    import torch
+
+    from momij_amd._lib import MomijError
+
+    rng = np.random.default_rng(4)
+    H, nQ, nKV, D = 2048, 16, 4, 128
+    cfg = dict(H=H, nQ=nQ, nKV=nKV, D=D, rope_dim=64, rope_base=1e6, eps=1e-6, window=96, C=160,
+               gs=64)
+    aw = {k: dev(v) for k, v in synth.attn_weights(rng, H, nQ, nKV, D, 64).items()}
+    h, kc, vc = (dev(synth.normal_f16(rng, s)) for s in ((3, H), (nKV, 160, D), (nKV, 160, D)))
+    tok, am = dev(np.array([1, 2, 3], np.int32)), dev(np.array([2, 3, 9], np.int32))
+    out = torch.zeros(8, dtype=torch.int32, device="cuda")
+
+    def call():
+        if op == "attn_block":
+            ctx.attn_block(cfg, aw, h, kc, vc, 10, [-1, 0, 0], 3)
+        else:
+            ctx.accept_greedy(tok, [-1, 0, 1], am, 3, out)
+
+    torch.cuda.synchronize()
+    call()
+    ctx.sync()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(ctx.stream):
+        g.capture_begin(capture_error_mode="thread_local")
+        try:
+            with pytest.raises(MomijError):
+                call()
+        finally:
+            out.zero_()  # a captured graph of this alone
+            g.capture_end()
+    torch.cuda.synchronize()
+    call()
+    ctx.sync()
+    if op == "accept_greedy":
+        assert host(out).tolist() == [2, 9, 0, 1, 2, 2, 3, 9]
