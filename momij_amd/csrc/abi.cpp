@@ -102,10 +102,12 @@ mj_status mj_abort_end(mj_ctx* ctx, unsigned gen) {
     const unsigned now = ctx->abort_gen.load();
     const bool ab = ctx->abort_host.load() || now != gen;
     ctx->synced_gen = now;
+    // the kernels that set the fault word have completed: the caller has synchronised.  Either report
+    // voids the results since the previous one, so an aborted call leaves no fault to the next
+    const bool fault = ctx->fault && __atomic_load_n(ctx->fault, __ATOMIC_ACQUIRE) != 0;
+    if (fault) __atomic_store_n(ctx->fault, 0, __ATOMIC_RELEASE);
     if (ab) return mj_fail(ctx, MJ_ABORTED, "aborted by the abort word");
-    // the kernels that set the fault word have completed: the caller has synchronised
-    if (ctx->fault && __atomic_load_n(ctx->fault, __ATOMIC_ACQUIRE) != 0) {
-        __atomic_store_n(ctx->fault, 0, __ATOMIC_RELEASE);
+    if (fault) {
         return mj_fail(ctx, MJ_HIP_ERROR,
                        "fused MoE launch: a block's wait for the up product ran out its bound "
                        "(blocks not co-resident: another stream's kernels on the device?); the "

@@ -169,3 +169,39 @@ def test_host_trees_under_capture_are_refused(ctx, op):
     ctx.sync()
     if op == "accept_greedy":
         assert host(out).tolist() == [2, 9, 0, 1, 2, 2, 3, 9]
+
+
+def test_an_aborted_call_leaves_no_fault(ctx):
+    """A wait that ran out its bound (forced by a bound of 0) before a call that reports an abort:
+    the call after it reports neither."""
+    import torch
+
+    from momij_amd._lib import MomijError
+
+    rng = np.random.default_rng(6)
+    mw = {k: (dev(v) if isinstance(v, np.ndarray) else v)
+          for k, v in synth.moe_weights(rng, 64, 2048, 1024, 64).items()}
+    x = dev(synth.normal_f16(rng, (1, 2048)))
+    y = torch.empty_like(x)
+    torch.cuda.synchronize()
+    faults = 0
+    for abort in (False, True, False, True):
+        ctx.set_wait_limit(0)
+        try:
+            # one row: half of the blocks have no up item and check down items' rows at once
+            ctx.moe_block(mw, x, y, 1, 3)
+        finally:
+            ctx.set_wait_limit(1 << 17)
+        torch.cuda.synchronize()
+        if abort:
+            ctx.set_abort(True)
+            ctx.set_abort(False)
+        try:
+            ctx.sync()
+        except MomijError as e:
+            assert e.status == (5 if abort else 6), e
+            faults += not abort
+        else:
+            assert not abort
+        ctx.sync()
+    assert faults > 0  # the bound does report
